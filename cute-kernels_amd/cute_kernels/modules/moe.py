@@ -12,6 +12,7 @@ import torch.nn as nn
 from .. import _C
 from ..scattermoe import (
     _bias_in_epilogue,
+    choose_align,
     experts_down,
     experts_up,
     route_topk_softmax,
@@ -22,6 +23,7 @@ from ..scattermoe import (
 )
 from ..rmsnorm_route import rmsnorm_route_cute
 from ..swiglu import swiglu_packed_cute
+from ..utils import is_tracing
 
 
 class Experts(nn.Module):
@@ -195,7 +197,9 @@ class MoE(nn.Module):
     ) -> torch.Tensor:
         if hidden_states.size(0) == 0:  # no tokens: nothing to sort or multiply; the result stays in the autograd graph
             return hidden_states * 0
-        seg = sort_by_expert(selected_experts, self.num_experts)
+        inference = not torch.is_grad_enabled() and not is_tracing()
+        align = choose_align(selected_experts.numel(), self.num_experts, hidden_states.dtype, inference)
+        seg = sort_by_expert(selected_experts, self.num_experts, align)
         has_bias = self.c_fc.bias is not None or self.c_proj.bias is not None
 
         sixteen_bit = hidden_states.dtype != torch.float32  # fp32 layers take the unfused route on the fp32 GEMMs
