@@ -66,6 +66,11 @@ constexpr int kLineBM = 256, kLineK = 64;
 int launch_line(const GemmParams& prm, int mode, int bn, bool bt, int dtype, unsigned blocks, hipStream_t stream,
                 const char* name);
 
+// Tiles of 16, 32 or 64 rows (grouped_gemm_skinny.hip): forward GEMMs of inference batches with few rows per expert, modes
+// kGrouped, kScatter, kSwiglu, 16-bit or e4m3 operands; prm.align is the tile height.
+inline bool skinny_align(int align) { return align == 16 || align == 32 || align == 64; }
+int launch_skinny(const GemmParams& prm, int mode, int64_t max_rows, bool fp8, int dtype, hipStream_t stream, const char* name);
+
 namespace {
 
 // The dynamic-LDS limit of a kernel is a per-device attribute: set it once per (instantiation, device). `done` is the
@@ -223,10 +228,11 @@ __device__ inline void grouped_order(int r, int a_count, int b_count, int& a, in
 // conflicts both for 8 lanes over 32 banks and for 16 lanes over 64 banks.
 __device__ inline int lds_swizzle(int row) { return ((row >> 2) & 1) | ((((row >> 1) ^ (row >> 3)) & 1) << 1); }
 
-inline int check_segments(const ck_segments* seg, const char* name) {
+inline int check_segments(const ck_segments* seg, const char* name, bool small_tiles = false) {
   CK_REQUIRE(seg != nullptr, "%s: seg is NULL", name);
   CK_REQUIRE(seg->seg_starts && seg->counts && seg->tile_expert && seg->row_slot, "%s: NULL table in seg", name);
-  CK_REQUIRE(seg->align == 128 || seg->align == 256, "%s: align=%d must be 128 or 256", name, seg->align);
+  CK_REQUIRE(seg->align == 128 || seg->align == 256 || (small_tiles && skinny_align(seg->align)), "%s: align=%d must be %s128 or 256",
+             name, seg->align, small_tiles ? "16, 32, 64, " : "");
   CK_REQUIRE(seg->num_experts >= 1, "%s: num_experts=%d", name, seg->num_experts);
   CK_REQUIRE(seg->max_rows >= 0 && seg->max_rows % seg->align == 0, "%s: max_rows=%lld is not a multiple of align", name,
              (long long)seg->max_rows);

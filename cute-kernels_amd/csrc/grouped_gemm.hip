@@ -557,7 +557,7 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
         sync_slab();
         drain_rows([&](int r, int sc) -> T* {
           const int64_t p = m0 + r, n = (int64_t)nt * BN + tile_col(sc, pass);
-          if (p >= valid_end || n >= prm.N) return nullptr;
+          if (p >= valid_end || n >= prm.N || y == nullptr) return nullptr;
           const int64_t row = (MODE == kScatter) ? (int64_t)scatter_rows[r] : p;
           return y + row * prm.N + n;
         });
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
         sync_slab();
         drain_rows([&](int r, int sc) -> T* {
           const int64_t p = m0 + r, col = act_col(sc);
-          if (p >= valid_end || col >= prm.I) return nullptr;
+          if (p >= valid_end || col >= prm.I || (pass < 2 && pre == nullptr)) return nullptr;
           if (pass == 0) return pre + p * two_i + col;
           if (pass == 1) return pre + p * two_i + prm.I + col;
           return act + p * prm.I + col;
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
             static_for<4>([&](auto s) {
               v[s] = Elem<T>::down(acc[i][j][4 * q + s]);
               if (out_row[s] >= 0) {
-                y[out_row[s] * prm.N + n] = v[s];
+                if (y != nullptr) y[out_row[s] * prm.N + n] = v[s];
                 if (act != nullptr) act[out_row[s] * prm.N + n] = Elem<T>::down(gelu_tanh_fast(Elem<T>::up(v[s])));
               } else {
                 v[s] = Elem<T>::down(0.f);
@@ -689,8 +689,10 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
               const float sg = sigmoid_fast(gf);
               v[s] = Elem<T>::down(prm.act_kind == CK_ACT_GLU ? Elem<T>::up(up) * sg : Elem<T>::up(up) * gf * sg);  // same association as swiglu_fwd_kernel
               if (p < valid_end) {
-                pre[p * two_i + col] = up;
-                pre[p * two_i + prm.I + col] = gate;
+                if (pre != nullptr) {
+                  pre[p * two_i + col] = up;
+                  pre[p * two_i + prm.I + col] = gate;
+                }
                 act[p * prm.I + col] = v[s];
               } else {
                 v[s] = Elem<T>::down(0.f);
@@ -805,7 +807,7 @@ static int grouped_gemm_impl(const void* a, int32_t a_gather_div, const void* w,
                              const ck_segments* seg, int32_t epilogue, void* y, void* y_t, int64_t ld_t, void* aux,
                              const void* aux_in, int32_t dtype, void* stream, void* workspace, int64_t workspace_bytes) {
   const char* name = "ck_grouped_gemm";
-  if (int rc = check_segments(seg, name)) return rc;
+  if (int rc = check_segments(seg, name, true)) return rc;
   CK_REQUIRE(N >= 8 && K >= 8 && N % 8 == 0 && K % 8 == 0, "%s: N=%d and K=%d must be positive multiples of 8", name, N, K);
   CK_REQUIRE(a_gather_div >= 0, "%s: a_gather_div=%d is negative", name, a_gather_div);
   int act_kind = CK_ACT_SWIGLU;
@@ -822,7 +824,13 @@ static int grouped_gemm_impl(const void* a, int32_t a_gather_div, const void* w,
   }
   CK_REQUIRE(epilogue >= CK_EPI_GROUPED && epilogue <= CK_EPI_SWIGLU_BWD, "%s: unknown epilogue %d", name, epilogue);
   if (seg->max_rows == 0) return CK_OK;
-  CK_REQUIRE(a && w && y, "%s: a, w and y are required", name);
+  const bool skinny = skinny_align(seg->align);
+  const bool line_kernel = seg->align == kLineBM && K % kLineK == 0 && epilogue != CK_EPI_SWIGLU_BWD &&
+                           !force_register_pipeline() && line_kernel_enabled();
+  // y may be NULL where an activation epilogue's second output is all that is wanted (inference)
+  CK_REQUIRE(a && w && (y || (aux && epilogue != CK_EPI_SWIGLU_BWD)), "%s: a, w and y are required", name);
+  CK_REQUIRE(!skinny || (epilogue != CK_EPI_SWIGLU_BWD && y_t == nullptr),
+             "%s: tiles of fewer than 128 rows have no SwiGLU-backward epilogue and no transposed output", name);
   CK_REQUIRE(aligned16(a) && aligned16(w), "%s: a and w must be 16-byte aligned", name);
   CK_REQUIRE(y_t == nullptr || (ld_t >= seg->max_rows && ld_t % 8 == 0 && (reinterpret_cast<uintptr_t>(y_t) & 7) == 0),
              "%s: y_t needs ld_t >= max_rows, ld_t %% 8 == 0 and 8-byte alignment", name);
@@ -830,10 +838,8 @@ static int grouped_gemm_impl(const void* a, int32_t a_gather_div, const void* w,
 
   // rows are addressed with 32-bit byte offsets: from the operand base for a, from the expert's slice for w
   CK_REQUIRE((int64_t)N * K * 2 < ((int64_t)1 << 32), "%s: one expert's weight matrix must stay below 4 GiB", name);
-  const bool line_kernel = seg->align == kLineBM && K % kLineK == 0 && epilogue != CK_EPI_SWIGLU_BWD &&
-                           !force_register_pipeline() && line_kernel_enabled();
-  // the 128-byte-row kernel addresses a grouped input from each tile's first row; the general kernel from the operand base
-  CK_REQUIRE(a_gather_div > 0 || line_kernel || seg->max_rows * (int64_t)K * 2 < ((int64_t)1 << 32),
+  // the 128-byte-row and small-row kernels address a grouped input from each tile's first row; the general kernel from the operand base
+  CK_REQUIRE(a_gather_div > 0 || line_kernel || skinny || seg->max_rows * (int64_t)K * 2 < ((int64_t)1 << 32),
              "%s: the grouped input must stay below 4 GiB", name);
   GemmParams prm = {};
   prm.a = a;
@@ -867,6 +873,7 @@ static int grouped_gemm_impl(const void* a, int32_t a_gather_div, const void* w,
   auto n_tiles_for = [&](int bn) { return (int)ceil_div(out_cols, epilogue == CK_EPI_SWIGLU ? bn / 2 : bn); };
   CK_REQUIRE(aux_in == nullptr || epilogue != CK_EPI_SWIGLU,
              "%s: the bias operand (aux_in) goes with the grouped / scatter epilogues", name);
+  if (skinny) return launch_skinny(prm, epilogue, seg->max_rows, false, dtype, s, name);
   if (line_kernel) {
     const bool swiglu = epilogue == CK_EPI_SWIGLU;
     const int bn = 256;

@@ -520,8 +520,9 @@ extern "C" int ck_grouped_gemm_fp8(const void* a8, const float* a_scale, int32_t
                                    const float* w_scale, int32_t N, int32_t K, const ck_segments* seg, int32_t epilogue,
                                    void* y, void* aux, int32_t out_dtype, void* stream) {
   const char* name = "ck_grouped_gemm_fp8";
-  if (int rc = check_segments(seg, name)) return rc;
-  CK_REQUIRE(seg->align == 256, "%s: fp8 tiles are 256 rows high; sort with align = 256", name);
+  if (int rc = check_segments(seg, name, true)) return rc;
+  const bool skinny = skinny_align(seg->align);
+  CK_REQUIRE(skinny || seg->align == 256, "%s: fp8 tiles are 16, 32, 64 or 256 rows high; sort with such an align", name);
   CK_REQUIRE(N >= 8 && N % 8 == 0, "%s: N=%d must be a positive multiple of 8", name, N);
   CK_REQUIRE((reinterpret_cast<uintptr_t>(w_scale) & 15) == 0, "%s: w_scale must be 16-byte aligned", name);
   CK_REQUIRE(K >= 128 && K % 128 == 0, "%s: K=%d must be a positive multiple of 128", name, K);
@@ -531,7 +532,7 @@ extern "C" int ck_grouped_gemm_fp8(const void* a8, const float* a_scale, int32_t
   if (seg->max_rows == 0) return CK_OK;
   CK_REQUIRE(a8 && a_scale && w8 && w_scale, "%s: operands and scales are required", name);
   CK_REQUIRE(aligned16(a8) && aligned16(w8), "%s: a8 and w8 must be 16-byte aligned", name);
-  CK_REQUIRE((int64_t)N * K < ((int64_t)1 << 32) && (a_gather_div > 0 || seg->max_rows * (int64_t)K < ((int64_t)1 << 32)),
+  CK_REQUIRE((int64_t)N * K < ((int64_t)1 << 32) && (a_gather_div > 0 || skinny || seg->max_rows * (int64_t)K < ((int64_t)1 << 32)),
              "%s: operands are addressed with 32-bit byte offsets (4 GiB per expert matrix / grouped input)", name);
   GemmParams prm = {};
   prm.a = a8;
@@ -565,6 +566,7 @@ extern "C" int ck_grouped_gemm_fp8(const void* a8, const float* a_scale, int32_t
   const int64_t blocks = (seg->max_rows / seg->align) * prm.n_tiles;
   CK_REQUIRE(blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (skinny) return launch_skinny(prm, epilogue, seg->max_rows, true, out_dtype, s, name);
   CK_DISPATCH_HALF(out_dtype, name, {
     switch (epilogue) {
       case CK_EPI_GROUPED: return launch_fp8<scalar_t, kGrouped>(prm, (unsigned)blocks, s, name);

@@ -778,7 +778,7 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
           store_lines(v1, v2, 4 * jq, [&](int) { return row_a; }, [&](int r) { return i * 16 + r < rows_left; },
                       [&](int c) { return c < cols_left; });
         } else {
-          store_lines_at(v1, v2, 4 * jq, base, row_off, inside, i * 16 + lrow < rows_left, cols_left);
+          if (!EXTRA || y != nullptr) store_lines_at(v1, v2, 4 * jq, base, row_off, inside, i * 16 + lrow < rows_left, cols_left);
           if constexpr (EXTRA && !BT) if (act_base != nullptr) {  // CK_ACT_GELU_TANH: the activation of the rounded output
             store_lines_at(gelu8(v1), gelu8(v2), 4 * jq, act_base, row_off, inside, i * 16 + lrow < rows_left, cols_left);
           }
@@ -797,6 +797,7 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
     const int rows_left = (int)min((int64_t)WM, valid_end - tile_row0);
     constexpr int NH = NI / 2;  // column blocks per half
     static_assert(NH % 2 == 0, "whole block pairs in each half");
+    const bool keep_pre = pre != nullptr;  // NULL: inference, nothing reads the pre-activation again (two thirds of the stores)
     char* pre_base = uniform_out(reinterpret_cast<char*>(pre + tile_row0 * two_i + col0));
     char* act_base = uniform_out(reinterpret_cast<char*>(act + tile_row0 * prm.I + col0));
     const uint32_t pre_pitch = (uint32_t)two_i * 2u, act_pitch = (uint32_t)prm.I * 2u, gate_off = (uint32_t)prm.I * 2u;
@@ -838,8 +839,10 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
         vg_[jp] = vg;
         va_[jp] = va;
       });
-      store_lines_at(vu_[0], vu_[1], 0, pre_base, pre_off, inside, valid, cols_left);
-      store_lines_at(vg_[0], vg_[1], 0, pre_base, pre_off + gate_off, inside, valid, cols_left);
+      if (keep_pre) {
+        store_lines_at(vu_[0], vu_[1], 0, pre_base, pre_off, inside, valid, cols_left);
+        store_lines_at(vg_[0], vg_[1], 0, pre_base, pre_off + gate_off, inside, valid, cols_left);
+      }
       store_lines_at(va_[0], va_[1], 0, act_base, act_off, inside, valid, cols_left);
       pre_off += 16u * pre_pitch;
       act_off += 16u * act_pitch;

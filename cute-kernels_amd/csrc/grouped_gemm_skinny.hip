@@ -1,0 +1,307 @@
+// Grouped GEMM for few rows per expert (inference with small batches): 16-, 32- or 64-row tiles, bf16 / f16 or fp8 e4m3
+// operands, fp32 accumulation.
+//
+// What bounds it: the stream of expert weights out of HBM. A decoding step reads nearly every expert's matrices for a
+// handful of rows each, 2 to 64 multiply-adds per weight, far below what the matrix cores need to matter. So the kernel is
+// built around the weight stream and nothing else:
+//  * weights go straight from memory into MFMA operand registers: no LDS stage and no barrier in the main loop. A lane's
+//    16 bytes are 8 (fp8: 16) contraction values of one output column, which is the operand layout of
+//    v_mfma_f32_16x16x32 (v_mfma_f32_16x16x128_f8f6f4: two such pieces, the same two for both operands);
+//  * the four waves of a workgroup share the output tile and split the contraction, a quarter of every row each, in steps
+//    of one 128-byte line per row; no weight is read twice. The four partial tiles meet once, in LDS, in front of the
+//    epilogue (a fixed order of additions). Waves that take every fourth line instead, and lanes that take 16-byte pieces q
+//    and q + 4 of a line instead of 2 q and 2 q + 1, measured equal in bf16 and 2 to 8 % slower in fp8;
+//  * a wave keeps the next step's loads in flight under the current step's MFMAs (two register sets); with 2 to 4
+//    workgroups per CU that is 64 to 128 KiB of weights in flight per CU (eight waves per workgroup: 0 to 10 % slower,
+//    128-column tiles: equal, non-temporal weight loads: 5 to 20 % slower);
+//  * the activations, a few hundred KiB for the whole launch, are re-read by every column tile from L2.
+// An expert with more rows than a tile has several tiles; they are neighbours in launch order on one XCD, so that the
+// second reads the weights from that XCD's L2.
+// Measured, launch included: 8 experts of 28,672 x 4,096 with 2 rows each 317 us = 5.9 TB/s of weights, 8 x 4,096 x 14,336
+// 163 us = 5.8 TB/s, 64 x 2,816 x 2,048 with 8 rows 136 us = 5.4 TB/s (128-row tiles of the general kernel: 179 us), e4m3
+// 128 x 3,072 x 4,096 with 8 rows 288 us = 5.6 TB/s and 128 x 4,096 x 1,536 156 us = 5.2 TB/s (256-row tiles: 348, 205 us).
+#include "gemm_common.h"
+
+namespace ck {
+namespace {
+
+constexpr int kNT = 256, kWaves = kNT / kWave;
+constexpr int kStepBytes = 128;  // one cache line of every operand row per wave and step
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+
+struct fp8_t {};  // e4m3 operand bytes
+
+template <typename TI>
+struct Operand {
+  static constexpr int kBytes = 2;
+};
+template <>
+struct Operand<fp8_t> {
+  static constexpr int kBytes = 1;
+};
+
+// one step: 64 contraction values of 16 columns x 16 rows as two 16-bit MFMAs, or 128 values as one fp8 MFMA; the two
+// pieces are the lane's quarter of the row's line, 32 bytes; which contraction values those are does not matter as long as
+// both operands hold the same
+template <typename TI>
+__device__ inline void multiply(const vec16 (&w)[2], const vec16 (&a)[2], f32x4& c) {
+  if constexpr (std::is_same_v<TI, fp8_t>) {
+    union {
+      vec16 v[2];
+      i32x8_t f;
+    } uw, ua;
+    uw.v[0] = w[0];
+    uw.v[1] = w[1];
+    ua.v[0] = a[0];
+    ua.v[1] = a[1];
+    // both operands e4m3 (cbsz = blgp = 0), block scales 2^0 (127)
+    c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(uw.f, ua.f, c, 0, 0, 0, 127, 0, 127);
+  } else {
+    union {
+      vec16 v;
+      typename Mfma16<TI>::frag f;
+    } uw, ua;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uw.v = w[h];
+      ua.v = a[h];
+      c = Mfma16<TI>::run(uw.f, ua.f, c);
+    }
+  }
+}
+
+// TI: operand type, TO: output type; MB: row blocks of 16 per tile, NB: column blocks of 16 per tile. kSwiglu: half of the
+// column blocks are up columns, the other half the gate columns of the same outputs.
+template <typename TI, typename TO, int MODE, int MB, int NB>
+__global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
+  constexpr int BM = 16 * MB, kEl = Operand<TI>::kBytes;
+  constexpr int NH = MODE == kSwiglu ? NB / 2 : NB;  // column blocks of outputs per tile
+  static_assert(MODE != kSwiglu || NB % 2 == 0, "whole up / gate block pairs");
+  __shared__ f32x4 red[kWaves][MB * NB][kWave];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lrow = lane & 15, lq = lane >> 4;
+
+  // ---- which tile: every XCD owns a contiguous run of column tiles, all row tiles of one column tile in a row
+  const int live_m = prm.seg_starts[prm.num_experts] / BM;
+  const int total = live_m * prm.n_tiles;
+  int pid = blockIdx.x;
+  if (pid >= total) return;
+  const int per_xcd = total / kXcds;
+  if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;
+  const int nt = pid / live_m, mt = pid - nt * live_m;
+  const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[mt]);
+  const int m0 = mt * BM;
+  const int valid_end = prm.seg_starts[expert] + (int)prm.counts[expert];
+
+  // ---- operand rows of this lane, as 32-bit byte offsets from a uniform base (the host checks that they fit)
+  const char* w_base = static_cast<const char*>(prm.w) + (int64_t)expert * prm.w_expert_stride * kEl;
+  const char* a_base = static_cast<const char*>(prm.a);
+  if (prm.a_gather_div <= 0) a_base += (int64_t)m0 * prm.lda * kEl;
+  uint32_t w_off[NB], a_off[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int p = min(m0 + i * 16 + lrow, valid_end - 1);  // pad rows re-read a valid row; their results are never stored
+    const int row = prm.a_gather_div > 0 ? prm.row_slot[p] / prm.a_gather_div : p - m0;
+    a_off[i] = (uint32_t)row * (uint32_t)(prm.lda * kEl) + lq * 32;
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    int n;
+    if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(nt * (NH * 16) + (j % NH) * 16 + lrow, prm.I - 1);
+    else n = min(nt * (NB * 16) + j * 16 + lrow, prm.N - 1);
+    w_off[j] = (uint32_t)n * (uint32_t)(prm.ldw * kEl) + lq * 32;
+  }
+
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  struct Set {
+    vec16 w[NB][2], a[MB][2];
+  };
+  auto fetch = [&](Set& s, int step) __attribute__((always_inline)) {
+    const char* wp = w_base + (int64_t)step * kStepBytes;
+    const char* ap = a_base + (int64_t)step * kStepBytes;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) s.w[j][h] = load16(wp + w_off[j] + h * 16);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) s.a[i][h] = load16(ap + a_off[i] + h * 16);
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay in front of the products they overlap with
+  };
+  auto step_products = [&](const Set& s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) multiply<TI>(s.w[j], s.a[i], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  const int row_bytes = prm.K * kEl;
+  const int full = row_bytes / kStepBytes;  // whole steps; the rest of a row, if any, is one partial step
+  const int mine = __builtin_amdgcn_readfirstlane(full * (wave + 1) / kWaves - full * wave / kWaves);  // steps of this wave
+  const int first = __builtin_amdgcn_readfirstlane(full * wave / kWaves);
+  Set s0, s1;
+  if (mine > 0) {
+    fetch(s0, first);
+    int t = 0;
+    for (; t + 2 < mine; t += 2) {
+      fetch(s1, first + t + 1);
+      step_products(s0);
+      fetch(s0, first + t + 2);
+      step_products(s1);
+    }
+    if (mine - t == 2) {
+      fetch(s1, first + t + 1);
+      step_products(s0);
+      step_products(s1);
+    } else {
+      step_products(s0);
+    }
+  }
+  if (row_bytes % kStepBytes != 0 && wave == full % kWaves) {  // the partial step: pieces past the end of a row are zero
+    const int left = row_bytes - full * kStepBytes;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool in = (2 * lq + h) * 16 < left;
+#pragma unroll
+      for (int j = 0; j < NB; ++j) s0.w[j][h] = in ? load16(w_base + (int64_t)full * kStepBytes + w_off[j] + h * 16) : zero16();
+#pragma unroll
+      for (int i = 0; i < MB; ++i) s0.a[i][h] = in ? load16(a_base + (int64_t)full * kStepBytes + a_off[i] + h * 16) : zero16();
+    }
+    step_products(s0);
+  }
+
+  // ---- the four partial tiles meet in LDS; the weight operand is the MFMA's first, so a lane holds 4 consecutive output
+  // columns (16 j + 4 (lane / 16) ..) of tile row 16 i + lane % 16
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) red[wave][i * NB + j][lane] = acc[i][j];
+  __syncthreads();
+  auto total_of = [&](int b, int l) {
+    f32x4 v = red[0][b][l];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) v += red[w][b][l];
+    return v;
+  };
+  constexpr int kItems = MB * NH * kWave;
+  constexpr bool kFp8 = std::is_same_v<TI, fp8_t>;
+#pragma unroll
+  for (int it = tid; it < kItems; it += kNT) {
+    const int b = it / kWave, i = b / NH, j = b % NH;  // lane of the item: this thread's (kNT is a multiple of kWave)
+    const int p = m0 + i * 16 + lrow;
+    const int n = nt * (NH * 16) + j * 16 + 4 * lq;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
+    const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N);
+    f32x4 v = total_of(i * NB + j, lane);
+    [[maybe_unused]] f32x4 g = v;
+    if constexpr (MODE == kSwiglu) g = total_of(i * NB + j + NH, lane);
+    if (!inside) continue;
+    if constexpr (kFp8) {
+      const float rs = prm.a_scale[prm.a_gather_div > 0 ? prm.row_slot[p] / prm.a_gather_div : p];
+      const float4 cs = *reinterpret_cast<const float4*>(prm.w_scale + (int64_t)expert * prm.N + n);
+      v = f32x4{v[0] * rs * cs.x, v[1] * rs * cs.y, v[2] * rs * cs.z, v[3] * rs * cs.w};
+      if constexpr (MODE == kSwiglu) {
+        const float4 cg = *reinterpret_cast<const float4*>(prm.w_scale + (int64_t)expert * prm.N + prm.I + n);
+        g = f32x4{g[0] * rs * cg.x, g[1] * rs * cg.y, g[2] * rs * cg.z, g[3] * rs * cg.w};
+      }
+    } else if constexpr (MODE != kSwiglu) {
+      if (prm.aux_in != nullptr) {  // per-expert bias: joins the fp32 sum, one rounding
+        const TO* bias = static_cast<const TO*>(prm.aux_in) + (int64_t)expert * prm.N + n;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v[s] += Elem<TO>::up(bias[s]);
+      }
+    }
+    TO o[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) o[s] = Elem<TO>::down(v[s]);
+    if constexpr (MODE == kSwiglu) {  // from the rounded pre-activation, as if it had been a tensor
+      TO og[4], oa[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        og[s] = Elem<TO>::down(g[s]);
+        const float gf = Elem<TO>::up(og[s]), sg = sigmoid_fast(gf);
+        oa[s] = Elem<TO>::down(prm.act_kind == CK_ACT_GLU ? Elem<TO>::up(o[s]) * sg : Elem<TO>::up(o[s]) * gf * sg);
+      }
+      store4(static_cast<TO*>(prm.aux) + (int64_t)p * prm.I + n, oa[0], oa[1], oa[2], oa[3]);
+      if (prm.y != nullptr) {
+        TO* pre = static_cast<TO*>(prm.y) + (int64_t)p * 2 * prm.I + n;
+        store4(pre, o[0], o[1], o[2], o[3]);
+        store4(pre + prm.I, og[0], og[1], og[2], og[3]);
+      }
+    } else {
+      const int64_t row = MODE == kScatter ? prm.row_slot_out[p] : p;
+      if (MODE == kScatter || prm.y != nullptr) store4(static_cast<TO*>(prm.y) + row * prm.N + n, o[0], o[1], o[2], o[3]);
+      if constexpr (MODE == kGrouped && !kFp8) {
+        if (prm.aux != nullptr) {  // CK_ACT_GELU_TANH: the activation of the rounded output
+          TO oa[4];
+#pragma unroll
+          for (int s = 0; s < 4; ++s) oa[s] = Elem<TO>::down(gelu_tanh_fast(Elem<TO>::up(o[s])));
+          store4(static_cast<TO*>(prm.aux) + row * prm.N + n, oa[0], oa[1], oa[2], oa[3]);
+        }
+      }
+    }
+  }
+}
+
+template <typename TI, typename TO, int MODE, int MB, int NB>
+int launch_tile(const GemmParams& prm_in, int64_t m_tiles, int out_cols, hipStream_t s, const char* name) {
+  GemmParams prm = prm_in;
+  prm.n_tiles = (int)ceil_div(out_cols, 16 * (MODE == kSwiglu ? NB / 2 : NB));
+  const int64_t blocks = m_tiles * prm.n_tiles;
+  CK_REQUIRE(blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
+  hipLaunchKernelGGL((grouped_gemm_skinny_kernel<TI, TO, MODE, MB, NB>), dim3((unsigned)blocks), dim3(kNT), 0, s, prm);
+  CK_CHECK_LAUNCH(name);
+  return CK_OK;
+}
+
+template <typename TI, typename TO, int MODE>
+int launch_mode(const GemmParams& prm, int64_t rows, int64_t m_tiles, hipStream_t s, const char* name) {
+  const int out_cols = MODE == kSwiglu ? prm.I : prm.N;
+  switch (prm.align) {
+    case 16: {
+      // narrow column tiles while the launch would not fill the chip (256 CUs x 4 workgroups) with wide ones; the number of
+      // row tiles with work is at most one per row
+      const int64_t live = rows < m_tiles ? rows : m_tiles;
+      const bool narrow = live * ceil_div(out_cols, MODE == kSwiglu ? 32 : 64) < 1024;
+      if (narrow) return launch_tile<TI, TO, MODE, 1, 2>(prm, m_tiles, out_cols, s, name);
+      return launch_tile<TI, TO, MODE, 1, 4>(prm, m_tiles, out_cols, s, name);
+    }
+    case 32: return launch_tile<TI, TO, MODE, 2, 4>(prm, m_tiles, out_cols, s, name);
+    case 64: return launch_tile<TI, TO, MODE, 4, 4>(prm, m_tiles, out_cols, s, name);
+    default: set_error("%s: no small-row kernel for %d-row tiles", name, prm.align); return CK_ERR_ARG;
+  }
+}
+
+template <typename TI, typename TO>
+int launch_types(const GemmParams& prm, int mode, int64_t rows, int64_t m_tiles, hipStream_t s, const char* name) {
+  switch (mode) {
+    case kGrouped: return launch_mode<TI, TO, kGrouped>(prm, rows, m_tiles, s, name);
+    case kScatter: return launch_mode<TI, TO, kScatter>(prm, rows, m_tiles, s, name);
+    case kSwiglu: return launch_mode<TI, TO, kSwiglu>(prm, rows, m_tiles, s, name);
+    default: set_error("%s: the small-row kernel has no epilogue %d", name, mode); return CK_ERR_ARG;
+  }
+}
+
+}  // namespace
+
+int launch_skinny(const GemmParams& prm, int mode, int64_t max_rows, bool fp8, int dtype, hipStream_t stream, const char* name) {
+  const int64_t m_tiles = max_rows / prm.align;
+  // the padded layout holds at most max_rows - num_experts * (align - 1) rows (ck_sort_max_rows)
+  int64_t rows = max_rows - (int64_t)prm.num_experts * (prm.align - 1);
+  if (rows < 1) rows = 1;
+  CK_DISPATCH_HALF(dtype, name, {
+    if (fp8) return launch_types<fp8_t, scalar_t>(prm, mode, rows, m_tiles, stream, name);
+    return launch_types<scalar_t, scalar_t>(prm, mode, rows, m_tiles, stream, name);
+  });
+  return CK_ERR_ARG;
+}
+
+}  // namespace ck

@@ -525,7 +525,7 @@ def experts_up_gelu_backward(
     ctx = _Ctx((need_x, need_w, False, False, need_bias, False))
     ctx.seg, ctx.k, ctx.gelu = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align), k, True
     ctx.saved_tensors = (x.contiguous(), w.contiguous(), pre)
-    d_x, d_w, _, _, d_bias, _ = _moe._ExpertsUp.backward(ctx, d_act)
+    d_x, d_w, _, _, d_bias = _moe._ExpertsUp.backward(ctx, d_act)[:5]
     return _or_empty(d_x, x), _or_empty(d_w, x), _or_empty(d_bias, x)
 
 

@@ -14,7 +14,7 @@ import torch.nn as nn
 
 from . import _C
 from . import scattermoe
-from .scattermoe import ExpertSegments, _combine, route_topk_softmax, sort_by_expert
+from .scattermoe import ExpertSegments, _combine, choose_align, route_topk_softmax, sort_by_expert
 
 
 E4M3_MAX = 448.0
@@ -79,10 +79,11 @@ def swiglu_experts_e4m3(
 ) -> torch.Tensor:
     """out[t] = sum_j gates[t, j] * c_proj_e( swiglu_packed( c_fc_e( x[t] ) ) ) with e4m3 GEMM operands.
 
-    x [T, H] bf16 / fp16; w_fc8 [E, 2I, H] packed [up | gate]; w_proj8 [E, H, I]; seg from sort_by_expert(..., align=256).
+    x [T, H] bf16 / fp16; w_fc8 [E, 2I, H] packed [up | gate]; w_proj8 [E, H, I]; seg from sort_by_expert(..., align=256), or
+    a smaller tile height for few rows per expert (choose_align(rows, experts, inference=True)).
     x_quantized: (x8, scale) = quantize_rows_e4m3(x) if the caller has it already (rmsnorm_route_cute(..., quantize=True)).
     """
-    assert seg.align == 256, "the fp8 GEMMs use 256-row tiles: sort_by_expert(..., align=256)"
+    assert seg.align in (16, 32, 64, 256), "the fp8 GEMMs have tiles of 16, 32, 64 and 256 rows: sort_by_expert(..., align=256)"
     T, H = x.shape
     k = gates.size(1)
     E, two_i, _ = w_fc8.shape
@@ -125,7 +126,8 @@ class MoE_E4M3(nn.Module):
         hidden_states = hidden_states.view(-1, self.hidden_size)
         router_logits = self.gate(hidden_states)
         router_weights, selected_experts = route_topk_softmax(router_logits, self.top_k, long_indices=False)
-        seg = sort_by_expert(selected_experts, self.num_experts, 256)
+        align = choose_align(selected_experts.numel(), self.num_experts, hidden_states.dtype, inference=True)
+        seg = sort_by_expert(selected_experts, self.num_experts, align)
         out = swiglu_experts_e4m3(
             hidden_states, self.c_fc_weight_e4m3, self.c_fc_scale, self.c_proj_weight_e4m3, self.c_proj_scale,
             router_weights, seg,
@@ -145,7 +147,8 @@ class MoE_E4M3(nn.Module):
             hidden_states.view(-1, self.hidden_size), norm_weight, self.gate.weight, eps, quantize=True
         )
         router_weights, selected_experts = route_topk_softmax(router_logits, self.top_k, long_indices=False)
-        seg = sort_by_expert(selected_experts, self.num_experts, 256)
+        align = choose_align(selected_experts.numel(), self.num_experts, hidden_states.dtype, inference=True)
+        seg = sort_by_expert(selected_experts, self.num_experts, align)
         out = swiglu_experts_e4m3(
             normed, self.c_fc_weight_e4m3, self.c_fc_scale, self.c_proj_weight_e4m3, self.c_proj_scale, router_weights, seg,
             x_quantized=(x8, x_scale),

@@ -185,6 +185,9 @@ class ExpertSegments:
         return self.max_rows
 
 
+SMALL_TILES = ((6, 16), (14, 32), (30, 64))  # (rows per expert up to which, tile height) of inference batches
+
+
 def choose_align(
     num_rows: int, num_experts: int, dtype: torch.dtype | None = None, inference: bool = False
 ) -> int:
@@ -194,12 +197,20 @@ def choose_align(
     as stored instead of through transposed copies. Measured at 16 / 64 / 250 / 375 rows per expert, 128 against 256:
     training step of 8 wide experts (4,096 x 14,336) 3.44 / 4.13 / 5.56 / 6.93 against 2.24 / 2.41 / 3.24 / 3.94 ms, of 16
     experts (1,536 x 4,096) from 64 rows on 1.03 / 1.34 / 1.61 against 0.79 / 1.02 / 1.09 ms.
-    inference (no backward pass): 128 below 128 rows per expert, where the load is the weights' stream and smaller tiles
-    keep more of it in flight (8 wide experts, 8 tokens: 0.50 against 0.56 ms; at 256 rows per expert 1.52 against 0.96).
+    inference (no backward pass): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the stream
+    of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights fetched
+    once per tile, from L2 at best, so the height follows the load. Whole inference layers at 1 / 8 / 16 / 32 / 64 rows per
+    expert, tiles of 16, 32, 64, 256 rows: 128 experts of 4,096 x 1,536 in e4m3 286, 291, 299, 382 / 522, 509, 522, 607 / - /
+    872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 / 661, 609,
+    596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us.
     fp32 layers run on 64-row tiles either way: 128 below 512 rows per expert keeps their padding small."""
     if dtype is torch.float32:
         return 256 if num_rows >= 512 * num_experts else 128
-    return 128 if inference and num_rows < 128 * num_experts else 256
+    if inference:
+        for rows, align in SMALL_TILES:
+            if num_rows <= rows * num_experts:
+                return align
+    return 256
 
 
 @torch.no_grad()
@@ -551,24 +562,32 @@ def _check_expert_dtypes(x: torch.Tensor, *weights: torch.Tensor) -> None:
 # ---------------------------------------------------------------------------------------------------------------
 # generic expert linears (any activation between them)
 # ---------------------------------------------------------------------------------------------------------------
+def _experts_up_forward(x, w, seg: ExpertSegments, k: int, bias, gelu: bool, keep_pre: bool, zero_pads: bool):
+    """(y, act): the c_fc output in padded grouped order and, with gelu, its activation (y None unless keep_pre). Pad rows
+    are never written by the kernel: zero_pads makes them zeros, which keeps whatever is applied on top of them finite.
+    Without it they hold anything, which the expert GEMMs and their backward pass do not mind: they read valid rows only."""
+    N, K = w.shape[1:]
+    new = torch.zeros if zero_pads else torch.empty
+    y = new(seg.max_rows, N, dtype=x.dtype, device=x.device) if keep_pre or not gelu else None
+    act = new(seg.max_rows, N, dtype=x.dtype, device=x.device) if gelu else None
+    fused_bias = bias is not None and (gelu or _fp32(x) or _bias_in_epilogue(seg, K))
+    _gemm(x, k, w, seg, _C.CK_EPI_GELU_TANH if gelu else _C.CK_EPI_GROUPED, y, aux=act,
+          aux_in=bias.contiguous() if fused_bias else None)
+    if bias is not None and not fused_bias:
+        _add_expert_bias(y, bias.contiguous(), seg, None)
+    return y, act
+
+
 class _ExpertsUp(torch.autograd.Function):
     """x [T, H] (token order) -> y [max_rows, N] (padded grouped): the reference's c_fc with grouped_out=True.
     gelu=True: returns gelu_tanh(y) instead, computed in the GEMM's epilogue from the rounded y (the activation module
     applied to y would read the same values); y is kept for the backward pass only."""
 
     @staticmethod
-    def forward(ctx, x, w, seg: ExpertSegments, k: int, bias=None, gelu: bool = False):
+    def forward(ctx, x, w, seg: ExpertSegments, k: int, bias=None, gelu: bool = False, zero_pads: bool = True):
         x = x.contiguous()
         w = w.contiguous()
-        E, N, K = w.shape
-        # pad rows are never written by the kernel; zeros keep any activation applied on top finite
-        y = torch.zeros(seg.max_rows, N, dtype=x.dtype, device=x.device)
-        act = torch.zeros_like(y) if gelu else None
-        fused_bias = bias is not None and (gelu or _fp32(x) or _bias_in_epilogue(seg, K))
-        _gemm(x, k, w, seg, _C.CK_EPI_GELU_TANH if gelu else _C.CK_EPI_GROUPED, y, aux=act,
-              aux_in=bias.contiguous() if fused_bias else None)
-        if bias is not None and not fused_bias:
-            _add_expert_bias(y, bias.contiguous(), seg, None)
+        y, act = _experts_up_forward(x, w, seg, k, bias, gelu, True, zero_pads)
         ctx.gelu = gelu
         if gelu:
             ctx.save_for_backward(x, w, y)
@@ -605,15 +624,17 @@ class _ExpertsUp(torch.autograd.Function):
             d_expanded = torch.empty(T * k, K, dtype=x.dtype, device=x.device)
             _gemm_dx(d_y, w, seg, _C.CK_EPI_SCATTER, d_expanded)
             d_x = d_expanded if k == 1 else _combine(d_expanded, None, T, k, K)[0]
-        return d_x, d_w, None, None, d_bias, None
+        return d_x, d_w, None, None, d_bias, None, None
 
 
 class _ExpertsDown(torch.autograd.Function):
     """h [max_rows, I] (padded grouped), gates [T, k] -> out [T, H]: the reference's c_proj with grouped_in=True."""
 
     @staticmethod
-    def forward(ctx, h, w, gates, seg: ExpertSegments, bias=None, slot_expert=None, gate_slot=None):
-        ctx.gate_slot = gate_slot
+    def forward(
+        ctx, h, w, gates, seg: ExpertSegments, bias=None, slot_expert=None, gate_slot=None, zero_pads: bool = True
+    ):
+        ctx.gate_slot, ctx.zero_pads = gate_slot, zero_pads
         h = h.contiguous()
         w = w.contiguous()
         gates = gates.contiguous()
@@ -652,17 +673,19 @@ class _ExpertsDown(torch.autograd.Function):
                 _, h_t = _group_rows(h, None, 0, seg, False, True)
                 _gemm_dw(d_y_t, h_t, seg, d_w)
         if ctx.needs_input_grad[0]:
-            d_h = torch.zeros(seg.max_rows, K, dtype=h.dtype, device=h.device)
+            new = torch.zeros if getattr(ctx, "zero_pads", True) else torch.empty
+            d_h = new(seg.max_rows, K, dtype=h.dtype, device=h.device)
             _gemm_dx(d_y, w, seg, _C.CK_EPI_GROUPED, d_h)
-        return d_h, d_w, d_gates, None, d_bias, None, None
+        return d_h, d_w, d_gates, None, d_bias, None, None, None
 
 
 def experts_up(
     x: torch.Tensor, weight: torch.Tensor, seg: ExpertSegments, k: int, bias: torch.Tensor | None = None,
-    gelu_tanh: bool = False,
+    gelu_tanh: bool = False, zero_pads: bool = True,
 ) -> torch.Tensor:
     """x [T, H] -> c_fc output in padded grouped order [max_rows, N] (+ bias[e] on expert e's rows); with gelu_tanh, the
-    tanh-approximated GELU of that output, applied in the GEMM's epilogue."""
+    tanh-approximated GELU of that output, applied in the GEMM's epilogue. Pad rows are zero; zero_pads=False leaves them
+    unwritten, for a caller that hands the result straight to experts_down(..., zero_pads=False)."""
     _check_expert_dtypes(x, weight)
     assert bias is None or (bias.dtype == x.dtype and bias.shape == weight.shape[:2]), "bias should be [E, out] in x.dtype"
     if is_tracing():
@@ -673,13 +696,18 @@ def experts_up(
         )
         return out[0] if gelu_tanh else out
     _C.require_gpu(x, weight, bias)
-    return _ExpertsUp.apply(x, weight, seg, k, bias, gelu_tanh)
+    if not torch.is_grad_enabled():
+        y, act = _experts_up_forward(x.contiguous(), weight.contiguous(), seg, k, bias, gelu_tanh, False, zero_pads)
+        return act if gelu_tanh else y
+    return _ExpertsUp.apply(x, weight, seg, k, bias, gelu_tanh, zero_pads)
 
 
 def experts_down(
-    h: torch.Tensor, weight: torch.Tensor, gates: torch.Tensor, seg: ExpertSegments, bias: torch.Tensor | None = None
+    h: torch.Tensor, weight: torch.Tensor, gates: torch.Tensor, seg: ExpertSegments, bias: torch.Tensor | None = None,
+    zero_pads: bool = True,
 ) -> torch.Tensor:
-    """h [max_rows, I] (padded grouped) -> sum_k gates * (c_proj output + bias[e]) in token order [T, N]."""
+    """h [max_rows, I] (padded grouped) -> sum_k gates * (c_proj output + bias[e]) in token order [T, N]. Pad rows of the
+    gradient of h are zero; zero_pads=False leaves them unwritten."""
     _check_expert_dtypes(h, weight)
     assert bias is None or (bias.dtype == h.dtype and bias.shape == weight.shape[:2]), "bias should be [E, out] in h.dtype"
     if is_tracing():
@@ -689,12 +717,33 @@ def experts_down(
             seg.max_rows, seg.num_experts, seg.align,
         )[0]
     _C.require_gpu(h, weight, gates, bias)
-    return _ExpertsDown.apply(h, weight, gates.to(h.dtype), seg, bias, None, _gate_slot(gates))
+    return _ExpertsDown.apply(h, weight, gates.to(h.dtype), seg, bias, None, _gate_slot(gates), zero_pads)
 
 
 # ---------------------------------------------------------------------------------------------------------------
 # fused SwiGLU expert block
 # ---------------------------------------------------------------------------------------------------------------
+def _swiglu_experts_forward(x, w_fc, w_proj, gates, seg: ExpertSegments, act_kind: int, keep_pre: bool, keep_act: bool):
+    """(out, pre, act, act_t, expanded) of the fused expert block on contiguous tensors. keep_pre: whether the c_fc GEMM
+    also writes its pre-activation (a backward pass reads it; without one, two thirds of that GEMM's stores go away).
+    keep_act: d_w_proj needs the activation, as it is or, where its GEMM has no row-major form, transposed (act_t, a second
+    output of the same epilogue)."""
+    T, H = x.shape
+    k = gates.size(1)
+    E, two_i, _ = w_fc.shape
+    I = two_i // 2
+    dev, dt = x.device, x.dtype
+    pre = torch.empty(seg.max_rows, two_i, dtype=dt, device=dev) if keep_pre else None
+    act = torch.empty(seg.max_rows, I, dtype=dt, device=dev)
+    rows_form = _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, (H, I), (two_i, H))
+    act_t = torch.empty(I, seg.ld_t, dtype=dt, device=dev) if keep_act and not rows_form else None
+    _gemm(x, k, w_fc, seg, _C.CK_EPI_GLU if act_kind == _C.CK_ACT_GLU else _C.CK_EPI_SWIGLU, pre, y_t=act_t, aux=act)
+    expanded = torch.empty(T * k, H, dtype=dt, device=dev)
+    _gemm(act, 0, w_proj, seg, _C.CK_EPI_SCATTER, expanded)
+    out, _ = _combine(expanded, gates, T, k, H)
+    return out, pre, act, act_t, expanded
+
+
 class _SwigluExperts(torch.autograd.Function):
     """out = combine_k( gates * c_proj( swiglu_packed( c_fc(x) ) ) ) with the SwiGLU forward fused into the c_fc
     epilogue and the SwiGLU backward fused into the epilogue of the c_proj input-gradient GEMM."""
@@ -702,30 +751,13 @@ class _SwigluExperts(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_fc, w_proj, gates, seg: ExpertSegments, act_kind: int = _C.CK_ACT_SWIGLU, gate_slot=None):
         ctx.gate_slot = gate_slot
-        x = x.contiguous()
-        w_fc = w_fc.contiguous()
-        w_proj = w_proj.contiguous()
-        gates = gates.contiguous()
-        T, H = x.shape
-        k = gates.size(1)
-        E, two_i, _ = w_fc.shape
-        I = two_i // 2
-        dev, dt = x.device, x.dtype
+        x, w_fc, w_proj, gates = (t.contiguous() for t in (x, w_fc, w_proj, gates))
         need_grad = any(ctx.needs_input_grad[:4])
-
-        pre = torch.empty(seg.max_rows, two_i, dtype=dt, device=dev)
-        act = torch.empty(seg.max_rows, I, dtype=dt, device=dev)
-        # d_w_proj needs the activation: transposed (written by the same epilogue) or, in the row-major form, as it is
-        rows_form = _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, (H, I), (two_i, H))
-        act_t = torch.empty(I, seg.ld_t, dtype=dt, device=dev) if ctx.needs_input_grad[2] and not rows_form else None
-        _gemm(x, k, w_fc, seg, _C.CK_EPI_GLU if act_kind == _C.CK_ACT_GLU else _C.CK_EPI_SWIGLU, pre, y_t=act_t, aux=act)
-
-        expanded = torch.empty(T * k, H, dtype=dt, device=dev)
-        _gemm(act, 0, w_proj, seg, _C.CK_EPI_SCATTER, expanded)
-        out, _ = _combine(expanded, gates, T, k, H)
-
+        out, pre, act, act_t, expanded = _swiglu_experts_forward(
+            x, w_fc, w_proj, gates, seg, act_kind, True, ctx.needs_input_grad[2]
+        )
         if need_grad:
-            act_saved = (act if ctx.needs_input_grad[2] else None) if rows_form else act_t
+            act_saved = act_t if act_t is not None else (act if ctx.needs_input_grad[2] else None)
             ctx.save_for_backward(x, w_fc, w_proj, gates, pre, act_saved, expanded)
         ctx.seg, ctx.act_kind = seg, act_kind
         return out
@@ -809,6 +841,9 @@ def swiglu_experts(
             grad and w_proj.requires_grad, grad and gates.requires_grad, act_kind,
         )[0]
     _C.require_gpu(x, w_fc, w_proj, gates)
+    if not torch.is_grad_enabled():
+        tensors = (t.contiguous() for t in (x, w_fc, w_proj, gates.to(x.dtype)))
+        return _swiglu_experts_forward(*tensors, seg, act_kind, False, False)[0]
     return _SwigluExperts.apply(x, w_fc, w_proj, gates.to(x.dtype), seg, act_kind, _gate_slot(gates))
 
 

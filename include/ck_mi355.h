@@ -183,7 +183,8 @@ int ck_transpose_batched(const void* src, int64_t batch, int32_t rows, int32_t c
  * Replaces: scatter2scatter + scatter2scatter_triton_kernel -- triton_implementation/ops.py:31-78, kernels.py:12-133 --
  *           group_bwd_W + groupXtY_triton_kernel -- ops.py:81-105, kernels.py:136-222 -- and the per-expert
  *           F.linear loop of torch_implementation.py:32-49.
- * Shared layout arguments come from ck_sort_by_expert (same `align`; align must be 128 or 256).
+ * Shared layout arguments come from ck_sort_by_expert (same `align`; align must be 128 or 256, for the forward
+ * GEMMs of an inference batch also 16, 32 or 64: see ck_grouped_gemm).
  * K and N must be multiples of 8.
  * ------------------------------------------------------------------------------------------------------------- */
 typedef struct ck_segments {
@@ -219,6 +220,9 @@ typedef struct ck_segments {
  *   CK_EPI_SWIGLU_BWD     : the GEMM result is d_act [rows, N = I]; aux_in = saved pre-activation [max_rows, 2I];
  *                           writes d_preact to y [max_rows, 2I] and its transpose to y_t [2I, ld_t] (optional)
  *                           (backward formula: cute_kernels/kernels/swiglu/cuda_implementation/backward.cu:27-41)
+ * y may be NULL in the GELU, SwiGLU and GLU epilogues (inference: only the activation is written).
+ * align 16, 32, 64: few rows per expert, the weights streamed from memory without an LDS stage; no y_t, no
+ * CK_EPI_SWIGLU_BWD. (The fp8 GEMM takes these three and 256.)
  */
 #define CK_EPI_GROUPED 0
 #define CK_EPI_SCATTER 1
@@ -299,7 +303,7 @@ int ck_grouped_gemm_dw_rows(const void* a, const void* b, int32_t M, int32_t N, 
  * round to nearest even. x [rows, cols] bf16 / f16, q [rows, cols] bytes, cols % 16 == 0. Used per token for
  * activations and per output channel ([E * out, in] rows) for expert weights. */
 int ck_quant_rows_e4m3(const void* x, int64_t rows, int32_t cols, void* q, float* scales, int32_t dtype, void* stream);
-/* Y = (A_e * diag(a_scale)) * (W[e] * diag(w_scale[e]))^T over tile-aligned expert segments (align must be 256).
+/* Y = (A_e * diag(a_scale)) * (W[e] * diag(w_scale[e]))^T over tile-aligned expert segments (align 16, 32, 64 or 256).
  * a8: e4m3 rows [*, K], gathered like ck_grouped_gemm (a_gather_div); a_scale is indexed by the row of a8 that is read.
  * w8 [E, N, K] e4m3, w_scale [E, N]. K % 128 == 0. Epilogues: CK_EPI_GROUPED (y [max_rows, N]), CK_EPI_SCATTER
  * (y [R, N]), CK_EPI_SWIGLU (N = 2I packed [up | gate]; only the activation is written, to aux [max_rows, I]).

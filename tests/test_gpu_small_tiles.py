@@ -1,0 +1,97 @@
+"""GPU parity of the small-row grouped GEMMs (16-, 32- and 64-row tiles: inference batches with few rows per expert), through
+the C ABI, against fp32 products of the same operands."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import cute_kernels
+from cute_kernels import _C, fp8, scattermoe
+from oracle import moe_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+# outputs are fp32 sums rounded once to 16 bits: half a step of bf16 is 2^-9 of the value; 1e-2 as in the other GEMM tests
+RTOL = ATOL = 1e-2
+
+
+def _case(device, T, k, E, align, seed):
+    g = torch.Generator().manual_seed(seed)
+    ids = torch.randint(0, E, (T * k,), generator=g, dtype=torch.int32)
+    ids[ids == 1] = 0  # one empty expert, one with more rows than a tile
+    seg = cute_kernels.sort_by_expert(ids.to(device), E, align)
+    return g, seg
+
+
+def _rows(seg):
+    """(padded row, expert, flat slot) of every valid row."""
+    starts, counts, slot = seg.seg_starts.cpu(), seg.counts.cpu().to(torch.int64), seg.row_slot.cpu()
+    return [(p, e, int(slot[p])) for e in range(seg.num_experts) for p in range(int(starts[e]), int(starts[e]) + int(counts[e]))]
+
+
+# T: a single row, less than a tile, several ragged tiles. K: one step of one wave, a partial step only, an uneven split of
+# the steps over the waves with a partial step behind it. N: less than a column tile, ragged, several tiles.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("align", [16, 32, 64])
+@pytest.mark.parametrize("T,K,N", [(1, 64, 80), (9, 8, 144), (60, 200, 128), (150, 648, 272)])
+@pytest.mark.parametrize("epilogue", ["grouped_bias", "scatter", "swiglu", "swiglu_no_pre", "glu", "gelu"])
+def test_small_tiles_match_fp32(device, dtype, align, T, K, N, epilogue):
+    k, E = 2, 5
+    g, seg = _case(device, T, k, E, align, seed=T + K)
+    x = torch.randn(T, K, generator=g).to(dtype)
+    w = (0.1 * torch.randn(E, N, K, generator=g)).to(dtype)
+    bias = torch.randn(E, N, generator=g).to(dtype)
+    rows = _rows(seg)
+    want = torch.stack([F.linear(x[s // k].float(), w[e].float()) for _, e, s in rows])
+    experts = torch.tensor([e for _, e, _ in rows])
+    padded = torch.tensor([p for p, _, _ in rows])
+    xd, wd = x.to(device), w.to(device)
+    nan = lambda *shape: torch.full(shape, float("nan"), dtype=dtype, device=device)  # noqa: E731
+    if epilogue == "scatter":  # grouped input, (token, slot) output
+        a = nan(seg.max_rows, K)
+        a[padded.to(device)] = torch.stack([x[s // k] for _, _, s in rows]).to(device)
+        y = nan(T * k, N)
+        scattermoe._gemm(a, 0, wd, seg, _C.CK_EPI_SCATTER, y)
+        torch.testing.assert_close(y.cpu().float()[[s for _, _, s in rows]], want, rtol=RTOL, atol=ATOL)
+    elif epilogue == "grouped_bias":
+        y = nan(seg.max_rows, N)
+        scattermoe._gemm(xd, k, wd, seg, _C.CK_EPI_GROUPED, y, aux_in=bias.to(device))
+        torch.testing.assert_close(y.cpu().float()[padded], want + bias.float()[experts], rtol=RTOL, atol=ATOL)
+        assert torch.isnan(y).sum() == N * (seg.max_rows - len(rows))  # pad rows are left alone
+    elif epilogue == "gelu":
+        act = nan(seg.max_rows, N)
+        scattermoe._gemm(xd, k, wd, seg, _C.CK_EPI_GELU_TANH, None, aux=act)
+        torch.testing.assert_close(act.cpu().float()[padded], F.gelu(want.to(dtype).float(), approximate="tanh"), rtol=RTOL, atol=ATOL)
+    else:
+        act = nan(seg.max_rows, N // 2)
+        pre = None if epilogue == "swiglu_no_pre" else nan(seg.max_rows, N)
+        scattermoe._gemm(xd, k, wd, seg, _C.CK_EPI_GLU if epilogue == "glu" else _C.CK_EPI_SWIGLU, pre, aux=act)
+        fn = (lambda t: F.glu(t, dim=-1)) if epilogue == "glu" else mo.swiglu_packed_torch
+        torch.testing.assert_close(act.cpu().float()[padded], fn(want), rtol=2 * RTOL, atol=ATOL)  # two rounded factors
+        if pre is not None:
+            torch.testing.assert_close(pre.cpu().float()[padded], want, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("align", [16, 32, 64])
+@pytest.mark.parametrize("T,K,N", [(1, 128, 80), (40, 640, 272), (150, 1152, 128)])
+def test_small_tiles_fp8(device, align, T, K, N):
+    """The same products on e4m3 operands: against the de-quantised fp32 product (exact products, fp32 sums, one rounding)."""
+    k, E, dtype = 2, 5, torch.bfloat16
+    g, seg = _case(device, T, k, E, align, seed=T + K)
+    x8, xs = cute_kernels.quantize_rows_e4m3(torch.randn(T, K, generator=g).to(dtype).to(device))
+    w8, ws = cute_kernels.quantize_expert_weights_e4m3((0.1 * torch.randn(E, N, K, generator=g)).to(dtype).to(device))
+    xd, wd = x8.cpu().float() * xs.cpu()[:, None], w8.cpu().float() * ws.cpu()[:, :, None]
+    rows = _rows(seg)
+    want = torch.stack([F.linear(xd[s // k], wd[e]) for _, e, s in rows])
+    padded = torch.tensor([p for p, _, _ in rows])
+    act = torch.full((seg.max_rows, N // 2), float("nan"), dtype=dtype, device=device)
+    fp8._gemm_fp8(x8, xs, k, w8, ws, seg, _C.CK_EPI_SWIGLU, None, act, dtype)
+    torch.testing.assert_close(act.cpu().float()[padded], mo.swiglu_packed_torch(want), rtol=2 * RTOL, atol=ATOL)
+    a8 = torch.zeros(seg.max_rows, K, dtype=torch.uint8, device=device)
+    scale = torch.ones(seg.max_rows, device=device)
+    at = padded.to(device)
+    src = torch.tensor([s // k for _, _, s in rows], device=device)
+    a8[at], scale[at] = x8.view(torch.uint8)[src], xs[src]
+    y = torch.full((T * k, N), float("nan"), dtype=dtype, device=device)
+    fp8._gemm_fp8(a8.view(torch.float8_e4m3fn), scale, 0, w8, ws, seg, _C.CK_EPI_SCATTER, y, None, dtype)
+    torch.testing.assert_close(y.cpu().float()[[s for _, _, s in rows]], want, rtol=RTOL, atol=ATOL)
