@@ -448,8 +448,9 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_bwd_kernel(const T* __restrict
 // of the rows (256-byte coalesced reads, 8 independent partial sums so that 8 loads are in flight per wave), then the
 // sixteen results are added through LDS.
 constexpr int kReduceBlock = 1024, kReduceWaves = kReduceBlock / kWave, kReduceUnroll = 8;
+template <typename OUT>
 __global__ __launch_bounds__(kReduceBlock) void rmsnorm_dw_reduce_kernel(const float* __restrict__ partial, int64_t workers,
-                                                                          int H, float* __restrict__ d_weight) {
+                                                                          int H, OUT* __restrict__ d_weight) {
   __shared__ float part[kReduceWaves][kWave];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int h = blockIdx.x * kWave + lane;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(kReduceBlock) void rmsnorm_dw_reduce_kernel(const f
     float t = 0.f;
 #pragma unroll
     for (int g = 0; g < kReduceWaves; ++g) t += part[g][lane];
-    d_weight[h] = t;
+    d_weight[h] = Elem<OUT>::down(t);
   }
 }
 
@@ -611,20 +612,30 @@ extern "C" int64_t ck_rmsnorm_bwd_partial_rows(int64_t B) {
 
 static int rmsnorm_bwd_impl(const char* name, const void* x, const void* weight, const void* d_out, const void* d_added,
                             const float* rstd, float eps, float multiplier, int64_t B, int32_t H, void* d_x,
-                            void* d_residual, float* d_weight_partial, float* d_weight, int32_t dtype, void* stream) {
+                            void* d_residual, float* d_weight_partial, void* d_weight, bool d_weight_typed, int32_t dtype,
+                            void* stream) {
   CK_REQUIRE(B >= 0 && H >= 1, "%s: bad sizes B=%lld H=%d", name, (long long)B, H);
   CK_REQUIRE((weight == nullptr) == (d_weight == nullptr) && (weight == nullptr) == (d_weight_partial == nullptr),
              "%s: weight, d_weight and d_weight_partial must be given together", name);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // d_weight in fp32, or rounded to the weight's own dtype (one launch less for a caller that wants it there)
+#define CK_RMS_REDUCE(ROWS)                                                                                                 \
+  do {                                                                                                                      \
+    if (d_weight_typed)                                                                                                     \
+      hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<scalar_t>), dim3((unsigned)ceil_div(H, kWave)), dim3(kReduceBlock), 0, s, \
+                         d_weight_partial, ROWS, (int)H, static_cast<scalar_t*>(d_weight));                                 \
+    else                                                                                                                    \
+      hipLaunchKernelGGL((rmsnorm_dw_reduce_kernel<float>), dim3((unsigned)ceil_div(H, kWave)), dim3(kReduceBlock), 0, s,   \
+                         d_weight_partial, ROWS, (int)H, static_cast<float*>(d_weight));                                    \
+  } while (0)
   if (B == 0) {
     if (d_weight != nullptr) {  // no rows: the sum over zero partial rows is zero
-      hipLaunchKernelGGL(rmsnorm_dw_reduce_kernel, dim3((unsigned)ceil_div(H, kWave)), dim3(kReduceBlock), 0,
-                         static_cast<hipStream_t>(stream), d_weight_partial, (int64_t)0, (int)H, d_weight);
+      CK_DISPATCH_FLOAT(dtype, name, CK_RMS_REDUCE((int64_t)0));
       CK_CHECK_LAUNCH(name);
     }
     return CK_OK;
   }
   CK_REQUIRE(x && d_out && d_x, "%s: NULL argument", name);
-  hipStream_t s = static_cast<hipStream_t>(stream);
   CK_DISPATCH_FLOAT(dtype, name, {
     const bool aligned = aligned16(x) && aligned16(d_out) && aligned16(d_x) && (weight == nullptr || aligned16(weight)) &&
                          (d_added == nullptr || aligned16(d_added)) && (d_residual == nullptr || aligned16(d_residual));
@@ -634,11 +645,9 @@ static int rmsnorm_bwd_impl(const char* name, const void* x, const void* weight,
     const int64_t blocks = workers / rows_per_block;
     const BwdFuse<scalar_t> fuse = {static_cast<const scalar_t*>(d_added), static_cast<scalar_t*>(d_residual), multiplier};
     CK_RMS_DISPATCH(CK_RMS_BWD, 0);
-    if (d_weight != nullptr) {
-      hipLaunchKernelGGL(rmsnorm_dw_reduce_kernel, dim3((unsigned)ceil_div(H, kWave)), dim3(kReduceBlock), 0, s,
-                         d_weight_partial, workers, (int)H, d_weight);
-    }
+    if (d_weight != nullptr) CK_RMS_REDUCE(workers);
   });
+#undef CK_RMS_REDUCE
   CK_CHECK_LAUNCH(name);
   return CK_OK;
 }
@@ -647,7 +656,17 @@ extern "C" int ck_rmsnorm_bwd(const void* x, const void* weight, const void* d_o
                               int64_t B, int32_t H, void* d_x, float* d_weight_partial, float* d_weight, int32_t dtype,
                               void* stream) {
   return rmsnorm_bwd_impl("ck_rmsnorm_bwd", x, weight, d_out, nullptr, rstd, eps, 1.0f, B, H, d_x, nullptr,
-                          d_weight_partial, d_weight, dtype, stream);
+                          d_weight_partial, d_weight, false, dtype, stream);
+}
+
+extern "C" int ck_rmsnorm_bwd_typed(const void* x, const void* weight, const void* d_out, const void* d_added,
+                                    const float* rstd, float eps, float multiplier, int64_t B, int32_t H, void* d_x,
+                                    void* d_residual, float* d_weight_partial, void* d_weight, int32_t dtype, void* stream) {
+  const char* name = "ck_rmsnorm_bwd_typed";
+  CK_REQUIRE((d_residual != nullptr && d_residual != d_x) || multiplier == 1.0f,
+             "%s: d_x stands for both gradients only when multiplier is 1", name);
+  return rmsnorm_bwd_impl(name, x, weight, d_out, d_added, rstd, eps, multiplier, B, H, d_x,
+                          d_residual == d_x ? nullptr : d_residual, d_weight_partial, d_weight, true, dtype, stream);
 }
 
 extern "C" int ck_fused_residual_add_rmsnorm_bwd(const void* added, const void* weight, const void* d_out,
@@ -659,5 +678,5 @@ extern "C" int ck_fused_residual_add_rmsnorm_bwd(const void* added, const void* 
   CK_REQUIRE(d_residual != d_x || multiplier == 1.0f, "%s: d_x and d_residual may be one buffer only when multiplier is 1", name);
   // multiplier == 1: both gradients are the same values; a caller that passes one buffer for both gets one store
   return rmsnorm_bwd_impl(name, added, weight, d_out, d_added, rstd, eps, multiplier, B, H, d_x,
-                          d_residual == d_x ? nullptr : d_residual, d_weight_partial, d_weight, dtype, stream);
+                          d_residual == d_x ? nullptr : d_residual, d_weight_partial, d_weight, false, dtype, stream);
 }

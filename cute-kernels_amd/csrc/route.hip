@@ -19,10 +19,22 @@ __device__ inline uint32_t float_order_bits(float v) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-template <typename T, int PER>
+// the value behind float_order_bits (-0.0 comes back as +0.0)
+__device__ inline float float_from_order_bits(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+}
+
+// What bounds it: latency. A token's k selections depend on each other, so everything inside one is kept short: the selected
+// logit comes back out of its key (a second read of the row was a memory round trip per selection) and the exponentials
+// stay in registers until the denominator is known (KMAX of them; the group's lanes all hold them). Every output a caller
+// wants is written here, the 16-bit gates and 64-bit ids included: each was a launch of its own behind this one.
+// KMAX: upper bound of k in this instantiation.
+template <typename T, int PER, int KMAX>
 __global__ __launch_bounds__(kBlock) void route_topk_softmax_kernel(const T* __restrict__ logits, int64_t T_tokens,
                                                                      int E, int k, int G, int32_t* __restrict__ selected,
-                                                                     float* __restrict__ gates, T* __restrict__ topk_values) {
+                                                                     int64_t* __restrict__ selected_long,
+                                                                     float* __restrict__ gates, T* __restrict__ gates_rounded,
+                                                                     T* __restrict__ topk_values) {
   const int lane_in_group = threadIdx.x & (G - 1);
   const int64_t token = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / G;
   const bool live = token < T_tokens;
@@ -39,8 +51,11 @@ __global__ __launch_bounds__(kBlock) void route_topk_softmax_kernel(const T* __r
     }
   }
 
-  float vmax = 0.f, denom = 0.f;
-  for (int j = 0; j < k; ++j) {
+  float vmax = 0.f, denom = 0.f, ex[KMAX];
+  const bool writer = live && lane_in_group == 0;
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j) {
+    if (j >= k) break;
     uint64_t best = 0ull;
 #pragma unroll
     for (int p = 0; p < PER; ++p) best = key[p] > best ? key[p] : best;
@@ -54,19 +69,24 @@ __global__ __launch_bounds__(kBlock) void route_topk_softmax_kernel(const T* __r
 #pragma unroll
     for (int p = 0; p < PER; ++p)
       if (key[p] == best) key[p] = 0ull;  // keys are unique (they embed the expert index)
-    float v = 0.f;
-    if (live) v = Elem<T>::up(row[e < (uint32_t)E ? e : 0]);
+    const float v = live ? float_from_order_bits((uint32_t)(best >> 32)) : 0.f;
     if (j == 0) vmax = v;
-    const float ex = expf(v - vmax);
-    denom += ex;
-    if (live && lane_in_group == 0) {
-      gates[token * k + j] = ex;  // normalised below by the same lane
-      selected[token * k + j] = (int32_t)e;
-      if (topk_values) topk_values[token * k + j] = Elem<T>::down(v);
+    ex[j] = expf(v - vmax);
+    denom += ex[j];
+    if (writer) {
+      if (selected) selected[token * k + j] = (int32_t)e;
+      if (selected_long) selected_long[token * k + j] = (int64_t)e;
+      if (topk_values) topk_values[token * k + j] = row[e < (uint32_t)E ? e : 0];  // as stored: keeps the sign of a zero
     }
   }
-  if (live && lane_in_group == 0) {
-    for (int j = 0; j < k; ++j) gates[token * k + j] = gates[token * k + j] / denom;
+  if (writer) {
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      if (j >= k) break;
+      const float g = ex[j] / denom;
+      if (gates) gates[token * k + j] = g;
+      if (gates_rounded) gates_rounded[token * k + j] = Elem<T>::down(g);
+    }
   }
 }
 
@@ -106,13 +126,15 @@ __global__ __launch_bounds__(kBlock) void route_bwd_kernel(const float* __restri
 
 using namespace ck;
 
-extern "C" int ck_route_topk_softmax(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,
-                                     int32_t* selected, float* gates, void* topk_values, void* stream) {
-  CK_REQUIRE(E >= 1 && E <= kWave * kMaxPerLane, "ck_route_topk_softmax: E=%d outside [1, %d]", E, kWave * kMaxPerLane);
-  CK_REQUIRE(k >= 1 && k <= E && k <= kMaxTopK, "ck_route_topk_softmax: k=%d outside [1, min(E, %d)]", k, kMaxTopK);
-  CK_REQUIRE(T >= 0, "ck_route_topk_softmax: T is negative");
+static int route_impl(const char* name, const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,
+                      int32_t* selected, int64_t* selected_long, float* gates, void* gates_rounded, void* topk_values,
+                      void* stream) {
+  CK_REQUIRE(E >= 1 && E <= kWave * kMaxPerLane, "%s: E=%d outside [1, %d]", name, E, kWave * kMaxPerLane);
+  CK_REQUIRE(k >= 1 && k <= E && k <= kMaxTopK, "%s: k=%d outside [1, min(E, %d)]", name, k, kMaxTopK);
+  CK_REQUIRE(T >= 0, "%s: T is negative", name);
   if (T == 0) return CK_OK;
-  CK_REQUIRE(logits && selected && gates, "ck_route_topk_softmax: logits, selected and gates are required");
+  CK_REQUIRE(logits && (selected || selected_long) && (gates || gates_rounded),
+             "%s: logits, the selection and the gates are required", name);
   // Lanes per token: as few as keep at most 8 logits per lane (fewer lanes = fewer shuffle rounds per selection and more
   // tokens per wave; measured at T = 65,536, E = 128, k = 8: 85 us with a whole wave per token). Wide rows fall back to
   // whole waves with up to 16 logits per lane.
@@ -121,20 +143,39 @@ extern "C" int ck_route_topk_softmax(const void* logits, int32_t dtype, int64_t 
   const int per = (E + G - 1) / G;
   const int64_t blocks = ceil_div(T * G, kBlock);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CK_LAUNCH_ROUTE(PER)                                                                                      \
-  hipLaunchKernelGGL((route_topk_softmax_kernel<scalar_t, PER>), dim3((unsigned)blocks), dim3(kBlock), 0, s,      \
-                     static_cast<const scalar_t*>(logits), T, (int)E, (int)k, G, selected, gates,                 \
-                     static_cast<scalar_t*>(topk_values))
-  CK_DISPATCH_FLOAT(dtype, "ck_route_topk_softmax", {
-    if (per == 1) CK_LAUNCH_ROUTE(1);
-    else if (per == 2) CK_LAUNCH_ROUTE(2);
-    else if (per <= 4) CK_LAUNCH_ROUTE(4);
-    else if (per <= 8) CK_LAUNCH_ROUTE(8);
-    else CK_LAUNCH_ROUTE(16);
+#define CK_LAUNCH_ROUTE(PER, KMAX)                                                                                \
+  hipLaunchKernelGGL((route_topk_softmax_kernel<scalar_t, PER, KMAX>), dim3((unsigned)blocks), dim3(kBlock), 0, s, \
+                     static_cast<const scalar_t*>(logits), T, (int)E, (int)k, G, selected, selected_long, gates,  \
+                     static_cast<scalar_t*>(gates_rounded), static_cast<scalar_t*>(topk_values))
+#define CK_LAUNCH_ROUTE_K(PER)                                       \
+  do {                                                               \
+    if (k <= 2) CK_LAUNCH_ROUTE(PER, 2);                             \
+    else if (k <= 8) CK_LAUNCH_ROUTE(PER, 8);                        \
+    else CK_LAUNCH_ROUTE(PER, kMaxTopK);                             \
+  } while (0)
+  CK_DISPATCH_FLOAT(dtype, name, {
+    if (per <= 4) CK_LAUNCH_ROUTE_K(4);
+    else if (per <= 8) CK_LAUNCH_ROUTE_K(8);
+    else CK_LAUNCH_ROUTE_K(16);
   });
+#undef CK_LAUNCH_ROUTE_K
 #undef CK_LAUNCH_ROUTE
-  CK_CHECK_LAUNCH("ck_route_topk_softmax");
+  CK_CHECK_LAUNCH(name);
   return CK_OK;
+}
+
+extern "C" int ck_route_topk_softmax(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,
+                                     int32_t* selected, float* gates, void* topk_values, void* stream) {
+  const char* name = "ck_route_topk_softmax";
+  CK_REQUIRE(T <= 0 || (selected && gates), "%s: logits, selected and gates are required", name);
+  return route_impl(name, logits, dtype, T, E, k, selected, nullptr, gates, nullptr, topk_values, stream);
+}
+
+extern "C" int ck_route_topk_softmax_all(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,
+                                         int32_t* selected, int64_t* selected_long, float* gates, void* gates_rounded,
+                                         void* stream) {
+  return route_impl("ck_route_topk_softmax_all", logits, dtype, T, E, k, selected, selected_long, gates, gates_rounded,
+                    nullptr, stream);
 }
 
 static int route_bwd_impl(const char* name, const float* gates, const float* d_gates, const void* d_gates_rounded,

@@ -67,11 +67,11 @@ __global__ __launch_bounds__(kBlock) void combine_rows_kernel(const T* __restric
   }
 }
 
-// d_gates[t, j] = <expanded[t, j, :], grad_out[t, :]>, one wave per (t, j)
+// d_gates[t, j] = <expanded[t, j, :], grad_out[t, :]>, one wave per (t, j); rounded (optional): the same in the rows' type
 template <typename T, typename OUT>
 __global__ __launch_bounds__(kBlock) void gate_grad_kernel(const T* __restrict__ expanded, const T* __restrict__ grad_out,
                                                             int64_t pairs, int k, int chunks_per_row,
-                                                            OUT* __restrict__ d_gates) {
+                                                            OUT* __restrict__ d_gates, T* __restrict__ rounded) {
   constexpr int P = Elem<T>::per16;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t pair = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
@@ -86,7 +86,10 @@ __global__ __launch_bounds__(kBlock) void gate_grad_kernel(const T* __restrict__
     for (int i = 0; i < P; ++i) acc += Elem<T>::up(a.e[i]) * Elem<T>::up(b.e[i]);
   }
   acc = wave_sum(acc);
-  if (lane == 0) d_gates[pair] = Elem<OUT>::down(acc);
+  if (lane == 0) {
+    d_gates[pair] = Elem<OUT>::down(acc);
+    if (rounded != nullptr) rounded[pair] = Elem<T>::down(acc);
+  }
 }
 
 // ---- 64x64 tiles of 16-bit elements through LDS ---------------------------------------------------------------
@@ -422,30 +425,42 @@ extern "C" int ck_combine_rows(const void* expanded, const void* gates, int64_t 
       const int64_t pairs = T * k;
       hipLaunchKernelGGL((gate_grad_kernel<scalar_t, scalar_t>), dim3((unsigned)ceil_div(pairs, kBlock / kWave)), dim3(kBlock),
                          0, s, static_cast<const scalar_t*>(expanded), static_cast<const scalar_t*>(grad_out), pairs,
-                         (int)k, cpr, static_cast<scalar_t*>(d_gates_out));
+                         (int)k, cpr, static_cast<scalar_t*>(d_gates_out), static_cast<scalar_t*>(nullptr));
     }
   });
   CK_CHECK_LAUNCH("ck_combine_rows");
   return CK_OK;
 }
 
-extern "C" int ck_gate_grad_f32(const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H,
-                                float* d_gates, int32_t dtype, void* stream) {
-  CK_REQUIRE(T >= 0 && k >= 1 && H >= 1, "ck_gate_grad_f32: bad sizes T=%lld k=%d H=%d", (long long)T, k, H);
+static int gate_grad_impl(const char* name, const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H,
+                          float* d_gates, void* rounded, int32_t dtype, void* stream) {
+  CK_REQUIRE(T >= 0 && k >= 1 && H >= 1, "%s: bad sizes T=%lld k=%d H=%d", name, (long long)T, k, H);
   if (T == 0) return CK_OK;
-  CK_REQUIRE(expanded && grad_out && d_gates, "ck_gate_grad_f32: NULL argument");
-  CK_REQUIRE(aligned16(expanded) && aligned16(grad_out), "ck_gate_grad_f32: expanded / grad_out must be 16-byte aligned");
+  CK_REQUIRE(expanded && grad_out && d_gates, "%s: NULL argument", name);
+  CK_REQUIRE(aligned16(expanded) && aligned16(grad_out), "%s: expanded / grad_out must be 16-byte aligned", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  CK_DISPATCH_FLOAT(dtype, "ck_gate_grad_f32", {
+  CK_DISPATCH_FLOAT(dtype, name, {
     constexpr int P = Elem<scalar_t>::per16;
-    CK_REQUIRE(H % P == 0, "ck_gate_grad_f32: H=%d is not a multiple of %d", H, P);
+    CK_REQUIRE(H % P == 0, "%s: H=%d is not a multiple of %d", name, H, P);
     const int64_t pairs = T * k;
     hipLaunchKernelGGL((gate_grad_kernel<scalar_t, float>), dim3((unsigned)ceil_div(pairs, kBlock / kWave)), dim3(kBlock), 0,
                        s, static_cast<const scalar_t*>(expanded), static_cast<const scalar_t*>(grad_out), pairs, (int)k,
-                       H / P, d_gates);
+                       H / P, d_gates, static_cast<scalar_t*>(rounded));
   });
-  CK_CHECK_LAUNCH("ck_gate_grad_f32");
+  CK_CHECK_LAUNCH(name);
   return CK_OK;
+}
+
+extern "C" int ck_gate_grad_f32(const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H,
+                                float* d_gates, int32_t dtype, void* stream) {
+  return gate_grad_impl("ck_gate_grad_f32", expanded, grad_out, T, k, H, d_gates, nullptr, dtype, stream);
+}
+
+extern "C" int ck_gate_grad_both(const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H,
+                                 float* d_gates, void* d_gates_rounded, int32_t dtype, void* stream) {
+  const char* name = "ck_gate_grad_both";
+  CK_REQUIRE(T <= 0 || d_gates_rounded != nullptr, "%s: d_gates_rounded is required", name);
+  return gate_grad_impl(name, expanded, grad_out, T, k, H, d_gates, d_gates_rounded, dtype, stream);
 }
 
 extern "C" int ck_group_rows_padded(const void* src, const void* coeff, int32_t fan_out, int32_t H,

@@ -47,6 +47,7 @@ _SIGNATURES = {
     "ck_count_offsets": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ck_count_offsets_static": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ck_route_topk_softmax": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ck_route_topk_softmax_all": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ck_route_topk_softmax_bwd": (c_int32, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
     "ck_route_topk_softmax_bwd_exact": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
     "ck_sort_max_rows": (c_int64, [c_int64, c_int32, c_int32]),
@@ -59,6 +60,7 @@ _SIGNATURES = {
     "ck_gather_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p, c_int32, c_void_p]),
     "ck_combine_rows": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p]),
     "ck_gate_grad_f32": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
+    "ck_gate_grad_both": (c_int32, [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_int32, c_void_p]),
     "ck_group_rows_padded": (
         c_int32,
         [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_int64, c_int32, c_void_p],
@@ -107,6 +109,7 @@ _SIGNATURES = {
     "ck_rmsnorm_fwd": (c_int32, [c_void_p, c_void_p, c_float, c_int64, c_int32, c_void_p, c_void_p, c_int32, c_void_p]),
     "ck_rmsnorm_bwd_partial_rows": (c_int64, [c_int64]),
     "ck_rmsnorm_bwd": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p]),
+    "ck_rmsnorm_bwd_typed": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p]),
     "ck_add_expert_bias": (c_int32, [c_void_p, c_int64, c_int32, c_void_p, c_void_p, POINTER(ck_segments), c_int32, c_void_p]),
     "ck_expert_bias_grad": (c_int32, [c_void_p, c_int32, POINTER(ck_segments), c_void_p, c_int32, c_void_p]),
     "ck_softmax_fwd": (c_int32, [c_void_p, c_float, c_int64, c_int32, c_void_p, c_int32, c_void_p]),

@@ -54,19 +54,16 @@ class _RMSNorm_Cute(torch.autograd.Function):
         lib = _C.lib()
         weight_grad = partial = None
         if weight is not None:
-            weight_grad = torch.empty(H, device=x.device, dtype=torch.float32)
+            weight_grad = torch.empty(H, device=x.device, dtype=x.dtype)
             partial = torch.empty(max(lib.ck_rmsnorm_bwd_partial_rows(B), 1), H, device=x.device, dtype=torch.float32)
 
         with torch.cuda.device(x.device):
             _C.check(
-                lib.ck_rmsnorm_bwd(
-                    _C.ptr(x), _C.ptr(weight), _C.ptr(output_grad), _C.ptr(rstd), ctx.eps, B, H, _C.ptr(x_grad),
-                    _C.ptr(partial), _C.ptr(weight_grad), _C.dtype_code(x.dtype), _C.stream(),
+                lib.ck_rmsnorm_bwd_typed(
+                    _C.ptr(x), _C.ptr(weight), _C.ptr(output_grad), None, _C.ptr(rstd), ctx.eps, 1.0, B, H, _C.ptr(x_grad),
+                    None, _C.ptr(partial), _C.ptr(weight_grad), _C.dtype_code(x.dtype), _C.stream(),
                 )
             )
-
-        if weight_grad is not None:
-            weight_grad = weight_grad.type_as(weight)
 
         return x_grad, weight_grad, None, None
 

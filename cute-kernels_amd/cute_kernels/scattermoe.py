@@ -63,23 +63,28 @@ class _RouteTopKSoftmax(torch.autograd.Function):
         T, E = logits.shape
         selected = torch.empty(T, k, dtype=torch.int32, device=logits.device)
         gates = torch.empty(T, k, dtype=torch.float32, device=logits.device)
-        lib = _C.lib()
+        selected_long = torch.empty(T, k, dtype=torch.int64, device=logits.device) if long_indices else None
+        rounded = torch.empty(T, k, dtype=logits.dtype, device=logits.device) if logits.dtype != torch.float32 else None
         with torch.cuda.device(logits.device):
             _C.check(
-                lib.ck_route_topk_softmax(
-                    _C.ptr(logits), _C.dtype_code(logits.dtype), T, E, k, _C.ptr(selected), _C.ptr(gates), None, _C.stream()
+                _C.lib().ck_route_topk_softmax_all(
+                    _C.ptr(logits), _C.dtype_code(logits.dtype), T, E, k, _C.ptr(selected), _C.ptr(selected_long), _C.ptr(gates),
+                    _C.ptr(rounded), _C.stream(),
                 )
             )
         ctx.save_for_backward(gates, selected)
         ctx.E = E
         ctx.dtype = logits.dtype
         ctx.slot = slot
-        selected_out = selected.long() if long_indices else selected
+        selected_out = selected_long if long_indices else selected
         ctx.mark_non_differentiable(selected_out)
-        return gates.to(logits.dtype), selected_out
+        ctx.set_materialize_grads(False)  # no zero-filled gradient for the selection
+        return gates if rounded is None else rounded, selected_out
 
     @staticmethod
     def backward(ctx, d_gates: torch.Tensor, _d_selected):
+        if d_gates is None:
+            return None, None, None, None
         gates, selected = ctx.saved_tensors
         T, k = gates.shape
         exact = ctx.slot.d_gates_f32 if ctx.slot is not None else None
@@ -493,15 +498,18 @@ def _combine(expanded, gates, T, k, H, grad_out=None, want_out=True, want_d_gate
 def _gate_grad(expanded, grad_out, T, k, H, gates_dtype, slot):
     """d_gates in fp32 (kept in `slot` for the router's backward) and rounded to the gates' dtype for autograd."""
     d32 = torch.empty(T, k, dtype=torch.float32, device=expanded.device)
+    rounded = torch.empty(T, k, dtype=gates_dtype, device=expanded.device)
+    assert gates_dtype == expanded.dtype, "gates and expert outputs should have the same dtype"
     with torch.cuda.device(expanded.device):
         _C.check(
-            _C.lib().ck_gate_grad_f32(
-                _C.ptr(expanded), _C.ptr(grad_out), T, k, H, _C.ptr(d32), _C.dtype_code(expanded.dtype), _C.stream()
+            _C.lib().ck_gate_grad_both(
+                _C.ptr(expanded), _C.ptr(grad_out), T, k, H, _C.ptr(d32), _C.ptr(rounded), _C.dtype_code(expanded.dtype),
+                _C.stream(),
             )
         )
     if slot is not None:
         slot.d_gates_f32 = d32
-    return d32.to(gates_dtype)
+    return rounded
 
 
 def gather_rows(src: torch.Tensor, idx: torch.Tensor, coeff: torch.Tensor | None = None, fan_out: int = 1) -> torch.Tensor:

@@ -80,6 +80,10 @@ int ck_count_offsets_static(const void* ids, int32_t ids_are_i64, int64_t n, int
  * ------------------------------------------------------------------------------------------------------------- */
 int ck_route_topk_softmax(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k, int32_t* selected,
                           float* gates, void* topk_values, void* stream);
+/* The same in every form a caller may want, in one launch: selected int32 and / or selected_long int64 (at least one), gates
+ * fp32 and / or gates_rounded of `dtype` (at least one), all [T, k]. */
+int ck_route_topk_softmax_all(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k, int32_t* selected,
+                              int64_t* selected_long, float* gates, void* gates_rounded, void* stream);
 /* Backward of the above with respect to the logits (autograd of topk + softmax at
  * torch_implementation.py:127-133): d_logits [T, E] of `dtype`, every element written (zeros off the selection).
  * d_gates [T, k] fp32. */
@@ -155,6 +159,9 @@ int ck_combine_rows(const void* expanded, const void* gates, int64_t T, int32_t 
  * numbers. expanded [T * k, H], grad_out [T, H], d_gates [T, k]. */
 int ck_gate_grad_f32(const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H, float* d_gates,
                      int32_t dtype, void* stream);
+/* The same, and d_gates_rounded [T, k] of `dtype`: what autograd hands on next to the unrounded values. */
+int ck_gate_grad_both(const void* expanded, const void* grad_out, int64_t T, int32_t k, int32_t H, float* d_gates,
+                      void* d_gates_rounded, int32_t dtype, void* stream);
 /* Padded grouped copy of token rows and (optionally) its transpose, for the grouped GEMMs below:
  *   row p valid : grouped[p, :] = src[row_slot[p] / fan_out, :] * (coeff ? coeff[row_slot[p]] : 1)
  *   row p pad   : zeros
@@ -394,6 +401,11 @@ int ck_fused_residual_add_rmsnorm_bwd(const void* added, const void* weight, con
                                       const float* rstd, float eps, float multiplier, int64_t B, int32_t H, void* d_x,
                                       void* d_residual, float* d_weight_partial, float* d_weight, int32_t dtype,
                                       void* stream);
+/* Both backward passes with d_weight [H] in the tensors' `dtype` (what autograd wants for a weight of that dtype). d_added
+ * and d_residual may be NULL (plain RMSNorm); d_residual NULL or == d_x: one buffer for both gradients, multiplier 1. */
+int ck_rmsnorm_bwd_typed(const void* x, const void* weight, const void* d_out, const void* d_added, const float* rstd,
+                         float eps, float multiplier, int64_t B, int32_t H, void* d_x, void* d_residual,
+                         float* d_weight_partial, void* d_weight, int32_t dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------------
  * Softmax over the last dimension (what a load-balancing loss applies to the router logits the MoE layer returns)
