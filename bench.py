@@ -422,9 +422,9 @@ def secondary_hbm_kernels(dev):
 
     dt = timed(step5, iters=5)
     timer = scattermoe.LaunchTimer()
-    scattermoe.launch_timer = timer
+    scattermoe.set_launch_timer(timer)
     step5()
-    scattermoe.launch_timer = None
+    scattermoe.set_launch_timer(None)
     torch.cuda.synchronize()
     f5 = 6.0 * T5 * K5 * H5 * I5
     launches = {}
@@ -601,13 +601,13 @@ def main() -> int:
     torch.cuda.synchronize()
 
     timer = scattermoe.LaunchTimer()
-    scattermoe.launch_timer = timer
+    scattermoe.set_launch_timer(timer)
     t0 = time.perf_counter()
     for _ in range(args.steps):
         step(moe, x, grad_out)
     torch.cuda.synchronize()
     dt = (time.perf_counter() - t0) / args.steps
-    scattermoe.launch_timer = None
+    scattermoe.set_launch_timer(None)
 
     R = T * TOP_K
     flops_step = 18.0 * R * H * I

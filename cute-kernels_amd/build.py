@@ -3,7 +3,8 @@
     python cute-kernels_amd/build.py [--jobs N] [--force] [--define NAME=VALUE ...] [--output FILE.so]
 
 Every translation unit under csrc/ is compiled with hipcc to an object file (in parallel) and linked into
-cute_kernels/libck_mi355.so. Nothing is compiled at import time: the package only ever dlopens the result.
+cute_kernels/libck_mi355.so; csrc/host is compiled with g++ into cute_kernels/_ck_host.so, the Python package's native
+host side. Nothing is compiled at import time: the package only ever dlopens the result.
 
 Measurement builds: `--define CK_ABLATE=2 --output /some/dir/libck_ablate2.so` compiles the same sources with the given
 preprocessor definitions into an object directory of their own and links the library where --output says (outside
@@ -24,6 +25,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(ROOT, "csrc")
 INCLUDE = os.path.join(os.path.dirname(ROOT), "include")
 OBJ_DIR = os.path.join(ROOT, "build")
+HOST_SOURCE = os.path.join(CSRC, "host", "host_ops.cpp")
+HOST_PATH = os.path.join(ROOT, "cute_kernels", "_ck_host.so")
 LIB_PATH = os.path.join(ROOT, "cute_kernels", "libck_mi355.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -58,6 +61,35 @@ def _compile(src: str, force: bool, defines: tuple[str, ...] = (), obj_dir: str 
     return obj
 
 
+def _host_command(output: str) -> list[str]:
+    """g++ line of the native host module (csrc/host): plain C++ against torch's headers, no device code."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = os.path.dirname(torch.__file__)
+    include = os.path.join(torch_dir, "include")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_EXTENSION_NAME=_ck_host"]
+    for d in (INCLUDE, include, os.path.join(include, "torch", "csrc", "api", "include"), "/opt/rocm/include",
+              sysconfig.get_paths()["include"]):
+        cmd += ["-I", d]
+    lib = os.path.join(torch_dir, "lib")
+    return cmd + [HOST_SOURCE, "-o", output, "-L", lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+                  "-ldl", f"-Wl,-rpath,{lib}"]
+
+
+def build_host(force: bool = False) -> str:
+    header = os.path.join(INCLUDE, "ck_mi355.h")
+    if not force and os.path.exists(HOST_PATH):
+        if os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(HOST_SOURCE), os.path.getmtime(header)):
+            return HOST_PATH
+    proc = subprocess.run(_host_command(HOST_PATH), capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on {HOST_SOURCE}:\n{proc.stdout}\n{proc.stderr}")
+    return HOST_PATH
+
+
 def build(jobs: int = 8, force: bool = False, defines: tuple[str, ...] = (), output: str | None = None) -> str:
     if defines and not output:
         raise ValueError("a build with --define needs its own --output name: the product library takes no definitions")
@@ -68,7 +100,10 @@ def build(jobs: int = 8, force: bool = False, defines: tuple[str, ...] = (), out
     os.makedirs(os.path.dirname(lib_path), exist_ok=True)
     os.makedirs(obj_dir, exist_ok=True)
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
+        host = None if output else pool.submit(build_host, force)  # measurement builds share the product's host module
         objs = list(pool.map(lambda s: _compile(s, force, tuple(defines), obj_dir), _sources()))
+        if host is not None:
+            host.result()
     cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", lib_path, *objs]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -166,9 +166,7 @@ static int route_impl(const char* name, const void* logits, int32_t dtype, int64
 
 extern "C" int ck_route_topk_softmax(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,
                                      int32_t* selected, float* gates, void* topk_values, void* stream) {
-  const char* name = "ck_route_topk_softmax";
-  CK_REQUIRE(T <= 0 || (selected && gates), "%s: logits, selected and gates are required", name);
-  return route_impl(name, logits, dtype, T, E, k, selected, nullptr, gates, nullptr, topk_values, stream);
+  return route_impl("ck_route_topk_softmax", logits, dtype, T, E, k, selected, nullptr, gates, nullptr, topk_values, stream);
 }
 
 extern "C" int ck_route_topk_softmax_all(const void* logits, int32_t dtype, int64_t T, int32_t E, int32_t k,

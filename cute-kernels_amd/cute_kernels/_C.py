@@ -160,6 +160,24 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host module (csrc/host): output allocation, launches and autograd nodes of the eager path. Built next to
+    the library; loaded, and pointed at the library, on first use."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _ck_host
+        except ImportError as e:
+            raise RuntimeError(f"the native host module is not built ({e}). Run `python cute-kernels_amd/build.py`.") from e
+        _ck_host.init(_LIB_PATH)
+        _host = _ck_host
+    return _host
+
+
 def check(rc: int) -> None:
     if rc != 0:
         raise RuntimeError(lib().ck_last_error_string().decode())
@@ -189,20 +207,3 @@ def require_gpu(*tensors: torch.Tensor) -> None:
 
 def stream() -> int:
     return torch.cuda.current_stream().cuda_stream
-
-
-_zero_workspaces: dict = {}
-
-
-def zero_workspace(device: torch.device, words: int, kind: str) -> torch.Tensor:
-    """A uint32 workspace that starts all-zero; the kernels using it restore the words they require to be zero.
-
-    One buffer per (kind, device, stream): calls on one stream are ordered, calls on different streams never share
-    it, and kernels with different zero-invariants (kind) never share it either.
-    """
-    key = (kind, device.index, stream())
-    buf = _zero_workspaces.get(key)
-    if buf is None or buf.numel() < words:
-        buf = torch.zeros(max(words, 1 << 16), dtype=torch.int32, device=device)
-        _zero_workspaces[key] = buf
-    return buf

@@ -18,12 +18,7 @@ from torch import Tensor
 from torch.library import custom_op
 
 from . import _C
-from . import continuous_count as _count
-from . import fused_residual_add_rmsnorm as _frn
-from . import rmsnorm as _rms
 from . import scattermoe as _moe
-from . import softmax as _softmax
-from . import swiglu as _swiglu
 
 NS = "ck_mi355"
 
@@ -56,7 +51,7 @@ def _or_empty(t, like, dtype=None):
 # ---------------------------------------------------------------------------------------------------------------
 @custom_op(f"{NS}::continuous_count", mutates_args=())
 def continuous_count(x: Tensor, size: int) -> Tensor:
-    return _count._launch(x, size, want_offsets=False)[0]
+    return _C.host().count(x, size, False)[0]
 
 
 @continuous_count.register_fake
@@ -69,7 +64,7 @@ def _(x, size):
 # ---------------------------------------------------------------------------------------------------------------
 @custom_op(f"{NS}::swiglu", mutates_args=())
 def swiglu(gate: Tensor, up: Tensor) -> Tensor:
-    return _swiglu._Swiglu_Cute.forward(_Ctx(), gate, up)
+    return _C.host().swiglu_forward(gate, up)
 
 
 @swiglu.register_fake
@@ -79,9 +74,7 @@ def _(gate, up):
 
 @custom_op(f"{NS}::swiglu_backward", mutates_args=())
 def swiglu_backward(gate: Tensor, up: Tensor, output_grad: Tensor) -> tuple[Tensor, Tensor]:
-    ctx = _Ctx()
-    ctx.saved_tensors = (gate.contiguous(), up.contiguous())
-    return _swiglu._Swiglu_Cute.backward(ctx, output_grad)
+    return _C.host().swiglu_backward(gate, up, output_grad)
 
 
 @swiglu_backward.register_fake
@@ -105,7 +98,7 @@ swiglu.register_autograd(_swiglu_bwd, setup_context=_swiglu_setup)
 
 @custom_op(f"{NS}::swiglu_packed", mutates_args=())
 def swiglu_packed(x: Tensor) -> Tensor:
-    return _swiglu._SwigluPacked_Cute.forward(_Ctx(), x)
+    return _C.host().swiglu_packed_forward(x)
 
 
 @swiglu_packed.register_fake
@@ -115,9 +108,7 @@ def _(x):
 
 @custom_op(f"{NS}::swiglu_packed_backward", mutates_args=())
 def swiglu_packed_backward(x: Tensor, output_grad: Tensor) -> Tensor:
-    ctx = _Ctx()
-    ctx.saved_tensors = (x.contiguous(),)
-    return _swiglu._SwigluPacked_Cute.backward(ctx, output_grad)
+    return _C.host().swiglu_packed_backward(x, output_grad)
 
 
 @swiglu_packed_backward.register_fake
@@ -141,9 +132,8 @@ swiglu_packed.register_autograd(_swiglu_packed_bwd, setup_context=_swiglu_packed
 # ---------------------------------------------------------------------------------------------------------------
 @custom_op(f"{NS}::rmsnorm", mutates_args=())
 def rmsnorm(x: Tensor, weight: Optional[Tensor], eps: float, memory_efficient: bool) -> tuple[Tensor, Tensor]:
-    ctx = _Ctx()
-    y = _rms._RMSNorm_Cute.forward(ctx, x, weight, eps, memory_efficient)
-    return y, _or_empty(ctx.saved_tensors[2], x, torch.float32)
+    y, rstd = _C.host().rmsnorm_forward(x, weight, eps, not memory_efficient)
+    return y, _or_empty(rstd, x, torch.float32)
 
 
 @rmsnorm.register_fake
@@ -156,10 +146,9 @@ def _(x, weight, eps, memory_efficient):
 def rmsnorm_backward(
     x: Tensor, weight: Optional[Tensor], rstd: Tensor, output_grad: Tensor, eps: float, memory_efficient: bool
 ) -> tuple[Tensor, Tensor]:
-    ctx = _Ctx()
-    ctx.saved_tensors = (x.contiguous(), weight, None if memory_efficient else rstd)
-    ctx.eps = eps
-    x_grad, weight_grad, _, _ = _rms._RMSNorm_Cute.backward(ctx, output_grad)
+    x_grad, _, weight_grad = _C.host().rmsnorm_backward(
+        x, weight, None if memory_efficient else rstd, output_grad, None, eps, 1.0, False
+    )
     return x_grad, _or_empty(weight_grad, x)
 
 
@@ -190,9 +179,8 @@ rmsnorm.register_autograd(_rmsnorm_bwd, setup_context=_rmsnorm_setup)
 def fused_residual_add_rmsnorm(
     x: Tensor, residual: Tensor, weight: Optional[Tensor], eps: float, multiplier: float, memory_efficient: bool
 ) -> tuple[Tensor, Tensor, Tensor]:
-    ctx = _Ctx()
-    y, added = _frn._FusedResidualAddRMSNorm_Cute.forward(ctx, x, residual, weight, eps, multiplier, memory_efficient)
-    return y, added, _or_empty(ctx.saved_tensors[2], x, torch.float32)
+    y, added, rstd = _C.host().residual_rmsnorm_forward(x, residual, weight, eps, multiplier, not memory_efficient)
+    return y, added, _or_empty(rstd, x, torch.float32)
 
 
 @fused_residual_add_rmsnorm.register_fake
@@ -216,11 +204,10 @@ def fused_residual_add_rmsnorm_backward(
     multiplier: float,
     memory_efficient: bool,
 ) -> tuple[Tensor, Tensor, Tensor]:
-    ctx = _Ctx()
-    ctx.saved_tensors = (added, weight, None if memory_efficient else rstd)
-    ctx.eps, ctx.multiplier = eps, multiplier
-    ctx.separate_outputs = True  # an operator's outputs may not alias each other
-    x_grad, residual_grad, weight_grad, *_ = _frn._FusedResidualAddRMSNorm_Cute.backward(ctx, output_grad, added_grad)
+    # two buffers, whatever the multiplier: an operator's outputs may not alias each other
+    x_grad, residual_grad, weight_grad = _C.host().rmsnorm_backward(
+        added, weight, None if memory_efficient else rstd, output_grad, added_grad, eps, multiplier, True
+    )
     return x_grad, residual_grad, _or_empty(weight_grad, added)
 
 
@@ -255,7 +242,7 @@ fused_residual_add_rmsnorm.register_autograd(_frn_bwd, setup_context=_frn_setup)
 # ---------------------------------------------------------------------------------------------------------------
 @custom_op(f"{NS}::softmax", mutates_args=())
 def softmax(x: Tensor, multiplier: float) -> Tensor:
-    return _softmax._Softmax_Cute.forward(_Ctx(), x, multiplier)
+    return _C.host().softmax_forward(x, multiplier)
 
 
 @softmax.register_fake
@@ -265,10 +252,7 @@ def _(x, multiplier):
 
 @custom_op(f"{NS}::softmax_backward", mutates_args=())
 def softmax_backward(output: Tensor, output_grad: Tensor, multiplier: float) -> Tensor:
-    ctx = _Ctx()
-    ctx.saved_tensors = (output,)
-    ctx.multiplier = multiplier
-    return _softmax._Softmax_Cute.backward(ctx, output_grad)[0]
+    return _C.host().softmax_backward(output, output_grad, multiplier)
 
 
 @softmax_backward.register_fake
@@ -294,9 +278,7 @@ softmax.register_autograd(_softmax_bwd, setup_context=_softmax_setup)
 @custom_op(f"{NS}::route_topk_softmax", mutates_args=())
 def route_topk_softmax(logits: Tensor, k: int) -> tuple[Tensor, Tensor]:
     """(gates fp32 [T, k], selected int32 [T, k])"""
-    ctx = _Ctx()
-    _moe._RouteTopKSoftmax.forward(ctx, logits, k)
-    return ctx.saved_tensors
+    return _C.host().route_forward(logits, k)
 
 
 @route_topk_softmax.register_fake
@@ -307,10 +289,7 @@ def _(logits, k):
 
 @custom_op(f"{NS}::route_topk_softmax_backward", mutates_args=())
 def route_topk_softmax_backward(gates: Tensor, selected: Tensor, gates_grad: Tensor, num_experts: int, like: Tensor) -> Tensor:
-    ctx = _Ctx()
-    ctx.saved_tensors = (gates, selected)
-    ctx.E, ctx.dtype = num_experts, like.dtype
-    return _moe._RouteTopKSoftmax.backward(ctx, gates_grad, None)[0]
+    return _C.host().route_backward(gates, selected, gates_grad, num_experts, like)
 
 
 @route_topk_softmax_backward.register_fake
@@ -381,13 +360,14 @@ def swiglu_experts(
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(out [T, H], pre [max_rows, 2I], the activation for d_w_proj ([I, max_rows] transposed, or [max_rows, I] when the
     weight gradients read row-major operands) or empty, expanded [T * k, H])"""
-    ctx = _Ctx((need_x, need_fc, need_proj, need_gates, False))
     seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    out = _moe._SwigluExperts.forward(ctx, x, w_fc, w_proj, gates, seg, act_kind)
-    if not ctx.saved_tensors:
+    keep = need_x or need_fc or need_proj or need_gates
+    out, pre, act, expanded = _C.host().swiglu_experts_forward(
+        x, w_fc, w_proj, gates, seg, act_kind, keep, need_proj, _moe._flags()
+    )
+    if not keep:
         return out, x.new_empty(0), x.new_empty(0), x.new_empty(0)
-    pre, act_t, expanded = ctx.saved_tensors[4:]
-    return out, pre, _or_empty(act_t, x), expanded
+    return out, pre, _or_empty(act, x), expanded
 
 
 @swiglu_experts.register_fake
@@ -414,13 +394,11 @@ def swiglu_experts_backward(
     seg_starts: Tensor, counts: Tensor, tile_expert: Tensor, row_slot: Tensor, max_rows: int, num_experts: int, align: int,
     need_x: bool, need_fc: bool, need_proj: bool, need_gates: bool, act_kind: int,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    ctx = _Ctx((need_x, need_fc, need_proj, need_gates, False))
-    ctx.act_kind = act_kind
-    ctx.seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    ctx.saved_tensors = (
-        x.contiguous(), w_fc.contiguous(), w_proj.contiguous(), gates.contiguous(), pre, act_t if need_proj else None, expanded,
+    seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
+    d_x, d_w_fc, d_w_proj, d_gates = _C.host().swiglu_experts_backward(
+        grad_out, x, w_fc, w_proj, gates, pre, act_t if need_proj else None, expanded, seg, act_kind, need_x, need_fc,
+        need_proj, need_gates, _moe._flags(),
     )
-    d_x, d_w_fc, d_w_proj, d_gates = _moe._SwigluExperts.backward(ctx, grad_out)[:4]
     return _or_empty(d_x, x), _or_empty(d_w_fc, x), _or_empty(d_w_proj, x), _or_empty(d_gates, x)
 
 
@@ -459,7 +437,7 @@ def experts_up(
     max_rows: int, num_experts: int, align: int, k: int,
 ) -> Tensor:
     seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    return _moe._ExpertsUp.forward(_Ctx(), x, w, seg, k, bias)
+    return _C.host().experts_up_forward(x, w, bias, seg, k, False, _moe._flags())[0]
 
 
 @experts_up.register_fake
@@ -472,10 +450,8 @@ def experts_up_backward(
     d_y: Tensor, x: Tensor, w: Tensor, seg_starts: Tensor, counts: Tensor, tile_expert: Tensor, row_slot: Tensor,
     max_rows: int, num_experts: int, align: int, k: int, need_x: bool, need_w: bool, need_bias: bool,
 ) -> tuple[Tensor, Tensor, Tensor]:
-    ctx = _Ctx((need_x, need_w, False, False, need_bias))
-    ctx.seg, ctx.k = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align), k
-    ctx.saved_tensors = (x.contiguous(), w.contiguous())
-    d_x, d_w, _, _, d_bias = _moe._ExpertsUp.backward(ctx, d_y)[:5]
+    seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
+    d_x, d_w, d_bias = _C.host().experts_up_backward(d_y, x, w, None, seg, k, need_x, need_w, need_bias, _moe._flags())
     return _or_empty(d_x, x), _or_empty(d_w, x), _or_empty(d_bias, x)
 
 
@@ -510,10 +486,9 @@ def experts_up_gelu(
     max_rows: int, num_experts: int, align: int, k: int,
 ) -> tuple[Tensor, Tensor]:
     """(gelu_tanh(y) [max_rows, N], y [max_rows, N]): the c_fc GEMM with the activation in its epilogue"""
-    ctx = _Ctx()
     seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    act = _moe._ExpertsUp.forward(ctx, x, w, seg, k, bias, True)
-    return act, ctx.saved_tensors[2]
+    y, act = _C.host().experts_up_forward(x, w, bias, seg, k, True, _moe._flags())
+    return act, y
 
 
 @experts_up_gelu.register_fake
@@ -526,10 +501,8 @@ def experts_up_gelu_backward(
     d_act: Tensor, pre: Tensor, x: Tensor, w: Tensor, seg_starts: Tensor, counts: Tensor, tile_expert: Tensor,
     row_slot: Tensor, max_rows: int, num_experts: int, align: int, k: int, need_x: bool, need_w: bool, need_bias: bool,
 ) -> tuple[Tensor, Tensor, Tensor]:
-    ctx = _Ctx((need_x, need_w, False, False, need_bias, False))
-    ctx.seg, ctx.k, ctx.gelu = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align), k, True
-    ctx.saved_tensors = (x.contiguous(), w.contiguous(), pre)
-    d_x, d_w, _, _, d_bias = _moe._ExpertsUp.backward(ctx, d_act)[:5]
+    seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
+    d_x, d_w, d_bias = _C.host().experts_up_backward(d_act, x, w, pre, seg, k, need_x, need_w, need_bias, _moe._flags())
     return _or_empty(d_x, x), _or_empty(d_w, x), _or_empty(d_bias, x)
 
 
@@ -564,10 +537,8 @@ def experts_down(
     counts: Tensor, tile_expert: Tensor, row_slot: Tensor, max_rows: int, num_experts: int, align: int,
 ) -> tuple[Tensor, Tensor]:
     """(out [T, N], expanded [T * k, N])"""
-    ctx = _Ctx()
     seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    out = _moe._ExpertsDown.forward(ctx, h, w, gates, seg, bias, slot_expert)
-    return out, ctx.saved_tensors[3]
+    return _C.host().experts_down_forward(h, w, gates, bias, slot_expert, seg, _moe._flags())
 
 
 @experts_down.register_fake
@@ -582,10 +553,10 @@ def experts_down_backward(
     tile_expert: Tensor, row_slot: Tensor, max_rows: int, num_experts: int, align: int, need_h: bool, need_w: bool,
     need_gates: bool, need_bias: bool,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    ctx = _Ctx((need_h, need_w, need_gates, False, need_bias))
-    ctx.seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
-    ctx.saved_tensors = (h.contiguous(), w.contiguous(), gates.contiguous(), expanded)
-    d_h, d_w, d_gates, _, d_bias = _moe._ExpertsDown.backward(ctx, grad_out)[:5]
+    seg = _segments(seg_starts, counts, tile_expert, row_slot, max_rows, num_experts, align)
+    d_h, d_w, d_gates, d_bias = _C.host().experts_down_backward(
+        grad_out, h, w, gates, expanded, seg, need_h, need_w, need_gates, need_bias, _moe._flags()
+    )
     return _or_empty(d_h, h), _or_empty(d_w, h), _or_empty(d_gates, h), _or_empty(d_bias, h)
 
 

@@ -7,14 +7,11 @@ torch_implementation.py:63-201) evaluated on the de-quantised operands". Routing
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 import torch.nn as nn
 
 from . import _C
-from . import scattermoe
-from .scattermoe import ExpertSegments, _combine, choose_align, route_topk_softmax, sort_by_expert
+from .scattermoe import ExpertSegments, choose_align, route_topk_softmax, sort_by_expert
 
 
 E4M3_MAX = 448.0
@@ -24,17 +21,8 @@ E4M3_MAX = 448.0
 def quantize_rows_e4m3(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """x [rows, cols] bf16 / fp16 -> (q [rows, cols] torch.float8_e4m3fn, scale [rows] fp32) with
     q = e4m3(x * (448 / amax_row)) and scale = amax_row / 448, so that x ~= q.float() * scale[:, None]."""
-    _C.require_gpu(x)
     assert x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16)
-    x = x.contiguous()
-    rows, cols = x.shape
-    q = torch.empty(rows, cols, dtype=torch.float8_e4m3fn, device=x.device)
-    scale = torch.empty(rows, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        _C.check(
-            _C.lib().ck_quant_rows_e4m3(_C.ptr(x), rows, cols, _C.ptr(q), _C.ptr(scale), _C.dtype_code(x.dtype), _C.stream())
-        )
-    return q, scale
+    return _C.host().quantize_rows(x)
 
 
 @torch.no_grad()
@@ -46,27 +34,10 @@ def quantize_expert_weights_e4m3(weight: torch.Tensor) -> tuple[torch.Tensor, to
 
 
 def _gemm_fp8(a8, a_scale, gather_div, w8, w_scale, seg: ExpertSegments, epilogue, y, aux, out_dtype):
-    E, N, K = w8.shape
-    cs = seg.c_struct()
-    if gather_div > 0:  # gathered rows are addressed with 32-bit byte offsets from the start of the token-order tensor
-        assert a8.numel() < 2**32, "the token-order fp8 input of a grouped GEMM must stay below 4 GiB"
-
-    def launch():
-        with torch.cuda.device(w8.device):
-            _C.check(
-                _C.lib().ck_grouped_gemm_fp8(
-                    _C.ptr(a8), _C.ptr(a_scale), gather_div, _C.ptr(w8), _C.ptr(w_scale), N, K, ctypes.byref(cs),
-                    epilogue, _C.ptr(y), _C.ptr(aux), _C.dtype_code(out_dtype), _C.stream(),
-                )
-            )
-
-    if scattermoe.launch_timer is None:
-        launch()
-    else:
-        scattermoe.launch_timer.time("fp8_" + scattermoe._EPILOGUE_NAMES[epilogue], (N, K), launch)
+    like = torch.empty(0, dtype=out_dtype, device=w8.device)
+    _C.host().gemm_fp8(a8, a_scale, gather_div, w8, w_scale, seg, epilogue, y, aux, like)
 
 
-@torch.no_grad()
 def swiglu_experts_e4m3(
     x: torch.Tensor,
     w_fc8: torch.Tensor,
@@ -84,18 +55,8 @@ def swiglu_experts_e4m3(
     x_quantized: (x8, scale) = quantize_rows_e4m3(x) if the caller has it already (rmsnorm_route_cute(..., quantize=True)).
     """
     assert seg.align in (16, 32, 64, 256), "the fp8 GEMMs have tiles of 16, 32, 64 and 256 rows: sort_by_expert(..., align=256)"
-    T, H = x.shape
-    k = gates.size(1)
-    E, two_i, _ = w_fc8.shape
-    I = two_i // 2
-    x8, x_scale = quantize_rows_e4m3(x) if x_quantized is None else x_quantized  # per token
-    act = torch.empty(seg.max_rows, I, dtype=x.dtype, device=x.device)  # pad rows: never written, quantised, never used
-    _gemm_fp8(x8, x_scale, k, w_fc8, w_fc_scale, seg, _C.CK_EPI_SWIGLU, None, act, x.dtype)
-    act8, act_scale = quantize_rows_e4m3(act)  # per routed row
-    expanded = torch.empty(T * k, H, dtype=x.dtype, device=x.device)
-    _gemm_fp8(act8, act_scale, 0, w_proj8, w_proj_scale, seg, _C.CK_EPI_SCATTER, expanded, None, x.dtype)
-    out, _ = _combine(expanded, gates.to(x.dtype).contiguous(), T, k, H)
-    return out
+    x8, x_scale = (None, None) if x_quantized is None else x_quantized
+    return _C.host().swiglu_experts_e4m3(x, w_fc8, w_fc_scale, w_proj8, w_proj_scale, gates, seg, x8, x_scale)
 
 
 class MoE_E4M3(nn.Module):

@@ -34,84 +34,18 @@ class Options:
 options = Options()
 
 
+def _flags() -> int:
+    """options as the native host module takes them (csrc/host/host_ops.cpp: Flags)"""
+    return options.gemm_split | options.bias_fused << 1 | options.gemm_nn << 2 | options.dw_rows << 3
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # routing
 # ---------------------------------------------------------------------------------------------------------------
-class _GateGradSlot:
-    """Side channel between the expert block's backward and the router's backward. Autograd hands a 16-bit gates tensor
-    a 16-bit gradient; the softmax backward then subtracts nearly equal rounded numbers and gate.weight.grad loses
-    digits. The expert block leaves its unrounded fp32 d_gates here, and the router's backward uses it when the gradient
-    it receives is exactly that tensor rounded (i.e. nothing else contributed to the gates' gradient)."""
-
-    __slots__ = ("d_gates_f32",)
-
-    def __init__(self):
-        self.d_gates_f32 = None
-
-
 def _gate_slot(gates: torch.Tensor):
+    """The side channel the router attached to these gates, if any: through it the expert block's backward hands the router's
+    its unrounded gate gradient (GateSlot in csrc/host/host_ops.cpp)."""
     return getattr(gates, "_ck_gate_slot", None)
-
-
-class _RouteTopKSoftmax(torch.autograd.Function):
-    """logits [T, E] -> gates [T, k] (softmax over the k largest logits, in logits.dtype), selected [T, k] int64."""
-
-    @staticmethod
-    def forward(ctx, logits: torch.Tensor, k: int, long_indices: bool = True, slot: _GateGradSlot | None = None):
-        _C.require_gpu(logits)
-        logits = logits.contiguous()
-        T, E = logits.shape
-        selected = torch.empty(T, k, dtype=torch.int32, device=logits.device)
-        gates = torch.empty(T, k, dtype=torch.float32, device=logits.device)
-        selected_long = torch.empty(T, k, dtype=torch.int64, device=logits.device) if long_indices else None
-        rounded = torch.empty(T, k, dtype=logits.dtype, device=logits.device) if logits.dtype != torch.float32 else None
-        with torch.cuda.device(logits.device):
-            _C.check(
-                _C.lib().ck_route_topk_softmax_all(
-                    _C.ptr(logits), _C.dtype_code(logits.dtype), T, E, k, _C.ptr(selected), _C.ptr(selected_long), _C.ptr(gates),
-                    _C.ptr(rounded), _C.stream(),
-                )
-            )
-        ctx.save_for_backward(gates, selected)
-        ctx.E = E
-        ctx.dtype = logits.dtype
-        ctx.slot = slot
-        selected_out = selected_long if long_indices else selected
-        ctx.mark_non_differentiable(selected_out)
-        ctx.set_materialize_grads(False)  # no zero-filled gradient for the selection
-        return gates if rounded is None else rounded, selected_out
-
-    @staticmethod
-    def backward(ctx, d_gates: torch.Tensor, _d_selected):
-        if d_gates is None:
-            return None, None, None, None
-        gates, selected = ctx.saved_tensors
-        T, k = gates.shape
-        exact = ctx.slot.d_gates_f32 if ctx.slot is not None else None
-        d_logits = torch.empty(T, ctx.E, dtype=ctx.dtype, device=gates.device)
-        lib = _C.lib()
-        if exact is not None and exact.shape == d_gates.shape and d_gates.dtype == ctx.dtype != torch.float32:
-            # the unrounded gradient wherever what arrived is that gradient rounded (decided per element inside the
-            # kernel: no host sync, no extra launches)
-            ctx.slot.d_gates_f32 = None
-            d_gates = d_gates.contiguous()
-            with torch.cuda.device(gates.device):
-                _C.check(
-                    lib.ck_route_topk_softmax_bwd_exact(
-                        _C.ptr(gates), _C.ptr(exact), _C.ptr(d_gates), _C.ptr(selected), T, ctx.E, k, _C.ptr(d_logits),
-                        _C.dtype_code(ctx.dtype), _C.stream(),
-                    )
-                )
-            return d_logits, None, None, None
-        d_gates = d_gates.float().contiguous()
-        with torch.cuda.device(gates.device):
-            _C.check(
-                lib.ck_route_topk_softmax_bwd(
-                    _C.ptr(gates), _C.ptr(d_gates), _C.ptr(selected), T, ctx.E, k, _C.ptr(d_logits),
-                    _C.dtype_code(ctx.dtype), _C.stream(),
-                )
-            )
-        return d_logits, None, None, None
 
 
 def route_topk_softmax(logits: torch.Tensor, k: int, long_indices: bool = True) -> tuple[torch.Tensor, torch.Tensor]:
@@ -121,9 +55,10 @@ def route_topk_softmax(logits: torch.Tensor, k: int, long_indices: bool = True) 
     if is_tracing():
         gates, selected = _ops.route_topk_softmax(logits, k)
         return gates.to(logits.dtype), (selected.long() if long_indices else selected)
-    slot = _GateGradSlot()
-    gates, selected = _RouteTopKSoftmax.apply(logits, k, long_indices, slot)
-    gates._ck_gate_slot = slot  # found again by the expert block that consumes these gates (see _GateGradSlot)
+    host = _C.host()
+    slot = host.GateSlot()
+    gates, selected = host.route(logits, k, long_indices, slot)
+    gates._ck_gate_slot = slot  # found again by the expert block that consumes these gates
     return gates, selected
 
 
@@ -218,7 +153,6 @@ def choose_align(
     return 256
 
 
-@torch.no_grad()
 def sort_by_expert(
     expert_ids: torch.Tensor, num_experts: int, align: int | None = None, validate: bool = False
 ) -> ExpertSegments:
@@ -245,37 +179,8 @@ def sort_by_expert(
 
 
 def _sort_by_expert_eager(expert_ids: torch.Tensor, num_experts: int, align: int) -> ExpertSegments:
-    _C.require_gpu(expert_ids)
-    ids = expert_ids.contiguous().view(-1)
-    R = ids.numel()
-    lib = _C.lib()
-    dev = ids.device
-    max_rows = lib.ck_sort_max_rows(R, num_experts, align)
-    i32 = dict(dtype=torch.int32, device=dev)
-    u32 = dict(dtype=torch.uint32, device=dev)
-    seg = ExpertSegments(
-        sorted_expert_idxs=torch.empty(R, **i32),
-        sorted_scattered_idxs=torch.empty(R, **i32),
-        counts=torch.empty(num_experts, **u32),
-        ends=torch.empty(num_experts, **u32),
-        starts=torch.empty(num_experts, **u32),
-        seg_starts=torch.empty(num_experts + 1, **i32),
-        row_slot=torch.empty(max(max_rows, 1), **i32),
-        tile_expert=torch.empty(max(max_rows // align, 1), **i32),
-        max_rows=max_rows,
-        num_experts=num_experts,
-        align=align,
-    )
-    ws = _C.zero_workspace(dev, lib.ck_sort_workspace_words(R, num_experts), "sort")
-    with torch.cuda.device(dev):
-        _C.check(
-            lib.ck_sort_by_expert(
-                _C.ptr(ids), int(ids.dtype == torch.long), R, num_experts, align, _C.ptr(seg.sorted_expert_idxs),
-                _C.ptr(seg.sorted_scattered_idxs), _C.ptr(seg.counts), _C.ptr(seg.ends), _C.ptr(seg.starts),
-                _C.ptr(seg.seg_starts), _C.ptr(seg.row_slot), _C.ptr(seg.tile_expert), _C.ptr(ws), _C.stream(),
-            )
-        )
-    return seg
+    *tables, max_rows = _C.host().sort_by_expert(expert_ids, num_experts, align)
+    return ExpertSegments(*tables, max_rows, num_experts, align)
 
 
 # ---------------------------------------------------------------------------------------------------------------
@@ -299,70 +204,25 @@ class LaunchTimer:
         self.records.append((name, dims, start, end))
 
 
-launch_timer: LaunchTimer | None = None
 
-_EPILOGUE_NAMES = {
-    _C.CK_EPI_GROUPED: "grouped_gemm<grouped>",
-    _C.CK_EPI_SCATTER: "grouped_gemm<scatter>",
-    _C.CK_EPI_SWIGLU: "grouped_gemm<swiglu>",
-    _C.CK_EPI_SWIGLU_BWD: "grouped_gemm<swiglu_bwd>",
-    _C.CK_EPI_GLU: "grouped_gemm<swiglu>",
-    _C.CK_EPI_GELU_TANH: "grouped_gemm<grouped>",
-}
-
-
-_split_workspaces: dict = {}
+def set_launch_timer(timer: LaunchTimer | None) -> None:
+    """Every expert GEMM launched from now on goes through timer.time (None: no timing)."""
+    _C.host().set_launch_timer(timer)
 
 
 def _split_workspace(device: torch.device) -> torch.Tensor:
-    """Workspace of ck_grouped_gemm_ws / ck_grouped_gemm_nn_ws (split last round of tiles): one buffer per device and
-    stream (launches that may overlap must not share one; it needs no initial contents)."""
-    if not options.gemm_split:
-        return None
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
-    ws = _split_workspaces.get(key)
-    if ws is None:
-        ws = _split_workspaces[key] = torch.empty(_C.lib().ck_grouped_gemm_workspace_bytes(), dtype=torch.uint8, device=device)
-    return ws
+    """Workspace of ck_grouped_gemm_ws / ck_grouped_gemm_nn_ws (split last round of tiles) on this device and stream."""
+    return _C.host().split_workspace(torch.empty(0, device=device))
 
 
 def _gemm_f32(a, gather_div, w, w_is_kn: bool, N: int, K: int, seg: ExpertSegments, scatter: bool, y, bias=None,
               rows_in=None, rows_out=None):
     """The grouped GEMMs of fp32 tensors (fp32 MFMA; see ck_grouped_gemm_f32)."""
-    cs = seg.c_struct(rows_in, rows_out)
-    with torch.cuda.device(w.device):
-        _C.check(
-            _C.lib().ck_grouped_gemm_f32(
-                _C.ptr(a), gather_div, _C.ptr(w), int(w_is_kn), N, K, ctypes.byref(cs), int(scatter), _C.ptr(y), _C.ptr(bias),
-                _C.stream(),
-            )
-        )
+    _C.host().gemm_f32(a, gather_div, w, w_is_kn, N, K, seg, scatter, y, bias, rows_in, rows_out)
 
 
 def _gemm(a, gather_div, w, seg: ExpertSegments, epilogue, y, y_t=None, aux=None, aux_in=None, rows_in=None, rows_out=None):
-    E, N, K = w.shape
-    if w.dtype == torch.float32:
-        assert epilogue in (_C.CK_EPI_GROUPED, _C.CK_EPI_SCATTER) and y_t is None and aux is None
-        return _gemm_f32(a, gather_div, w, False, N, K, seg, epilogue == _C.CK_EPI_SCATTER, y, aux_in, rows_in, rows_out)
-    cs = seg.c_struct(rows_in, rows_out)
-    if gather_div > 0:  # gathered rows are addressed with 32-bit byte offsets from the start of `a` (the library is not
-        # told how many rows `a` has, so this limit is checked here)
-        assert a.numel() * a.element_size() < 2**32, "the token-order input of a grouped GEMM must stay below 4 GiB"
-
-    def launch():
-        with torch.cuda.device(w.device):
-            ws = _split_workspace(w.device) if epilogue in (_C.CK_EPI_GROUPED, _C.CK_EPI_SCATTER) else None
-            _C.check(
-                _C.lib().ck_grouped_gemm_ws(
-                    _C.ptr(a), gather_div, _C.ptr(w), N, K, ctypes.byref(cs), epilogue, _C.ptr(y), _C.ptr(y_t), seg.ld_t,
-                    _C.ptr(aux), _C.ptr(aux_in), _C.dtype_code(w.dtype), _C.stream(), _C.ptr(ws), 0 if ws is None else ws.numel(),
-                )
-            )
-
-    if launch_timer is None:
-        launch()
-    else:
-        launch_timer.time(_EPILOGUE_NAMES[epilogue], (N, K), launch)
+    _C.host().gemm(a, gather_div, w, seg, epilogue, y, y_t, aux, aux_in, rows_in, rows_out, _flags())
 
 
 def _bias_in_epilogue(seg: ExpertSegments, K: int) -> bool:
@@ -380,72 +240,17 @@ def _fp32(t: torch.Tensor) -> bool:
 
 def _gemm_dx(d_y, w, seg: ExpertSegments, epilogue, out, rows_out=None):
     """out = d_y @ w[e] per expert, w [E, out_features, in_features] as the forward stores it: the input-gradient GEMM.
-    Reads w contraction-strided where the kernel for that exists (256-row tiles, out_features % 64 == 0); otherwise
-    through a transposed copy. rows_out: the table a scatter epilogue writes through (default seg.row_slot)."""
-    E, n_out, n_in = w.shape
-    if w.dtype == torch.float32:
-        return _gemm_f32(d_y, 0, w, True, n_in, n_out, seg, epilogue == _C.CK_EPI_SCATTER, out, None, None, rows_out)
-    if seg.align == 256 and n_out % 64 == 0 and options.gemm_nn:
-        cs = seg.c_struct(None, rows_out)
-
-        def launch():
-            with torch.cuda.device(w.device):
-                ws = _split_workspace(w.device)
-                _C.check(
-                    _C.lib().ck_grouped_gemm_nn_ws(
-                        _C.ptr(d_y), _C.ptr(w), n_in, n_out, ctypes.byref(cs), epilogue, _C.ptr(out), _C.dtype_code(w.dtype),
-                        _C.stream(), _C.ptr(ws), 0 if ws is None else ws.numel(),
-                    )
-                )
-
-        if launch_timer is None:
-            launch()
-        else:
-            launch_timer.time(_EPILOGUE_NAMES[epilogue].replace("grouped_gemm<", "grouped_gemm_nn<"), (n_in, n_out), launch)
-        return
-    _gemm(d_y, 0, _transpose_weights(w), seg, epilogue, out, rows_out=rows_out)
+    rows_out: the table a scatter epilogue writes through (default seg.row_slot)."""
+    _C.host().gemm_dx(d_y, w, seg, epilogue, out, rows_out, _flags())
 
 
 def _gemm_dw(a_t, b_t, seg: ExpertSegments, dw):
-    E, M, N = dw.shape
-    cs = seg.c_struct()
-
-    def launch():
-        with torch.cuda.device(dw.device):
-            _C.check(
-                _C.lib().ck_grouped_gemm_dw(
-                    _C.ptr(a_t), _C.ptr(b_t), seg.ld_t, M, N, ctypes.byref(cs), _C.ptr(dw), _C.dtype_code(dw.dtype),
-                    _C.stream(),
-                )
-            )
-
-    if launch_timer is None:
-        launch()
-    else:
-        launch_timer.time("grouped_gemm<dw>", (M, N), launch)
+    _C.host().gemm_dw(a_t, b_t, seg, dw)
 
 
 def _gemm_dw_rows(a, b, seg: ExpertSegments, dw):
     """dw[e] = a[rows of e]^T @ b[rows of e] from row-major padded-grouped operands (no transposed copies)."""
-    E, M, N = dw.shape
-    cs = seg.c_struct()
-    if dw.dtype == torch.float32:
-        with torch.cuda.device(dw.device):
-            _C.check(_C.lib().ck_grouped_gemm_dw_f32(_C.ptr(a), _C.ptr(b), M, N, ctypes.byref(cs), _C.ptr(dw), _C.stream()))
-        return
-
-    def launch():
-        with torch.cuda.device(dw.device):
-            _C.check(
-                _C.lib().ck_grouped_gemm_dw_rows(
-                    _C.ptr(a), _C.ptr(b), M, N, ctypes.byref(cs), _C.ptr(dw), _C.dtype_code(dw.dtype), _C.stream()
-                )
-            )
-
-    if launch_timer is None:
-        launch()
-    else:
-        launch_timer.time("grouped_gemm_dw_rows", (M, N), launch)
+    _C.host().gemm_dw_rows(a, b, seg, dw)
 
 
 def _dw_from_rows(max_rows: int, num_experts: int, align: int, *shapes: tuple[int, int]) -> bool:
@@ -460,26 +265,11 @@ def _dw_from_rows(max_rows: int, num_experts: int, align: int, *shapes: tuple[in
 def _group_rows(src, coeff, fan_out, seg: ExpertSegments, want_grouped: bool, want_transposed: bool, rows=None):
     """Padded grouped copy of `src` rows (fan_out == 0: src is already padded-grouped) and / or its transpose. rows: the
     table the rows are read through (default seg.row_slot)."""
-    H = src.size(-1)
-    grouped = torch.empty(seg.max_rows, H, dtype=src.dtype, device=src.device) if want_grouped else None
-    grouped_t = torch.empty(H, seg.ld_t, dtype=src.dtype, device=src.device) if want_transposed else None
-    with torch.cuda.device(src.device):
-        _C.check(
-            _C.lib().ck_group_rows_padded(
-                _C.ptr(src), _C.ptr(coeff), fan_out, H, _C.ptr(seg.row_slot if rows is None else rows), _C.ptr(seg.seg_starts), _C.ptr(seg.counts),
-                _C.ptr(seg.tile_expert), seg.align, seg.max_rows, _C.ptr(grouped), _C.ptr(grouped_t), seg.ld_t,
-                _C.dtype_code(src.dtype), _C.stream(),
-            )
-        )
-    return grouped, grouped_t
+    return _C.host().group_rows(src, coeff, fan_out, seg, want_grouped, want_transposed, rows)
 
 
 def _transpose_weights(w: torch.Tensor) -> torch.Tensor:
-    E, N, K = w.shape
-    w_t = torch.empty(E, K, N, dtype=w.dtype, device=w.device)
-    with torch.cuda.device(w.device):
-        _C.check(_C.lib().ck_transpose_batched(_C.ptr(w), E, N, K, _C.ptr(w_t), _C.dtype_code(w.dtype), _C.stream()))
-    return w_t
+    return _C.host().transpose_weights(w)
 
 
 def _combine(expanded, gates, T, k, H, grad_out=None, want_out=True, want_d_gates=False):
@@ -497,19 +287,8 @@ def _combine(expanded, gates, T, k, H, grad_out=None, want_out=True, want_d_gate
 
 def _gate_grad(expanded, grad_out, T, k, H, gates_dtype, slot):
     """d_gates in fp32 (kept in `slot` for the router's backward) and rounded to the gates' dtype for autograd."""
-    d32 = torch.empty(T, k, dtype=torch.float32, device=expanded.device)
-    rounded = torch.empty(T, k, dtype=gates_dtype, device=expanded.device)
     assert gates_dtype == expanded.dtype, "gates and expert outputs should have the same dtype"
-    with torch.cuda.device(expanded.device):
-        _C.check(
-            _C.lib().ck_gate_grad_both(
-                _C.ptr(expanded), _C.ptr(grad_out), T, k, H, _C.ptr(d32), _C.ptr(rounded), _C.dtype_code(expanded.dtype),
-                _C.stream(),
-            )
-        )
-    if slot is not None:
-        slot.d_gates_f32 = d32
-    return rounded
+    return _C.host().gate_grad(expanded, grad_out, T, k, H, slot)
 
 
 def gather_rows(src: torch.Tensor, idx: torch.Tensor, coeff: torch.Tensor | None = None, fan_out: int = 1) -> torch.Tensor:
@@ -529,27 +308,12 @@ def gather_rows(src: torch.Tensor, idx: torch.Tensor, coeff: torch.Tensor | None
 
 def _add_expert_bias(y: torch.Tensor, bias: torch.Tensor, seg: ExpertSegments, row_expert: torch.Tensor | None) -> None:
     """y[r] += bias[expert of row r] in place: padded grouped rows (row_expert None) or token-order rows."""
-    cs = seg.c_struct()
-    with torch.cuda.device(y.device):
-        _C.check(
-            _C.lib().ck_add_expert_bias(
-                _C.ptr(y), y.size(0), y.size(1), _C.ptr(bias), _C.ptr(row_expert), None if row_expert is not None else ctypes.byref(cs),
-                _C.dtype_code(y.dtype), _C.stream(),
-            )
-        )
+    _C.host().add_expert_bias(y, bias, seg, row_expert)
 
 
 def _expert_bias_grad(d_y: torch.Tensor, seg: ExpertSegments) -> torch.Tensor:
     """[E, N] column sums of the padded grouped rows of every expert."""
-    d_bias = torch.empty(seg.num_experts, d_y.size(1), dtype=d_y.dtype, device=d_y.device)
-    cs = seg.c_struct()
-    with torch.cuda.device(d_y.device):
-        _C.check(
-            _C.lib().ck_expert_bias_grad(
-                _C.ptr(d_y), d_y.size(1), ctypes.byref(cs), _C.ptr(d_bias), _C.dtype_code(d_y.dtype), _C.stream()
-            )
-        )
-    return d_bias
+    return _C.host().expert_bias_grad(d_y, seg)
 
 
 def _slot_experts(seg: ExpertSegments) -> torch.Tensor:
@@ -570,123 +334,6 @@ def _check_expert_dtypes(x: torch.Tensor, *weights: torch.Tensor) -> None:
 # ---------------------------------------------------------------------------------------------------------------
 # generic expert linears (any activation between them)
 # ---------------------------------------------------------------------------------------------------------------
-def _experts_up_forward(x, w, seg: ExpertSegments, k: int, bias, gelu: bool, keep_pre: bool, zero_pads: bool):
-    """(y, act): the c_fc output in padded grouped order and, with gelu, its activation (y None unless keep_pre). Pad rows
-    are never written by the kernel: zero_pads makes them zeros, which keeps whatever is applied on top of them finite.
-    Without it they hold anything, which the expert GEMMs and their backward pass do not mind: they read valid rows only."""
-    N, K = w.shape[1:]
-    new = torch.zeros if zero_pads else torch.empty
-    y = new(seg.max_rows, N, dtype=x.dtype, device=x.device) if keep_pre or not gelu else None
-    act = new(seg.max_rows, N, dtype=x.dtype, device=x.device) if gelu else None
-    fused_bias = bias is not None and (gelu or _fp32(x) or _bias_in_epilogue(seg, K))
-    _gemm(x, k, w, seg, _C.CK_EPI_GELU_TANH if gelu else _C.CK_EPI_GROUPED, y, aux=act,
-          aux_in=bias.contiguous() if fused_bias else None)
-    if bias is not None and not fused_bias:
-        _add_expert_bias(y, bias.contiguous(), seg, None)
-    return y, act
-
-
-class _ExpertsUp(torch.autograd.Function):
-    """x [T, H] (token order) -> y [max_rows, N] (padded grouped): the reference's c_fc with grouped_out=True.
-    gelu=True: returns gelu_tanh(y) instead, computed in the GEMM's epilogue from the rounded y (the activation module
-    applied to y would read the same values); y is kept for the backward pass only."""
-
-    @staticmethod
-    def forward(ctx, x, w, seg: ExpertSegments, k: int, bias=None, gelu: bool = False, zero_pads: bool = True):
-        x = x.contiguous()
-        w = w.contiguous()
-        y, act = _experts_up_forward(x, w, seg, k, bias, gelu, True, zero_pads)
-        ctx.gelu = gelu
-        if gelu:
-            ctx.save_for_backward(x, w, y)
-        else:
-            ctx.save_for_backward(x, w)
-        ctx.seg, ctx.k = seg, k
-        return act if gelu else y
-
-    @staticmethod
-    def backward(ctx, d_y):
-        x, w = ctx.saved_tensors[:2]
-        seg, k = ctx.seg, ctx.k
-        T, K = x.shape
-        d_y = d_y.contiguous()
-        if getattr(ctx, "gelu", False):  # d_y arrives as d_act: through the activation first
-            pre, d_act = ctx.saved_tensors[2], d_y
-            d_y = torch.empty_like(d_act)
-            with torch.cuda.device(d_act.device):
-                _C.check(_C.lib().ck_gelu_tanh_bwd(_C.ptr(pre), _C.ptr(d_act), _C.ptr(d_y), d_act.numel(),
-                                                   _C.dtype_code(d_act.dtype), _C.stream()))
-        d_x = d_w = d_bias = None
-        if len(ctx.needs_input_grad) > 4 and ctx.needs_input_grad[4]:
-            d_bias = _expert_bias_grad(d_y, seg)
-        if ctx.needs_input_grad[1]:
-            d_w = torch.empty_like(w)
-            if _fp32(x) or _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, tuple(w.shape[1:])):
-                x_g, _ = _group_rows(x, None, k, seg, True, False)
-                _gemm_dw_rows(d_y, x_g, seg, d_w)
-            else:
-                _, d_y_t = _group_rows(d_y, None, 0, seg, False, True)
-                _, x_t = _group_rows(x, None, k, seg, False, True)
-                _gemm_dw(d_y_t, x_t, seg, d_w)
-        if ctx.needs_input_grad[0]:
-            d_expanded = torch.empty(T * k, K, dtype=x.dtype, device=x.device)
-            _gemm_dx(d_y, w, seg, _C.CK_EPI_SCATTER, d_expanded)
-            d_x = d_expanded if k == 1 else _combine(d_expanded, None, T, k, K)[0]
-        return d_x, d_w, None, None, d_bias, None, None
-
-
-class _ExpertsDown(torch.autograd.Function):
-    """h [max_rows, I] (padded grouped), gates [T, k] -> out [T, H]: the reference's c_proj with grouped_in=True."""
-
-    @staticmethod
-    def forward(
-        ctx, h, w, gates, seg: ExpertSegments, bias=None, slot_expert=None, gate_slot=None, zero_pads: bool = True
-    ):
-        ctx.gate_slot, ctx.zero_pads = gate_slot, zero_pads
-        h = h.contiguous()
-        w = w.contiguous()
-        gates = gates.contiguous()
-        T, k = gates.shape
-        E, N, K = w.shape
-        expanded = torch.empty(T * k, N, dtype=h.dtype, device=h.device)
-        fused_bias = bias is not None and (_fp32(h) or _bias_in_epilogue(seg, K))
-        _gemm(h, 0, w, seg, _C.CK_EPI_SCATTER, expanded, aux_in=bias.contiguous() if fused_bias else None)
-        if bias is not None and not fused_bias:  # before the gate multiply, as torch_implementation.py:160-163
-            _add_expert_bias(expanded, bias.contiguous(), seg, slot_expert if slot_expert is not None else _slot_experts(seg))
-        out, _ = _combine(expanded, gates, T, k, N)
-        ctx.save_for_backward(h, w, gates, expanded)
-        ctx.seg = seg
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        h, w, gates, expanded = ctx.saved_tensors
-        seg = ctx.seg
-        T, k = gates.shape
-        E, N, K = w.shape
-        grad_out = grad_out.contiguous()
-        d_h = d_w = d_gates = d_bias = None
-        if ctx.needs_input_grad[2]:
-            d_gates = _gate_grad(expanded, grad_out, T, k, N, gates.dtype, ctx.gate_slot)
-        need_w = ctx.needs_input_grad[1]
-        rows_form = _fp32(h) or _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, (N, K))
-        d_y, d_y_t = _group_rows(grad_out, gates, k, seg, True, need_w and not rows_form)
-        if len(ctx.needs_input_grad) > 4 and ctx.needs_input_grad[4]:
-            d_bias = _expert_bias_grad(d_y, seg)  # d_y: the gate-scaled grad_out rows in padded grouped order
-        if need_w:
-            d_w = torch.empty_like(w)
-            if rows_form:
-                _gemm_dw_rows(d_y, h, seg, d_w)
-            else:
-                _, h_t = _group_rows(h, None, 0, seg, False, True)
-                _gemm_dw(d_y_t, h_t, seg, d_w)
-        if ctx.needs_input_grad[0]:
-            new = torch.zeros if getattr(ctx, "zero_pads", True) else torch.empty
-            d_h = new(seg.max_rows, K, dtype=h.dtype, device=h.device)
-            _gemm_dx(d_y, w, seg, _C.CK_EPI_GROUPED, d_h)
-        return d_h, d_w, d_gates, None, d_bias, None, None, None
-
-
 def experts_up(
     x: torch.Tensor, weight: torch.Tensor, seg: ExpertSegments, k: int, bias: torch.Tensor | None = None,
     gelu_tanh: bool = False, zero_pads: bool = True,
@@ -703,11 +350,7 @@ def experts_up(
             seg.align, k,
         )
         return out[0] if gelu_tanh else out
-    _C.require_gpu(x, weight, bias)
-    if not torch.is_grad_enabled():
-        y, act = _experts_up_forward(x.contiguous(), weight.contiguous(), seg, k, bias, gelu_tanh, False, zero_pads)
-        return act if gelu_tanh else y
-    return _ExpertsUp.apply(x, weight, seg, k, bias, gelu_tanh, zero_pads)
+    return _C.host().experts_up(x, weight, bias, seg, k, gelu_tanh, zero_pads, _flags())
 
 
 def experts_down(
@@ -724,114 +367,12 @@ def experts_down(
             h, weight, gates.to(h.dtype), bias, slot_expert, seg.seg_starts, seg.counts, seg.tile_expert, seg.row_slot,
             seg.max_rows, seg.num_experts, seg.align,
         )[0]
-    _C.require_gpu(h, weight, gates, bias)
-    return _ExpertsDown.apply(h, weight, gates.to(h.dtype), seg, bias, None, _gate_slot(gates), zero_pads)
+    return _C.host().experts_down(h, weight, gates.to(h.dtype), bias, seg, _gate_slot(gates), zero_pads, _flags())
 
 
 # ---------------------------------------------------------------------------------------------------------------
 # fused SwiGLU expert block
 # ---------------------------------------------------------------------------------------------------------------
-def _swiglu_experts_forward(x, w_fc, w_proj, gates, seg: ExpertSegments, act_kind: int, keep_pre: bool, keep_act: bool):
-    """(out, pre, act, act_t, expanded) of the fused expert block on contiguous tensors. keep_pre: whether the c_fc GEMM
-    also writes its pre-activation (a backward pass reads it; without one, two thirds of that GEMM's stores go away).
-    keep_act: d_w_proj needs the activation, as it is or, where its GEMM has no row-major form, transposed (act_t, a second
-    output of the same epilogue)."""
-    T, H = x.shape
-    k = gates.size(1)
-    E, two_i, _ = w_fc.shape
-    I = two_i // 2
-    dev, dt = x.device, x.dtype
-    pre = torch.empty(seg.max_rows, two_i, dtype=dt, device=dev) if keep_pre else None
-    act = torch.empty(seg.max_rows, I, dtype=dt, device=dev)
-    rows_form = _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, (H, I), (two_i, H))
-    act_t = torch.empty(I, seg.ld_t, dtype=dt, device=dev) if keep_act and not rows_form else None
-    _gemm(x, k, w_fc, seg, _C.CK_EPI_GLU if act_kind == _C.CK_ACT_GLU else _C.CK_EPI_SWIGLU, pre, y_t=act_t, aux=act)
-    expanded = torch.empty(T * k, H, dtype=dt, device=dev)
-    _gemm(act, 0, w_proj, seg, _C.CK_EPI_SCATTER, expanded)
-    out, _ = _combine(expanded, gates, T, k, H)
-    return out, pre, act, act_t, expanded
-
-
-class _SwigluExperts(torch.autograd.Function):
-    """out = combine_k( gates * c_proj( swiglu_packed( c_fc(x) ) ) ) with the SwiGLU forward fused into the c_fc
-    epilogue and the SwiGLU backward fused into the epilogue of the c_proj input-gradient GEMM."""
-
-    @staticmethod
-    def forward(ctx, x, w_fc, w_proj, gates, seg: ExpertSegments, act_kind: int = _C.CK_ACT_SWIGLU, gate_slot=None):
-        ctx.gate_slot = gate_slot
-        x, w_fc, w_proj, gates = (t.contiguous() for t in (x, w_fc, w_proj, gates))
-        need_grad = any(ctx.needs_input_grad[:4])
-        out, pre, act, act_t, expanded = _swiglu_experts_forward(
-            x, w_fc, w_proj, gates, seg, act_kind, True, ctx.needs_input_grad[2]
-        )
-        if need_grad:
-            act_saved = act_t if act_t is not None else (act if ctx.needs_input_grad[2] else None)
-            ctx.save_for_backward(x, w_fc, w_proj, gates, pre, act_saved, expanded)
-        ctx.seg, ctx.act_kind = seg, act_kind
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        x, w_fc, w_proj, gates, pre, act_saved, expanded = ctx.saved_tensors
-        seg, act_kind = ctx.seg, ctx.act_kind
-        T, H = x.shape
-        k = gates.size(1)
-        E, two_i, _ = w_fc.shape
-        I = two_i // 2
-        dev, dt = x.device, x.dtype
-        grad_out = grad_out.contiguous()
-        need_x, need_fc, need_proj, need_gates = ctx.needs_input_grad[:4]
-        d_x = d_w_fc = d_w_proj = d_gates = None
-        rows_form = _dw_from_rows(seg.max_rows, seg.num_experts, seg.align, (H, I), (two_i, H))  # as in forward
-
-        if need_gates:
-            d_gates = _gate_grad(expanded, grad_out, T, k, H, gates.dtype, ctx.gate_slot)
-
-        # gate-scaled grad_out rows in padded grouped order (+ transpose for d_w_proj unless it reads rows)
-        d_y, d_y_t = _group_rows(grad_out, gates, k, seg, True, need_proj and not rows_form)
-        if need_proj:
-            d_w_proj = torch.empty_like(w_proj)
-            if rows_form:
-                _gemm_dw_rows(d_y, act_saved, seg, d_w_proj)
-            else:
-                _gemm_dw(d_y_t, act_saved, seg, d_w_proj)
-            del d_y_t
-
-        if need_x or need_fc:
-            # d_act = d_y @ w_proj with the leanest epilogue, then one streaming pass for the SwiGLU backward and the
-            # transpose d_w_fc needs. (The GEMM can also do this in its epilogue, CK_EPI_SWIGLU_BWD, but with one
-            # workgroup per CU the epilogue is time the MFMA units idle, while the streaming pass runs at HBM speed.)
-            d_act = torch.empty(seg.max_rows, I, dtype=dt, device=dev)
-            _gemm_dx(d_y, w_proj, seg, _C.CK_EPI_GROUPED, d_act)
-            del d_y
-            d_pre = torch.empty(seg.max_rows, two_i, dtype=dt, device=dev)
-            d_pre_t = torch.empty(two_i, seg.ld_t, dtype=dt, device=dev) if need_fc and not rows_form else None
-            with torch.cuda.device(dev):
-                _C.check(
-                    _C.lib().ck_swiglu_bwd_grouped(
-                        _C.ptr(pre), _C.ptr(d_act), I, _C.ptr(seg.seg_starts), _C.ptr(seg.counts), _C.ptr(seg.tile_expert),
-                        seg.align, seg.max_rows, _C.ptr(d_pre), _C.ptr(d_pre_t), seg.ld_t, act_kind, _C.dtype_code(dt),
-                        _C.stream(),
-                    )
-                )
-            del d_act
-            if need_fc:
-                d_w_fc = torch.empty_like(w_fc)
-                if rows_form:
-                    x_g, _ = _group_rows(x, None, k, seg, True, False)
-                    _gemm_dw_rows(d_pre, x_g, seg, d_w_fc)
-                    del x_g
-                else:
-                    _, x_t = _group_rows(x, None, k, seg, False, True)
-                    _gemm_dw(d_pre_t, x_t, seg, d_w_fc)
-                    del d_pre_t, x_t
-            if need_x:
-                d_expanded = torch.empty(T * k, H, dtype=dt, device=dev)
-                _gemm_dx(d_pre, w_fc, seg, _C.CK_EPI_SCATTER, d_expanded)
-                d_x = d_expanded if k == 1 else _combine(d_expanded, None, T, k, H)[0]
-        return d_x, d_w_fc, d_w_proj, d_gates, None, None, None
-
-
 def swiglu_experts(
     x: torch.Tensor, w_fc: torch.Tensor, w_proj: torch.Tensor, gates: torch.Tensor, seg: ExpertSegments,
     act_kind: int = _C.CK_ACT_SWIGLU,
@@ -848,11 +389,7 @@ def swiglu_experts(
             seg.num_experts, seg.align, grad and x.requires_grad, grad and w_fc.requires_grad,
             grad and w_proj.requires_grad, grad and gates.requires_grad, act_kind,
         )[0]
-    _C.require_gpu(x, w_fc, w_proj, gates)
-    if not torch.is_grad_enabled():
-        tensors = (t.contiguous() for t in (x, w_fc, w_proj, gates.to(x.dtype)))
-        return _swiglu_experts_forward(*tensors, seg, act_kind, False, False)[0]
-    return _SwigluExperts.apply(x, w_fc, w_proj, gates.to(x.dtype), seg, act_kind, _gate_slot(gates))
+    return _C.host().swiglu_experts(x, w_fc, w_proj, gates.to(x.dtype), seg, act_kind, _gate_slot(gates), _flags())
 
 
 # ---------------------------------------------------------------------------------------------------------------
