@@ -97,6 +97,20 @@ Tensor new_empty(at::IntArrayRef size, const Tensor& like, at::ScalarType t) { r
 Tensor new_empty(at::IntArrayRef size, const Tensor& like) { return at::empty(size, like.options()); }
 Tensor like_contiguous(const Tensor& t) { return at::empty(t.sizes(), t.options()); }
 
+// Whether a call is recorded for autograd. Forward-mode tangents count, in every grad mode: the nodes have no forward-mode
+// rule, and recording is what makes torch refuse such a call instead of losing the tangent.
+bool any_requires_grad(std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t->defined() && ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined())) return true;
+  return false;
+}
+
+// rows of a tensor whose last dimension is one row
+int64_t row_count(const Tensor& x) {
+  TORCH_CHECK(x.size(-1) > 0, "rows of a tensor of shape ", x.sizes(), " are empty");
+  return x.numel() / x.size(-1);
+}
+
 // ---- workspaces: one per kind, device and stream. "count" and "sort" start zero and their kernels leave them so; "split"
 // needs no initial contents. Never freed (torch's allocator may be gone at exit); torch has a bounded number of streams.
 enum WorkspaceKind { kCountWs, kSortWs, kSplitWs };
@@ -238,7 +252,7 @@ struct Route : torch::autograd::Function<Route> {
 };
 
 std::tuple<Tensor, Tensor> route(const Tensor& logits, int64_t k, bool long_indices, SlotPtr slot) {
-  if (at::GradMode::is_enabled() && logits.requires_grad()) {
+  if (any_requires_grad({&logits})) {
     auto out = Route::apply(logits, k, long_indices, std::move(slot));
     return {out[0], out[1]};
   }
@@ -553,13 +567,6 @@ struct SwigluExperts : torch::autograd::Function<SwigluExperts> {
   }
 };
 
-bool any_requires_grad(std::initializer_list<const Tensor*> ts) {
-  if (!at::GradMode::is_enabled()) return false;
-  for (const Tensor* t : ts)
-    if (t->defined() && t->requires_grad()) return true;
-  return false;
-}
-
 Tensor swiglu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, const Tensor& gates, py::object seg, int64_t act_kind,
                       std::optional<SlotPtr> slot, int64_t flags) {
   require_gpu(x, w_fc, w_proj, gates);
@@ -859,7 +866,7 @@ Tensor swiglu_packed(const Tensor& x) {
 // ---- RMSNorm, with and without the residual add ------------------------------------------------------------------
 std::tuple<Tensor, Tensor> rmsnorm_forward(const Tensor& x, const Tensor& weight, double eps, bool want_rstd) {
   const Launch l(x);
-  const int64_t H = x.size(-1), B = x.numel() / H;
+  const int64_t H = x.size(-1), B = row_count(x);
   const Tensor out = like_contiguous(x);
   Tensor rstd;
   if (want_rstd) rstd = new_empty({B}, x, at::kFloat);
@@ -869,7 +876,7 @@ std::tuple<Tensor, Tensor> rmsnorm_forward(const Tensor& x, const Tensor& weight
 std::tuple<Tensor, Tensor, Tensor> residual_rmsnorm_forward(const Tensor& x, const Tensor& residual, const Tensor& weight, double eps,
                                                             double multiplier, bool want_rstd) {
   const Launch l(x);
-  const int64_t H = x.size(-1), B = x.numel() / H;
+  const int64_t H = x.size(-1), B = row_count(x);
   const Tensor out = like_contiguous(x), added = like_contiguous(x);
   Tensor rstd;
   if (want_rstd) rstd = new_empty({B}, x, at::kFloat);
@@ -883,7 +890,7 @@ std::tuple<Tensor, Tensor, Tensor> rmsnorm_backward(const Tensor& x, const Tenso
                                                     const Tensor& d_added_in, double eps, double multiplier, bool residual, bool one_buffer) {
   const Tensor d_out = d_out_in.contiguous(), d_added = contiguous(d_added_in);
   const Launch l(x);
-  const int64_t H = x.size(-1), B = x.numel() / H;
+  const int64_t H = x.size(-1), B = row_count(x);
   const Tensor d_x = like_contiguous(x);
   Tensor d_residual, d_weight, partial;
   if (residual) d_residual = one_buffer ? d_x : like_contiguous(x);
@@ -1037,14 +1044,14 @@ Tensor softmax_forward(const Tensor& x, double multiplier) {
   const Launch l(x);
   const int64_t H = x.size(-1);
   const Tensor out = like_contiguous(x);
-  check(api.ck_softmax_fwd(ptr(x), (float)multiplier, x.numel() / H, (int32_t)H, ptr(out), dtype_code(x), l.stream));
+  check(api.ck_softmax_fwd(ptr(x), (float)multiplier, row_count(x), (int32_t)H, ptr(out), dtype_code(x), l.stream));
   return out;
 }
 Tensor softmax_backward(const Tensor& y, const Tensor& grad_in, double multiplier) {
   const Tensor grad = grad_in.contiguous(), d_x = like_contiguous(y);
   const Launch l(y);
   const int64_t H = y.size(-1);
-  check(api.ck_softmax_bwd(ptr(y), ptr(grad), (float)multiplier, y.numel() / H, (int32_t)H, ptr(d_x), dtype_code(y), l.stream));
+  check(api.ck_softmax_bwd(ptr(y), ptr(grad), (float)multiplier, row_count(y), (int32_t)H, ptr(d_x), dtype_code(y), l.stream));
   return d_x;
 }
 struct Softmax : torch::autograd::Function<Softmax> {

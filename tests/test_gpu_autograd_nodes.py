@@ -87,3 +87,29 @@ def test_layer_with_a_frozen_part(device, frozen):
     for n in leaves:
         if n != frozen:
             assert torch.equal(part[n], full[n]), n
+
+
+@pytest.mark.parametrize("grad_mode", [True, False])
+def test_forward_mode_is_refused(device, grad_mode):
+    """The nodes have no forward-mode rule: a call on a dual tensor raises, whatever the grad mode, and never drops the tangent."""
+    x, w = torch.randn(8, 64, device=device), torch.ones(64, device=device)
+    calls = [
+        lambda d: cute_kernels.rmsnorm_cute(d, w, 1e-6),
+        lambda d: cute_kernels.rmsnorm_cute(x, d[0].contiguous(), 1e-6),
+        lambda d: cute_kernels.fused_residual_add_rmsnorm_cute(x, d, w, 1e-6),
+        lambda d: cute_kernels.swiglu_cute(x, d),
+        lambda d: cute_kernels.swiglu_packed_cute(d),
+        lambda d: cute_kernels.softmax_cute(d),
+        lambda d: cute_kernels.route_topk_softmax(d, 2),
+    ]
+    with torch.autograd.forward_ad.dual_level(), torch.set_grad_enabled(grad_mode):
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        for call in calls:
+            with pytest.raises(RuntimeError, match="jvp"):
+                call(dual)
+
+
+@pytest.mark.parametrize("fn", [cute_kernels.softmax_cute, lambda x: cute_kernels.rmsnorm_cute(x, None, 1e-6)])
+def test_rows_without_elements_are_refused(device, fn):
+    with pytest.raises(RuntimeError, match="are empty"):
+        fn(torch.empty(3, 0, device=device))
