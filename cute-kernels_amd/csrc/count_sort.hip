@@ -4,7 +4,7 @@
 //         copies up to 1024 bins, one LDS copy beyond), blocks merge into a zero-initialised global accumulator, and the
 //         last block to finish (ticket counter) scans the bins, writes counts / inclusive ends / exclusive starts and
 //         puts the accumulator back to zero.
-// sort:   two launches. (1) every wave histograms its contiguous segment of the ids into a bin-major table
+// sort:   up to 4,096 ids one launch of one block (sort_small_kernel), beyond that two. (1) every wave histograms its contiguous segment of the ids into a bin-major table
 //         [bin][segment]; the last block scans that flattened table, which is exactly the destination of the first id of
 //         every (bin, segment) pair in a stable sort, and derives counts / offsets / tile-aligned segment starts /
 //         tile->expert table. (2) every wave re-reads its segment in order and ranks ids 64 at a time with bit-ballots.
@@ -21,10 +21,11 @@ constexpr int kMaxCountBins = 16384;
 constexpr int kMaxSortBins = 4096;
 constexpr int kSortTableWords = 16384;  // bins * segments held in LDS by the scanning block
 
-// Exclusive scan, in place, of data[0..n) (LDS) by a block of kBlock threads. Returns the total. tmp: kWavesPerBlock words.
+// Exclusive scan, in place, of data[0..n) (LDS) by a block of BLOCK threads. Returns the total. tmp: BLOCK / kWave words.
+template <int BLOCK = kBlock>
 __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  const int per = (n + kBlock - 1) / kBlock;
+  const int per = (n + BLOCK - 1) / BLOCK;
   const int b = min(n, t * per), e = min(n, b + per);
   uint32_t s = 0;
   for (int i = b; i < e; ++i) s += data[i];
@@ -39,7 +40,7 @@ __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
   __syncthreads();
   uint32_t wave_off = 0, total = 0;
 #pragma unroll
-  for (int w = 0; w < kWavesPerBlock; ++w) {
+  for (int w = 0; w < BLOCK / kWave; ++w) {
     const uint32_t v = tmp[w];
     if (w < wave) wave_off += v;
     total += v;
@@ -246,6 +247,36 @@ SortPlan make_sort_plan(int64_t R, int E) {
   return p;
 }
 
+// tile_expert[tile]: the expert whose padded segment holds the tile's rows, -1 past the last one. padded: [E + 1] starts (LDS)
+__device__ inline void write_tile_experts(const uint32_t* padded, int E, uint32_t padded_total, int align, int64_t max_tiles,
+                                          int32_t* __restrict__ tile_expert, int t, int threads) {
+  for (int64_t tile = t; tile < max_tiles; tile += threads) {
+    const uint32_t row = (uint32_t)(tile * align);
+    int32_t owner = -1;
+    if (row < padded_total) {
+      // last e with padded[e] <= row; empty experts share a start with their successor and are skipped by "last"
+      int lo = 0, hi = E - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (padded[mid] <= row) lo = mid; else hi = mid - 1;
+      }
+      owner = lo;
+    }
+    tile_expert[tile] = owner;
+  }
+}
+
+// ranks of 64 ids (one per lane): the lanes of the wave that hold the same id
+__device__ inline uint64_t lanes_with_same_id(int id, bool valid, int id_bits) {
+  uint64_t peers = __ballot(valid);
+  for (int b = 0; b < id_bits; ++b) {
+    const bool bit = (id >> b) & 1;
+    const uint64_t m = __ballot(bit);
+    peers &= bit ? m : ~m;
+  }
+  return peers;
+}
+
 // ws layout (uint32 words): [0] ticket, [1 .. 1 + E*S) bin-major table, scanned in place by the last block.
 template <typename id_t>
 __global__ __launch_bounds__(kBlock) void sort_hist_kernel(const id_t* __restrict__ ids, int64_t R, int E, int S,
@@ -303,20 +334,7 @@ __global__ __launch_bounds__(kBlock) void sort_hist_kernel(const id_t* __restric
   if (t == 0) padded[E] = padded_total;
   __syncthreads();
   for (int e = t; e <= E; e += kBlock) seg_starts[e] = (int32_t)padded[e];
-  for (int64_t tile = t; tile < max_tiles; tile += kBlock) {
-    const uint32_t row = (uint32_t)(tile * align);
-    int32_t owner = -1;
-    if (row < padded_total) {
-      // last e with padded[e] <= row; empty experts share a start with their successor and are skipped by "last"
-      int lo = 0, hi = E - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (padded[mid] <= row) lo = mid; else hi = mid - 1;
-      }
-      owner = lo;
-    }
-    tile_expert[tile] = owner;
-  }
+  write_tile_experts(padded, E, padded_total, align, max_tiles, tile_expert, t, kBlock);
   if (t == 0) ws[0] = 0u;
 }
 
@@ -353,12 +371,7 @@ __global__ __launch_bounds__(kBlock) void sort_scatter_kernel(const id_t* __rest
     const int64_t i = base + lane;
     const int id = ids_ahead[u];
     const bool valid = (unsigned)id < (unsigned)E;
-    uint64_t peers = __ballot(valid);
-    for (int b = 0; b < id_bits; ++b) {
-      const bool bit = (id >> b) & 1;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
+    const uint64_t peers = lanes_with_same_id(id, valid, id_bits);
     if (valid) {
       const uint32_t rank = (uint32_t)__popcll(peers & lanes_below);
       const uint32_t group = (uint32_t)__popcll(peers);
@@ -368,6 +381,76 @@ __global__ __launch_bounds__(kBlock) void sort_scatter_kernel(const id_t* __rest
       sorted_scattered_idxs[pos] = (int32_t)i;
       row_slot[(uint32_t)seg_starts[id] + (pos - starts[id])] = (int32_t)i;
     }
+    }
+  }
+}
+
+// The whole sort in one block and one launch, for the few ids of a decoding step or a small batch. What bounds it: latency.
+// The two launches above are a dozen dependent memory round trips (table out, fence, ticket, table back in, table out, launch
+// gap, table in) around a few hundred ids; here an id is read once and stays in registers, and the table in LDS.
+// Measured, a call behind others on its stream: 16 / 512 / 4,096 ids over 64 experts 7.9 / 8.5 / 16.6 -> 4.6 / 4.8 / 9.2 us,
+// over 512 experts 11.5 / 13.0 / 23.1 -> 7.6 / 8.0 / 13.3. The line: past 4,096 ids one block's rounds of 64 take as long as
+// two launches that spread them over the chip.
+constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
+constexpr int kSmallPer = 4;                                  // ids per lane
+constexpr int kSmallIds = kSmallBlock * kSmallPer;            // R up to which the one-block sort runs
+constexpr int kSmallBins = 512;                               // E up to which it runs: 36 KiB of LDS
+
+template <typename id_t>
+__global__ __launch_bounds__(kSmallBlock) void sort_small_kernel(const id_t* __restrict__ ids, int R, int E, int align, int64_t max_tiles,
+                                                                  int id_bits, int32_t* __restrict__ sorted_expert_idxs,
+                                                                  int32_t* __restrict__ sorted_scattered_idxs, uint32_t* __restrict__ counts,
+                                                                  uint32_t* __restrict__ ends, uint32_t* __restrict__ starts,
+                                                                  int32_t* __restrict__ seg_starts, int32_t* __restrict__ row_slot,
+                                                                  int32_t* __restrict__ tile_expert) {
+  extern __shared__ uint32_t lds[];  // table [E][waves], start [E], padded [E + 1], scan scratch [waves]
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
+  const int words = E * kSmallWaves;
+  uint32_t *table = lds, *start = lds + words, *padded = start + E, *tmp = padded + E + 1;
+  // a wave's ids are neighbours and the waves are in order, so that the flattened table, scanned, is a stable sort's first
+  // destination of every (id, wave)
+  const int per_wave = (R + kSmallBlock - 1) / kSmallBlock * kWave;
+  int id[kSmallPer];
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int i = wave * per_wave + u * kWave + lane;
+    id[u] = u * kWave < per_wave && i < R ? load_id(ids + i) : -1;
+  }
+  for (int i = t; i < words; i += kSmallBlock) table[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u)
+    if ((unsigned)id[u] < (unsigned)E) atomicAdd(&table[id[u] * kSmallWaves + wave], 1u);
+  __syncthreads();
+  const uint32_t total = block_exclusive_scan<kSmallBlock>(table, words, tmp);
+  for (int e = t; e < E; e += kSmallBlock) {
+    const uint32_t s = table[e * kSmallWaves], nxt = e + 1 < E ? table[(e + 1) * kSmallWaves] : total;
+    start[e] = s;
+    counts[e] = nxt - s;
+    starts[e] = s;
+    ends[e] = nxt;
+    padded[e] = (nxt - s + (uint32_t)align - 1) / (uint32_t)align * (uint32_t)align;
+  }
+  __syncthreads();
+  const uint32_t padded_total = block_exclusive_scan<kSmallBlock>(padded, E, tmp);
+  if (t == 0) padded[E] = padded_total;
+  __syncthreads();
+  for (int e = t; e <= E; e += kSmallBlock) seg_starts[e] = (int32_t)padded[e];
+  write_tile_experts(padded, E, padded_total, align, max_tiles, tile_expert, t, kSmallBlock);
+  const uint64_t lanes_below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    if (u * kWave >= per_wave) break;
+    const bool valid = (unsigned)id[u] < (unsigned)E;
+    const uint64_t peers = lanes_with_same_id(id[u], valid, id_bits);
+    if (valid) {
+      uint32_t* next = &table[id[u] * kSmallWaves + wave];  // this wave's word alone; its LDS operations keep their order
+      const uint32_t pos = *next + (uint32_t)__popcll(peers & lanes_below);
+      if ((peers >> lane) == 1ull) *next = pos + 1;  // the highest lane of the group advances the bin
+      const int i = wave * per_wave + u * kWave + lane;
+      sorted_expert_idxs[pos] = id[u];
+      sorted_scattered_idxs[pos] = i;
+      row_slot[padded[id[u]] + (pos - start[id[u]])] = i;
     }
   }
 }
@@ -604,11 +687,23 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
   CK_REQUIRE(sorted_expert_idxs && sorted_scattered_idxs && counts && ends && starts && seg_starts && row_slot &&
                  tile_expert && workspace,
              "ck_sort_by_expert: every output and the workspace are required");
-  const SortPlan p = make_sort_plan(R, E);
-  const int blocks = p.segments / kWavesPerBlock;
   const int64_t max_tiles = ck_sort_max_rows(R, E, align) / align;
   int id_bits = 0;
   while ((1 << id_bits) < E) ++id_bits;
+  if (R <= kSmallIds && E <= kSmallBins) {
+    const size_t lds = ((size_t)E * (kSmallWaves + 2) + 1 + kSmallWaves) * sizeof(uint32_t);
+#define CK_LAUNCH_SMALL(ID_T)                                                                                                \
+  hipLaunchKernelGGL((sort_small_kernel<ID_T>), dim3(1), dim3(kSmallBlock), lds, static_cast<hipStream_t>(stream),           \
+                     static_cast<const ID_T*>(expert_ids), (int)R, (int)E, (int)align, max_tiles, id_bits, sorted_expert_idxs, \
+                     sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert)
+    if (ids_are_i64) CK_LAUNCH_SMALL(int64_t);
+    else CK_LAUNCH_SMALL(int32_t);
+#undef CK_LAUNCH_SMALL
+    CK_CHECK_LAUNCH("ck_sort_by_expert");
+    return CK_OK;
+  }
+  const SortPlan p = make_sort_plan(R, E);
+  const int blocks = p.segments / kWavesPerBlock;
   const size_t table_words = (size_t)E * p.segments;
   size_t lds_words = (size_t)kWavesPerBlock * E;
   if (table_words + E + 1 > lds_words) lds_words = table_words + E + 1;

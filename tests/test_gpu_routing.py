@@ -249,3 +249,21 @@ def test_sort_by_expert_out_of_range_ids_are_dropped_and_can_be_detected(device)
     with pytest.raises(ValueError, match="outside"):
         cute_kernels.sort_by_expert(ids.to(device), E, 128, validate=True)
     cute_kernels.sort_by_expert(ids[keep].to(device), E, 128, validate=True)  # all in range: no error
+
+
+@pytest.mark.parametrize("R,E", [(1, 1), (63, 2), (65, 60), (1023, 8), (1025, 512), (2049, 128), (4096, 64), (4096, 513), (4097, 64)])
+@pytest.mark.parametrize("align", [16, 256])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.long])
+def test_sort_of_few_ids_in_one_block(device, R, E, align, dtype):
+    """Both sides of the lines (ids, experts) up to which one block does the whole sort, skewed so that waves meet runs of one
+    id and some experts stay empty; and the same ids with some out of range, which both forms drop."""
+    g = torch.Generator().manual_seed(R + E)
+    ids = (torch.rand(R, generator=g) ** 3 * E).to(dtype).clamp_(max=E - 1)
+    _check_sort(device, ids, E, align)
+    ids[::3] = torch.tensor([-1, E, 2**31 - 1], dtype=dtype).repeat(R)[: ids[::3].numel()]
+    seg = cute_kernels.sort_by_expert(ids.to(device), E, align)
+    kept = ((ids >= 0) & (ids < E)).nonzero().flatten()
+    order = kept[torch.sort(ids[kept], stable=True).indices]
+    assert int(seg.ends[-1]) == order.numel()
+    assert torch.equal(seg.sorted_scattered_idxs.cpu()[: order.numel()].long(), order)
+    assert torch.equal(seg.counts.cpu().long(), torch.bincount(ids[kept].long(), minlength=E))
