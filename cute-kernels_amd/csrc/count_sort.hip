@@ -4,10 +4,10 @@
 //         copies up to 1024 bins, one LDS copy beyond), blocks merge into a zero-initialised global accumulator, and the
 //         last block to finish (ticket counter) scans the bins, writes counts / inclusive ends / exclusive starts and
 //         puts the accumulator back to zero.
-// sort:   up to 4,096 ids one launch of one block (sort_small_kernel), beyond that two. (1) every wave histograms its contiguous segment of the ids into a bin-major table
-//         [bin][segment]; the last block scans that flattened table, which is exactly the destination of the first id of
-//         every (bin, segment) pair in a stable sort, and derives counts / offsets / tile-aligned segment starts /
-//         tile->expert table. (2) every wave re-reads its segment in order and ranks ids 64 at a time with bit-ballots.
+// sort:   up to 4,096 ids one launch of one block (sort_small_kernel), beyond that two. (1) every block histograms its
+//         contiguous segment of the ids into its row of a table. (2) every block sums the table's columns, which with a scan
+//         over the bins is the destination of its first id of every bin in a stable sort, and ranks its ids 64 at a time
+//         with bit-ballots; block 0 writes counts / offsets / tile-aligned segment starts.
 #include <stdlib.h>
 
 #include "ck_common.h"
@@ -19,7 +19,11 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxCountBins = 16384;
 constexpr int kMaxSortBins = 4096;
-constexpr int kSortTableWords = 16384;  // bins * segments held in LDS by the scanning block
+// The sort's table of counts holds at most this many words (bins * blocks). Half as many: 524,288 ids over 128 experts 17.7 ->
+// 17.9 us, 32,768 over 513 16.4 -> 20.6, 131,072 over 4,096 97 -> 161.
+constexpr int kSortTableWords = 32768;
+constexpr int kSortMaxBlocks = 256;            // one per CU
+constexpr int64_t kSortIdsPerBlock = 1024;     // 2,048: 32,768 ids over 64 experts 10.0 -> 10.7 us, 65,536 over 128 10.8 -> 12.3
 
 // Exclusive scan, in place, of data[0..n) (LDS) by a block of BLOCK threads. Returns the total. tmp: BLOCK / kWave words.
 template <int BLOCK = kBlock>
@@ -56,22 +60,17 @@ __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
 }
 
 // Returns true in every thread of exactly one block: the last one to arrive. Blocks must have made their global
-// writes before calling; the caller may read other blocks' writes after a true return.
-// FENCE = false is for blocks that publish their data only through device-scope atomics: those are coherent across the
-// XCDs by themselves and are complete once the barrier below has drained the wave's memory counters, so the L2
-// write-back + invalidate of a full fence (about 0.2 us per block, serialised) is not needed.
-template <bool FENCE>
+// writes before calling; the caller may read other blocks' writes after a true return. Blocks publish their data only through device-scope atomics: those are coherent across the XCDs by themselves and are
+// complete once the barrier below has drained the wave's memory counters, so the L2 write-back + invalidate of a full fence
+// (about 0.2 us per block, serialised) is not needed.
 __device__ bool last_block_ticket(uint32_t* ticket, uint32_t* lds_flag) {
-  if constexpr (FENCE) __threadfence();
   __syncthreads();
   if (threadIdx.x == 0) {
     const uint32_t prev = atomicAdd(ticket, 1u);
     *lds_flag = (prev == gridDim.x - 1) ? 1u : 0u;
   }
   __syncthreads();
-  const bool last = (*lds_flag != 0u);
-  if (FENCE && last) __threadfence();
-  return last;
+  return *lds_flag != 0u;
 }
 
 template <typename id_t>
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
     uint32_t* my_acc = acc + (size_t)(blockIdx.x % replicas) * num_bins;
     for (int e = t; e < num_bins; e += kBlock)
       if (hist[e]) atomicAdd(&my_acc[e], hist[e]);
-    if (!last_block_ticket<false>(ws, tmp + kWavesPerBlock)) return;
+    if (!last_block_ticket(ws, tmp + kWavesPerBlock)) return;
     // Sum the replicas that were used and put them back to zero. Device-scope atomic loads read the values where the
     // other blocks' atomics left them; the loads of one thread are independent, so their latencies overlap.
     const int used = min(replicas, (int)gridDim.x);
@@ -225,31 +224,32 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
 // ------------------------------------------------------------------------------------------------------------
 // sort
 // ------------------------------------------------------------------------------------------------------------
-constexpr int kSortUnroll = 8;  // ids a lane fetches before it consumes them
+// Blocks of the two-launch sort. Up to kSmallBins bins a block has 16 waves; beyond, 4, as its counters are one word per bin
+// and wave in LDS. Every block of the second launch reads the whole table of per-block counts: E * blocks words.
+constexpr int kSortPer = 4;  // ids a lane holds in registers
+constexpr int kWideWaves = 16, kNarrowWaves = 4;
+constexpr int kSmallBins = 512;
 
 struct SortPlan {
-  int segments;    // multiple of kWavesPerBlock
-  int64_t seg_len; // multiple of kWave
+  int blocks;
+  int64_t seg_len;  // ids of one block: a multiple of 64 per wave
 };
 
-// ids per wave segment (measured at 256 .. 4096: more, shorter segments lengthen the last block's scan; 1024 is fastest)
-constexpr int64_t kSortIdsPerSegment = 1024;
-
 SortPlan make_sort_plan(int64_t R, int E) {
+  const int64_t unit = (int64_t)(E <= kSmallBins ? kWideWaves : kNarrowWaves) * kWave;
   int64_t cap = kSortTableWords / (E > 0 ? E : 1);
-  cap = (cap / kWavesPerBlock) * kWavesPerBlock;
-  if (cap < kWavesPerBlock) cap = kWavesPerBlock;
-  int64_t want = ceil_div(R > 0 ? R : 1, kSortIdsPerSegment);
-  want = round_up(want, kWavesPerBlock);
+  if (cap > kSortMaxBlocks) cap = kSortMaxBlocks;
+  if (cap < 1) cap = 1;
+  const int64_t want = ceil_div(R > 0 ? R : 1, kSortIdsPerBlock);
   SortPlan p;
-  p.segments = (int)(want < cap ? want : cap);
-  p.seg_len = round_up(ceil_div(R > 0 ? R : 1, p.segments), kWave);
+  p.blocks = (int)(want < cap ? want : cap);
+  p.seg_len = round_up(ceil_div(R > 0 ? R : 1, p.blocks), unit);
   return p;
 }
 
 // tile_expert[tile]: the expert whose padded segment holds the tile's rows, -1 past the last one. padded: [E + 1] starts (LDS)
 __device__ inline void write_tile_experts(const uint32_t* padded, int E, uint32_t padded_total, int align, int64_t max_tiles,
-                                          int32_t* __restrict__ tile_expert, int t, int threads) {
+                                          int32_t* __restrict__ tile_expert, int64_t t, int64_t threads) {
   for (int64_t tile = t; tile < max_tiles; tile += threads) {
     const uint32_t row = (uint32_t)(tile * align);
     int32_t owner = -1;
@@ -277,124 +277,150 @@ __device__ inline uint64_t lanes_with_same_id(int id, bool valid, int id_bits) {
   return peers;
 }
 
-// ws layout (uint32 words): [0] ticket, [1 .. 1 + E*S) bin-major table, scanned in place by the last block.
-template <typename id_t>
-__global__ __launch_bounds__(kBlock) void sort_hist_kernel(const id_t* __restrict__ ids, int64_t R, int E, int S,
-                                                            int64_t seg_len, int align, int64_t max_tiles,
-                                                            uint32_t* __restrict__ counts, uint32_t* __restrict__ ends,
-                                                            uint32_t* __restrict__ starts, int32_t* __restrict__ seg_starts,
-                                                            int32_t* __restrict__ tile_expert, uint32_t* __restrict__ ws) {
-  extern __shared__ uint32_t lds[];  // max(4*E, E*S + E + 1) words + scan scratch (placed at the end)
-  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  uint32_t* my_hist = lds + (size_t)wave * E;
-  for (int i = t; i < kWavesPerBlock * E; i += kBlock) lds[i] = 0;
-  __syncthreads();
-
-  const int seg = blockIdx.x * kWavesPerBlock + wave;
-  const int64_t begin = (int64_t)seg * seg_len;
+// First launch of the sort: table[block][bin] = how often the bin occurs in the block's contiguous segment of the ids.
+template <typename id_t, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void sort_hist_kernel(const id_t* __restrict__ ids, int64_t R, int E, int64_t seg_len,
+                                                                  uint32_t* __restrict__ table) {
+  constexpr int BLOCK = WAVES * kWave;
+  extern __shared__ uint32_t lds[];  // [WAVES][E]: a wave's own counters, so that few bins do not serialise the whole block
+  const int t = threadIdx.x, wave = t / kWave;
+  for (int i = t; i < WAVES * E; i += BLOCK) lds[i] = 0;
+  const int64_t begin = (int64_t)blockIdx.x * seg_len;
   const int64_t end = min(R, begin + seg_len);
-  // kSortUnroll loads in flight per lane: a segment is a handful of dependent-latency round trips otherwise
-  for (int64_t base = begin + lane; base < end; base += kSortUnroll * kWave) {
-    int id[kSortUnroll];
+  bool cleared = false;
+  for (int64_t base = begin + t; base - t < end; base += kSortPer * BLOCK) {
+    int id[kSortPer];
 #pragma unroll
-    for (int u = 0; u < kSortUnroll; ++u) {
-      const int64_t i = base + u * kWave;
+    for (int u = 0; u < kSortPer; ++u) {
+      const int64_t i = base + u * BLOCK;
       id[u] = i < end ? load_id(ids + i) : -1;
     }
+    if (!cleared) __syncthreads();  // block-uniform; the first ids are under way meanwhile
+    cleared = true;
 #pragma unroll
-    for (int u = 0; u < kSortUnroll; ++u)
-      if ((unsigned)id[u] < (unsigned)E) atomicAdd(&my_hist[id[u]], 1u);
+    for (int u = 0; u < kSortPer; ++u)
+      if ((unsigned)id[u] < (unsigned)E) atomicAdd(&lds[wave * E + id[u]], 1u);
   }
   __syncthreads();
-  uint32_t* table = ws + 1;
-  for (int e = lane; e < E; e += kWave) table[(size_t)e * S + seg] = my_hist[e];
-
-  const int table_words = E * S;
-  uint32_t* tmp = lds + max(kWavesPerBlock * E, table_words + E + 1);
-  if (!last_block_ticket<true>(ws, tmp + kWavesPerBlock)) return;
-
-  // ---- last block: scan the flattened bin-major table in LDS
-  uint32_t* tab = lds;
-  for (int i = t; i < table_words; i += kBlock) tab[i] = table[i];
-  __syncthreads();
-  const uint32_t total = block_exclusive_scan(tab, table_words, tmp);
-  for (int i = t; i < table_words; i += kBlock) table[i] = tab[i];
-  uint32_t* padded = tab + table_words;  // [E + 1]
-  for (int e = t; e < E; e += kBlock) {
-    const uint32_t s = tab[(size_t)e * S];
-    const uint32_t nxt = (e + 1 < E) ? tab[(size_t)(e + 1) * S] : total;
-    const uint32_t c = nxt - s;
-    counts[e] = c;
-    starts[e] = s;
-    ends[e] = nxt;
-    padded[e] = (c + (uint32_t)align - 1) / (uint32_t)align * (uint32_t)align;
+  for (int e = t; e < E; e += BLOCK) {
+    uint32_t n = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) n += lds[w * E + e];
+    table[(int64_t)blockIdx.x * E + e] = n;
   }
-  __syncthreads();
-  const uint32_t padded_total = block_exclusive_scan(padded, E, tmp);
-  if (t == 0) padded[E] = padded_total;
-  __syncthreads();
-  for (int e = t; e <= E; e += kBlock) seg_starts[e] = (int32_t)padded[e];
-  write_tile_experts(padded, E, padded_total, align, max_tiles, tile_expert, t, kBlock);
-  if (t == 0) ws[0] = 0u;
 }
 
-template <typename id_t>
-__global__ __launch_bounds__(kBlock) void sort_scatter_kernel(const id_t* __restrict__ ids, int64_t R, int E, int S,
-                                                               int64_t seg_len, int id_bits,
-                                                               const uint32_t* __restrict__ starts,
-                                                               const int32_t* __restrict__ seg_starts,
-                                                               int32_t* __restrict__ sorted_expert_idxs,
-                                                               int32_t* __restrict__ sorted_scattered_idxs,
-                                                               int32_t* __restrict__ row_slot,
-                                                               const uint32_t* __restrict__ ws) {
-  extern __shared__ uint32_t lds[];  // [kWavesPerBlock][E] running destination of the next id of each bin
+// Second launch: every block sums the table's columns (all blocks, and those ahead of it), scans the bins, ranks its ids 64
+// at a time with bit-ballots and writes them to their places; the outputs per bin come from block 0, the tiles' experts
+// from all blocks.
+// What bounds the sort: latency. In the form before, one block scanned the table of all waves' counts behind a device-wide
+// fence and ticket, and wrote it back for the second launch; here the launch boundary is the only wait between blocks, the
+// table has one row per block instead of per wave, and reading all of it takes a block less time than the hand-over did.
+// The blocks' number is free of that one block's scan, so that a wave ranks 64 to 256 ids instead of 1,024 to 4,096.
+// Measured, both launches, before -> now (host included, under which a call does not get below 9.8 us): 8,192 ids over 64
+// experts 17.8 -> 9.8 us, 32,768 over 64 20.8 -> 10.0, 32,768 over 512 64 -> 12.8, 524,288 over 128 94 -> 17.7, 2,000,003 over
+// 60 135 -> 32, 131,072 over 4,096 488 -> 97.
+template <typename id_t, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void sort_scatter_kernel(
+    const id_t* __restrict__ ids, int64_t R, int E, int64_t seg_len, int id_bits, int align, int64_t max_tiles,
+    const uint32_t* __restrict__ table, int32_t* __restrict__ sorted_expert_idxs, int32_t* __restrict__ sorted_scattered_idxs,
+    uint32_t* __restrict__ counts, uint32_t* __restrict__ ends, uint32_t* __restrict__ starts, int32_t* __restrict__ seg_starts,
+    int32_t* __restrict__ row_slot, int32_t* __restrict__ tile_expert) {
+  constexpr int BLOCK = WAVES * kWave, STRIDE = WAVES + 1;  // a spare word per bin (always zero) spreads the bins over the banks
+  extern __shared__ uint32_t lds[];  // next [E][STRIDE], ahead [E], start [E], padded [E + 1], scan scratch [WAVES]
+  uint32_t *next = lds, *ahead = lds + STRIDE * E, *start = ahead + E, *padded = start + E, *tmp = padded + E + 1;
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-  uint32_t* next = lds + (size_t)wave * E;
-  const int seg = blockIdx.x * kWavesPerBlock + wave;
-  const uint32_t* table = ws + 1;
-  for (int e = lane; e < E; e += kWave) next[e] = table[(size_t)e * S + seg];
-  // LDS traffic below is wave-private and a wave's LDS operations complete in program order: no barrier needed.
-  const int64_t begin = (int64_t)seg * seg_len;
-  const int64_t end = min(R, begin + seg_len);
+  const int S = gridDim.x, me = blockIdx.x;
+  const int64_t per_wave = seg_len / WAVES;
+  const int64_t begin = (int64_t)me * seg_len + wave * per_wave, end = min(R, begin + per_wave);
+  constexpr int kRound = kSortPer * kWave;  // ids of a wave per round trip
+  int id[kSortPer];
+  auto fetch = [&](int64_t base) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kSortPer; ++u) {
+      const int64_t i = base + u * kWave + lane;
+      id[u] = i < end ? load_id(ids + i) : -1;
+    }
+  };
+  fetch(begin);
+  for (int i = t; i < (STRIDE + 2) * E; i += BLOCK) lds[i] = 0;  // next, ahead, start
+  __syncthreads();
+
+  // ---- column sums: BLOCK / E threads share a bin where there are fewer bins than threads
+  const int parts = E < BLOCK ? BLOCK / E : 1, part = E < BLOCK ? t / E : 0;
+  if (part < parts) {
+    for (int e = t - part * E; e < E; e += BLOCK) {
+      uint32_t all = 0, before = 0;
+#pragma unroll 8
+      for (int s = part; s < S; s += parts) {
+        const uint32_t n = table[(int64_t)s * E + e];
+        all += n;
+        if (s < me) before += n;
+      }
+      atomicAdd(&start[e], all);
+      atomicAdd(&ahead[e], before);
+    }
+  }
+  // ---- this block's ids by bin and wave
+  for (int64_t base = begin; base < end; base += kRound) {
+    if (base > begin) fetch(base);
+#pragma unroll
+    for (int u = 0; u < kSortPer; ++u)
+      if ((unsigned)id[u] < (unsigned)E) atomicAdd(&next[id[u] * STRIDE + wave], 1u);
+  }
+  __syncthreads();
+  for (int e = t; e < E; e += BLOCK) {
+    const uint32_t c = start[e];
+    padded[e] = (c + (uint32_t)align - 1) / (uint32_t)align * (uint32_t)align;
+    if (me == 0) counts[e] = c;
+  }
+  __syncthreads();
+  block_exclusive_scan<BLOCK>(start, E, tmp);
+  const uint32_t padded_total = block_exclusive_scan<BLOCK>(padded, E, tmp);
+  block_exclusive_scan<BLOCK>(next, E * STRIDE, tmp);
+  if (me == 0) {
+    for (int e = t; e < E; e += BLOCK) {
+      starts[e] = start[e];
+      ends[e] = start[e] + counts[e];  // counts[e] was written by this same thread above
+      seg_starts[e] = (int32_t)padded[e];
+    }
+    if (t == 0) seg_starts[E] = (int32_t)padded_total;
+  }
+  // next[e][w] counts from the block's first id on: to the bin's place among all blocks
+  for (int e = t; e < E; e += BLOCK) ahead[e] += start[e] - next[e * STRIDE];
+  __syncthreads();
+  write_tile_experts(padded, E, padded_total, align, max_tiles, tile_expert, (int64_t)me * BLOCK + t, (int64_t)S * BLOCK);
   const uint64_t lanes_below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
-  for (int64_t chunk = begin; chunk < end; chunk += kSortUnroll * kWave) {
-    int ids_ahead[kSortUnroll];  // the ids of the next kSortUnroll rounds, fetched together
+  const bool again = per_wave > kRound;  // more than the registers hold: read once more, out of L2
+  for (int64_t base = begin; base < end; base += kRound) {
+    if (again) fetch(base);
 #pragma unroll
-    for (int u = 0; u < kSortUnroll; ++u) {
-      const int64_t i = chunk + u * kWave + lane;
-      ids_ahead[u] = i < end ? load_id(ids + i) : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < kSortUnroll; ++u) {
-    const int64_t base = chunk + u * kWave;
-    if (base >= end) break;
-    const int64_t i = base + lane;
-    const int id = ids_ahead[u];
-    const bool valid = (unsigned)id < (unsigned)E;
-    const uint64_t peers = lanes_with_same_id(id, valid, id_bits);
-    if (valid) {
-      const uint32_t rank = (uint32_t)__popcll(peers & lanes_below);
-      const uint32_t group = (uint32_t)__popcll(peers);
-      const uint32_t pos = next[id] + rank;
-      if (rank == group - 1) next[id] = pos + 1;  // highest lane of the group advances the bin
-      sorted_expert_idxs[pos] = id;
-      sorted_scattered_idxs[pos] = (int32_t)i;
-      row_slot[(uint32_t)seg_starts[id] + (pos - starts[id])] = (int32_t)i;
-    }
+    for (int u = 0; u < kSortPer; ++u) {
+      if (base + u * kWave >= end) break;
+      const bool valid = (unsigned)id[u] < (unsigned)E;
+      const uint64_t peers = lanes_with_same_id(id[u], valid, id_bits);
+      if (valid) {
+        uint32_t* mine = &next[id[u] * STRIDE + wave];  // this wave's word alone; its LDS operations keep their order
+        const uint32_t local = *mine + (uint32_t)__popcll(peers & lanes_below);
+        if ((peers >> lane) == 1ull) *mine = local + 1;  // the highest lane of the group advances the bin
+        const uint32_t pos = ahead[id[u]] + local;
+        const int32_t i = (int32_t)(base + u * kWave + lane);
+        sorted_expert_idxs[pos] = id[u];
+        sorted_scattered_idxs[pos] = i;
+        row_slot[padded[id[u]] + (pos - start[id[u]])] = i;
+      }
     }
   }
 }
 
 // The whole sort in one block and one launch, for the few ids of a decoding step or a small batch. What bounds it: latency.
-// The two launches above are a dozen dependent memory round trips (table out, fence, ticket, table back in, table out, launch
-// gap, table in) around a few hundred ids; here an id is read once and stays in registers, and the table in LDS.
-// Measured, a call behind others on its stream: 16 / 512 / 4,096 ids over 64 experts 7.9 / 8.5 / 16.6 -> 4.6 / 4.8 / 9.2 us,
-// over 512 experts 11.5 / 13.0 / 23.1 -> 7.6 / 8.0 / 13.3. The line: past 4,096 ids one block's rounds of 64 take as long as
-// two launches that spread them over the chip.
+// An id is read once and stays in registers, and the table in LDS; the second launch and the way of the table through memory
+// go. Measured, a call behind others on its stream: 16 / 512 / 4,096 ids over 64 experts 4.6 / 4.8 / 9.2 us, over 512 experts
+// 7.6 / 8.0 / 13.3. The line: at 4,096 ids over 64 experts 8.6 us against the two launches' 9.8, and past it one block's
+// rounds of 64 take longer than launches that spread them over the chip.
 constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallPer = 4;                                  // ids per lane
-constexpr int kSmallIds = kSmallBlock * kSmallPer;            // R up to which the one-block sort runs
-constexpr int kSmallBins = 512;                               // E up to which it runs: 36 KiB of LDS
+constexpr int kSmallIds = kSmallBlock * kSmallPer;            // R up to which the one-block sort runs, up to kSmallBins bins
 
 template <typename id_t>
 __global__ __launch_bounds__(kSmallBlock) void sort_small_kernel(const id_t* __restrict__ ids, int R, int E, int align, int64_t max_tiles,
@@ -672,7 +698,7 @@ extern "C" int64_t ck_sort_max_rows(int64_t R, int32_t E, int32_t align) {
 extern "C" int64_t ck_sort_workspace_words(int64_t R, int32_t E) {
   if (E < 1) return 1;
   const SortPlan p = make_sort_plan(R, E);
-  return 1 + (int64_t)E * p.segments;
+  return 1 + (int64_t)E * p.blocks;
 }
 
 extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, int64_t R, int32_t E, int32_t align,
@@ -703,30 +729,26 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
     return CK_OK;
   }
   const SortPlan p = make_sort_plan(R, E);
-  const int blocks = p.segments / kWavesPerBlock;
-  const size_t table_words = (size_t)E * p.segments;
-  size_t lds_words = (size_t)kWavesPerBlock * E;
-  if (table_words + E + 1 > lds_words) lds_words = table_words + E + 1;
-  const size_t lds_hist = (lds_words + kWavesPerBlock + 2) * sizeof(uint32_t);
-  const size_t lds_scatter = (size_t)kWavesPerBlock * E * sizeof(uint32_t);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (ids_are_i64) {
-    const int64_t* ids = static_cast<const int64_t*>(expert_ids);
-    hipLaunchKernelGGL((sort_hist_kernel<int64_t>), dim3(blocks), dim3(kBlock), lds_hist, s, ids, R, (int)E,
-                       p.segments, p.seg_len, (int)align, max_tiles, counts, ends, starts, seg_starts, tile_expert,
-                       workspace);
-    hipLaunchKernelGGL((sort_scatter_kernel<int64_t>), dim3(blocks), dim3(kBlock), lds_scatter, s, ids, R, (int)E,
-                       p.segments, p.seg_len, id_bits, starts, seg_starts, sorted_expert_idxs, sorted_scattered_idxs,
-                       row_slot, workspace);
+  uint32_t* table = workspace + 1;  // word 0 stays zero, as the interface says
+#define CK_LAUNCH_SORT(ID_T, WAVES)                                                                                            \
+  do {                                                                                                                         \
+    const ID_T* ids = static_cast<const ID_T*>(expert_ids);                                                                    \
+    const size_t hist_words = (size_t)WAVES * E, words = (size_t)(WAVES + 4) * E + 1 + WAVES;                                  \
+    hipLaunchKernelGGL((sort_hist_kernel<ID_T, WAVES>), dim3(p.blocks), dim3(WAVES * kWave), hist_words * sizeof(uint32_t), s, \
+                       ids, R, (int)E, p.seg_len, table);                                                                      \
+    hipLaunchKernelGGL((sort_scatter_kernel<ID_T, WAVES>), dim3(p.blocks), dim3(WAVES * kWave), words * sizeof(uint32_t), s,   \
+                       ids, R, (int)E, p.seg_len, id_bits, (int)align, max_tiles, table, sorted_expert_idxs,                   \
+                       sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert);                        \
+  } while (0)
+  if (E <= kSmallBins) {
+    if (ids_are_i64) CK_LAUNCH_SORT(int64_t, kWideWaves);
+    else CK_LAUNCH_SORT(int32_t, kWideWaves);
   } else {
-    const int32_t* ids = static_cast<const int32_t*>(expert_ids);
-    hipLaunchKernelGGL((sort_hist_kernel<int32_t>), dim3(blocks), dim3(kBlock), lds_hist, s, ids, R, (int)E,
-                       p.segments, p.seg_len, (int)align, max_tiles, counts, ends, starts, seg_starts, tile_expert,
-                       workspace);
-    hipLaunchKernelGGL((sort_scatter_kernel<int32_t>), dim3(blocks), dim3(kBlock), lds_scatter, s, ids, R, (int)E,
-                       p.segments, p.seg_len, id_bits, starts, seg_starts, sorted_expert_idxs, sorted_scattered_idxs,
-                       row_slot, workspace);
+    if (ids_are_i64) CK_LAUNCH_SORT(int64_t, kNarrowWaves);
+    else CK_LAUNCH_SORT(int32_t, kNarrowWaves);
   }
+#undef CK_LAUNCH_SORT
   CK_CHECK_LAUNCH("ck_sort_by_expert");
   return CK_OK;
 }

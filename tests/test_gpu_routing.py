@@ -267,3 +267,11 @@ def test_sort_of_few_ids_in_one_block(device, R, E, align, dtype):
     assert int(seg.ends[-1]) == order.numel()
     assert torch.equal(seg.sorted_scattered_idxs.cpu()[: order.numel()].long(), order)
     assert torch.equal(seg.counts.cpu().long(), torch.bincount(ids[kept].long(), minlength=E))
+
+
+@pytest.mark.parametrize("R,E", [(5121, 60), (4099, 512), (4099, 513), (66000, 1), (262145, 512), (131073, 384), (20001, 4096), (300001, 128)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.long])
+def test_sort_over_many_blocks(device, R, E, dtype):
+    """Two launches: a ragged last block and one with no ids left, both widths of block (to 512 bins and beyond), bins that do
+    not divide the block, the most blocks that the table of counts allows, and segments longer than the registers hold."""
+    test_sort_of_few_ids_in_one_block(device, R, E, 128, dtype)
