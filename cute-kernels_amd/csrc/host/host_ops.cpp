@@ -38,7 +38,7 @@ using torch::autograd::variable_list;
   X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
   X(ck_grouped_gemm_f32) X(ck_grouped_gemm_dw_f32) X(ck_grouped_gemm_dw) X(ck_grouped_gemm_dw_rows)                     \
   X(ck_quant_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) \
-  X(ck_fused_residual_add_rmsnorm_fwd) X(ck_rmsnorm_fwd) X(ck_rmsnorm_bwd_partial_rows) X(ck_rmsnorm_bwd_typed)         \
+  X(ck_gelu_tanh_bwd_grouped) X(ck_fused_residual_add_rmsnorm_fwd) X(ck_rmsnorm_fwd) X(ck_rmsnorm_bwd_partial_rows) X(ck_rmsnorm_bwd_typed)         \
   X(ck_softmax_fwd) X(ck_softmax_bwd) X(ck_add_expert_bias) X(ck_expert_bias_grad)
 
 struct Api {
@@ -607,7 +607,14 @@ LinearGrads experts_up_backward(const Tensor& d_y_in, const Tensor& x, const Ten
     const Tensor d_act = d_y;
     d_y = like_contiguous(d_act);
     const Launch l(d_act);
-    check(api.ck_gelu_tanh_bwd(ptr(pre), ptr(d_act), ptr(d_y), d_act.numel(), dtype_code(d_act), l.stream));
+    const int64_t N = pre.size(1);
+    const auto aligned = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    if (N % 8 == 0 && aligned(pre) && aligned(d_act) && aligned(d_y)) {  // whole 16-byte pieces of rows: the pad rows are left out
+      const ck_segments cs = seg.c();
+      check(api.ck_gelu_tanh_bwd_grouped(ptr(pre), ptr(d_act), (int32_t)N, &cs, ptr(d_y), dtype_code(d_act), l.stream));
+    } else {
+      check(api.ck_gelu_tanh_bwd(ptr(pre), ptr(d_act), ptr(d_y), d_act.numel(), dtype_code(d_act), l.stream));
+    }
   }
   LinearGrads g;
   if (need_bias) g.d_bias = expert_bias_grad(d_y, seg);

