@@ -198,7 +198,10 @@ class MoE(nn.Module):
         if hidden_states.size(0) == 0:  # no tokens: nothing to sort or multiply; the result stays in the autograd graph
             return hidden_states * 0
         inference = not torch.is_grad_enabled() and not is_tracing()
-        align = choose_align(selected_experts.numel(), self.num_experts, hidden_states.dtype, inference)
+        align = choose_align(
+            selected_experts.numel(), self.num_experts, hidden_states.dtype, inference,
+            (self.hidden_size, self.intermediate_size, self.is_glu),
+        )
         seg = sort_by_expert(selected_experts, self.num_experts, align)
         has_bias = self.c_fc.bias is not None or self.c_proj.bias is not None
 

@@ -129,7 +129,8 @@ SMALL_TILES = ((6, 16), (14, 32), (30, 64))  # (rows per expert up to which, til
 
 
 def choose_align(
-    num_rows: int, num_experts: int, dtype: torch.dtype | None = None, inference: bool = False
+    num_rows: int, num_experts: int, dtype: torch.dtype | None = None, inference: bool = False,
+    widths: tuple[int, int, bool] | None = None,
 ) -> int:
     """Tile height of the padded layout. 16-bit layers: 256 rows wherever a backward pass follows. A 256-row tile runs on
     the 128-byte-row kernel, which does a 256 x 256 tile in the time the 128-row kernel takes for two 128 x 128 ones, so
@@ -143,6 +144,12 @@ def choose_align(
     expert, tiles of 16, 32, 64, 256 rows: 128 experts of 4,096 x 1,536 in e4m3 286, 291, 299, 382 / 522, 509, 522, 607 / - /
     872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 / 661, 609,
     596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us.
+    widths (hidden, intermediate, gated) of a 16-bit inference layer: below 512 rows per expert, 128 rows where 256 x 256 tiles
+    of c_proj would leave half of the 256 CUs idle or contract too little to pay for their split last round, and, up to 100 rows
+    per expert (one 128-row tile each), unless a gated layer has them by the thousand. 128 against 256: 8 experts of 1,664 x
+    5,632 at 40 / 128 / 256 rows per expert 166 / 189 / 234 against 260 / 268 / 298 us, 32 of 1,024 x 1,024 at 64 / 192 / 500
+    65 / 99 / 193 against 152 / 173 / 258; the other side: 8 of 4,096 x 14,336 at 128 rows 1,014 against 691, 64 of 2,048 x
+    1,408 437 against 337, 128 of 4,096 x 1,536 at 64 rows 1,148 against 991.
     fp32 layers run on 64-row tiles either way: 128 below 512 rows per expert keeps their padding small."""
     if dtype is torch.float32:
         return 256 if num_rows >= 512 * num_experts else 128
@@ -150,6 +157,13 @@ def choose_align(
         for rows, align in SMALL_TILES:
             if num_rows <= rows * num_experts:
                 return align
+        if widths is not None and num_rows < 512 * num_experts:
+            hidden, inter, gated = widths
+            columns = num_experts * -(-hidden // 256)
+            if num_rows <= 100 * num_experts:
+                return 256 if gated and columns >= 1024 else 128
+            tiles = columns * -(-(num_rows + 32 * num_experts) // (256 * num_experts))  # + 32: the load is not even
+            return 256 if tiles >= 128 and hidden * inter > 1 << 20 else 128
     return 256
 
 
