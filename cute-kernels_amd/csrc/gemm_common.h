@@ -43,19 +43,20 @@ struct GemmParams {
   void* trace;           // measurement builds only (CK_STAMP): per-wave cycle counts, 8 x uint64 each, else NULL
   // Split contraction for the last, partial round of tiles (128-byte-row kernel, grouped / scatter epilogues):
   // split_ws = [tiles][parts][4 waves][64 blocks][64 lanes] f32x4 partial accumulators (at most kSplitMaxTail tiles in
-  // kSplitParts parts or twice as many in half as many parts), followed by 2 * kSplitMaxTail arrival words; NULL = never
-  // split. split_base = the launch's grid without the extra workgroups (they are blockIdx split_base ..).
-  // An arrival word holds (launch epoch << 4) | parts arrived. A part that finds another epoch in the word starts the
-  // count afresh, so the words need no initial value and nothing resets them: whatever an earlier launch (or one that
-  // was cut short) left behind reads as "nobody has arrived yet". split_epoch: 1 .. 2^28 - 1, unique per launch.
+  // kSplitParts parts or twice as many in half as many parts), followed by 2 * kSplitMaxTail 64-bit arrival words; NULL =
+  // never split. split_base = the launch's grid without the extra workgroups (they are blockIdx split_base ..).
+  // An arrival word holds (launch tag << 4) | parts arrived. A part that finds another tag in the word starts the
+  // count afresh, so the words need no initial value: whatever another launch, one that was cut short or the memory's former
+  // owner left behind reads as "nobody has arrived yet". The last part to arrive puts the word to 0 (no launch's tag): a
+  // launch in a captured graph has the same tag in every replay. split_tag: 60 bits, never 0.
   float* split_ws;
   int split_base;
-  uint32_t split_epoch;
+  uint64_t split_tag;
 };
-uint32_t next_split_epoch();  // process-wide launch counter (grouped_gemm.hip)
+uint64_t next_split_tag();  // grouped_gemm.hip
 constexpr int kSplitParts = 4, kSplitMaxTail = 64, kSplitMaxRounds = 64, kSplitMinSteps = 16;
 constexpr int64_t kSplitPartFloats = 4 * 64 * 64 * 4;  // one workgroup's 256 x 256 fp32 tile
-constexpr int64_t kSplitWorkspaceBytes = kSplitMaxTail * kSplitParts * kSplitPartFloats * 4 + 2 * kSplitMaxTail * 4;
+constexpr int64_t kSplitWorkspaceBytes = kSplitMaxTail * kSplitParts * kSplitPartFloats * 4 + 2 * kSplitMaxTail * 8;
 
 // The 16-bit kernel with 128-byte LDS rows (grouped_gemm_line.hip): 256 x bn tiles, bn = 256 or 384, contraction length a
 // multiple of 64, modes kGrouped, kScatter, kSwiglu, kDw. The caller fills `prm` for these tile dimensions (n_tiles,

@@ -11,6 +11,7 @@
 // tiles built from 32x32 MFMA blocks, and two pipelines -- K step 32 straight from global memory into four swizzled LDS
 // stages (K % 32 == 0), or K step 64 through registers into two padded LDS stages (any K % 8 == 0).
 #include <atomic>
+#include <random>
 
 #include "gemm_common.h"
 
@@ -775,11 +776,17 @@ int launch_by_tile(const GemmParams& prm, int align, unsigned blocks_256, unsign
 }  // namespace ck
 
 namespace ck {
-uint32_t next_split_epoch() {
-  static std::atomic<uint32_t> counter{0};
-  uint32_t e;
-  do e = counter.fetch_add(1, std::memory_order_relaxed) + 1u; while ((e & 0x0fffffffu) == 0);
-  return e & 0x0fffffffu;
+// The tag of one split launch: consecutive numbers from a random start, so that recycled memory that holds small integers,
+// addresses or 16-bit tensors does not look like a launch's own arrivals.
+uint64_t next_split_tag() {
+  constexpr uint64_t kMask = ~0ull >> 4;
+  static std::atomic<uint64_t> counter{[] {
+    std::random_device random;
+    return (uint64_t)random() << 32 | random();
+  }()};
+  uint64_t tag;
+  do tag = counter.fetch_add(1, std::memory_order_relaxed) & kMask; while (tag == 0);
+  return tag;
 }
 }  // namespace ck
 
@@ -796,7 +803,7 @@ inline void fill_segments(GemmParams& prm, const ck_segments* seg) {
   prm.row_slot_out = seg->row_slot_out != nullptr ? seg->row_slot_out : seg->row_slot;
   prm.trace = debug_options().trace_buffer.load(std::memory_order_relaxed);  // NULL unless a measurement build was given one
 }
-// workspace for the split last round (NULL: never split): kSplitWorkspaceBytes, 16-byte aligned, counters zero
+// workspace for the split last round (NULL: never split): kSplitWorkspaceBytes, 16-byte aligned, any contents
 inline float* split_workspace(void* workspace, int64_t workspace_bytes) {
   if (workspace == nullptr || workspace_bytes < kSplitWorkspaceBytes || !aligned16(workspace)) return nullptr;
   return static_cast<float*>(workspace);

@@ -589,20 +589,22 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NI; ++j) *reinterpret_cast<f32x4*>(mine + (i * NI + j) * kWave * 4) = acc[i][j];
-      uint32_t* arrivals = reinterpret_cast<uint32_t*>(prm.split_ws + (int64_t)kSplitMaxTail * kSplitParts * kSplitPartFloats);
+      uint64_t* arrivals = reinterpret_cast<uint64_t*>(prm.split_ws + (int64_t)kSplitMaxTail * kSplitParts * kSplitPartFloats);
       uint32_t* flag = reinterpret_cast<uint32_t*>(lds_c);  // the stages are dead
       __threadfence();  // the partial tile is visible device-wide before the ticket is taken
       __syncthreads();
       if (tid == 0) {
-        // ticket = arrivals of THIS launch so far: a word left by another launch (any epoch but ours) counts as zero
-        uint32_t cur = __hip_atomic_load(&arrivals[split_slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), nxt;
+        // ticket = arrivals of THIS launch so far: a word left by another launch (any tag but ours) counts as zero
+        uint64_t cur = __hip_atomic_load(&arrivals[split_slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), nxt;
         for (;;) {  // bounded: another part of this tile (at most three) changed the word in between
-          nxt = (cur >> 4) == prm.split_epoch ? cur + 1u : ((prm.split_epoch << 4) | 1u);
-          const uint32_t seen = atomicCAS(&arrivals[split_slot], cur, nxt);
+          nxt = (cur >> 4) == prm.split_tag ? cur + 1u : ((prm.split_tag << 4) | 1u);
+          const uint64_t seen = atomicCAS(reinterpret_cast<unsigned long long*>(&arrivals[split_slot]), cur, nxt);
           if (seen == cur) break;
           cur = seen;
         }
-        *flag = nxt & 15u;
+        *flag = (uint32_t)nxt & 15u;
+        // the last one leaves the word as no launch's: a replayed graph runs this launch again under the same tag
+        if (*flag == (uint32_t)split_parts) __hip_atomic_store(&arrivals[split_slot], (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       __syncthreads();
       const bool last = *flag == (uint32_t)split_parts;
@@ -913,7 +915,7 @@ int launch_line(const GemmParams& prm_in, int mode, int bn, bool bt, int dtype, 
   GemmParams prm = prm_in;
   if (prm.split_ws != nullptr && (mode == kGrouped || mode == kScatter)) {
     prm.split_base = (int)blocks;  // the extra workgroups of a split last round sit behind the regular grid
-    prm.split_epoch = next_split_epoch();
+    prm.split_tag = next_split_tag();
     blocks += kSplitMaxTail * (kSplitParts - 1);
   } else {
     prm.split_ws = nullptr;

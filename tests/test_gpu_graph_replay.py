@@ -1,0 +1,40 @@
+"""Captured HIP graphs: a replay computes from the inputs it finds, whatever earlier replays and eager calls left behind."""
+
+import pytest
+import torch
+
+import cute_kernels
+from cute_kernels import scattermoe
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tokens,hidden,inter", [(300, 1024, 1024), (520, 2048, 2048)])
+def test_replays_of_a_layer_with_a_split_last_round(device, tokens, hidden, inter):
+    """A layer whose c_proj GEMM is the graph's only launch that splits its last round of tiles, on a stream that runs nothing
+    else: every replay finds the workspace as the replay before left it. Each one equals the eager layer bit for bit (the
+    same kernels on the same layout; the parts of a split tile are added in a fixed order)."""
+    E, k = 4, 2
+    g = torch.Generator(device=device).manual_seed(7)
+    rand = lambda *shape: torch.randn(*shape, device=device, generator=g)
+    w_fc, w_proj = (0.03 * rand(E, 2 * inter, hidden)).bfloat16(), (0.03 * rand(E, hidden, inter)).bfloat16()
+    ids = torch.stack([torch.randperm(E, device=device, generator=g)[:k] for _ in range(tokens)]).int()
+    x, gates = rand(tokens, hidden).bfloat16(), torch.rand(tokens, k, device=device, generator=g).bfloat16()
+
+    def layer():
+        return scattermoe.swiglu_experts(x, w_fc, w_proj, gates, cute_kernels.sort_by_expert(ids, E, 256))
+
+    with torch.no_grad():
+        seg = cute_kernels.sort_by_expert(ids, E, 256)
+        tail = int(seg.seg_starts[-1]) // 256 * (hidden // 256) % 256
+        assert 0 < tail <= 128 and inter // 64 >= 16  # the c_proj launch splits
+        layer()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=torch.cuda.Stream(device)):
+            out = layer()
+        for _ in range(4):
+            x.copy_(rand(tokens, hidden))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, layer())
