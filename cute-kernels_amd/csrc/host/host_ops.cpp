@@ -81,6 +81,13 @@ void require_gpu(const Tensor& t, const Rest&... rest) {
   require_gpu(rest...);
 }
 
+// A tensor whose sizes a launch is derived from has as many dimensions as the code takes it to have: rows of a [B, S, H]
+// tensor read as [T, K] would be addressed past its end.
+void require_dims(std::initializer_list<std::pair<const Tensor*, int64_t>> ts) {
+  for (const auto& [t, dims] : ts)
+    TORCH_CHECK_VALUE(t->dim() == dims, "expected a tensor with ", dims, " dimensions, got shape ", t->sizes());
+}
+
 // the device of a call made current, and torch's current stream on it
 struct Launch {
   c10::OptionalDeviceGuard guard;
@@ -191,6 +198,7 @@ using SlotPtr = c10::intrusive_ptr<GateSlot>;
 
 // (gates fp32, gates in logits.dtype, selected int32, selected int64); what is not wanted stays undefined
 std::tuple<Tensor, Tensor, Tensor, Tensor> route_forward(const Tensor& logits_in, int64_t k, bool want_f32, bool want_i32, bool want_i64) {
+  require_dims({{&logits_in, 2}});
   require_gpu(logits_in);
   const Tensor logits = logits_in.contiguous();
   const Launch l(logits);
@@ -450,6 +458,8 @@ struct Block {
 // transposed (act_t, a second output of the same epilogue).
 Block swiglu_experts_forward(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, const Tensor& gates, const Segments& seg,
                              int64_t act_kind, bool keep_pre, bool keep_act, int64_t flags) {
+  require_dims({{&x, 2}, {&w_fc, 3}, {&w_proj, 3}, {&gates, 2}});
+  require_gpu(x, w_fc, w_proj, gates);
   const int64_t T = x.size(0), H = x.size(1), k = gates.size(1), two_i = w_fc.size(1), I = two_i / 2;
   Block b;
   if (keep_pre) b.pre = new_empty({seg.max_rows, two_i}, x);
@@ -569,7 +579,6 @@ struct SwigluExperts : torch::autograd::Function<SwigluExperts> {
 
 Tensor swiglu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, const Tensor& gates, py::object seg, int64_t act_kind,
                       std::optional<SlotPtr> slot, int64_t flags) {
-  require_gpu(x, w_fc, w_proj, gates);
   const Segments g = Segments::of(seg);
   if (any_requires_grad({&x, &w_fc, &w_proj, &gates}))
     return SwigluExperts::apply(x, w_fc, w_proj, gates, g, act_kind, slot.value_or(SlotPtr()), flags);
@@ -581,6 +590,8 @@ Tensor swiglu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj,
 // them finite; without it they hold anything, which the expert GEMMs and their backward pass do not mind (valid rows only).
 std::pair<Tensor, Tensor> experts_up_forward(const Tensor& x, const Tensor& w, const Segments& seg, int64_t k, const Tensor& bias, bool gelu,
                                              bool keep_pre, bool zero_pads, int64_t flags) {
+  require_dims({{&w, 3}});
+  require_gpu(x, w, bias);
   const int64_t N = w.size(1);
   const auto rows = [&] { return zero_pads ? at::zeros({seg.max_rows, N}, x.options()) : at::empty({seg.max_rows, N}, x.options()); };
   Tensor y, act;
@@ -600,6 +611,7 @@ struct LinearGrads {
 // pre: the pre-activation where the GELU ran in the epilogue (d_y_in is then d_act), else undefined
 LinearGrads experts_up_backward(const Tensor& d_y_in, const Tensor& x, const Tensor& w, const Tensor& pre, const Segments& seg, int64_t k,
                                 bool need_x, bool need_w, bool need_bias, int64_t flags) {
+  require_dims({{&x, 2}});
   const int64_t T = x.size(0), K = x.size(1);
   Tensor d_y = d_y_in.contiguous();
   const Tensor none;
@@ -656,7 +668,6 @@ struct ExpertsUp : torch::autograd::Function<ExpertsUp> {
 
 Tensor experts_up(const Tensor& x, const Tensor& w, const OptTensor& bias, py::object seg, int64_t k, bool gelu, bool zero_pads, int64_t flags) {
   const Tensor b = value_or_undefined(bias);
-  require_gpu(x, w, b);
   const Segments g = Segments::of(seg);
   if (any_requires_grad({&x, &w, &b})) return ExpertsUp::apply(x, w, bias, g, k, gelu, zero_pads, flags);
   auto [y, act] = experts_up_forward(x.contiguous(), w.contiguous(), g, k, contiguous(b), gelu, false, zero_pads, flags);
@@ -674,6 +685,8 @@ Tensor slot_experts(const Tensor& sorted_expert_idxs, const Tensor& sorted_scatt
 // slot, needed where the bias is added by its own kernel
 std::pair<Tensor, Tensor> experts_down_forward(const Tensor& h, const Tensor& w, const Tensor& gates, const Segments& seg, const Tensor& bias,
                                                const Tensor& slot_expert, int64_t flags) {
+  require_dims({{&w, 3}, {&gates, 2}});
+  require_gpu(h, w, gates, bias);
   const int64_t T = gates.size(0), k = gates.size(1), N = w.size(1);
   const Tensor expanded = new_empty({T * k, N}, h), none;
   const bool fused_bias = bias.defined() && (is_f32(h) || (flags & kBiasFused));
@@ -737,7 +750,6 @@ struct ExpertsDown : torch::autograd::Function<ExpertsDown> {
 Tensor experts_down(const Tensor& h, const Tensor& w, const Tensor& gates, const OptTensor& bias, py::object seg, std::optional<SlotPtr> slot,
                     bool zero_pads, int64_t flags) {
   const Tensor b = value_or_undefined(bias);
-  require_gpu(h, w, gates, b);
   const Segments g = Segments::of(seg);
   Tensor slot_expert;
   if (b.defined() && !is_f32(h) && !(flags & kBiasFused))
@@ -772,6 +784,7 @@ void gemm_fp8(const Tensor& a8, const Tensor& a_scale, int64_t gather_div, const
 
 Tensor swiglu_experts_e4m3(const Tensor& x, const Tensor& w_fc8, const Tensor& w_fc_scale, const Tensor& w_proj8, const Tensor& w_proj_scale,
                            const Tensor& gates_in, py::object seg, const OptTensor& x8_in, const OptTensor& x_scale_in) {
+  require_dims({{&x, 2}, {&w_fc8, 3}, {&w_proj8, 3}, {&gates_in, 2}});
   require_gpu(x, w_fc8, w_proj8, gates_in);
   const at::NoGradGuard no_grad;
   const Segments g = Segments::of(seg);
@@ -1137,7 +1150,6 @@ PYBIND11_MODULE(_ck_host, m) {
   DEF("softmax_backward", ([](const Tensor& y, const Tensor& grad, double multiplier) { return softmax_backward(y.contiguous(), grad, multiplier); }));
   DEF("swiglu_experts_forward", ([](const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, const Tensor& gates, py::object seg, int64_t act_kind,
                                     bool keep_pre, bool keep_act, int64_t flags) {
-        require_gpu(x, w_fc, w_proj, gates);
         Block b = swiglu_experts_forward(x.contiguous(), w_fc.contiguous(), w_proj.contiguous(), gates.contiguous(), Segments::of(seg), act_kind,
                                          keep_pre, keep_act, flags);
         return std::make_tuple(b.out, to_opt(b.pre), to_opt(b.act_t.defined() ? b.act_t : keep_act ? b.act : Tensor()), b.expanded);
@@ -1150,7 +1162,6 @@ PYBIND11_MODULE(_ck_host, m) {
         return std::make_tuple(to_opt(g.d_x), to_opt(g.d_w_fc), to_opt(g.d_w_proj), to_opt(g.d_gates));
       }));
   DEF("experts_up_forward", ([](const Tensor& x, const Tensor& w, const OptTensor& bias, py::object seg, int64_t k, bool gelu, int64_t flags) {
-        require_gpu(x, w, value_or_undefined(bias));
         auto [y, act] = experts_up_forward(x.contiguous(), w.contiguous(), Segments::of(seg), k, contiguous(value_or_undefined(bias)), gelu, true, true, flags);
         return std::make_tuple(y, to_opt(act));
       }));
@@ -1161,7 +1172,6 @@ PYBIND11_MODULE(_ck_host, m) {
       }));
   DEF("experts_down_forward", ([](const Tensor& h, const Tensor& w, const Tensor& gates, const OptTensor& bias, const OptTensor& slot_expert, py::object seg,
                                   int64_t flags) {
-        require_gpu(h, w, gates, value_or_undefined(bias));
         return experts_down_forward(h.contiguous(), w.contiguous(), gates.contiguous(), Segments::of(seg), contiguous(value_or_undefined(bias)),
                                     value_or_undefined(slot_expert), flags);
       }));

@@ -1,0 +1,73 @@
+"""What the native host module refuses before it looks at a device: shapes the kernels would read or write past."""
+
+import pytest
+import torch
+
+import cute_kernels as ck
+from cute_kernels import _C, scattermoe
+
+
+def _segments(rows, experts, align=128):
+    max_rows = _C.lib().ck_sort_max_rows(rows, experts, align)
+    i32 = lambda n: torch.zeros(n, dtype=torch.int32)
+    return scattermoe.ExpertSegments(
+        i32(rows), i32(rows), i32(experts), i32(experts), i32(experts), i32(experts + 1), i32(max_rows), i32(max_rows // align),
+        max_rows, experts, align,
+    )
+
+
+E, T, k, H, I = 4, 6, 2, 64, 128
+bf16 = dict(dtype=torch.bfloat16)
+X, GATES = torch.zeros(T, H, **bf16), torch.zeros(T, k, **bf16)
+W_FC, W_PROJ = torch.zeros(E, 2 * I, H, **bf16), torch.zeros(E, H, I, **bf16)
+W8 = [torch.zeros(E, 2 * I, H, dtype=torch.float8_e4m3fn), torch.zeros(E, 2 * I), torch.zeros(E, H, I, dtype=torch.float8_e4m3fn), torch.zeros(E, H)]
+
+
+def test_matching_shapes_get_as_far_as_the_device():
+    seg = _segments(T * k, E)
+    for call in (
+        lambda: scattermoe.swiglu_experts(X, W_FC, W_PROJ, GATES, seg),
+        lambda: scattermoe.experts_down(torch.zeros(seg.max_rows, I, **bf16), W_PROJ, GATES, seg),
+        lambda: ck.swiglu_experts_e4m3(X, *W8, GATES, _segments(T * k, E, 256)),
+        lambda: ck.route_topk_softmax(torch.zeros(T, E), k),
+    ):
+        with pytest.raises(RuntimeError, match="GPU only"):
+            call()
+
+
+@pytest.mark.parametrize("x", [X.view(2, 3, H), X[0]])
+def test_token_rows_are_a_matrix(x):
+    with pytest.raises(ValueError):
+        scattermoe.swiglu_experts(x, W_FC, W_PROJ, GATES, _segments(T * k, E))
+    with pytest.raises(ValueError):
+        ck.swiglu_experts_e4m3(x, *W8, GATES, _segments(T * k, E, 256))
+    if x.dim() == 3:  # the forward of one linear reads rows only; its backward writes an [T, K] gradient
+        with pytest.raises(ValueError):
+            _C.host().experts_up_backward(
+                torch.zeros(640, 2 * I, **bf16), x, W_FC, None, _segments(T * k, E), k, True, False, False, scattermoe._flags()
+            )
+
+
+def test_gates_and_weights_have_their_dimensions():
+    seg = _segments(T * k, E)
+    h = torch.zeros(seg.max_rows, I, **bf16)
+    for gates in (GATES.flatten(), GATES.view(2, 3, k)):
+        with pytest.raises(ValueError):
+            scattermoe.swiglu_experts(X, W_FC, W_PROJ, gates, seg)
+        with pytest.raises(ValueError):
+            scattermoe.experts_down(h, W_PROJ, gates, seg)
+        with pytest.raises(ValueError):
+            ck.swiglu_experts_e4m3(X, *W8, gates, _segments(T * k, E, 256))
+    for w_fc, w_proj in ((W_FC.flatten(0, 1), W_PROJ), (W_FC, W_PROJ.flatten(0, 1))):
+        with pytest.raises(ValueError):
+            scattermoe.swiglu_experts(X, w_fc, w_proj, GATES, seg)
+    with pytest.raises(ValueError):
+        scattermoe.experts_down(h, W_PROJ.flatten(0, 1), GATES, seg)
+    with pytest.raises(ValueError):
+        scattermoe.experts_up(X, W_FC.flatten(0, 1), seg, k)
+
+
+@pytest.mark.parametrize("shape", [(E,), (2, 3, E)])
+def test_router_logits_are_a_matrix(shape):
+    with pytest.raises(ValueError):
+        ck.route_topk_softmax(torch.zeros(shape), 2)
