@@ -586,8 +586,9 @@ Tensor swiglu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj,
 }
 
 // ---- c_fc with any activation behind it: y [max_rows, N] (padded grouped), and with gelu the tanh GELU of it, computed in the
-// GEMM's epilogue. Pad rows are never written by the kernel: zero_pads makes them zeros, which keeps whatever is applied on top of
-// them finite; without it they hold anything, which the expert GEMMs and their backward pass do not mind (valid rows only).
+// GEMM's epilogue. Pad rows are never written by the kernel: zero_pads makes them zeros, which keeps whatever a caller applies on
+// top of them finite; without it they hold anything, which the expert GEMMs and their backward pass do not mind (valid rows
+// only), but nobody else may see: inside the node of the whole GELU block.
 std::pair<Tensor, Tensor> experts_up_forward(const Tensor& x, const Tensor& w, const Segments& seg, int64_t k, const Tensor& bias, bool gelu,
                                              bool keep_pre, bool zero_pads, int64_t flags) {
   require_dims({{&w, 3}});
@@ -645,16 +646,16 @@ LinearGrads experts_up_backward(const Tensor& d_y_in, const Tensor& x, const Ten
 
 struct ExpertsUp : torch::autograd::Function<ExpertsUp> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& w_in, const OptTensor& bias, const Segments& seg, int64_t k,
-                        bool gelu, bool zero_pads, int64_t flags) {
+                        bool gelu, int64_t flags) {
     const Tensor x = x_in.contiguous(), w = w_in.contiguous();
-    auto [y, act] = experts_up_forward(x, w, seg, k, contiguous(value_or_undefined(bias)), gelu, true, zero_pads, flags);
+    auto [y, act] = experts_up_forward(x, w, seg, k, contiguous(value_or_undefined(bias)), gelu, true, true, flags);
     save_segments(ctx, {x, w, gelu ? y : Tensor()}, seg,
                   {k, flags, x_in.requires_grad(), w_in.requires_grad(), bias.has_value() && bias->requires_grad()});
     ctx->set_materialize_grads(false);
     return gelu ? act : y;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    variable_list out(8);
+    variable_list out(7);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
@@ -666,11 +667,11 @@ struct ExpertsUp : torch::autograd::Function<ExpertsUp> {
   }
 };
 
-Tensor experts_up(const Tensor& x, const Tensor& w, const OptTensor& bias, py::object seg, int64_t k, bool gelu, bool zero_pads, int64_t flags) {
+Tensor experts_up(const Tensor& x, const Tensor& w, const OptTensor& bias, py::object seg, int64_t k, bool gelu, int64_t flags) {
   const Tensor b = value_or_undefined(bias);
   const Segments g = Segments::of(seg);
-  if (any_requires_grad({&x, &w, &b})) return ExpertsUp::apply(x, w, bias, g, k, gelu, zero_pads, flags);
-  auto [y, act] = experts_up_forward(x.contiguous(), w.contiguous(), g, k, contiguous(b), gelu, false, zero_pads, flags);
+  if (any_requires_grad({&x, &w, &b})) return ExpertsUp::apply(x, w, bias, g, k, gelu, flags);
+  auto [y, act] = experts_up_forward(x.contiguous(), w.contiguous(), g, k, contiguous(b), gelu, false, true, flags);
   return gelu ? act : y;
 }
 
@@ -721,23 +722,23 @@ LinearGrads experts_down_backward(const Tensor& grad_out_in, const Tensor& h, co
 
 struct ExpertsDown : torch::autograd::Function<ExpertsDown> {
   static Tensor forward(AutogradContext* ctx, const Tensor& h_in, const Tensor& w_in, const Tensor& gates_in, const OptTensor& bias,
-                        const Segments& seg, const OptTensor& slot_expert, SlotPtr slot, bool zero_pads, int64_t flags) {
+                        const Segments& seg, const OptTensor& slot_expert, SlotPtr slot, int64_t flags) {
     const Tensor h = h_in.contiguous(), w = w_in.contiguous(), gates = gates_in.contiguous();
     auto [out, expanded] = experts_down_forward(h, w, gates, seg, contiguous(value_or_undefined(bias)),
                                                 value_or_undefined(slot_expert), flags);
     save_segments(ctx, {h, w, gates, expanded}, seg,
-                  {flags, zero_pads, h_in.requires_grad(), w_in.requires_grad(), gates_in.requires_grad(),
+                  {flags, h_in.requires_grad(), w_in.requires_grad(), gates_in.requires_grad(),
                    bias.has_value() && bias->requires_grad()});
     ctx->saved_data["slot"] = slot_capsule(slot);
     ctx->set_materialize_grads(false);
     return out;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    variable_list out(9);
+    variable_list out(8);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
-    const LinearGrads g = experts_down_backward(grads[0], s[0], s[1], s[2], s[3], saved_segments(s, n), n[2], n[3], n[4], n[5], n[1],
+    const LinearGrads g = experts_down_backward(grads[0], s[0], s[1], s[2], s[3], saved_segments(s, n), n[1], n[2], n[3], n[4], true,
                                                 slot_of(ctx->saved_data["slot"]), n[0]);
     out[0] = g.d_in;
     out[1] = g.d_w;
@@ -748,15 +749,65 @@ struct ExpertsDown : torch::autograd::Function<ExpertsDown> {
 };
 
 Tensor experts_down(const Tensor& h, const Tensor& w, const Tensor& gates, const OptTensor& bias, py::object seg, std::optional<SlotPtr> slot,
-                    bool zero_pads, int64_t flags) {
+                    int64_t flags) {
   const Tensor b = value_or_undefined(bias);
   const Segments g = Segments::of(seg);
   Tensor slot_expert;
   if (b.defined() && !is_f32(h) && !(flags & kBiasFused))
     slot_expert = slot_experts(seg.attr("sorted_expert_idxs").cast<Tensor>(), seg.attr("sorted_scattered_idxs").cast<Tensor>());
   if (any_requires_grad({&h, &w, &gates, &b}))
-    return ExpertsDown::apply(h, w, gates, bias, g, to_opt(slot_expert), slot.value_or(SlotPtr()), zero_pads, flags);
+    return ExpertsDown::apply(h, w, gates, bias, g, to_opt(slot_expert), slot.value_or(SlotPtr()), flags);
   return experts_down_forward(h.contiguous(), w.contiguous(), gates.contiguous(), g, contiguous(b), slot_expert, flags).first;
+}
+
+// ---- the tanh-GELU block as one node: out = combine_k( gates * c_proj( gelu( c_fc(x) ) ) ). The activation's gradient, whose
+// pad rows nothing writes, stays inside: between two nodes a hook or anomaly mode would read them.
+struct GeluExperts : torch::autograd::Function<GeluExperts> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& w_fc_in, const Tensor& w_proj_in, const Tensor& gates_in,
+                        const OptTensor& bias_fc, const OptTensor& bias_proj, const Segments& seg, SlotPtr slot, int64_t flags) {
+    const Tensor x = x_in.contiguous(), w_fc = w_fc_in.contiguous(), w_proj = w_proj_in.contiguous(), gates = gates_in.contiguous();
+    auto [pre, act] = experts_up_forward(x, w_fc, seg, gates.size(1), contiguous(value_or_undefined(bias_fc)), true, true, false, flags);
+    auto [out, expanded] = experts_down_forward(act, w_proj, gates, seg, contiguous(value_or_undefined(bias_proj)), Tensor(), flags);
+    const auto needs = [](const OptTensor& b) { return b.has_value() && b->requires_grad(); };
+    save_segments(ctx, {x, w_fc, w_proj, gates, pre, act, expanded}, seg,
+                  {flags, x_in.requires_grad(), w_fc_in.requires_grad(), w_proj_in.requires_grad(), gates_in.requires_grad(),
+                   needs(bias_fc), needs(bias_proj)});
+    ctx->saved_data["slot"] = slot_capsule(slot);
+    ctx->set_materialize_grads(false);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    variable_list out(9);
+    if (!grads[0].defined()) return out;
+    const auto s = ctx->get_saved_variables();
+    const auto n = ctx->saved_data["ints"].toIntVector();
+    const Segments seg = saved_segments(s, n);
+    const bool need_act = n[1] || n[2] || n[5];
+    const LinearGrads down = experts_down_backward(grads[0], s[5], s[2], s[3], s[6], seg, need_act, n[3], n[4], n[6], false,
+                                                   slot_of(ctx->saved_data["slot"]), n[0]);
+    out[2] = down.d_w;
+    out[3] = down.d_gates;
+    out[5] = down.d_bias;
+    if (need_act) {
+      const LinearGrads up = experts_up_backward(down.d_in, s[0], s[1], s[4], seg, s[3].size(1), n[1], n[2], n[5], n[0]);
+      out[0] = up.d_in;
+      out[1] = up.d_w;
+      out[4] = up.d_bias;
+    }
+    return out;
+  }
+};
+
+// both biases join the accumulators (kBiasFused)
+Tensor gelu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, const Tensor& gates, const OptTensor& bias_fc,
+                    const OptTensor& bias_proj, py::object seg, std::optional<SlotPtr> slot, int64_t flags) {
+  require_dims({{&x, 2}, {&w_fc, 3}, {&w_proj, 3}, {&gates, 2}});
+  const Tensor b_fc = value_or_undefined(bias_fc), b_proj = value_or_undefined(bias_proj);
+  const Segments g = Segments::of(seg);
+  if (any_requires_grad({&x, &w_fc, &w_proj, &gates, &b_fc, &b_proj}))
+    return GeluExperts::apply(x, w_fc, w_proj, gates, bias_fc, bias_proj, g, slot.value_or(SlotPtr()), flags);
+  const Tensor act = experts_up_forward(x.contiguous(), w_fc.contiguous(), g, gates.size(1), contiguous(b_fc), true, false, false, flags).second;
+  return experts_down_forward(act, w_proj.contiguous(), gates.contiguous(), g, contiguous(b_proj), Tensor(), flags).first;
 }
 
 // ---- quantised-expert forward (inference) ------------------------------------------------------------------------
@@ -1110,6 +1161,7 @@ PYBIND11_MODULE(_ck_host, m) {
   DEF("swiglu_experts", swiglu_experts);
   DEF("experts_up", experts_up);
   DEF("experts_down", experts_down);
+  DEF("gelu_experts", gelu_experts);
   DEF("quantize_rows", quantize_rows);
   DEF("swiglu_experts_e4m3", swiglu_experts_e4m3);
   DEF("swiglu", swiglu);

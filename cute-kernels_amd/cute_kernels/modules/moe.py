@@ -228,18 +228,13 @@ class MoE(nn.Module):
             and (self.c_fc.bias is None or _bias_in_epilogue(seg, self.hidden_size))
         ):
             # the non-GLU activation of the reference's layer test (tests/test_commons.py:85-86) runs in the c_fc epilogue
-            # (nothing else touches the grouped rows in between, so their pad rows need no zeros)
-            fused_gelu = True
-            hidden_states = experts_up(
-                hidden_states, self.c_fc.weight, seg, self.top_k, self.c_fc.bias, gelu_tanh=True, zero_pads=False
+            return experts_up(
+                hidden_states, self.c_fc.weight, seg, self.top_k, self.c_fc.bias, gelu_tanh=True,
+                down=(self.c_proj.weight, router_weights, self.c_proj.bias),
             )
-        else:
-            fused_gelu = False
-            hidden_states = experts_up(hidden_states, self.c_fc.weight, seg, self.top_k, self.c_fc.bias)
-            hidden_states = self.act(hidden_states)
-        hidden_states = experts_down(
-            hidden_states, self.c_proj.weight, router_weights, seg, self.c_proj.bias, zero_pads=not fused_gelu
-        )
+        hidden_states = experts_up(hidden_states, self.c_fc.weight, seg, self.top_k, self.c_fc.bias)
+        hidden_states = self.act(hidden_states)
+        hidden_states = experts_down(hidden_states, self.c_proj.weight, router_weights, seg, self.c_proj.bias)
         return hidden_states
 
 

@@ -350,13 +350,25 @@ def _check_expert_dtypes(x: torch.Tensor, *weights: torch.Tensor) -> None:
 # ---------------------------------------------------------------------------------------------------------------
 def experts_up(
     x: torch.Tensor, weight: torch.Tensor, seg: ExpertSegments, k: int, bias: torch.Tensor | None = None,
-    gelu_tanh: bool = False, zero_pads: bool = True,
+    gelu_tanh: bool = False, down: tuple[torch.Tensor, torch.Tensor, torch.Tensor | None] | None = None,
 ) -> torch.Tensor:
-    """x [T, H] -> c_fc output in padded grouped order [max_rows, N] (+ bias[e] on expert e's rows); with gelu_tanh, the
-    tanh-approximated GELU of that output, applied in the GEMM's epilogue. Pad rows are zero; zero_pads=False leaves them
-    unwritten, for a caller that hands the result straight to experts_down(..., zero_pads=False)."""
+    """x [T, H] -> c_fc output in padded grouped order [max_rows, N] (+ bias[e] on expert e's rows; pad rows are zero); with
+    gelu_tanh, the tanh-approximated GELU of that output, applied in the GEMM's epilogue.
+    down: (weight, gates, bias) of the experts_down that follows a gelu_tanh c_fc of a 16-bit layer. Both then are one
+    autograd node and the result is experts_down's: nothing outside sees the grouped rows in between, so that neither they
+    nor their gradient need zeros in the pad rows."""
     _check_expert_dtypes(x, weight)
     assert bias is None or (bias.dtype == x.dtype and bias.shape == weight.shape[:2]), "bias should be [E, out] in x.dtype"
+    if down is not None:
+        w_down, gates, bias_down = down
+        if is_tracing() or not options.bias_fused:
+            return experts_down(experts_up(x, weight, seg, k, bias, gelu_tanh), w_down, gates, seg, bias_down)
+        assert gelu_tanh and x.dtype != torch.float32, "only the tanh GELU of a 16-bit layer is one node with its c_proj"
+        _check_expert_dtypes(x, w_down)
+        assert bias_down is None or (bias_down.dtype == x.dtype and bias_down.shape == w_down.shape[:2]), (
+            "bias should be [E, out] in x.dtype"
+        )
+        return _C.host().gelu_experts(x, weight, w_down, gates.to(x.dtype), bias, bias_down, seg, _gate_slot(gates), _flags())
     if is_tracing():
         op = _ops.experts_up_gelu if gelu_tanh else _ops.experts_up
         out = op(
@@ -364,15 +376,14 @@ def experts_up(
             seg.align, k,
         )
         return out[0] if gelu_tanh else out
-    return _C.host().experts_up(x, weight, bias, seg, k, gelu_tanh, zero_pads, _flags())
+    return _C.host().experts_up(x, weight, bias, seg, k, gelu_tanh, _flags())
 
 
 def experts_down(
-    h: torch.Tensor, weight: torch.Tensor, gates: torch.Tensor, seg: ExpertSegments, bias: torch.Tensor | None = None,
-    zero_pads: bool = True,
+    h: torch.Tensor, weight: torch.Tensor, gates: torch.Tensor, seg: ExpertSegments, bias: torch.Tensor | None = None
 ) -> torch.Tensor:
     """h [max_rows, I] (padded grouped) -> sum_k gates * (c_proj output + bias[e]) in token order [T, N]. Pad rows of the
-    gradient of h are zero; zero_pads=False leaves them unwritten."""
+    gradient of h are zero."""
     _check_expert_dtypes(h, weight)
     assert bias is None or (bias.dtype == h.dtype and bias.shape == weight.shape[:2]), "bias should be [E, out] in h.dtype"
     if is_tracing():
@@ -381,7 +392,7 @@ def experts_down(
             h, weight, gates.to(h.dtype), bias, slot_expert, seg.seg_starts, seg.counts, seg.tile_expert, seg.row_slot,
             seg.max_rows, seg.num_experts, seg.align,
         )[0]
-    return _C.host().experts_down(h, weight, gates.to(h.dtype), bias, seg, _gate_slot(gates), zero_pads, _flags())
+    return _C.host().experts_down(h, weight, gates.to(h.dtype), bias, seg, _gate_slot(gates), _flags())
 
 
 # ---------------------------------------------------------------------------------------------------------------
