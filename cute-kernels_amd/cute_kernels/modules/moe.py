@@ -23,7 +23,6 @@ from ..scattermoe import (
 )
 from ..rmsnorm_route import rmsnorm_route_cute
 from ..swiglu import swiglu_packed_cute
-from ..utils import is_tracing
 
 
 class Experts(nn.Module):
@@ -197,7 +196,12 @@ class MoE(nn.Module):
     ) -> torch.Tensor:
         if hidden_states.size(0) == 0:  # no tokens: nothing to sort or multiply; the result stays in the autograd graph
             return hidden_states * 0
-        inference = not torch.is_grad_enabled() and not is_tracing()
+        weights = (self.c_fc.weight, self.c_proj.weight, self.c_fc.bias, self.c_proj.bias)
+        # with gradients enabled, an activation of the caller's may hold parameters of its own
+        inference = not torch.is_grad_enabled() or (
+            (self.act is swiglu_packed_cute or type(self.act) in (torch.nn.GLU, torch.nn.GELU))
+            and not any(t is not None and t.requires_grad for t in (hidden_states, router_weights, *weights))
+        )
         align = choose_align(
             selected_experts.numel(), self.num_experts, hidden_states.dtype, inference,
             (self.hidden_size, self.intermediate_size, self.is_glu),

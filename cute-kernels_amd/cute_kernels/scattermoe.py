@@ -10,9 +10,11 @@ contraction-contiguous on both operands.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import torch
+from torch.fx.experimental.symbolic_shapes import statically_known_true
 
 from . import _C
 from .utils import is_tracing
@@ -128,43 +130,90 @@ class ExpertSegments:
 SMALL_TILES = ((6, 16), (14, 32), (30, 64))  # (rows per expert up to which, tile height) of inference batches
 
 
+def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
+    """256 or 128 rows for 16-bit layers below 512 rows per expert, whichever makes the sum of the layer's launches shorter.
+    launches: (columns, contraction, whether the epilogue may split its last round, input gradient) of every grouped GEMM
+    that depends on the height. In us, with the constants fitted to layers of 8 to 128 experts, 768 to 4,096 wide, 512 to
+    14,336 inside, gated and not, at 16 to 450 rows per expert (1,850 training steps, 2,590 inference calls):
+      * a 64-deep step of a 256 x 256 tile takes 1.7 on a CU; contractions that are no multiple of 64 run on the general
+        kernel, 1.6 with fewer loads in flight and no split; of a 128 x 128 tile 0.7, or 1.4 for the two that share a CU;
+      * splitting the last round of 256-row tiles costs 60 for its device-wide fences (32 experts of 1,024 x 1,024 at 64 rows:
+        137 us in 256-row tiles, 53 in 128-row ones);
+      * no launch is shorter than its weights' stream, 4.2 TB/s, and the input gradient of 128-row tiles (or of such a
+        contraction) transposes the weights first.
+    The chosen height is 0.3 % slower than the better one on average in training and 0.8 % in inference; always 256 was 11 and
+    26 %, always 128 17 and 11 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
+    4,096 x 14,336 at 8 / 96 / 400 rows 3,217 / 3,548 / 6,801 against 2,132 / 2,416 / 3,980 us; 32 of 1,024 x 1,024 304 / 335 /
+    622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. Inference: 8 of 4,096 x
+    14,336 at 34 / 64 / 100 / 128 rows 606 / 630 / 686 / 1,014 against 631 / 643 / 658 / 686; 8 of 1,664 x 5,632 at 64 / 200 /
+    300 rows 154 / 214 / 301 against 243 / 265 / 279; 16 of 1,536 x 4,096 without a gate at 64 / 300 rows 121 / 264 against
+    193 / 188."""
+    cost = {}
+    for height in (128, 256):
+        tile_rows = num_experts * -(-(num_rows + 24 * num_experts) // (height * num_experts))
+        total = 0.0
+        for columns, contraction, splits, input_gradient in launches:
+            tiles, steps = tile_rows * -(-columns // height), -(-contraction // 64)
+            stream = num_experts * columns * contraction * 2 / 4.2e6
+            nt_only = height == 128 or contraction % 64 != 0
+            if height == 128:
+                pairs, left = tiles // 512, tiles % 512
+                time = steps * (1.4 * pairs + (0.0 if left == 0 else 0.7 if left <= 256 else 1.4))
+            elif nt_only:
+                time = 1.6 * steps * -(-tiles // 256)
+            elif splits and 0 < tiles % 256 <= 128 and steps >= 16:
+                time = 1.7 * (steps * (tiles // 256) + -(-steps // min(4, 256 // (tiles % 256)))) + 60.0
+            else:
+                time = 1.7 * steps * -(-tiles // 256)
+            total += max(time, stream) + (2 * stream if input_gradient and nt_only else 0.0)
+        cost[height] = total
+    return 256 if cost[256] < cost[128] else 128
+
+
+_height_of_large_tiles_kept = functools.lru_cache(4096)(_height_of_large_tiles)  # a function of sizes alone
+
+
+def _large_tiles(
+    num_rows: int, num_experts: int, dtype: torch.dtype, launches: tuple[tuple[int, int, bool, bool], ...]
+) -> int:
+    # fp32 GEMMs run on 64-row tiles either way. A traced row count that stands for many takes part in one comparison only,
+    # so that a graph is compiled for two ranges of it and no more.
+    many = is_tracing() and not statically_known_true(num_rows < 1 << 48)
+    if dtype is torch.float32 or many or num_rows >= 512 * num_experts:
+        return 256 if num_rows >= 512 * num_experts else 128
+    return (_height_of_large_tiles if is_tracing() else _height_of_large_tiles_kept)(num_rows, num_experts, launches)
+
+
 def choose_align(
     num_rows: int, num_experts: int, dtype: torch.dtype | None = None, inference: bool = False,
     widths: tuple[int, int, bool] | None = None,
 ) -> int:
-    """Tile height of the padded layout. 16-bit layers: 256 rows wherever a backward pass follows. A 256-row tile runs on
-    the 128-byte-row kernel, which does a 256 x 256 tile in the time the 128-row kernel takes for two 128 x 128 ones, so
-    that even one ragged tile per expert costs no more than two of the small ones, and the backward pass reads the weights
-    as stored instead of through transposed copies. Measured at 16 / 64 / 250 / 375 rows per expert, 128 against 256:
-    training step of 8 wide experts (4,096 x 14,336) 3.44 / 4.13 / 5.56 / 6.93 against 2.24 / 2.41 / 3.24 / 3.94 ms, of 16
-    experts (1,536 x 4,096) from 64 rows on 1.03 / 1.34 / 1.61 against 0.79 / 1.02 / 1.09 ms.
-    inference (no backward pass): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the stream
-    of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights fetched
-    once per tile, from L2 at best, so the height follows the load. Whole inference layers at 1 / 8 / 16 / 32 / 64 rows per
-    expert, tiles of 16, 32, 64, 256 rows: 128 experts of 4,096 x 1,536 in e4m3 286, 291, 299, 382 / 522, 509, 522, 607 / - /
-    872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 / 661, 609,
-    596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us.
-    widths (hidden, intermediate, gated) of a 16-bit inference layer: below 512 rows per expert, 128 rows where 256 x 256 tiles
-    of c_proj would leave half of the 256 CUs idle or contract too little to pay for their split last round, and, up to 100 rows
-    per expert (one 128-row tile each), unless a gated layer has them by the thousand. 128 against 256: 8 experts of 1,664 x
-    5,632 at 40 / 128 / 256 rows per expert 166 / 189 / 234 against 260 / 268 / 298 us, 32 of 1,024 x 1,024 at 64 / 192 / 500
-    65 / 99 / 193 against 152 / 173 / 258; the other side: 8 of 4,096 x 14,336 at 128 rows 1,014 against 691, 64 of 2,048 x
-    1,408 437 against 337, 128 of 4,096 x 1,536 at 64 rows 1,148 against 991.
-    fp32 layers run on 64-row tiles either way: 128 below 512 rows per expert keeps their padding small."""
-    if dtype is torch.float32:
+    """Tile height of the padded layout.
+    A caller that says no more than the sizes, and every fp32 layer: 256 rows from 512 rows per expert on, else 128, which
+    keeps the padding small.
+    widths: (hidden, intermediate, whether the activation is the gated epilogue's) of a 16-bit layer. Below 512 rows per
+    expert its GEMMs decide (_height_of_large_tiles), those of a training step or of the forward alone.
+    inference (no gradient is asked for): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the
+    stream of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights
+    fetched once per tile, from L2 at best, so the height follows the load. Whole inference layers at 1 / 8 / 16 / 32 / 64
+    rows per expert, tiles of 16, 32, 64, 256 rows: 128 experts of 4,096 x 1,536 in e4m3 286, 291, 299, 382 / 522, 509, 522,
+    607 / - / 872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 /
+    661, 609, 596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us. Without widths, 256 rows beyond: the e4m3 GEMMs have
+    tiles of 16, 32, 64 and 256 rows."""
+    if dtype is torch.float32 or (widths is None and not inference):
         return 256 if num_rows >= 512 * num_experts else 128
-    if inference:
+    if inference and not (is_tracing() and not statically_known_true(num_rows < 1 << 48)):
         for rows, align in SMALL_TILES:
             if num_rows <= rows * num_experts:
                 return align
-        if widths is not None and num_rows < 512 * num_experts:
-            hidden, inter, gated = widths
-            columns = num_experts * -(-hidden // 256)
-            if num_rows <= 100 * num_experts:
-                return 256 if gated and columns >= 1024 else 128
-            tiles = columns * -(-(num_rows + 32 * num_experts) // (256 * num_experts))  # + 32: the load is not even
-            return 256 if tiles >= 128 and hidden * inter > 1 << 20 else 128
-    return 256
+    if widths is None:
+        return 256
+    hidden, inter, gated = widths
+    c_fc = 2 * inter if gated else inter
+    launches = ((c_fc, hidden, not gated, False), (hidden, inter, True, False))
+    if not inference:
+        launches += ((inter, hidden, True, True), (hidden, c_fc, True, True))
+    return _large_tiles(num_rows, num_experts, dtype, launches)
 
 
 def sort_by_expert(
@@ -485,9 +534,9 @@ class _ScatteredExperts(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, k, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out,
-                bias=None, gate_slot=None):
+                bias=None, gate_slot=None, align=None):
         assert not (gates is not None and grouped_out), "gated outputs are combined per token, not grouped"
-        seg = segments_from_sorted(sorted_expert_idxs, sorted_scattered_idxs, expert_offsets)
+        seg = segments_from_sorted(sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, align)
         x = x.contiguous()
         w = w.contiguous()
         E, N, K = w.shape
@@ -530,7 +579,7 @@ class _ScatteredExperts(torch.autograd.Function):
             return (
                 torch.zeros_like(x) if need_x else None, torch.zeros_like(w) if need_w else None, None, None, None, None,
                 torch.zeros_like(gates) if need_gates and gates is not None else None, None, None,
-                torch.zeros(E, N, dtype=w.dtype, device=w.device) if need_bias else None, None,
+                torch.zeros(E, N, dtype=w.dtype, device=w.device) if need_bias else None, None, None,
             )
         # the output gradient as padded grouped rows: what both the weight- and the input-gradient GEMM read
         if gates is not None:
@@ -558,7 +607,7 @@ class _ScatteredExperts(torch.autograd.Function):
             d_rows = torch.empty(R, K, dtype=x.dtype, device=x.device)
             _gemm_dx(d_y, w, seg, _C.CK_EPI_SCATTER, d_rows, rows_out=seg.row_pos if grouped_in else seg.row_slot)
             d_x = d_rows if grouped_in or k == 1 else _combine(d_rows, None, x.size(0), k, K)[0]
-        return d_x, d_w, None, None, None, None, d_gates, None, None, d_bias, None
+        return d_x, d_w, None, None, None, None, d_gates, None, None, d_bias, None, None
 
 
 def scattered_experts(
@@ -575,13 +624,18 @@ def scattered_experts(
     if gates is not None:
         gates_in = gates
         gates = gates.to(inputs.dtype)
+    E, N, K = w.shape
+    launches = ((N, K, True, False),)
+    if torch.is_grad_enabled() and inputs.requires_grad:
+        launches += ((K, N, True, True),)
+    align = _large_tiles(sorted_expert_idxs.numel(), E, inputs.dtype, launches)
     if is_tracing():
         out = _ops.scattered_experts(
-            inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out
+            inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align
         )
         return out[0]
     _C.require_gpu(inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets)
     return _ScatteredExperts.apply(
         inputs, w, k, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out, bias,
-        _gate_slot(gates_in) if gates is not None else None,
+        _gate_slot(gates_in) if gates is not None else None, align,
     )

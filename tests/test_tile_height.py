@@ -1,0 +1,147 @@
+"""Which tile height a call gets (scattermoe.choose_align): one rule for the eager layer, the traced one and the reference's
+expert-linear interface. Nothing is launched; traced calls end at the first real operator, which refuses the CPU tensor."""
+
+import pytest
+import torch
+
+import cute_kernels as ck
+from cute_kernels import scattermoe
+from cute_kernels.modules import moe as moe_module
+
+BF16 = torch.bfloat16
+E = 8
+
+
+def _layer(act="swiglu", H=256, I=320, dtype=BF16):
+    fn, gated = {"swiglu": (ck.swiglu_packed_cute, True), "gelu": (torch.nn.GELU("tanh"), False), "silu": (torch.nn.SiLU(), False),
+                 "prelu": (torch.nn.PReLU(), False)}[act]
+    return ck.MoE(E, 2, H, I, fn, gated, False, 0.02).to(dtype)
+
+
+class _Stop(Exception):
+    pass
+
+
+def _eager_align(monkeypatch, moe, rows, grad):
+    """the height the eager layer sorts with"""
+    seen = []
+    monkeypatch.setattr(moe_module, "route_topk_softmax", lambda x, k, **kw: (x.softmax(-1).topk(k)[0], x.topk(k)[1]))
+
+    def sort(ids, experts, align=None):
+        seen.append(align)
+        raise _Stop
+
+    monkeypatch.setattr(moe_module, "sort_by_expert", sort)
+    with torch.set_grad_enabled(grad), pytest.raises(_Stop):
+        moe(torch.randn(rows * E // 2, moe.hidden_size, dtype=moe.gate.weight.dtype))
+    return seen[0]
+
+
+class _Backend:
+    """Keeps the `align` argument of every sort (or of every expert linear) in the graphs it is given."""
+
+    def __init__(self):
+        self.aligns, self.graphs = [], 0
+
+    def __call__(self, gm, inputs):
+        self.graphs += 1
+        ops = torch.ops.ck_mi355
+        for n in gm.graph.nodes:
+            if n.target in (ops.sort_by_expert, ops.sort_by_expert.default):
+                self.aligns.append(n.args[2])
+            if n.target in (ops.scattered_experts, ops.scattered_experts.default):
+                self.aligns.append(n.args[10])
+        return gm.forward
+
+
+def _traced(fn, x, backend, grad, **kw):
+    torch._dynamo.reset()
+    compiled = torch.compile(fn, fullgraph=True, backend=backend, **kw)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="runs on the GPU only"):
+        compiled(x)
+    return compiled
+
+
+def test_a_caller_that_says_only_the_sizes():
+    for dtype, inference, widths in ((None, False, None), (torch.float32, True, (256, 320, True)), (torch.float32, False, (4096, 14336, True))):
+        for rows in (1, 40, 192, 511):
+            assert scattermoe.choose_align(rows * E, E, dtype, inference, widths) == 128
+        assert scattermoe.choose_align(512 * E, E, dtype, inference, widths) == 256
+
+
+def test_the_quantised_layer_never_gets_128_rows():
+    aligns = [scattermoe.choose_align(rows * E, E, BF16, inference=True) for rows in range(1, 600)]
+    assert set(aligns) == {16, 32, 64, 256}
+
+
+@pytest.mark.parametrize("H,I,gated,rows,training,height", [
+    (4096, 14336, True, 8, True, 256), (4096, 14336, True, 400, True, 256), (1024, 1024, True, 96, True, 128),
+    (3200, 1120, True, 32, True, 128), (3200, 1120, True, 400, True, 256), (1024, 1024, False, 16, True, 128),
+    (4096, 14336, True, 128, False, 256), (1664, 5632, True, 40, False, 128), (1664, 5632, True, 300, False, 256),
+])
+def test_sixteen_bit_layers_take_the_faster_height(H, I, gated, rows, training, height):
+    """8 experts, far from where the two heights meet (the times beside the rule: 1.15 to 2.7 times apart)."""
+    assert scattermoe.choose_align(rows * E, E, BF16, not training, (H, I, gated)) == height
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu", "silu", "prelu"])
+@pytest.mark.parametrize("rows", [4, 40, 200, 600])
+def test_nothing_to_differentiate_is_inference(monkeypatch, act, rows):
+    """Gradients enabled, but no tensor asks for one: the inference heights, except where the activation is a callable that
+    may hold parameters (its output then needs a gradient, which the small tiles' GEMMs do not have)."""
+    moe = _layer(act)
+    want = {grad: _eager_align(monkeypatch, moe, rows, grad) for grad in (False, True)}
+    for p in moe.parameters():
+        p.requires_grad_(False)
+    if act == "prelu":
+        moe.act.weight.requires_grad_(True)
+    assert _eager_align(monkeypatch, moe, rows, True) == want[act in ("silu", "prelu")]
+    assert _eager_align(monkeypatch, moe, rows, False) == want[False]
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu", "silu"])
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("rows", [4, 20, 40, 200, 600])
+def test_the_traced_layer_takes_the_eager_height(monkeypatch, act, grad, rows):
+    moe, backend = _layer(act), _Backend()
+    _traced(lambda x: moe(x)[0], torch.randn(rows * E // 2, moe.hidden_size, dtype=BF16), backend, grad, dynamic=False)
+    assert backend.aligns == [_eager_align(monkeypatch, moe, rows, grad)]
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_dynamic_row_count_compiles_two_graphs(grad):
+    """128 rows below 512 rows per expert, 256 from there on, and not a graph for every line of the rule."""
+    moe, backend = _layer(), _Backend()
+    shapes = [rows * E // 2 for rows in (4, 10, 20, 40, 120, 300, 511, 512, 700, 2000)]
+    compiled = _traced(lambda x: moe(x)[0], torch.randn(shapes[0], 256, dtype=BF16), backend, grad, dynamic=True)
+    for T in shapes[1:]:
+        with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="runs on the GPU only"):
+            compiled(torch.randn(T, 256, dtype=BF16))
+    assert backend.aligns == [128, 256] and backend.graphs == 2
+
+
+@pytest.mark.parametrize("dtype,rows,grad,height", [
+    (torch.float32, 40, False, 128), (torch.float32, 192, True, 128), (torch.float32, 512, False, 256), (BF16, 40, False, 128),
+    (BF16, 192, False, 128), (BF16, 40, True, 128), (BF16, 512, True, 256),
+])
+def test_the_reference_interface(monkeypatch, dtype, rows, grad, height):
+    """scattered_experts and an Experts module, eager and traced, at 8 experts of 256 x 320."""
+    experts, R = ck.Experts(E, 256, 320, False, 0.02).to(dtype), rows * E
+    x = torch.randn(R, 256, dtype=dtype, requires_grad=grad)
+    se, ss = torch.arange(E).repeat_interleave(rows), torch.arange(R)
+    off = torch.full((E,), rows).cumsum(0)
+    seen = []
+
+    def segments(*args):
+        seen.append(args[3])
+        raise _Stop
+
+    call = lambda x: experts(x, 1, se, ss, off, grouped_in=True, grouped_out=True)
+    backend = _Backend()
+    _traced(call, x, backend, grad, dynamic=False)
+    assert backend.aligns == [height]
+    monkeypatch.setattr(scattermoe, "segments_from_sorted", segments)
+    monkeypatch.setattr(scattermoe._C, "require_gpu", lambda *t: None)
+    with torch.set_grad_enabled(grad), pytest.raises(_Stop):
+        call(x)
+    assert seen == [height]
