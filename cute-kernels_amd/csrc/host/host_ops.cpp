@@ -1151,7 +1151,10 @@ PYBIND11_MODULE(_ck_host, m) {
       .def(py::init([] { return c10::make_intrusive<GateSlot>(); }))
       .def_property(
           "d_gates_f32", [](const GateSlot& s) { return to_opt(s.d_gates_f32); },
-          [](GateSlot& s, const OptTensor& t) { s.d_gates_f32 = value_or_undefined(t); });
+          [](GateSlot& s, const OptTensor& t) { s.d_gates_f32 = value_or_undefined(t); })
+      // gates are copied and saved with their attributes; what is in a slot belongs to one backward pass: a copy is empty
+      .def("__reduce__", [](const py::object& s) { return py::make_tuple(py::type::of(s), py::tuple()); })
+      .attr("__module__") = "cute_kernels._ck_host";
 #define DEF(name, fn) m.def(name, torch::wrap_pybind_function(fn))
   DEF("init", init);
   m.def("set_launch_timer", set_launch_timer);

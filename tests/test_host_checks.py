@@ -1,5 +1,11 @@
 """What the native host module refuses before it looks at a device: shapes the kernels would read or write past."""
 
+import copy
+import os
+import pickle
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -71,3 +77,22 @@ def test_gates_and_weights_have_their_dimensions():
 def test_router_logits_are_a_matrix(shape):
     with pytest.raises(ValueError):
         ck.route_topk_softmax(torch.zeros(shape), 2)
+
+
+def test_gates_can_be_copied_and_saved(tmp_path):
+    """The router's gates carry a slot of the native module as an attribute. It belongs to one backward pass: a copy of the
+    gates gets an empty one of its own."""
+    gates = torch.rand(3, 2)
+    gates._ck_gate_slot = _C.host().GateSlot()
+    gates._ck_gate_slot.d_gates_f32 = torch.ones(3, 2)
+    torch.save(gates, tmp_path / "gates.pt")
+    for other in (copy.deepcopy(gates), pickle.loads(pickle.dumps(gates)), torch.load(tmp_path / "gates.pt", weights_only=False)):
+        assert torch.equal(other, gates)
+        slot = other._ck_gate_slot
+        assert type(slot) is type(gates._ck_gate_slot) and slot is not gates._ck_gate_slot and slot.d_gates_f32 is None
+    assert gates._ck_gate_slot.d_gates_f32 is not None
+    # another process finds the class where the package is on its path
+    load = "import pickle, sys; print(type(pickle.load(sys.stdin.buffer)._ck_gate_slot).__module__)"
+    env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(_C.__file__)))
+    out = subprocess.run([sys.executable, "-c", load], input=pickle.dumps(gates), capture_output=True, env=env, timeout=100)
+    assert out.stdout.split() == [b"cute_kernels._ck_host"], out.stderr.decode()
