@@ -134,6 +134,8 @@ Tensor workspace(WorkspaceKind kind, const Tensor& like, void* stream, int64_t w
 }
 
 // ---- optional per-launch timing of the expert GEMMs (scattermoe.set_launch_timer): timer.time(name, (N, K), launch)
+// The backward pass launches from threads that do not hold the interpreter lock, and the timer may be taken off meanwhile:
+// the atomic says whether to ask for the lock, the pointer is read under it, and a call keeps a reference of its own.
 std::atomic<bool> timed_launches{false};
 py::object* launch_timer = nullptr;
 void set_launch_timer(py::object timer) {
@@ -144,9 +146,15 @@ void set_launch_timer(py::object timer) {
 }
 template <typename F>
 void timed(const char* name, int64_t a, int64_t b, F&& launch) {
-  if (!timed_launches) return launch();
-  const py::gil_scoped_acquire gil;
-  launch_timer->attr("time")(name, py::make_tuple(a, b), py::cpp_function([&] { launch(); }));
+  if (timed_launches) {
+    const py::gil_scoped_acquire gil;
+    if (launch_timer != nullptr) {
+      const py::object timer = *launch_timer;
+      timer.attr("time")(name, py::make_tuple(a, b), py::cpp_function([&] { launch(); }));
+      return;
+    }
+  }
+  launch();
 }
 
 // ---- count, sort ------------------------------------------------------------------------------------------------
@@ -1158,6 +1166,14 @@ PYBIND11_MODULE(_ck_host, m) {
 #define DEF(name, fn) m.def(name, torch::wrap_pybind_function(fn))
   DEF("init", init);
   m.def("set_launch_timer", set_launch_timer);
+  // for tests: a launch as the autograd engine's threads make it, without the interpreter lock
+  m.def("timed_without_lock", [](const std::string& name, int64_t a, int64_t b, const py::function& launch) {
+    const py::gil_scoped_release release;
+    timed(name.c_str(), a, b, [&] {
+      const py::gil_scoped_acquire gil;
+      launch();
+    });
+  });
   DEF("count", count);
   DEF("sort_by_expert", sort_by_expert);
   DEF("route", route);

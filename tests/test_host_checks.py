@@ -5,6 +5,7 @@ import os
 import pickle
 import subprocess
 import sys
+import threading
 
 import pytest
 import torch
@@ -96,3 +97,37 @@ def test_gates_can_be_copied_and_saved(tmp_path):
     env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(_C.__file__)))
     out = subprocess.run([sys.executable, "-c", load], input=pickle.dumps(gates), capture_output=True, env=env, timeout=100)
     assert out.stdout.split() == [b"cute_kernels._ck_host"], out.stderr.decode()
+
+
+class _Timer:
+    def __init__(self):
+        self.names = []
+
+    def time(self, name, dims, launch):
+        self.names.append((name, dims))
+        launch()
+
+
+def test_launch_timer_may_be_taken_off_while_another_thread_launches():
+    """Every launch happens once, with the timer or without: a thread that saw a timer and then waited for the interpreter lock
+    finds out whether it is still there."""
+    host, launched = _C.host(), []
+    timer = _Timer()
+    host.set_launch_timer(timer)
+    host.timed_without_lock("gemm", 2, 3, lambda: launched.append(0))
+    host.set_launch_timer(None)
+    host.timed_without_lock("gemm", 2, 3, lambda: launched.append(0))
+    assert timer.names == [("gemm", (2, 3))] and len(launched) == 2
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        for i in range(2000):
+            host.set_launch_timer(_Timer())
+            thread = threading.Thread(target=host.timed_without_lock, args=("gemm", 2, 3, lambda: launched.append(i)))
+            thread.start()
+            host.set_launch_timer(None)
+            thread.join()
+    finally:
+        sys.setswitchinterval(interval)
+        host.set_launch_timer(None)
+    assert len(launched) == 2002
