@@ -75,7 +75,7 @@ def _host_command(output: str) -> list[str]:
               sysconfig.get_paths()["include"]):
         cmd += ["-I", d]
     lib = os.path.join(torch_dir, "lib")
-    return cmd + [HOST_SOURCE, "-o", output, "-L", lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+    return cmd + [HOST_SOURCE, "-o", output, "-L", lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-lamdhip64",
                   "-ldl", f"-Wl,-rpath,{lib}"]
 
 

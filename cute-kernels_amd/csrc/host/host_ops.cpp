@@ -10,6 +10,7 @@
 // stream (calls on one stream are ordered, calls on different streams never share one).
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <dlfcn.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
@@ -118,18 +119,29 @@ int64_t row_count(const Tensor& x) {
   return x.numel() / x.size(-1);
 }
 
-// ---- workspaces: one per kind, device and stream. "count" and "sort" start zero and their kernels leave them so; "split"
-// needs no initial contents. Never freed (torch's allocator may be gone at exit); torch has a bounded number of streams.
+// ---- workspaces: one per kind, device and stream. "count" starts zero and its kernel leaves it so; "sort" and "split" need no
+// initial contents. Never freed (torch's allocator may be gone at exit); torch has a bounded number of streams.
+// A call that is being captured gets a workspace of its own, in the graph's memory: a graph may be replayed on any stream,
+// beside eager calls on the one it was captured on, and the zeros of a kept one would be written by the replays of the graph
+// that happened to ask first.
 enum WorkspaceKind { kCountWs, kSortWs, kSplitWs };
 Tensor workspace(WorkspaceKind kind, const Tensor& like, void* stream, int64_t words) {
   static std::mutex mutex;
   static auto* table = new std::map<std::tuple<int, int, void*>, Tensor>();
-  const std::lock_guard<std::mutex> lock(mutex);
-  Tensor& ws = (*table)[{(int)kind, (int)like.device().index(), stream}];
-  if (!ws.defined() || ws.numel() < words) {
-    const auto options = at::TensorOptions().dtype(at::kInt).device(like.device());
-    ws = kind == kSplitWs ? at::empty({words}, options) : at::zeros({std::max<int64_t>(words, 1 << 16)}, options);
+  const auto options = at::TensorOptions().dtype(at::kInt).device(like.device());
+  const auto made = [&](int64_t n) { return kind == kCountWs ? at::zeros({n}, options) : at::empty({n}, options); };
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return made(words);
+  const std::tuple<int, int, void*> key{(int)kind, (int)like.device().index(), stream};
+  {
+    const std::lock_guard<std::mutex> lock(mutex);
+    const Tensor& ws = (*table)[key];
+    if (ws.defined() && ws.numel() >= words) return ws;
   }
+  // not under the lock: making a tensor may run Python (dispatch modes) and wait for its lock
+  const Tensor fresh = made(kind == kSplitWs ? words : std::max<int64_t>(words, 1 << 16));
+  const std::lock_guard<std::mutex> lock(mutex);
+  Tensor& ws = (*table)[key];
+  if (!ws.defined() || ws.numel() < words) ws = fresh;
   return ws;
 }
 

@@ -38,3 +38,33 @@ def test_replays_of_a_layer_with_a_split_last_round(device, tokens, hidden, inte
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, layer())
+
+
+def test_graphs_that_count_do_not_depend_on_each_other(device):
+    """Two graphs captured on one stream, in memory that earlier replays have used: the second one replayed first, then either,
+    with eager calls on the capture stream in between."""
+    stream = torch.cuda.Stream(device)
+    ids = torch.randint(0, 60, (50000,), device=device, dtype=torch.int32)
+    want = torch.bincount(ids, minlength=60)
+    dirty = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(dirty, stream=stream):
+        used = [torch.full((1 << 18,), 7, dtype=torch.int32, device=device) for _ in range(4)]
+    dirty.replay()
+    torch.cuda.synchronize()
+    del used
+    graphs = []
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, pool=dirty.pool()):
+            out = cute_kernels.continuous_count_cute(ids, 60)
+        graphs.append((graph, out))
+    for i in (1, 0, 1, 1, 0):
+        graph, out = graphs[i]
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.long(), want), i
+        with torch.cuda.stream(stream):
+            eager = cute_kernels.continuous_count_cute(ids, 60)
+        torch.cuda.synchronize()
+        assert torch.equal(eager.long(), want)
