@@ -19,6 +19,7 @@ from torch.library import custom_op
 
 from . import _C
 from . import scattermoe as _moe
+from .utils import plain_size
 
 NS = "ck_mi355"
 
@@ -340,7 +341,7 @@ def _(expert_ids, num_experts, align):
 
 def sort_by_expert_segments(expert_ids: Tensor, num_experts: int, align: int) -> "_moe.ExpertSegments":
     out = sort_by_expert(expert_ids, num_experts, align)
-    max_rows = _max_rows(expert_ids.numel(), num_experts, align)
+    max_rows = _max_rows(plain_size(expert_ids.numel()), num_experts, align)
     return _moe.ExpertSegments(*out, max_rows=max_rows, num_experts=num_experts, align=align)
 
 

@@ -23,6 +23,7 @@ from ..scattermoe import (
 )
 from ..rmsnorm_route import rmsnorm_route_cute
 from ..swiglu import swiglu_packed_cute
+from ..utils import plain_size
 
 
 class Experts(nn.Module):
@@ -203,7 +204,7 @@ class MoE(nn.Module):
             and not any(t is not None and t.requires_grad for t in (hidden_states, router_weights, *weights))
         )
         align = choose_align(
-            selected_experts.numel(), self.num_experts, hidden_states.dtype, inference,
+            plain_size(selected_experts.numel()), self.num_experts, hidden_states.dtype, inference,
             (self.hidden_size, self.intermediate_size, self.is_glu),
         )
         seg = sort_by_expert(selected_experts, self.num_experts, align)

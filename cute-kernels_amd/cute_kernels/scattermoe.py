@@ -17,7 +17,7 @@ import torch
 from torch.fx.experimental.symbolic_shapes import statically_known_true
 
 from . import _C
-from .utils import is_tracing
+from .utils import is_tracing, plain_size
 
 _ops = None  # cute_kernels.compile_ops, set by the package once it is imported (used only while torch.compile traces)
 
@@ -228,7 +228,7 @@ def sort_by_expert(
     on a mismatch; it costs a device-to-host read, so the layer does not ask for it."""
     assert expert_ids.dtype in (torch.int32, torch.long)
     if align is None:
-        align = choose_align(expert_ids.numel(), num_experts)
+        align = choose_align(plain_size(expert_ids.numel()), num_experts)
     if is_tracing():
         return _ops.sort_by_expert_segments(expert_ids, num_experts, align)
     seg = _sort_by_expert_eager(expert_ids, num_experts, align)
@@ -624,11 +624,11 @@ def scattered_experts(
     if gates is not None:
         gates_in = gates
         gates = gates.to(inputs.dtype)
-    E, N, K = w.shape
+    E, N, K = (plain_size(n) for n in w.shape)
     launches = ((N, K, True, False),)
     if torch.is_grad_enabled() and inputs.requires_grad:
         launches += ((K, N, True, True),)
-    align = _large_tiles(sorted_expert_idxs.numel(), E, inputs.dtype, launches)
+    align = _large_tiles(plain_size(sorted_expert_idxs.numel()), E, inputs.dtype, launches)
     if is_tracing():
         out = _ops.scattered_experts(
             inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align

@@ -27,9 +27,14 @@ def enable_cute_tracing():
 
 
 def is_tracing() -> bool:
-    """Whether the public functions must dispatch to their torch.library custom ops (dynamo or cute tracing) instead of
-    the eager autograd.Function path. Reference: cute_kernels/utils/custom_op.py:26."""
-    return _IS_CUTE_TRACING or torch.compiler.is_compiling()
+    """Whether the public functions must dispatch to their torch.library custom ops (dynamo, cute tracing or torch.jit.trace)
+    instead of the eager path, whose launches a trace does not see. Reference: cute_kernels/utils/custom_op.py:26."""
+    return _IS_CUTE_TRACING or torch.compiler.is_compiling() or torch.jit.is_tracing()
+
+
+def plain_size(n) -> int:
+    """A size that decides what is launched: torch.jit.trace hands sizes out as tensors, and a trace is made for its own."""
+    return int(n) if isinstance(n, torch.Tensor) else n
 
 
 class KernelBackend(enum.Enum):
