@@ -549,20 +549,22 @@ BlockGrads swiglu_experts_backward(const Tensor& grad_out_in, const Tensor& x, c
 c10::IValue slot_capsule(const SlotPtr& slot) { return slot.defined() ? c10::IValue::make_capsule(slot) : c10::IValue(); }
 GateSlot* slot_of(const c10::IValue& v) { return v.isNone() ? nullptr : static_cast<GateSlot*>(v.toCapsule().get()); }
 
-// segment tables and integers of a node
+// Tensors, segment tables and integers of a node. The tables are whole numbers that address memory: they are kept beside the
+// saved tensors, where no saved-tensor hook (compression, conversion) gets at them.
 void save_segments(AutogradContext* ctx, variable_list tensors, const Segments& seg, std::vector<int64_t> ints) {
-  tensors.insert(tensors.end(), {seg.seg_starts, seg.counts, seg.tile_expert, seg.row_slot});
   ctx->save_for_backward(std::move(tensors));
+  ctx->saved_data["tables"] = std::vector<Tensor>{seg.seg_starts, seg.counts, seg.tile_expert, seg.row_slot};
   ints.insert(ints.end(), {seg.max_rows, seg.experts, seg.align});
   ctx->saved_data["ints"] = std::move(ints);
 }
-Segments saved_segments(const variable_list& saved, const std::vector<int64_t>& ints) {
-  const size_t t = saved.size() - 4, i = ints.size() - 3;
+Segments saved_segments(AutogradContext* ctx, const std::vector<int64_t>& ints) {
+  const std::vector<Tensor> tables = ctx->saved_data["tables"].toTensorVector();
+  const size_t i = ints.size() - 3;
   Segments g;
-  g.seg_starts = saved[t];
-  g.counts = saved[t + 1];
-  g.tile_expert = saved[t + 2];
-  g.row_slot = saved[t + 3];
+  g.seg_starts = tables[0];
+  g.counts = tables[1];
+  g.tile_expert = tables[2];
+  g.row_slot = tables[3];
   g.max_rows = ints[i];
   g.experts = ints[i + 1];
   g.align = ints[i + 2];
@@ -587,7 +589,7 @@ struct SwigluExperts : torch::autograd::Function<SwigluExperts> {
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
-    const BlockGrads g = swiglu_experts_backward(grads[0], s[0], s[1], s[2], s[3], s[4], s[5], s[6], saved_segments(s, n), n[0], n[2], n[3],
+    const BlockGrads g = swiglu_experts_backward(grads[0], s[0], s[1], s[2], s[3], s[4], s[5], s[6], saved_segments(ctx, n), n[0], n[2], n[3],
                                                  n[4], n[5], slot_of(ctx->saved_data["slot"]), n[1]);
     out[0] = g.d_x;
     out[1] = g.d_w_fc;
@@ -679,7 +681,7 @@ struct ExpertsUp : torch::autograd::Function<ExpertsUp> {
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
-    const LinearGrads g = experts_up_backward(grads[0], s[0], s[1], s[2], saved_segments(s, n), n[0], n[2], n[3], n[4], n[1]);
+    const LinearGrads g = experts_up_backward(grads[0], s[0], s[1], s[2], saved_segments(ctx, n), n[0], n[2], n[3], n[4], n[1]);
     out[0] = g.d_in;
     out[1] = g.d_w;
     out[2] = g.d_bias;
@@ -758,7 +760,7 @@ struct ExpertsDown : torch::autograd::Function<ExpertsDown> {
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
-    const LinearGrads g = experts_down_backward(grads[0], s[0], s[1], s[2], s[3], saved_segments(s, n), n[1], n[2], n[3], n[4], true,
+    const LinearGrads g = experts_down_backward(grads[0], s[0], s[1], s[2], s[3], saved_segments(ctx, n), n[1], n[2], n[3], n[4], true,
                                                 slot_of(ctx->saved_data["slot"]), n[0]);
     out[0] = g.d_in;
     out[1] = g.d_w;
@@ -801,7 +803,7 @@ struct GeluExperts : torch::autograd::Function<GeluExperts> {
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto n = ctx->saved_data["ints"].toIntVector();
-    const Segments seg = saved_segments(s, n);
+    const Segments seg = saved_segments(ctx, n);
     const bool need_act = n[1] || n[2] || n[5];
     const LinearGrads down = experts_down_backward(grads[0], s[5], s[2], s[3], s[6], seg, need_act, n[3], n[4], n[6], false,
                                                    slot_of(ctx->saved_data["slot"]), n[0]);
