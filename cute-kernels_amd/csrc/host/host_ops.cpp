@@ -409,10 +409,11 @@ void gemm_dw_rows(const Tensor& a, const Tensor& b, const Segments& seg, const T
   });
 }
 
-// Whether the weight-gradient GEMMs of shapes (M, N), ... read row-major operands instead of transposed copies: whenever that
-// kernel takes the shapes (not writing the transposes outweighs the wider tiles the transposed form can use). A function of
-// sizes only, so that forward, backward and the traced (fake) implementations agree on which tensors exist.
-bool dw_from_rows(int64_t align, int64_t flags, std::initializer_list<std::pair<int64_t, int64_t>> shapes) {
+// Whether the weight-gradient GEMMs of shapes (M, N), ... read row-major operands (ck_grouped_gemm_dw_rows) instead of
+// transposed copies: whenever that kernel takes the shapes. Not writing (and not holding) the transposes outweighs the wider
+// tiles the transposed form can use (fine-grained layer 4 % faster, Mixtral-shape layer 0.4 %). A function of sizes only, and
+// the one for forward, backward and the traced (fake) implementations, which have to agree on which tensors exist.
+bool dw_from_rows(int64_t align, int64_t flags, const std::vector<std::pair<int64_t, int64_t>>& shapes) {
   if (!(flags & kDwRows) || align % 64 != 0) return false;
   for (const auto& [m, n] : shapes)
     if (std::min(m, n) < 256 || m % 8 != 0 || n % 8 != 0) return false;
@@ -1285,6 +1286,7 @@ PYBIND11_MODULE(_ck_host, m) {
                       const OptTensor& y, const OptTensor& aux, const Tensor& like) {
         gemm_fp8(a8, a_scale, gather_div, w8, w_scale, Segments::of(seg), epilogue, value_or_undefined(y), value_or_undefined(aux), like.scalar_type());
       }));
+  m.def("dw_from_rows", dw_from_rows);
   DEF("transpose_weights", transpose_weights);
   DEF("group_rows", ([](const Tensor& src, const OptTensor& coeff, int64_t fan_out, py::object seg, bool want_grouped, bool want_transposed,
                         const OptTensor& rows) {

@@ -382,7 +382,7 @@ def _(x, w_fc, w_proj, gates, seg_starts, counts, tile_expert, row_slot, max_row
     I = two_i // 2
     if not need_proj:
         act_t = x.new_empty(0)
-    elif _moe._dw_from_rows(max_rows, num_experts, align, (H, I), (two_i, H)):
+    elif _moe._dw_from_rows(align, (H, I), (two_i, H)):
         act_t = x.new_empty(max_rows, I)  # the activation itself: d_w_proj reads row-major operands
     else:
         act_t = x.new_empty(I, max_rows)

@@ -316,13 +316,10 @@ def _gemm_dw_rows(a, b, seg: ExpertSegments, dw):
     _C.host().gemm_dw_rows(a, b, seg, dw)
 
 
-def _dw_from_rows(max_rows: int, num_experts: int, align: int, *shapes: tuple[int, int]) -> bool:
-    """Whether the weight-gradient GEMMs of shapes (M, N), ... read row-major operands (ck_grouped_gemm_dw_rows) instead
-    of transposed copies: whenever that kernel takes the shapes. Not writing (and not holding) the transposes outweighs
-    the 384-wide tiles the transposed form can use (measured: fine-grained layer 4 % faster, Mixtral-shape layer 0.4 %).
-    A function of sizes only, so that forward, backward and the traced (fake) implementations agree on which tensors
-    exist."""
-    return options.dw_rows and align % 64 == 0 and all(min(m, n) >= 256 and m % 8 == 0 and n % 8 == 0 for m, n in shapes)
+def _dw_from_rows(align: int, *shapes: tuple[int, int]) -> bool:
+    """Whether the weight-gradient GEMMs of shapes (M, N), ... read row-major operands instead of transposed copies
+    (csrc/host/host_ops.cpp)."""
+    return _C.host().dw_from_rows(align, _flags(), [(int(m), int(n)) for m, n in shapes])
 
 
 def _group_rows(src, coeff, fan_out, seg: ExpertSegments, want_grouped: bool, want_transposed: bool, rows=None):
@@ -596,7 +593,7 @@ class _ScatteredExperts(torch.autograd.Function):
         if need_w:
             x_g, _ = _group_rows(x, None, 1 if grouped_in else k, seg, True, False, rows=seg.row_pos if grouped_in else None)
             d_w = torch.empty_like(w)
-            if _fp32(x) or _dw_from_rows(seg.max_rows, E, seg.align, (N, K)):
+            if _fp32(x) or _dw_from_rows(seg.align, (N, K)):
                 _gemm_dw_rows(d_y, x_g, seg, d_w)
             else:
                 _, d_y_t = _group_rows(d_y, None, 0, seg, False, True)

@@ -63,3 +63,21 @@ class _LayerOnTheReferenceInterface(ck.MoE):
 def test_layer_on_the_reference_interface_traces():
     moe = _LayerOnTheReferenceInterface(4, 2, 64, 32, torch.nn.GLU(), True, False, 0.02).to(torch.bfloat16)
     _traces(lambda a: moe(a)[0], torch.randn(16, 64, dtype=torch.bfloat16, requires_grad=True))
+
+
+@pytest.mark.parametrize("dw_rows", [True, False])
+@pytest.mark.parametrize("align,H,I,rows_form", [(128, 256, 256, True), (256, 256, 256, True), (256, 248, 256, False), (128, 256, 128, False)])
+def test_traced_activation_has_the_shape_the_library_writes(monkeypatch, align, H, I, rows_form, dw_rows):
+    """swiglu_experts announces its saved activation in the form the weight gradients will read, by the library's own rule."""
+    monkeypatch.setattr(ck.scattermoe.options, "dw_rows", dw_rows)
+    T, k, E = 40, 2, 4
+    max_rows = compile_ops._max_rows(T * k, E, align)
+    e = lambda *s, dtype=torch.bfloat16: torch.empty(*s, dtype=dtype, device="meta")
+    i32 = dict(dtype=torch.int32)
+    _, pre, act, _ = compile_ops.swiglu_experts(
+        e(T, H), e(E, 2 * I, H), e(E, H, I), e(T, k), e(E + 1, **i32), e(E, **i32), e(max_rows // align, **i32), e(max_rows, **i32),
+        max_rows, E, align, True, True, True, True, 0,
+    )
+    assert pre.shape == (max_rows, 2 * I)
+    assert act.shape == ((max_rows, I) if rows_form and dw_rows else (I, max_rows))
+    assert _C.host().dw_from_rows(align, ck.scattermoe._flags(), [(H, I), (2 * I, H)]) == (rows_form and dw_rows)
