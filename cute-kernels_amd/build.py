@@ -80,13 +80,24 @@ def _host_command(output: str) -> list[str]:
 
 
 def build_host(force: bool = False) -> str:
-    header = os.path.join(INCLUDE, "ck_mi355.h")
-    if not force and os.path.exists(HOST_PATH):
-        if os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(HOST_SOURCE), os.path.getmtime(header)):
-            return HOST_PATH
-    proc = subprocess.run(_host_command(HOST_PATH), capture_output=True, text=True)
+    """Compiles the host module unless it is newer than its sources and was made by the same command against the same torch:
+    it links against torch's C++ interface, which has no stable ABI."""
+    import torch
+
+    sources = (HOST_SOURCE, os.path.join(INCLUDE, "ck_mi355.h"))
+    command = _host_command(HOST_PATH)
+    made_by = f"{torch.__version__} {torch.version.git_version}\n{' '.join(command)}\n"
+    stamp = os.path.join(OBJ_DIR, "_ck_host.made_by")
+    if not force and os.path.exists(HOST_PATH) and os.path.exists(stamp):
+        with open(stamp) as f:
+            if f.read() == made_by and os.path.getmtime(HOST_PATH) >= max(os.path.getmtime(s) for s in sources):
+                return HOST_PATH
+    proc = subprocess.run(command, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed on {HOST_SOURCE}:\n{proc.stdout}\n{proc.stderr}")
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    with open(stamp, "w") as f:
+        f.write(made_by)
     return HOST_PATH
 
 
