@@ -30,16 +30,12 @@ class _Ctx:
     def __init__(self, needs_input_grad=()) -> None:
         self.needs_input_grad = tuple(needs_input_grad)
         self.saved_tensors = ()
-        self.leaf = False
         self.gate_slot = self.slot = None  # traced graphs pass d_gates in the gates' dtype (no fp32 side channel)
 
     def save_for_backward(self, *tensors) -> None:
         self.saved_tensors = tensors
 
     def mark_non_differentiable(self, *tensors) -> None:
-        pass
-
-    def set_materialize_grads(self, value: bool) -> None:
         pass
 
 
