@@ -19,11 +19,11 @@ constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxCountBins = 16384;
 constexpr int kMaxSortBins = 4096;
-// The sort's table of counts holds at most this many words (bins * blocks). Half as many: 524,288 ids over 128 experts 17.7 ->
-// 17.9 us, 32,768 over 513 16.4 -> 20.6, 131,072 over 4,096 97 -> 161.
+// The sort's table of counts holds at most this many words (bins * blocks). Half as many: 524,288 ids over 128 experts 1 %
+// slower, 32,768 over 513 1.26 times, 131,072 over 4,096 1.66 times.
 constexpr int kSortTableWords = 32768;
 constexpr int kSortMaxBlocks = 256;            // one per CU
-constexpr int64_t kSortIdsPerBlock = 1024;     // 2,048: 32,768 ids over 64 experts 10.0 -> 10.7 us, 65,536 over 128 10.8 -> 12.3
+constexpr int64_t kSortIdsPerBlock = 1024;     // 2,048: 32,768 ids over 64 experts 7 % slower, 65,536 over 128 14 %
 
 // Exclusive scan, in place, of data[0..n) (LDS) by a block of BLOCK threads. Returns the total. tmp: BLOCK / kWave words.
 template <int BLOCK = kBlock>
@@ -59,10 +59,10 @@ __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
   return total;
 }
 
-// Returns true in every thread of exactly one block: the last one to arrive. Blocks must have made their global
-// writes before calling; the caller may read other blocks' writes after a true return. Blocks publish their data only through device-scope atomics: those are coherent across the XCDs by themselves and are
-// complete once the barrier below has drained the wave's memory counters, so the L2 write-back + invalidate of a full fence
-// (about 0.2 us per block, serialised) is not needed.
+// Returns true in every thread of exactly one block: the last one to arrive. Blocks must have made their global writes before
+// calling; the caller may read other blocks' writes after a true return. Blocks publish their data only through device-scope
+// atomics: those are coherent across the XCDs by themselves and are complete once the barrier below has drained the wave's
+// memory counters, so the L2 write-back + invalidate of a full fence (about 0.2 us per block, serialised) is not needed.
 __device__ bool last_block_ticket(uint32_t* ticket, uint32_t* lds_flag) {
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -317,9 +317,9 @@ __global__ __launch_bounds__(WAVES * kWave) void sort_hist_kernel(const id_t* __
 // fence and ticket, and wrote it back for the second launch; here the launch boundary is the only wait between blocks, the
 // table has one row per block instead of per wave, and reading all of it takes a block less time than the hand-over did.
 // The blocks' number is free of that one block's scan, so that a wave ranks 64 to 256 ids instead of 1,024 to 4,096.
-// Measured, both launches, before -> now (host included, under which a call does not get below 9.8 us): 8,192 ids over 64
-// experts 17.8 -> 9.8 us, 32,768 over 64 20.8 -> 10.0, 32,768 over 512 64 -> 12.8, 524,288 over 128 94 -> 17.7, 2,000,003 over
-// 60 135 -> 32, 131,072 over 4,096 488 -> 97.
+// Measured, both launches, 50 sorts in a replayed graph (no host time), before -> now: 8,192 ids over 64 experts 17.7 -> 9.2 us,
+// 32,768 over 64 21.2 -> 9.8, 32,768 over 512 64 -> 12.6, 65,536 over 128 39.9 -> 10.6, 524,288 over 128 99 -> 18.1, 2,000,003
+// over 60 150 -> 35, 131,072 over 4,096 494 -> 96.
 template <typename id_t, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void sort_scatter_kernel(
     const id_t* __restrict__ ids, int64_t R, int E, int64_t seg_len, int id_bits, int align, int64_t max_tiles,
@@ -415,9 +415,9 @@ __global__ __launch_bounds__(WAVES * kWave) void sort_scatter_kernel(
 
 // The whole sort in one block and one launch, for the few ids of a decoding step or a small batch. What bounds it: latency.
 // An id is read once and stays in registers, and the table in LDS; the second launch and the way of the table through memory
-// go. Measured, a call behind others on its stream: 16 / 512 / 4,096 ids over 64 experts 4.6 / 4.8 / 9.2 us, over 512 experts
-// 7.6 / 8.0 / 13.3. The line: at 4,096 ids over 64 experts 8.6 us against the two launches' 9.8, and past it one block's
-// rounds of 64 take longer than launches that spread them over the chip.
+// go. Measured, 50 sorts in a replayed graph, one launch against two: 16 / 512 / 4,096 ids over 64 experts 4.5 / 4.7 / 8.9
+// against 7.6 / 7.7 / 9.0 us, over 512 experts 7.6 / 8.0 / 13.0 against 9.5 / 9.9 / 11.3. The line lies where the two meet for
+// few experts; past it one block's rounds of 64 take longer than launches that spread them over the chip.
 constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallPer = 4;                                  // ids per lane
 constexpr int kSmallIds = kSmallBlock * kSmallPer;            // R up to which the one-block sort runs, up to kSmallBins bins
@@ -730,7 +730,7 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
   }
   const SortPlan p = make_sort_plan(R, E);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  uint32_t* table = workspace + 1;  // word 0 stays zero, as the interface says
+  uint32_t* table = workspace + 1;  // word 0 is left alone
 #define CK_LAUNCH_SORT(ID_T, WAVES)                                                                                            \
   do {                                                                                                                         \
     const ID_T* ids = static_cast<const ID_T*>(expert_ids);                                                                    \

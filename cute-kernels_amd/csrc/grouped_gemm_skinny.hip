@@ -17,9 +17,10 @@
 //  * the activations, a few hundred KiB for the whole launch, are re-read by every column tile from L2.
 // An expert with more rows than a tile has several tiles; they are neighbours in launch order on one XCD, so that the
 // second reads the weights from that XCD's L2.
-// Measured, launch included: 8 experts of 28,672 x 4,096 with 2 rows each 317 us = 5.9 TB/s of weights, 8 x 4,096 x 14,336
-// 163 us = 5.8 TB/s, 64 x 2,816 x 2,048 with 8 rows 136 us = 5.4 TB/s (128-row tiles of the general kernel: 179 us), e4m3
-// 128 x 3,072 x 4,096 with 8 rows 288 us = 5.6 TB/s and 128 x 4,096 x 1,536 156 us = 5.2 TB/s (256-row tiles: 348, 205 us).
+// Measured (kernel trace; the rate is the weights' bytes by the time): 8 experts of 28,672 x 4,096 with 2 rows each 308 us =
+// 6.1 TB/s, 8 x 4,096 x 14,336 163 us = 5.8, 64 x 2,816 x 2,048 with 8 rows 130 us = 5.7 (128-row tiles of the general kernel:
+// 179), 64 x 2,048 x 1,408 69 us = 5.3, e4m3 128 x 3,072 x 4,096 with 8 rows 281 us = 5.7 and 128 x 4,096 x 1,536 157 us = 5.1
+// (256-row tiles: 348, 205). The memory reads 1.01 to 1.13 times the weights' bytes, most where the activations weigh most.
 #include "gemm_common.h"
 
 namespace ck {
