@@ -115,7 +115,7 @@ int ck_route_topk_softmax_bwd_exact(const float* gates, const float* d_gates_exa
  *                         are left unwritten
  *   tile_expert[max_tiles] -- expert that owns rows [t*align, (t+1)*align) of the padded layout, -1 past the end
  * max_rows = ck_sort_max_rows(R, E, align), max_tiles = max_rows / align.
- * workspace: ck_sort_workspace_words(R, E) uint32 words; word 0 must be zero on entry and is zero again on exit.
+ * workspace: ck_sort_workspace_words(R, E) uint32 words, no initial contents required.
  * ------------------------------------------------------------------------------------------------------------- */
 int64_t ck_sort_max_rows(int64_t R, int32_t E, int32_t align);
 int64_t ck_sort_workspace_words(int64_t R, int32_t E);
