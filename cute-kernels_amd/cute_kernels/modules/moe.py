@@ -192,17 +192,20 @@ class MoE(nn.Module):
         selected, _, values = route_topk_softmax_raw(x, self.top_k)
         return values, selected.long()
 
+    def _needs_grad(self, hidden_states: torch.Tensor, router_weights: torch.Tensor) -> bool:
+        """Whether a backward pass may come through the experts. An activation that is the caller's own may hold parameters."""
+        if hidden_states.requires_grad or router_weights.requires_grad:
+            return True
+        if self.act is not swiglu_packed_cute and type(self.act) not in (torch.nn.GLU, torch.nn.GELU):
+            return True
+        return any(p.requires_grad for p in (*self.c_fc.parameters(), *self.c_proj.parameters()))
+
     def _compute_experts(
         self, hidden_states: torch.Tensor, router_weights: torch.Tensor, selected_experts: torch.Tensor
     ) -> torch.Tensor:
         if hidden_states.size(0) == 0:  # no tokens: nothing to sort or multiply; the result stays in the autograd graph
             return hidden_states * 0
-        weights = (self.c_fc.weight, self.c_proj.weight, self.c_fc.bias, self.c_proj.bias)
-        # with gradients enabled, an activation of the caller's may hold parameters of its own
-        inference = not torch.is_grad_enabled() or (
-            (self.act is swiglu_packed_cute or type(self.act) in (torch.nn.GLU, torch.nn.GELU))
-            and not any(t is not None and t.requires_grad for t in (hidden_states, router_weights, *weights))
-        )
+        inference = not (torch.is_grad_enabled() and self._needs_grad(hidden_states, router_weights))
         align = choose_align(
             plain_size(selected_experts.numel()), self.num_experts, hidden_states.dtype, inference,
             (self.hidden_size, self.intermediate_size, self.is_glu),

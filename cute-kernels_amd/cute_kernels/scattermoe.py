@@ -170,18 +170,46 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tupl
     return 256 if cost[256] < cost[128] else 128
 
 
-_height_of_large_tiles_kept = functools.lru_cache(4096)(_height_of_large_tiles)  # a function of sizes alone
+def _plain_tiles(num_rows: int, num_experts: int) -> int:
+    return 256 if num_rows >= 512 * num_experts else 128
 
 
 def _large_tiles(
-    num_rows: int, num_experts: int, dtype: torch.dtype, launches: tuple[tuple[int, int, bool, bool], ...]
+    num_rows: int, num_experts: int, dtype: torch.dtype | None, launches: tuple[tuple[int, int, bool, bool], ...], many: bool
 ) -> int:
-    # fp32 GEMMs run on 64-row tiles either way. A traced row count that stands for many takes part in one comparison only,
-    # so that a graph is compiled for two ranges of it and no more.
-    many = is_tracing() and not statically_known_true(num_rows < 1 << 48)
-    if dtype is torch.float32 or many or num_rows >= 512 * num_experts:
-        return 256 if num_rows >= 512 * num_experts else 128
-    return (_height_of_large_tiles if is_tracing() else _height_of_large_tiles_kept)(num_rows, num_experts, launches)
+    if many or dtype is torch.float32 or num_rows >= 512 * num_experts:  # fp32 GEMMs run on 64-row tiles either way
+        return _plain_tiles(num_rows, num_experts)
+    return _height_of_large_tiles(num_rows, num_experts, launches)
+
+
+def _layer_tiles(
+    num_rows: int, num_experts: int, dtype: torch.dtype | None, inference: bool, widths: tuple[int, int, bool] | None, many: bool
+) -> int:
+    if dtype is torch.float32 or (widths is None and not inference):
+        return _plain_tiles(num_rows, num_experts)
+    if inference and not many:
+        for rows, align in SMALL_TILES:
+            if num_rows <= rows * num_experts:
+                return align
+    if widths is None:
+        return 256
+    hidden, inter, gated = widths
+    c_fc = 2 * inter if gated else inter
+    launches = ((c_fc, hidden, not gated, False), (hidden, inter, True, False))
+    if not inference:
+        launches += ((inter, hidden, True, True), (hidden, c_fc, True, True))
+    return _large_tiles(num_rows, num_experts, dtype, launches, many)
+
+
+_large_tiles_kept, _layer_tiles_kept = functools.lru_cache(4096)(_large_tiles), functools.lru_cache(4096)(_layer_tiles)
+
+
+def _height(rule, kept, num_rows: int, *rest) -> int:
+    """A rule of sizes alone, looked up where it has been asked before. A traced row count that stands for many takes part in
+    one comparison only (many), so that a graph is compiled for two ranges of it and no more."""
+    if not is_tracing():
+        return kept(num_rows, *rest, False)
+    return rule(num_rows, *rest, not statically_known_true(num_rows < 1 << 48))
 
 
 def choose_align(
@@ -200,20 +228,7 @@ def choose_align(
     607 / - / 872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 /
     661, 609, 596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us. Without widths, 256 rows beyond: the e4m3 GEMMs have
     tiles of 16, 32, 64 and 256 rows."""
-    if dtype is torch.float32 or (widths is None and not inference):
-        return 256 if num_rows >= 512 * num_experts else 128
-    if inference and not (is_tracing() and not statically_known_true(num_rows < 1 << 48)):
-        for rows, align in SMALL_TILES:
-            if num_rows <= rows * num_experts:
-                return align
-    if widths is None:
-        return 256
-    hidden, inter, gated = widths
-    c_fc = 2 * inter if gated else inter
-    launches = ((c_fc, hidden, not gated, False), (hidden, inter, True, False))
-    if not inference:
-        launches += ((inter, hidden, True, True), (hidden, c_fc, True, True))
-    return _large_tiles(num_rows, num_experts, dtype, launches)
+    return _height(_layer_tiles, _layer_tiles_kept, num_rows, num_experts, dtype, inference, widths)
 
 
 def sort_by_expert(
@@ -228,7 +243,7 @@ def sort_by_expert(
     on a mismatch; it costs a device-to-host read, so the layer does not ask for it."""
     assert expert_ids.dtype in (torch.int32, torch.long)
     if align is None:
-        align = choose_align(plain_size(expert_ids.numel()), num_experts)
+        align = _plain_tiles(plain_size(expert_ids.numel()), num_experts)
     if is_tracing():
         return _ops.sort_by_expert_segments(expert_ids, num_experts, align)
     seg = _sort_by_expert_eager(expert_ids, num_experts, align)
@@ -492,7 +507,7 @@ def segments_from_sorted(
     assert expert_offsets.dim() == 1 and expert_offsets.dtype in (torch.int32, torch.uint32, torch.long)
     R, E = sorted_expert_idxs.numel(), expert_offsets.numel()
     if align is None:
-        align = choose_align(R, E)
+        align = _plain_tiles(R, E)
     tensors = (sorted_expert_idxs, sorted_scattered_idxs, expert_offsets)
     versions = tuple(t._version for t in tensors)
     for entry in _segments_cache:
@@ -625,7 +640,7 @@ def scattered_experts(
     launches = ((N, K, True, False),)
     if torch.is_grad_enabled() and inputs.requires_grad:
         launches += ((K, N, True, True),)
-    align = _large_tiles(plain_size(sorted_expert_idxs.numel()), E, inputs.dtype, launches)
+    align = _height(_large_tiles, _large_tiles_kept, plain_size(sorted_expert_idxs.numel()), E, inputs.dtype, launches)
     if is_tracing():
         out = _ops.scattered_experts(
             inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align

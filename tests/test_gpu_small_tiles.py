@@ -7,6 +7,7 @@ import torch.nn.functional as F
 
 import cute_kernels
 from cute_kernels import _C, fp8, scattermoe
+from cute_kernels.modules import moe as moe_module
 from oracle import moe_oracle as mo
 
 pytestmark = pytest.mark.gpu
@@ -99,16 +100,17 @@ def test_small_tiles_fp8(device, align, T, K, N):
 
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("rows", [31, 100, 101, 300])
-def test_inference_on_128_row_tiles_matches_the_training_forward(device, gated, rows):
-    """Narrow layers between the small tiles and 512 rows per expert: the same sums as on the 256-row tiles that a backward
-    pass takes, in another order at most."""
+def test_inference_on_128_row_tiles_matches_a_forward_on_256(device, monkeypatch, gated, rows):
+    """Narrow layers between the small tiles and 512 rows per expert: the same sums as on 256-row tiles with what a backward
+    pass needs kept, in another order at most."""
     E, H, I = 8, 256, 320
     assert scattermoe.choose_align(rows * E, E, torch.bfloat16, True, (H, I, gated)) == 128
     torch.manual_seed(rows)
     act = cute_kernels.swiglu_packed_cute if gated else torch.nn.GELU(approximate="tanh")
     moe = cute_kernels.MoE(E, 2, H, I, act, gated, not gated, 0.05).to(device, torch.bfloat16)
     x = torch.randn(rows * E // 2, H, device=device).to(torch.bfloat16)
-    want, _ = moe(x)
     with torch.no_grad():
         got, _ = moe(x)
+    monkeypatch.setattr(moe_module, "choose_align", lambda *args: 256)
+    want, _ = moe(x)
     torch.testing.assert_close(got.float(), want.detach().float(), rtol=RTOL, atol=ATOL)
