@@ -68,3 +68,46 @@ def test_graphs_that_count_do_not_depend_on_each_other(device):
             eager = cute_kernels.continuous_count_cute(ids, 60)
         torch.cuda.synchronize()
         assert torch.equal(eager.long(), want)
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu"])
+@pytest.mark.parametrize("tokens", [40, 700])  # tiles of 128 rows; of 256 rows with split last rounds
+def test_replays_of_a_training_step_of_the_experts(device, act, tokens):
+    """Forward and backward of the expert block in one graph (the backward launches from the autograd engine's thread), replayed
+    on other inputs with eager steps in between: outputs and gradients bit for bit those of an eager step."""
+    E, k, hidden, inter = 4, 2, 1024, 1024
+    g = torch.Generator(device=device).manual_seed(3)
+    rand = lambda *shape: torch.randn(*shape, device=device, generator=g)
+    w_fc = (0.03 * rand(E, 2 * inter if act == "swiglu" else inter, hidden)).bfloat16().requires_grad_()
+    w_proj = (0.03 * rand(E, hidden, inter)).bfloat16().requires_grad_()
+    ids = torch.stack([torch.randperm(E, device=device, generator=g)[:k] for _ in range(tokens)]).int()
+    x, dy = rand(tokens, hidden).bfloat16().requires_grad_(), rand(tokens, hidden).bfloat16()
+    gates = torch.rand(tokens, k, device=device, generator=g).bfloat16().requires_grad_()
+    leaves = (x, gates, w_fc, w_proj)
+    align = 128 if tokens < 100 else 256
+
+    def step():
+        seg = cute_kernels.sort_by_expert(ids, E, align)
+        if act == "swiglu":
+            y = scattermoe.swiglu_experts(x, w_fc, w_proj, gates, seg)
+        else:
+            y = scattermoe.experts_up(x, w_fc, seg, k, gelu_tanh=True, down=(w_proj, gates, None))
+        return [y.detach(), *torch.autograd.grad(y, leaves, dy)]
+
+    warm = torch.cuda.Stream(device)
+    warm.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(warm):
+        step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for _ in range(4):
+        with torch.no_grad():
+            x.copy_(rand(tokens, hidden))
+            dy.copy_(rand(tokens, hidden))
+            w_fc.mul_(0.99)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, step()):
+            assert torch.equal(a, b)
