@@ -595,19 +595,21 @@ experts_down.register_autograd(_experts_down_bwd, setup_context=_experts_down_se
 @custom_op(f"{NS}::scattered_experts", mutates_args=())
 def scattered_experts(
     x: Tensor, w: Tensor, gates: Optional[Tensor], bias: Optional[Tensor], sorted_expert_idxs: Tensor,
-    sorted_scattered_idxs: Tensor, expert_offsets: Tensor, k: int, grouped_in: bool, grouped_out: bool, align: int,
+    sorted_scattered_idxs: Tensor, expert_offsets: Tensor, k: int, grouped_in: bool, grouped_out: bool,
+    align: int = 0,
 ) -> tuple[Tensor, Tensor]:
-    """(out, the ungated rows [R, N] that the gates' gradient needs, or empty)"""
+    """(out, the ungated rows [R, N] that the gates' gradient needs, or empty). align 0 (graphs saved before there was the
+    argument): by the sizes."""
     ctx = _Ctx()
     out = _moe._ScatteredExperts.forward(
         ctx, x, w, k, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, gates, grouped_in, grouped_out, bias,
-        align=align,
+        align=align or None,
     )
     return out, _or_empty(ctx.saved_tensors[3], x)
 
 
 @scattered_experts.register_fake
-def _(x, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align):
+def _(x, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align=0):
     R, N = sorted_expert_idxs.shape[0], w.shape[1]
     if gates is None:
         return x.new_empty(R, N), x.new_empty(0)
@@ -617,11 +619,11 @@ def _(x, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offse
 @custom_op(f"{NS}::scattered_experts_backward", mutates_args=())
 def scattered_experts_backward(
     grad_out: Tensor, x: Tensor, w: Tensor, gates: Optional[Tensor], expanded: Tensor, sorted_expert_idxs: Tensor,
-    sorted_scattered_idxs: Tensor, expert_offsets: Tensor, k: int, grouped_in: bool, grouped_out: bool, align: int, need_x: bool,
-    need_w: bool, need_gates: bool, need_bias: bool,
+    sorted_scattered_idxs: Tensor, expert_offsets: Tensor, k: int, grouped_in: bool, grouped_out: bool, need_x: bool,
+    need_w: bool, need_gates: bool, need_bias: bool, align: int = 0,
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     ctx = _Ctx((need_x, need_w, False, False, False, False, need_gates, False, False, need_bias, False, False))
-    ctx.seg = _moe.segments_from_sorted(sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, align)
+    ctx.seg = _moe.segments_from_sorted(sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, align or None)
     ctx.k, ctx.grouped_in, ctx.grouped_out = k, grouped_in, grouped_out
     ctx.saved_tensors = (x.contiguous(), w.contiguous(), None if gates is None else gates.contiguous(), expanded)
     grads = _moe._ScatteredExperts.backward(ctx, grad_out)
@@ -629,8 +631,8 @@ def scattered_experts_backward(
 
 
 @scattered_experts_backward.register_fake
-def _(grad_out, x, w, gates, expanded, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align,
-      need_x, need_w, need_gates, need_bias):
+def _(grad_out, x, w, gates, expanded, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out,
+      need_x, need_w, need_gates, need_bias, align=0):
     e = x.new_empty(0)
     return (
         torch.empty_like(x) if need_x else e,
@@ -644,13 +646,15 @@ def _scattered_experts_setup(ctx, inputs, output):
     x, w, gates, _bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, *rest = inputs
     ctx.has_gates = gates is not None
     ctx.save_for_backward(x, w, gates, output[1], sorted_expert_idxs, sorted_scattered_idxs, expert_offsets)
+    *rest, ctx.align = rest
     ctx.rest = tuple(rest)
 
 
 def _scattered_experts_bwd(ctx, grad_out, _expanded_grad):
     need_x, need_w, need_gates, need_bias = ctx.needs_input_grad[:4]
     d_x, d_w, d_gates, d_bias = scattered_experts_backward(
-        grad_out.contiguous(), *ctx.saved_tensors, *ctx.rest, need_x, need_w, need_gates and ctx.has_gates, need_bias
+        grad_out.contiguous(), *ctx.saved_tensors, *ctx.rest, need_x, need_w, need_gates and ctx.has_gates, need_bias,
+        ctx.align,
     )
     return (
         (d_x if need_x else None), (d_w if need_w else None), (d_gates if need_gates and ctx.has_gates else None),

@@ -145,3 +145,14 @@ def test_the_reference_interface(monkeypatch, dtype, rows, grad, height):
     with torch.set_grad_enabled(grad), pytest.raises(_Stop):
         call(x)
     assert seen == [height]
+
+
+def test_graphs_saved_without_a_height_still_call():
+    """The operators of the reference's interface took no `align` argument once."""
+    for op in (torch.ops.ck_mi355.scattered_experts, torch.ops.ck_mi355.scattered_experts_backward):
+        last = op.default._schema.arguments[-1]
+        assert last.name == "align" and last.default_value == 0
+    meta = lambda *s, dtype=BF16: torch.empty(*s, dtype=dtype, device="meta")
+    idx = lambda n: meta(n, dtype=torch.int64)
+    out, _ = torch.ops.ck_mi355.scattered_experts(meta(6, 16), meta(4, 8, 16), None, None, idx(12), idx(12), idx(4), 2, False, False)
+    assert out.shape == (12, 8)
