@@ -209,18 +209,76 @@ __device__ inline void store4(T* p, T v0, T v1, T v2, T v3) {
   *reinterpret_cast<uint2*>(p) = u;
 }
 
-// Tile order inside a run of tiles: groups of 8 along `a` (the side with a_count tiles), then `b`, with `a` fastest
+// Tile order inside a run of tiles: groups of at most 8 along `a` (the side with a_count tiles), then `b`, with `a` fastest
 // inside a group -- 32 consecutive tiles form an 8 x 4 block that shares 8 + 4 operand panels.
 // (measured at 4 / 8 / 16 / 32 tiles per group on the Mixtral-shape and fine-grained layers: 8 is fastest on both)
+// The groups are of even height (9 tiles are 5 + 4): a last group of one tile would share 1 + 32 panels.
+template <int GROUP = 8>
 __device__ inline void grouped_order(int r, int a_count, int b_count, int& a, int& b) {
-  constexpr int GROUP = 8;
-  const int group_sz = GROUP * b_count;
-  const int g = r / group_sz;
-  const int first = g * GROUP;
-  const int in_group = min(GROUP, a_count - first);
-  const int q = r - g * group_sz;
-  b = q / in_group;
-  a = first + (q - b * in_group);
+  const int groups = (a_count + GROUP - 1) / GROUP;
+  const int low = a_count / groups, taller = a_count - low * groups;  // `taller` groups of low + 1, then groups of low
+  const int taller_tiles = taller * (low + 1) * b_count;
+  int height = low, first = taller * (low + 1), q = r - taller_tiles;
+  if (q < 0) {
+    height = low + 1;
+    first = 0;
+    q = r;
+  }
+  const int group_sz = height * b_count;
+  const int g = q / group_sz;
+  q -= g * group_sz;
+  b = q / height;
+  a = first + g * height + (q - b * height);
+}
+
+// Tile `pid` of a forward launch's (m tiles x n_tiles) live tiles. Each XCD takes a contiguous run of them (workgroups are
+// dealt round-robin to the XCDs; the ragged end keeps its order), and the run goes expert by expert, each in groups
+// of its own m tiles: the 32 tiles an XCD computes at a time read one expert's weights where groups over all m tiles read
+// those of every expert the 8 m tiles belong to (4 tiles per expert: 4 + 8 operand panels against 8 + 8). 64 experts of
+// 2,048 x 1,408 at 1,024 rows each: 357 -> 346 us; 16 of 14,336 x 4,096: 1,557 -> 1,518, input gradients 1,537 -> 1,497.
+__device__ inline void forward_tile(const GemmParams& prm, int pid, int total, int& mt, int& nt, int& expert) {
+  const int per_xcd = total / kXcds;
+  if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;
+  expert = prm.tile_expert[pid / prm.n_tiles];  // an expert's tiles are consecutive: n_tiles for each of its m tiles
+  const int first = prm.seg_starts[expert] / prm.align, end = prm.seg_starts[expert + 1] / prm.align;
+  grouped_order(pid - first * prm.n_tiles, end - first, prm.n_tiles, mt, nt);
+  mt += first;
+}
+
+// Tile `pid` of a weight-gradient launch: `position` of its expert in the launch's order of experts, and its place in that
+// expert's m_tiles x n_tiles grid. Experts differ in contraction length, and which XCD computes a workgroup is fixed by its
+// index, so every XCD has to get its share of every length.
+// A grid of 4 or more tiles per XCD along its longer side is cut in 8 along it: the 32 tiles an XCD computes at a time are
+// then one s x 32 / s block (s = 4: 4 + 8 operand panels) and the shares are equal. Smaller grids (or sides that 8 does not
+// divide) would leave an XCD one row of an expert's tiles, or every eighth tile: 36 panels for 32 tiles of 11 x 8 per
+// expert. They go out in chunks of 16 consecutive tiles, 4 x 4 blocks of one expert, over the XCDs and back (8 + 8 panels;
+// the experts are sorted by length, so that turning back evens the shares out). 64 experts of 2,816 x 2,048 at 400 / 1,024 /
+// 2,048 rows each: 496 / 806 / 1,398 us -> 481 / 777 / 1,329, with Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393;
+// 32 of 2,048 x 2,048 178 / 282 / 498 -> 165 / 270 / 476. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at
+// even loads and 5 to 10 % slower at Zipf(0.8): too few of them to even out. Chunks on grids of 56 or 112 tiles along the
+// longer side lost 2 to 5 % to the slices.
+__device__ inline void dw_tile(const GemmParams& prm, int pid, int& position, int& mt, int& nt) {
+  constexpr int CHUNK = 16, CHUNK_HEIGHT = 4;
+  const bool m_major = prm.m_tiles >= prm.n_tiles;
+  const int major = m_major ? prm.m_tiles : prm.n_tiles, minor = m_major ? prm.n_tiles : prm.m_tiles;
+  const int xcd = pid % kXcds, j = pid / kXcds;
+  int a, b;
+  if (major % kXcds == 0 && major / kXcds >= CHUNK_HEIGHT) {
+    const int slice = major / kXcds, per_slice = slice * minor;
+    position = j / per_slice;
+    grouped_order(j - position * per_slice, slice, minor, a, b);
+    a += xcd * slice;
+  } else {
+    const int per_expert = major * minor, total = per_expert * prm.num_experts;
+    if (pid < total / (kXcds * CHUNK) * (kXcds * CHUNK)) {  // the last, partial round keeps its order
+      const int round = j / CHUNK;
+      pid = (round * kXcds + ((round & 1) ? kXcds - 1 - xcd : xcd)) * CHUNK + j % CHUNK;
+    }
+    position = pid / per_expert;
+    grouped_order<CHUNK_HEIGHT>(pid - position * per_expert, major, minor, a, b);
+  }
+  mt = m_major ? a : b;
+  nt = m_major ? b : a;
 }
 
 

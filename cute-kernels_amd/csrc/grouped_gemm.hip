@@ -65,40 +65,19 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int wm = wave >> 1, wn = wave & 1;
 
-  // ---- which tile: blocks are dealt round-robin to the 8 XCDs, so give each XCD a contiguous run of tiles
+  // ---- which tile (XCD-aware orders: gemm_common.h)
   int mt, nt, expert;
   int64_t k_begin = 0;
   int k_len;
   if constexpr (MODE == kDw) {
-    // Experts differ in contraction length (their row counts), so every XCD gets a slice of EVERY expert's tile grid:
-    // the grid is cut in 8 along its longer side, and a slice is walked in groups of 8 tiles along that side.
-    const int per_expert = prm.m_tiles * prm.n_tiles;
-    const bool m_major = prm.m_tiles >= prm.n_tiles;
-    const int major = m_major ? prm.m_tiles : prm.n_tiles, minor = m_major ? prm.n_tiles : prm.m_tiles;
-    int pid = blockIdx.x, a, b;  // a: index along the major side, b: along the minor side
-    if (major % kXcds == 0) {
-      const int xcd = pid % kXcds, j = pid / kXcds;
-      const int slice = major / kXcds, per_slice = slice * minor;
-      expert = j / per_slice;
-      grouped_order(j - expert * per_slice, slice, minor, a, b);
-      a += xcd * slice;
-    } else {
-      expert = pid / per_expert;
-      grouped_order(pid - expert * per_expert, major, minor, a, b);
-    }
-    mt = m_major ? a : b;
-    nt = m_major ? b : a;
+    dw_tile(prm, blockIdx.x, expert, mt, nt);
     k_begin = prm.seg_starts[expert];
     k_len = (int)((prm.counts[expert] + BK - 1) / BK * BK);
   } else {
     const int live_m = prm.seg_starts[prm.num_experts] / prm.align;
     const int total = live_m * prm.n_tiles;
-    int pid = blockIdx.x;
-    if (pid >= total) return;
-    const int per_xcd = total / kXcds;
-    if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;  // the ragged end keeps its order
-    grouped_order(pid, live_m, prm.n_tiles, mt, nt);
-    expert = prm.tile_expert[mt];
+    if ((int)blockIdx.x >= total) return;
+    forward_tile(prm, blockIdx.x, total, mt, nt, expert);
     k_len = prm.K;
   }
   const int64_t m0 = (int64_t)mt * BM;

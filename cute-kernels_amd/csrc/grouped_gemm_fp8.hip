@@ -57,16 +57,13 @@ __global__ __launch_bounds__(NT) void grouped_gemm_fp8_kernel(const GemmParams p
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave >> 1, wn = wave & 1;
 
-  // ---- which tile (same XCD-aware order as the 16-bit kernel)
+  // ---- which tile (XCD-aware order: gemm_common.h)
   const int live_m = prm.seg_starts[prm.num_experts] / prm.align;
   const int total = live_m * prm.n_tiles;
-  int pid = blockIdx.x;
+  const int pid = blockIdx.x;
   if (pid >= total) return;
-  const int per_xcd = total / kXcds;
-  if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;
-  int mt, nt;
-  grouped_order(pid, live_m, prm.n_tiles, mt, nt);
-  const int expert = prm.tile_expert[mt];
+  int mt, nt, expert;
+  forward_tile(prm, pid, total, mt, nt, expert);
   const int64_t m0 = (int64_t)mt * BM;
   const int64_t valid_end = (int64_t)prm.seg_starts[expert] + prm.counts[expert];
 

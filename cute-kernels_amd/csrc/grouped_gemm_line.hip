@@ -82,29 +82,14 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
   [[maybe_unused]] uint64_t st_begin = 0, st_loop = 0, st_end = 0, st_vm = 0, st_bar = 0, st_s0 = 0, st_s1 = 0, st_mark = 0;
   if constexpr (CK_STAMP != 0) st_begin = clock64();
 
-  // ---- which tile (same XCD-aware orders as the 256 x 256 kernel)
+  // ---- which tile (XCD-aware orders: gemm_common.h)
   constexpr bool kSplit = WGM == 2 && (MODE == kGrouped || MODE == kScatter);  // see the split below
   int mt, nt, expert;
   int64_t k_begin = 0;
   int k_len;
   [[maybe_unused]] int split_slot = -1, split_part = -1, split_parts = kSplitParts;
   if constexpr (MODE == kDw) {
-    const int per_expert = prm.m_tiles * prm.n_tiles;
-    const bool m_major = prm.m_tiles >= prm.n_tiles;
-    const int major = m_major ? prm.m_tiles : prm.n_tiles, minor = m_major ? prm.n_tiles : prm.m_tiles;
-    int pid = blockIdx.x, a, b;
-    if (major % kXcds == 0) {  // every XCD gets a slice of every expert's tile grid (experts differ in contraction length)
-      const int xcd = pid % kXcds, j = pid / kXcds;
-      const int slice = major / kXcds, per_slice = slice * minor;
-      expert = j / per_slice;
-      grouped_order(j - expert * per_slice, slice, minor, a, b);
-      a += xcd * slice;
-    } else {
-      expert = pid / per_expert;
-      grouped_order(pid - expert * per_expert, major, minor, a, b);
-    }
-    mt = m_major ? a : b;
-    nt = m_major ? b : a;
+    dw_tile(prm, blockIdx.x, expert, mt, nt);
     // `expert` so far is a position in the launch order. Experts differ in contraction length (their row counts), and
     // the hardware hands tiles out in block order: the longest contractions go first, so that the tiles still running
     // when the grid drains are the short ones (position r takes the expert with the r-th largest count, ties by index).
@@ -163,10 +148,7 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
       }
     }
     if (pid >= total) return;
-    const int per_xcd = total / kXcds;
-    if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;
-    grouped_order(pid, live_m, prm.n_tiles, mt, nt);
-    expert = prm.tile_expert[mt];
+    forward_tile(prm, pid, total, mt, nt, expert);
   }
   const int64_t m0 = (int64_t)mt * BM;
   int64_t valid_end = 0;  // forward modes: first pad row of this expert's segment

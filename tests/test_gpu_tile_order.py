@@ -1,0 +1,56 @@
+"""The order in which the workgroups of a grouped GEMM take its tiles: every tile of every expert once, whatever its number
+of row tiles (none, one, a whole group, one more than a group) and whichever split over the XCDs the grid gets."""
+
+import pytest
+import torch
+
+from cute_kernels import _C, scattermoe
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def _segments(counts, align=256):
+    ids = torch.arange(len(counts), dtype=torch.int32).repeat_interleave(torch.tensor(counts)).to(DEV)
+    return scattermoe.sort_by_expert(ids, len(counts), align)
+
+
+def _operand(seg, width, counts, g):
+    """Padded grouped rows with small whole numbers, so that products and sums are exact; and the rows of every expert."""
+    a = torch.full((seg.max_rows, width), float("nan"), dtype=torch.bfloat16)
+    starts = seg.seg_starts.cpu().tolist()
+    for e, c in enumerate(counts):
+        a[starts[e] : starts[e] + c] = torch.randint(-2, 3, (c, width), generator=g).to(torch.bfloat16)
+    return a.to(DEV), [a[starts[e] : starts[e] + c].float() for e, c in enumerate(counts)]
+
+
+@pytest.mark.parametrize("columns", [264, 2816])  # 2 and 11 column tiles
+@pytest.mark.parametrize("counts", [[2300, 0, 1, 256, 257, 2049], [0, 0, 5], [300] * 9])
+def test_forward_tiles(counts, columns):
+    g = torch.Generator().manual_seed(0)
+    seg = _segments(counts)
+    a, rows = _operand(seg, 64, counts, g)
+    w = torch.randint(-2, 3, (len(counts), columns, 64), generator=g).to(torch.bfloat16)
+    y = torch.full((seg.max_rows, columns), 1000.0, dtype=torch.bfloat16, device=DEV)
+    scattermoe._gemm(a, 0, w.to(DEV), seg, _C.CK_EPI_GROUPED, y)
+    y = y.cpu().float()
+    for e, c in enumerate(counts):
+        first = int(seg.seg_starts[e])
+        assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())  # |sum| <= 256: exact in bf16
+
+
+# tiles along the longer side: 32 (4 per XCD: slices), 16 and 11 (chunks of 16; 8 experts: 128 and 176 tiles, whole rounds of
+# chunks and a rest), 1; the longer side is the rows' or the columns'
+@pytest.mark.parametrize("M,N", [(8192, 256), (256, 4096), (2816, 512), (512, 2568), (256, 256)])
+@pytest.mark.parametrize("counts", [[70, 0, 64, 65, 1, 128, 3, 200], [33]])
+def test_weight_gradient_tiles(counts, M, N):
+    g = torch.Generator().manual_seed(1)
+    seg = _segments(counts)
+    a, a_rows = _operand(seg, M, counts, g)
+    b, b_rows = _operand(seg, N, counts, g)
+    dw = torch.full((len(counts), M, N), 1000.0, dtype=torch.bfloat16, device=DEV)
+    scattermoe._gemm_dw_rows(a, b, seg, dw)
+    for e in range(len(counts)):
+        expect = (a_rows[e].t().contiguous() @ b_rows[e]).to(torch.bfloat16)  # sums below 2^24: exact in fp32, one rounding
+        assert torch.equal(dw[e].cpu(), expect), e
