@@ -248,34 +248,42 @@ __device__ inline void forward_tile(const GemmParams& prm, int pid, int total, i
 // Tile `pid` of a weight-gradient launch: `position` of its expert in the launch's order of experts, and its place in that
 // expert's m_tiles x n_tiles grid. Experts differ in contraction length, and which XCD computes a workgroup is fixed by its
 // index, so every XCD has to get its share of every length.
-// A grid of 4 or more tiles per XCD along its longer side is cut in 8 along it: the 32 tiles an XCD computes at a time are
-// then one s x 32 / s block (s = 4: 4 + 8 operand panels) and the shares are equal. Smaller grids (or sides that 8 does not
-// divide) would leave an XCD one row of an expert's tiles, or every eighth tile: 36 panels for 32 tiles of 11 x 8 per
-// expert. They go out in chunks of 16 consecutive tiles, 4 x 4 blocks of one expert, over the XCDs and back (8 + 8 panels;
-// the experts are sorted by length, so that turning back evens the shares out). 64 experts of 2,816 x 2,048 at 400 / 1,024 /
-// 2,048 rows each: 496 / 806 / 1,398 us -> 481 / 777 / 1,329, with Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393;
-// 32 of 2,048 x 2,048 178 / 282 / 498 -> 165 / 270 / 476. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at
-// even loads and 5 to 10 % slower at Zipf(0.8): too few of them to even out. Chunks on grids of 56 or 112 tiles along the
-// longer side lost 2 to 5 % to the slices.
+// Chunks: runs of consecutive tiles (blocks of one expert's) go out over the XCDs and back; the experts are sorted by
+// length, so that turning back evens the shares out. Slices: every expert's grid is cut in 8 along its longer side, which
+// makes the shares equal, where each XCD gets 4 tiles or more of that side (4 + 8 operand panels for the 32 tiles an XCD
+// computes at a time). Smaller grids would leave an XCD one row of an expert's tiles, or every eighth tile: 36 panels for 32
+// tiles of 11 x 8 per expert.
+//   small grids: chunks of 16, 4 x 4 blocks (8 + 8 panels). 64 experts of 2,816 x 2,048 at 400 / 1,024 / 2,048 rows each: 496 /
+//     806 / 1,398 us -> 481 / 777 / 1,329, with Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393; 32 of 2,048 x 2,048 178 /
+//     282 / 498 -> 165 / 270 / 476. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at even loads and 5 to
+//     10 % slower at Zipf(0.8): too few of them to even out.
+//   large grids, 4,096 rows per expert and more: chunks of 32. All XCDs together then read 16 + 16 panels where slices read
+//     64 + 4, and the contraction is long enough for that to count. 8 experts of 28,672 x 4,096, slices / chunks at 1,024,
+//     2,048, 4,096, 8,192 rows each: 1,775 / 1,855, 3,029 / 3,079, 5,687 / 5,635, 11,342 / 10,958 us; Zipf(1.0) 1,768 / 1,821,
+//     3,080 / 3,079, 5,820 / 5,755, 11,393 / 11,066.
+template <int CHUNK, int HEIGHT>
+__device__ inline void dw_chunk_tile(int pid, int major, int minor, int num_experts, int& position, int& a, int& b) {
+  const int per_expert = major * minor, total = per_expert * num_experts;
+  if (pid < total / (kXcds * CHUNK) * (kXcds * CHUNK)) {  // the last, partial round keeps its order
+    const int xcd = pid % kXcds, j = pid / kXcds, round = j / CHUNK;
+    pid = (round * kXcds + ((round & 1) ? kXcds - 1 - xcd : xcd)) * CHUNK + j % CHUNK;
+  }
+  position = pid / per_expert;
+  grouped_order<HEIGHT>(pid - position * per_expert, major, minor, a, b);
+}
 __device__ inline void dw_tile(const GemmParams& prm, int pid, int& position, int& mt, int& nt) {
-  constexpr int CHUNK = 16, CHUNK_HEIGHT = 4;
   const bool m_major = prm.m_tiles >= prm.n_tiles;
   const int major = m_major ? prm.m_tiles : prm.n_tiles, minor = m_major ? prm.n_tiles : prm.m_tiles;
-  const int xcd = pid % kXcds, j = pid / kXcds;
   int a, b;
-  if (major % kXcds == 0 && major / kXcds >= CHUNK_HEIGHT) {
-    const int slice = major / kXcds, per_slice = slice * minor;
+  if (major % kXcds != 0 || major / kXcds < 4) {
+    dw_chunk_tile<16, 4>(pid, major, minor, prm.num_experts, position, a, b);
+  } else if (prm.seg_starts[prm.num_experts] / prm.num_experts >= 4096) {
+    dw_chunk_tile<32, 8>(pid, major, minor, prm.num_experts, position, a, b);
+  } else {
+    const int slice = major / kXcds, per_slice = slice * minor, j = pid / kXcds;
     position = j / per_slice;
     grouped_order(j - position * per_slice, slice, minor, a, b);
-    a += xcd * slice;
-  } else {
-    const int per_expert = major * minor, total = per_expert * prm.num_experts;
-    if (pid < total / (kXcds * CHUNK) * (kXcds * CHUNK)) {  // the last, partial round keeps its order
-      const int round = j / CHUNK;
-      pid = (round * kXcds + ((round & 1) ? kXcds - 1 - xcd : xcd)) * CHUNK + j % CHUNK;
-    }
-    position = pid / per_expert;
-    grouped_order<CHUNK_HEIGHT>(pid - position * per_expert, major, minor, a, b);
+    a += pid % kXcds * slice;
   }
   mt = m_major ? a : b;
   nt = m_major ? b : a;

@@ -40,10 +40,10 @@ def test_forward_tiles(counts, columns):
         assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())  # |sum| <= 256: exact in bf16
 
 
-# tiles along the longer side: 32 (4 per XCD: slices), 16 and 11 (chunks of 16; 8 experts: 128 and 176 tiles, whole rounds of
+# tiles along the longer side: 32 (4 per XCD: slices, or chunks of 32 from 4,096 rows per expert on), 16 and 11 (chunks of 16; 8 experts: 128 and 176 tiles, whole rounds of
 # chunks and a rest), 1; the longer side is the rows' or the columns'
 @pytest.mark.parametrize("M,N", [(8192, 256), (256, 4096), (2816, 512), (512, 2568), (256, 256)])
-@pytest.mark.parametrize("counts", [[70, 0, 64, 65, 1, 128, 3, 200], [33]])
+@pytest.mark.parametrize("counts", [[70, 0, 64, 65, 1, 128, 3, 200], [33], [4000, 4200, 0, 8300]])
 def test_weight_gradient_tiles(counts, M, N):
     g = torch.Generator().manual_seed(1)
     seg = _segments(counts)
