@@ -1,8 +1,10 @@
 // Router: top-k over the logits of one token + softmax over the k selected logits, and its backward.
 //
 // A token is owned by a group of G lanes (a power of two, chosen on the host); each lane keeps ceil(E / G) logits in registers as
-// 64-bit keys (order-preserving float bits in the high word, ~expert index in the low word), so "largest value, lowest
-// expert index on ties" is a plain integer max that a butterfly of lane shuffles reduces in log2(G) steps.
+// integer keys (order-preserving float bits in the high half, ~expert index in the low half), so "largest value, lowest
+// expert index on ties" is a plain integer max that a butterfly over the lanes reduces in log2(G) steps. A 16-bit logit and
+// its index fit one 32-bit key, whose butterfly inside 16 lanes is one v_max with a DPP operand per step; fp32 logits take
+// 64-bit keys and two shuffles per step.
 #include "ck_common.h"
 
 namespace ck {
@@ -12,22 +14,76 @@ constexpr int kBlock = 256;
 constexpr int kMaxPerLane = 16;  // E <= 64 * 16
 constexpr int kMaxTopK = 32;
 
-__device__ inline uint32_t float_order_bits(float v) {
-  if (v != v) return 0xffffffffu;  // NaN sorts above everything, as torch does
-  v += 0.0f;                       // -0.0 -> +0.0 so that the two zeros tie
-  const uint32_t u = __float_as_uint(v);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
+// Key<T>: the sort key of a logit with its expert, the logit and the expert of a key. A key is never 0 (a real expert index is
+// below the low half's maximum).
+template <typename T>
+struct Key {  // 16-bit logits
+  typedef uint32_t type;
+  __device__ static type make(T value, int e) {
+    const float v = Elem<T>::up(value);
+    uint32_t u = (uint32_t)__builtin_bit_cast(unsigned short, value);
+    if (u == 0x8000u) u = 0;                                // -0.0 -> +0.0 so that the two zeros tie
+    u = (u & 0x8000u) ? (~u & 0xffffu) : (u | 0x8000u);
+    if (v != v) u = 0xffffu;                                // NaN sorts above everything, as torch does
+    return (u << 16) | (0xffffu - (uint32_t)e);
+  }
+  __device__ static float value(type key) {  // -0.0 comes back as +0.0
+    const uint32_t u = key >> 16;
+    return Elem<T>::up(__builtin_bit_cast(T, (unsigned short)((u & 0x8000u) ? (u & 0x7fffu) : (~u & 0xffffu))));
+  }
+  __device__ static uint32_t expert(type key) { return 0xffffu - (key & 0xffffu); }
+};
+template <>
+struct Key<float> {
+  typedef uint64_t type;
+  __device__ static type make(float v, int e) {
+    uint32_t u = 0xffffffffu;
+    if (v == v) {
+      u = __float_as_uint(v + 0.0f);
+      u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    }
+    return ((uint64_t)u << 32) | (uint32_t)(0xffffffffu - (uint32_t)e);
+  }
+  __device__ static float value(type key) {
+    const uint32_t u = (uint32_t)(key >> 32);
+    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+  }
+  __device__ static uint32_t expert(type key) { return 0xffffffffu - (uint32_t)key; }
+};
 
-// the value behind float_order_bits (-0.0 comes back as +0.0)
-__device__ inline float float_from_order_bits(uint32_t u) {
-  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+// the largest key of a group of G consecutive lanes, in all of them
+__device__ inline uint64_t group_max(uint64_t best, int G) {
+  for (int off = G >> 1; off > 0; off >>= 1) {
+    const uint32_t lo = __shfl_xor((uint32_t)best, off, kWave);
+    const uint32_t hi = __shfl_xor((uint32_t)(best >> 32), off, kWave);
+    const uint64_t other = ((uint64_t)hi << 32) | lo;
+    best = other > best ? other : best;
+  }
+  return best;
+}
+template <int CTRL>
+__device__ inline uint32_t max_dpp(uint32_t v) {
+  const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);
+  return other > v ? other : v;
+}
+__device__ inline uint32_t group_max(uint32_t best, int G) {
+  // lanes that differ in bit 0, bit 1, then the mirror images inside 8 and 16 lanes (whose halves are uniform by then)
+  if (G > 1) best = max_dpp<0xB1>(best);   // quad_perm 1 0 3 2
+  if (G > 2) best = max_dpp<0x4E>(best);   // quad_perm 2 3 0 1
+  if (G > 4) best = max_dpp<0x141>(best);  // row_half_mirror
+  if (G > 8) best = max_dpp<0x140>(best);  // row_mirror
+  for (int off = 16; off < G; off <<= 1) {
+    const uint32_t other = __shfl_xor(best, off, kWave);
+    best = other > best ? other : best;
+  }
+  return best;
 }
 
 // What bounds it: latency. A token's k selections depend on each other, so everything inside one is kept short: the selected
 // logit comes back out of its key (a second read of the row was a memory round trip per selection) and the exponentials
 // stay in registers until the denominator is known (KMAX of them; the group's lanes all hold them). Every output a caller
-// wants is written here, the 16-bit gates and 64-bit ids included: each was a launch of its own behind this one.
+// wants is written here, the 16-bit gates and 64-bit ids included: each was a launch of its own behind this one. Lane j of a
+// group of k lanes or more writes selection j, so that a store instruction takes whole groups.
 // KMAX: upper bound of k in this instantiation.
 template <typename T, int PER, int KMAX>
 __global__ __launch_bounds__(kBlock) void route_topk_softmax_kernel(const T* __restrict__ logits, int64_t T_tokens,
@@ -40,46 +96,56 @@ __global__ __launch_bounds__(kBlock) void route_topk_softmax_kernel(const T* __r
   const bool live = token < T_tokens;
   const T* row = logits + (live ? token : 0) * (int64_t)E;
 
-  uint64_t key[PER];
+  typedef typename Key<T>::type key_t;
+  key_t key[PER];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     const int e = p * G + lane_in_group;  // consecutive lanes read consecutive experts
-    key[p] = 0ull;                        // below every real key (real keys have a non-zero low word or high word)
-    if (live && e < E) {
-      const float v = Elem<T>::up(row[e]);
-      key[p] = ((uint64_t)float_order_bits(v) << 32) | (uint32_t)(0xffffffffu - (uint32_t)e);
-    }
+    key[p] = 0;                           // below every real key
+    if (live && e < E) key[p] = Key<T>::make(row[e], e);
   }
 
   float vmax = 0.f, denom = 0.f, ex[KMAX];
-  const bool writer = live && lane_in_group == 0;
+  const bool by_lane = G >= k;  // uniform
+  uint32_t my_expert = 0;
+  float my_ex = 0.f;
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j >= k) break;
-    uint64_t best = 0ull;
+    key_t best = 0;
 #pragma unroll
     for (int p = 0; p < PER; ++p) best = key[p] > best ? key[p] : best;
-    for (int off = G >> 1; off > 0; off >>= 1) {
-      const uint32_t lo = __shfl_xor((uint32_t)best, off, kWave);
-      const uint32_t hi = __shfl_xor((uint32_t)(best >> 32), off, kWave);
-      const uint64_t other = ((uint64_t)hi << 32) | lo;
-      best = other > best ? other : best;
-    }
-    const uint32_t e = 0xffffffffu - (uint32_t)best;
+    best = group_max(best, G);
 #pragma unroll
     for (int p = 0; p < PER; ++p)
-      if (key[p] == best) key[p] = 0ull;  // keys are unique (they embed the expert index)
-    const float v = live ? float_from_order_bits((uint32_t)(best >> 32)) : 0.f;
+      if (key[p] == best) key[p] = 0;  // keys are unique (they embed the expert index)
+    const uint32_t e = Key<T>::expert(best);
+    const float v = live ? Key<T>::value(best) : 0.f;
     if (j == 0) vmax = v;
     ex[j] = expf(v - vmax);
     denom += ex[j];
-    if (writer) {
+    if (by_lane) {
+      if (lane_in_group == j) {
+        my_expert = e;
+        my_ex = ex[j];
+      }
+    } else if (live && lane_in_group == 0) {
       if (selected) selected[token * k + j] = (int32_t)e;
       if (selected_long) selected_long[token * k + j] = (int64_t)e;
       if (topk_values) topk_values[token * k + j] = row[e < (uint32_t)E ? e : 0];  // as stored: keeps the sign of a zero
     }
   }
-  if (writer) {
+  if (!live) return;
+  if (by_lane) {
+    if (lane_in_group >= k) return;
+    const int64_t at = token * k + lane_in_group;
+    const float g = my_ex / denom;
+    if (selected) selected[at] = (int32_t)my_expert;
+    if (selected_long) selected_long[at] = (int64_t)my_expert;
+    if (topk_values) topk_values[at] = row[my_expert < (uint32_t)E ? my_expert : 0];
+    if (gates) gates[at] = g;
+    if (gates_rounded) gates_rounded[at] = Elem<T>::down(g);
+  } else if (lane_in_group == 0) {
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) {
       if (j >= k) break;

@@ -110,6 +110,24 @@ def test_route_special_values(device):
     assert sel.tolist() == [[0, 1, 2, 3]]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,k", [(3, 3), (8, 2), (16, 6), (60, 8), (128, 8), (200, 4), (1000, 32), (1024, 9)])
+def test_route_16_bit_keys_order_every_value(device, E, k, dtype):
+    """16-bit logits are ordered by 32-bit keys of their own, fp32 ones by 64-bit keys: the same selections, values and gates
+    for every bit pattern (zeros of both signs, subnormals, infinities, NaNs), ties included."""
+    g = torch.Generator().manual_seed(E)
+    bits = torch.randint(-(1 << 15), 1 << 15, (331, E), generator=g, dtype=torch.int32).to(torch.int16)
+    special = torch.tensor([0, -32768, 1, -32767, 0x7F80, 0x7C00, 0x7FFF, -1], dtype=torch.int16)  # 0, -0, subnormals, inf, NaN
+    mask = torch.rand(331, E, generator=g) < torch.linspace(0, 1, 331)[:, None]
+    bits = torch.where(mask, special[torch.randint(0, 8, (331, E), generator=g)], bits)
+    logits = bits.view(dtype).to(device)
+    sel, gates, vals = cute_kernels.route_topk_softmax_raw(logits, k)
+    sel32, gates32, vals32 = cute_kernels.route_topk_softmax_raw(logits.float(), k)
+    assert torch.equal(sel, sel32)
+    torch.testing.assert_close(gates, gates32, rtol=0, atol=0, equal_nan=True)
+    torch.testing.assert_close(vals.float(), vals32, rtol=0, atol=0, equal_nan=True)
+
+
 def test_route_autograd_matches_torch(device):
     g = torch.Generator().manual_seed(1)
     logits = torch.randn(257, 16, generator=g)  # fp32, no ties
