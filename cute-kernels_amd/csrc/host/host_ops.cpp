@@ -38,7 +38,7 @@ using torch::autograd::variable_list;
   X(ck_sort_by_expert) X(ck_combine_rows) X(ck_gate_grad_both) X(ck_group_rows_padded) X(ck_swiglu_bwd_grouped)         \
   X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
   X(ck_grouped_gemm_f32) X(ck_grouped_gemm_dw_f32) X(ck_grouped_gemm_dw) X(ck_grouped_gemm_dw_rows)                     \
-  X(ck_quant_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) \
+  X(ck_quant_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) X(ck_router_rows) \
   X(ck_gelu_tanh_bwd_grouped) X(ck_fused_residual_add_rmsnorm_fwd) X(ck_rmsnorm_fwd) X(ck_rmsnorm_bwd_partial_rows) X(ck_rmsnorm_bwd_typed)         \
   X(ck_softmax_fwd) X(ck_softmax_bwd) X(ck_add_expert_bias) X(ck_expert_bias_grad)
 
@@ -1065,6 +1065,29 @@ std::tuple<Tensor, Tensor> residual_rmsnorm(const Tensor& x, const Tensor& resid
 struct NormRoute {
   Tensor y, logits, rstd, x8, scale8;
 };
+// Where ck_router_rows is the faster way from rows to router logits: while its workgroups (16 rows x 16 experts) do not outnumber
+// the compute units.
+bool router_rows_fit(int64_t B, int64_t H, int64_t E) {
+  return H >= 32 && H % 32 == 0 && H <= 4096 && ((B + 15) / 16) * ((E + 15) / 16) <= 256;
+}
+bool router_rows_take(const Tensor& x, const Tensor& gate_weight) {
+  if (x.dim() < 1 || gate_weight.dim() != 2 || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return false;
+  const int64_t H = x.size(-1);
+  return !any_requires_grad({&x, &gate_weight}) && H > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
+}
+// x @ gate_weight^T of few 16-bit rows (router_rows_take)
+Tensor router_rows(const Tensor& x_in, const Tensor& gate_weight_in) {
+  require_dims({{&x_in, 2}, {&gate_weight_in, 2}});
+  require_gpu(x_in, gate_weight_in);
+  const int64_t B = x_in.size(0), H = x_in.size(1), E = gate_weight_in.size(0);
+  TORCH_CHECK(gate_weight_in.size(1) == H && gate_weight_in.scalar_type() == x_in.scalar_type(), "router_rows: rows and weight disagree");
+  const Tensor x = x_in.contiguous(), gate_weight = gate_weight_in.contiguous();
+  const Launch l(x);
+  const Tensor logits = new_empty({B, E}, x);
+  check(api.ck_router_rows(ptr(x), nullptr, ptr(gate_weight), 0.f, 0, B, (int32_t)H, (int32_t)E, nullptr, nullptr, ptr(logits), nullptr, nullptr,
+                           dtype_code(x), l.stream));
+  return logits;
+}
 NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& gate_weight, double eps, bool quantize, bool want_rstd) {
   const Launch l(x);
   const int64_t B = x.size(0), H = x.size(1), E = gate_weight.size(0);
@@ -1075,6 +1098,11 @@ NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const T
   if (quantize) {
     r.x8 = new_empty({B, H}, x, at::kFloat8_e4m3fn);
     r.scale8 = new_empty({B}, x, at::kFloat);
+  }
+  if (router_rows_fit(B, H, E)) {
+    check(api.ck_router_rows(ptr(x), ptr(norm_weight), ptr(gate_weight), (float)eps, 1, B, (int32_t)H, (int32_t)E, ptr(r.y), (float*)ptr(r.rstd),
+                             ptr(r.logits), ptr(r.x8), (float*)ptr(r.scale8), dtype_code(x), l.stream));
+    return r;
   }
   const Tensor packed = new_empty({(E + 15) / 16 * 16 * H}, x);  // workspace of the call
   check(api.ck_rmsnorm_route(ptr(x), ptr(norm_weight), ptr(gate_weight), (float)eps, B, (int32_t)H, (int32_t)E, ptr(r.y), (float*)ptr(r.rstd),
@@ -1203,6 +1231,8 @@ PYBIND11_MODULE(_ck_host, m) {
   DEF("rmsnorm", rmsnorm);
   DEF("residual_rmsnorm", residual_rmsnorm);
   DEF("norm_route", norm_route);
+  DEF("router_rows_take", router_rows_take);
+  DEF("router_rows", router_rows);
   DEF("softmax", softmax);
   // without autograd, for the traced operators and the kernel tests
   DEF("route_forward", ([](const Tensor& logits, int64_t k) {

@@ -251,10 +251,173 @@ __global__ __launch_bounds__(kNT, 3) void rmsnorm_route_kernel(const T* __restri
   }
 }
 
+// ---- the same for few rows -----------------------------------------------------------------------------------------
+// What bounds it: latency. The kernel above gives 16 rows to one workgroup of 4 waves, each of which walks through a quarter
+// of the contraction for all experts, behind a launch that re-orders the gate weight; a handful of workgroups takes 13 us
+// for what is 1 MiB of reads. Here a workgroup owns 16 rows x 16 experts and has 16 waves: wave w takes the 64-column pieces
+// w, w + 16, ..., all of its loads (at most 8 of x, 8 of the gate weight) go out at once, and the 16 partial 16 x 16 blocks
+// are added through LDS in a fixed order. The workgroups of a row block all normalise it; the first writes y and rstd, the
+// last the e4m3 rows. The gate weight is read as stored: the channel conflicts of its row pitch do not show at this
+// size. In a decoding step: 64 rows x 2,048, 64 experts 8.0 us (re-ordering 4.2 + 12.9 above); 128 x 4,096, 128 experts with
+// e4m3 rows 17.5 (norm 4.5, library product 14.8, quantiser 4.4); without the norm, 8 rows x 4,096 and 8 experts 7.0 (library
+// 15.4), 2,000 rows 9.3 (16.1). A workgroup takes its 256 KiB at what one compute unit can fetch, which is most of the time:
+// more of them than compute units, and the kernels that read the gate weight once per more rows win (1,024 x 4,096, 128
+// experts: 28.5 us against 24.0 in separate kernels).
+constexpr int kRowWaves = 16;
+
+// S: 32-column pieces per wave, H <= 512 S and H % 32 == 0. NORM: rmsnorm(x) goes to the router (norm_w may be NULL), else x
+// itself.
+template <typename T, int S, bool NORM>
+__global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T* __restrict__ x, const T* __restrict__ norm_w,
+                                                                         const T* __restrict__ gate_w, float eps, int64_t B,
+                                                                         int H, int E, T* __restrict__ y,
+                                                                         float* __restrict__ rstd_out, T* __restrict__ logits,
+                                                                         uint8_t* __restrict__ x8, float* __restrict__ scale8) {
+  __shared__ float part[kRowWaves][kRows][17];  // 16 experts, one column of padding
+  __shared__ float red[2][kRowWaves][kRows];
+  __shared__ __attribute__((aligned(16))) T w_lds[NORM ? 512 * S : 8];  // the norm weight: read by all 16 rows of every wave
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t row0 = (int64_t)blockIdx.x * kRows, row = row0 + r;
+  const int e0 = blockIdx.y * 16;
+  const bool row_ok = row < B;
+  const bool writer = row_ok && blockIdx.y == 0;
+  const int pieces = H / 32;
+  const T* xr = x + (row_ok ? row : B - 1) * H + 8 * q;     // rows past the end re-read the last row
+  const T* gr = gate_w + (int64_t)min(e0 + r, E - 1) * H + 8 * q;  // experts past the end the last expert
+  auto piece = [&](int s) { return (s / 2 * kRowWaves + wave) * 2 + s % 2; };  // pairs: the halves of 128-byte lines
+
+  vec16 xa[S], g[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) xa[s] = piece(s) < pieces ? load16(xr + piece(s) * 32) : zero16();
+  if constexpr (NORM) {
+    if (norm_w != nullptr && tid < H / 8) *reinterpret_cast<vec16*>(&w_lds[8 * tid]) = load16(norm_w + 8 * tid);
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) g[s] = piece(s) < pieces ? load16(gr + piece(s) * 32) : zero16();
+
+  auto row_total = [&](float (&of)[kRowWaves][kRows], auto&& join) {  // over the waves, in order
+    float total = of[0][r];
+#pragma unroll
+    for (int w = 1; w < kRowWaves; ++w) total = join(total, of[w][r]);
+    return total;
+  };
+  if constexpr (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ss = dot2_acc<T>(xa[s].w[i], ss);
+    ss += __shfl_xor(ss, 16, kWave);
+    ss += __shfl_xor(ss, 32, kWave);
+    if (q == 0) red[0][wave][r] = ss;
+    __syncthreads();
+    ss = row_total(red[0], [](float a, float b) { return a + b; });
+    const float rs = rsqrtf(ss * (1.0f / (float)H) + eps);
+    if (rstd_out != nullptr && writer && wave == 0 && q == 0) rstd_out[row] = rs;
+    uint32_t amax_bits = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      Pack16<T> p, w;
+      p.v = xa[s];
+      if (norm_w != nullptr && piece(s) < pieces) w.v = *reinterpret_cast<const vec16*>(&w_lds[piece(s) * 32 + 8 * q]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float v0 = Elem<T>::up(p.e[2 * i]) * rs, v1 = Elem<T>::up(p.e[2 * i + 1]) * rs;
+        if (norm_w != nullptr) {
+          v0 *= Elem<T>::up(w.e[2 * i]);
+          v1 *= Elem<T>::up(w.e[2 * i + 1]);
+        }
+        xa[s].w[i] = piece(s) < pieces ? pack_pair<T>(v0, v1) : 0u;
+        amax_bits = pk_max_u16(amax_bits, xa[s].w[i] & 0x7fff7fffu);
+      }
+      if (writer && piece(s) < pieces) store16(y + row * H + piece(s) * 32 + 8 * q, xa[s]);
+    }
+    if (x8 != nullptr && blockIdx.y == gridDim.y - 1) {  // as ck_quant_rows_e4m3 computes them from the stored y
+      float amax = fmaxf(half_bits_to_float<T>(amax_bits & 0xffffu), half_bits_to_float<T>(amax_bits >> 16));
+      amax = fmaxf(amax, __shfl_xor(amax, 16, kWave));
+      amax = fmaxf(amax, __shfl_xor(amax, 32, kWave));
+      if (q == 0) red[1][wave][r] = amax;
+      __syncthreads();
+      amax = row_total(red[1], [](float a, float b) { return fmaxf(a, b); });
+      const float inv = amax > 0.f ? kE4M3Max / amax : 1.0f;
+      if (wave == 0 && q == 0 && row_ok) scale8[row] = amax > 0.f ? amax / kE4M3Max : 1.0f;
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        Pack16<T> a;
+        a.v = xa[s];
+        int lo = 0, hi = 0;
+        lo = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[0]) * inv, Elem<T>::up(a.e[1]) * inv, lo, false);
+        lo = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[2]) * inv, Elem<T>::up(a.e[3]) * inv, lo, true);
+        hi = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[4]) * inv, Elem<T>::up(a.e[5]) * inv, hi, false);
+        hi = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[6]) * inv, Elem<T>::up(a.e[7]) * inv, hi, true);
+        if (row_ok && piece(s) < pieces)
+          *reinterpret_cast<uint2*>(x8 + row * H + piece(s) * 32 + 8 * q) = uint2{(uint32_t)lo, (uint32_t)hi};
+      }
+    }
+  }
+
+  auto frag = [](const vec16& v) { return __builtin_bit_cast(typename Mfma16<T>::frag, v); };
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S; ++s) acc = Mfma16<T>::run(frag(g[s]), frag(xa[s]), acc);  // 4 consecutive experts of one row
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[wave][r][4 * q + i] = acc[i];
+  __syncthreads();
+  if (tid < kRows * 16) {
+    const int orow = tid >> 4, e = tid & 15;
+    float v = part[0][orow][e];
+#pragma unroll
+    for (int w = 1; w < kRowWaves; ++w) v += part[w][orow][e];
+    if (row0 + orow < B && e0 + e < E) logits[(row0 + orow) * E + e0 + e] = Elem<T>::down(v);
+  }
+}
+
 }  // namespace
 }  // namespace ck
 
 using namespace ck;
+
+extern "C" int ck_router_rows(const void* x, const void* norm_weight, const void* gate_weight, float eps, int32_t normalize,
+                              int64_t B, int32_t H, int32_t E, void* y, float* rstd, void* logits, void* x8, float* scale8,
+                              int32_t dtype, void* stream) {
+  const char* name = "ck_router_rows";
+  CK_REQUIRE(B >= 0, "%s: negative row count", name);
+  CK_REQUIRE(H >= 32 && H <= 4096 && H % 32 == 0, "%s: H=%d must be a multiple of 32, at most 4096", name, H);
+  CK_REQUIRE(E >= 1 && E <= 65535 * 16, "%s: E=%d must be in [1, %d]", name, E, 65535 * 16);
+  if (B == 0) return CK_OK;
+  CK_REQUIRE(x && gate_weight && logits, "%s: x, gate_weight and logits are required", name);
+  CK_REQUIRE((normalize != 0) == (y != nullptr), "%s: y goes with normalize", name);
+  CK_REQUIRE(normalize != 0 || (norm_weight == nullptr && rstd == nullptr && x8 == nullptr && scale8 == nullptr),
+             "%s: norm_weight, rstd, x8 and scale8 go with normalize", name);
+  CK_REQUIRE((x8 == nullptr) == (scale8 == nullptr), "%s: x8 and scale8 go together", name);
+  CK_REQUIRE(aligned16(x) && aligned16(gate_weight) && aligned16(y) && aligned16(norm_weight) && aligned16(x8),
+             "%s: pointers must be 16-byte aligned", name);
+  const int64_t row_blocks = ceil_div(B, kRows);
+  CK_REQUIRE(row_blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
+  const dim3 grid((unsigned)row_blocks, (unsigned)ceil_div(E, 16));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define CK_RR_N(S, NORM)                                                                                                   \
+  hipLaunchKernelGGL((router_rows_kernel<scalar_t, S, NORM>), grid, dim3(kRowWaves * kWave), 0, s,                         \
+                     static_cast<const scalar_t*>(x), static_cast<const scalar_t*>(norm_weight),                           \
+                     static_cast<const scalar_t*>(gate_weight), eps, B, (int)H, (int)E, static_cast<scalar_t*>(y), rstd,   \
+                     static_cast<scalar_t*>(logits), static_cast<uint8_t*>(x8), scale8)
+#define CK_RR(S)                     \
+  do {                               \
+    if (normalize) CK_RR_N(S, true); \
+    else CK_RR_N(S, false);          \
+  } while (0)
+  CK_DISPATCH_HALF(dtype, name, {
+    if (H <= 1024) CK_RR(2);
+    else if (H <= 2048) CK_RR(4);
+    else CK_RR(8);
+  });
+#undef CK_RR
+#undef CK_RR_N
+  CK_CHECK_LAUNCH(name);
+  return CK_OK;
+}
 
 extern "C" int ck_rmsnorm_route(const void* x, const void* norm_weight, const void* gate_weight, float eps, int64_t B,
                                 int32_t H, int32_t E, void* y, float* rstd, void* logits, void* x8, float* scale8,

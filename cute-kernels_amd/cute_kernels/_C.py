@@ -96,6 +96,10 @@ _SIGNATURES = {
         c_int32,
         [c_void_p, c_void_p, c_void_p, c_float, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p],
     ),
+    "ck_router_rows": (
+        c_int32,
+        [c_void_p, c_void_p, c_void_p, c_float, c_int32, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p],
+    ),
     "ck_grouped_gemm_f32": (
         c_int32,
         [c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, POINTER(ck_segments), c_int32, c_void_p, c_void_p, c_void_p],

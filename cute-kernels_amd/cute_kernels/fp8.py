@@ -11,6 +11,7 @@ import torch
 import torch.nn as nn
 
 from . import _C
+from .rmsnorm_route import router_logits
 from .scattermoe import ExpertSegments, choose_align, route_topk_softmax, sort_by_expert
 
 
@@ -85,15 +86,15 @@ class MoE_E4M3(nn.Module):
     def forward(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         original_shape = hidden_states.shape
         hidden_states = hidden_states.view(-1, self.hidden_size)
-        router_logits = self.gate(hidden_states)
-        router_weights, selected_experts = route_topk_softmax(router_logits, self.top_k, long_indices=False)
+        logits = router_logits(self.gate, hidden_states)
+        router_weights, selected_experts = route_topk_softmax(logits, self.top_k, long_indices=False)
         align = choose_align(selected_experts.numel(), self.num_experts, hidden_states.dtype, inference=True)
         seg = sort_by_expert(selected_experts, self.num_experts, align)
         out = swiglu_experts_e4m3(
             hidden_states, self.c_fc_weight_e4m3, self.c_fc_scale, self.c_proj_weight_e4m3, self.c_proj_scale,
             router_weights, seg,
         )
-        return out.view(original_shape), router_logits
+        return out.view(original_shape), logits
 
     @torch.no_grad()
     def forward_with_norm(

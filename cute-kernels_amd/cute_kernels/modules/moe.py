@@ -21,7 +21,7 @@ from ..scattermoe import (
     sort_by_expert,
     swiglu_experts,
 )
-from ..rmsnorm_route import rmsnorm_route_cute
+from ..rmsnorm_route import rmsnorm_route_cute, router_logits
 from ..swiglu import swiglu_packed_cute
 from ..utils import plain_size
 
@@ -167,12 +167,12 @@ class MoE(nn.Module):
         return out.view(original_shape), router_logits
 
     def _compute_routing_weights(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor]:
-        router_logits = self.gate(hidden_states)
+        logits = router_logits(self.gate, hidden_states)
         # top-k on the logits and softmax over the k selected logits in fp32, one kernel
         # (torch_implementation.py:127-133); equal logits resolve to the lowest expert index
-        router_weights, selected_experts = route_topk_softmax(router_logits, self.top_k)
+        router_weights, selected_experts = route_topk_softmax(logits, self.top_k)
         router_weights = router_weights.type_as(hidden_states)
-        return router_logits, router_weights, selected_experts
+        return logits, router_weights, selected_experts
 
     def _compute_expert_assignment(
         self, router_weights: torch.Tensor, selected_experts: torch.Tensor

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+import torch.nn.modules.module as _module
 
 from . import _C
 from .rmsnorm import rmsnorm_cute
@@ -18,9 +19,39 @@ from .utils import is_tracing
 MAX_EXPERTS, MAX_HIDDEN, HIDDEN_STEP = 128, 4096, 512
 
 
+def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
+    """Whether few enough 16-bit rows meet few enough experts for the kernel that gives 16 rows x 16 experts a workgroup of
+    their own (ck_router_rows, with or without the norm), and nothing but plain inference is asked for: a linear layer casts
+    under autocast, and gradients take the routes that they always took."""
+    return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight)
+
+
+def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """gate(x) for rows x [tokens, H]. A plain bias-free nn.Linear that nobody watches (hooks, a forward of its own, other
+    tensor types) runs as ck_router_rows where few rows come without gradients: the library's product takes 15 us there."""
+    weight = getattr(gate, "weight", None)
+    if (
+        type(gate) is torch.nn.Linear
+        and gate.bias is None
+        and type(weight) is torch.nn.Parameter
+        and type(x) is torch.Tensor
+        and x.is_cuda
+        and weight.device == x.device
+        and weight.dtype == x.dtype
+        and x.dim() == 2
+        and x.size(1) == weight.size(1)
+        and "forward" not in vars(gate)
+        and not (gate._forward_hooks or gate._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks)
+        and router_rows_fit(x, weight)
+    ):
+        return _C.host().router_rows(x, weight)
+    return gate(x)
+
+
 def rmsnorm_route_fused(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
     """Whether ck_rmsnorm_route takes this shape: 16-bit rows, hidden size a multiple of 512 up to 4096, at most 128 experts.
-    Other shapes run rmsnorm_cute followed by the linear layer (and quantize_rows_e4m3), with the same results contract."""
+    Other shapes run rmsnorm_cute followed by the linear layer (and quantize_rows_e4m3), with the same results contract, or,
+    few rows, ck_router_rows (router_rows_fit)."""
     H, E = x.size(-1), gate_weight.size(0)
     return (
         x.dtype in (torch.bfloat16, torch.float16)
@@ -49,7 +80,7 @@ def rmsnorm_route_cute(
     router_logits [tokens, E] is what `nn.Linear(H, E, bias=False)` with `gate_weight` returns for the 16-bit y (fp32
     accumulation, another summation order: equal within the rounding of the logits' dtype).
     fused: True takes the one-pass kernel wherever it supports the shape, False the separate kernels; None (default)
-    the one-pass kernel where it is the faster route (rmsnorm_route_pays)."""
+    the one-pass kernel where it is the faster route (router_rows_fit, rmsnorm_route_pays)."""
     if norm_weight is not None:
         assert norm_weight.dim() == 1 and norm_weight.size(0) == x.size(-1), "hidden size for x and weight tensor is different"
         assert norm_weight.dtype == x.dtype, "tensors weight and y should have same dtype"
@@ -58,9 +89,10 @@ def rmsnorm_route_cute(
     )
     if eps is None:
         eps = torch.finfo(x.dtype).eps
+    few_rows = fused is None and router_rows_fit(x, gate_weight)
     if fused is None:
         fused = rmsnorm_route_pays(x, gate_weight)
-    if fused and rmsnorm_route_fused(x, gate_weight):
+    if few_rows or (fused and rmsnorm_route_fused(x, gate_weight)):
         y, logits, x8, scale8 = _C.host().norm_route(x.reshape(-1, x.size(-1)), norm_weight, gate_weight, eps, quantize)
         y = y.view(x.shape)
     else:

@@ -373,6 +373,12 @@ int ck_rmsnorm_route(const void* x, const void* norm_weight, const void* gate_we
                      int32_t E, void* y, float* rstd, void* logits, void* x8, float* scale8, void* gate_packed,
                      int32_t dtype, void* stream);
 
+/* The same for few rows, and without the norm: every output as ck_rmsnorm_route defines it where normalize is non-zero (the
+ * norm's sums run in another order), else logits = x @ gate_weight^T alone, with y, norm_weight, rstd, x8 and scale8 NULL.
+ * bf16 / f16. Needs H % 32 == 0, H <= 4096; no workspace. */
+int ck_router_rows(const void* x, const void* norm_weight, const void* gate_weight, float eps, int32_t normalize, int64_t B,
+                   int32_t H, int32_t E, void* y, float* rstd, void* logits, void* x8, float* scale8, int32_t dtype, void* stream);
+
 /* ---------------------------------------------------------------------------------------------------------------
  * Expert biases
  * Replaces: the bias operand of F.linear in Experts_Torch.forward -- cute_kernels/kernels/scattermoe/

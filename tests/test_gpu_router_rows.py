@@ -1,0 +1,74 @@
+"""Router logits of few rows (ck_router_rows): against float64, with and without the norm ahead, and what keeps the layer's own
+gate module."""
+
+import pytest
+import torch
+
+import cute_kernels
+from cute_kernels import _C, rmsnorm_route
+from cute_kernels.fp8 import quantize_rows_e4m3
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _inputs(B, H, E, dtype):
+    g = torch.Generator().manual_seed(B * 7 + H + E)
+    x = torch.randn(B, H, generator=g).to(dtype).to(DEV)
+    return x, (0.02 * torch.randn(E, H, generator=g)).to(dtype).to(DEV), (1 + 0.1 * torch.randn(H, generator=g)).to(dtype).to(DEV)
+
+
+def _close_logits(logits, y, w):
+    """fp32 sums of H products of 16-bit values, rounded once: off by at most the unit roundoff (2 ** -8 in bf16's 8 bits, 2 ** -11
+    in fp16's 11; 2 ** -25 under fp16's smallest normal) and the sum's error, H * 2 ** -24 of the sum of magnitudes."""
+    exact = y.double() @ w.double().t().contiguous()
+    slack = y.size(1) * 2.0**-24 * (y.double().abs() @ w.double().abs().t().contiguous())
+    unit = 2.0**-8 if y.dtype == torch.bfloat16 else 2.0**-11
+    assert bool(((logits.double() - exact).abs() <= unit * exact.abs() + (1 + unit) * slack + 2.0**-25).all())
+
+
+# rows 1, 16, 17: edges of a row block; widths: one piece, an odd number of pieces, 64-column pairs left over, each
+# instantiation's largest; experts: one, a ragged block, whole blocks
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,E", [(1, 32, 1), (3, 1024, 8), (16, 1056, 16), (17, 2048, 60), (130, 2080, 128), (33, 4096, 17), (256, 4096, 8)])
+def test_logits_and_norm(B, H, E, dtype):
+    x, w, nw = _inputs(B, H, E, dtype)
+    assert _C.host().router_rows_take(x, w)
+    _close_logits(_C.host().router_rows(x, w), x, w)
+    for weight in (nw, None):
+        y, logits, x8, scale = rmsnorm_route.rmsnorm_route_cute(x, weight, w, 1e-6, quantize=True)
+        want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-6)
+        want = want if weight is None else want * weight.double()
+        unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+        assert bool(((y.double() - want).abs() <= want.abs() * (unit + (1 + unit) * (H + 4) * 2.0**-24) + 2.0**-25).all())
+        _close_logits(logits, y, w)
+        q, s = quantize_rows_e4m3(y)
+        assert torch.equal(x8.view(torch.uint8), q.view(torch.uint8)) and torch.equal(scale, s)
+
+
+def test_sizes_beyond_one_workgroup_per_compute_unit_keep_their_routes():
+    x, w, _ = _inputs(257, 512, 256, torch.bfloat16)
+    assert not _C.host().router_rows_take(x, w)  # 17 x 16 workgroups
+    assert _C.host().router_rows_take(x[:256], w)
+    assert not _C.host().router_rows_take(x[:16].float(), w.float())
+
+
+def test_a_watched_or_replaced_gate_is_called():
+    moe = cute_kernels.MoE(8, 2, 512, 256, cute_kernels.swiglu_packed_cute, True, False, 0.02).to(DEV).to(torch.bfloat16)
+    x = torch.randn(5, 512, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        plain = moe(x)[1]
+        _close_logits(plain, x, moe.gate.weight)
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert rmsnorm_route.router_logits(moe.gate, x).dtype == torch.float16
+        seen = []
+        handle = moe.gate.register_forward_hook(lambda m, a, out: seen.append(out))
+        moe(x)
+        handle.remove()
+        assert len(seen) == 1
+        moe.gate.forward = lambda rows: torch.zeros(rows.size(0), 8, device=DEV, dtype=rows.dtype)
+        assert not moe(x)[1].any()
+    del moe.gate.forward
+    x.requires_grad_()
+    moe(x)[1].float().sum().backward()
+    assert x.grad is not None and moe.gate.weight.grad is not None
