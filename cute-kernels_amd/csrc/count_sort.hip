@@ -1,9 +1,9 @@
 // Expert histogram, offset scans and the stable token->expert counting sort.
 //
-// count:  one launch. Waves privatise the histogram (ballot/popcount counters in registers for <= 16 bins, per-wave LDS
-//         copies up to 1024 bins, one LDS copy beyond), blocks merge into a zero-initialised global accumulator, and the
-//         last block to finish (ticket counter) scans the bins, writes counts / inclusive ends / exclusive starts and
-//         puts the accumulator back to zero.
+// count:  one launch. Waves privatise the histogram (ballot/popcount counters in registers for <= 8 bins, else LDS copies, one a
+//         wave while they fit), blocks merge into a zero-initialised global accumulator, and the last block to finish (ticket
+//         counters) scans the bins, writes counts / inclusive ends / exclusive starts and puts the accumulator back to
+//         zero.
 // sort:   up to 4,096 ids one launch of one block (sort_small_kernel), beyond that two. (1) every block histograms its
 //         contiguous segment of the ids into its row of a table. (2) every block sums the table's columns, which with a scan
 //         over the bins is the destination of its first id of every bin in a stable sort, and ranks its ids 64 at a time
@@ -63,11 +63,26 @@ __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
 // calling; the caller may read other blocks' writes after a true return. Blocks publish their data only through device-scope
 // atomics: those are coherent across the XCDs by themselves and are complete once the barrier below has drained the wave's
 // memory counters, so the L2 write-back + invalidate of a full fence (about 0.2 us per block, serialised) is not needed.
-__device__ bool last_block_ticket(uint32_t* ticket, uint32_t* lds_flag) {
+// Atomics on one address follow each other at about 9 ns, so the blocks take tickets of `groups` groups, each kTicketWords
+// apart, and only the last of a group one of the launch (groups = 0: all of the launch). tickets: 1 word, or (1 + groups) *
+// kTicketWords words, zero on entry and again when the last block has returned.
+constexpr int kTicketWords = 16;
+__device__ bool last_block_ticket(uint32_t* tickets, int groups, uint32_t* lds_flag) {
   __syncthreads();
   if (threadIdx.x == 0) {
-    const uint32_t prev = atomicAdd(ticket, 1u);
-    *lds_flag = (prev == gridDim.x - 1) ? 1u : 0u;
+    uint32_t arrivals = gridDim.x;  // at the launch's ticket
+    bool at_launch = true;
+    if (groups > 0) {
+      const uint32_t g = (uint32_t)groups, group = blockIdx.x % g, members = (gridDim.x - group + g - 1) / g;
+      uint32_t* mine = tickets + (1 + group) * kTicketWords;
+      arrivals = min(g, gridDim.x);
+      at_launch = atomicAdd(mine, 1u) == members - 1;
+      // nobody else of the group comes
+      if (at_launch) __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const bool last = at_launch && atomicAdd(tickets, 1u) == arrivals - 1;
+    if (last) __hip_atomic_store(tickets, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *lds_flag = last ? 1u : 0u;
   }
   __syncthreads();
   return *lds_flag != 0u;
@@ -84,6 +99,13 @@ __device__ inline int load_id(const id_t* p) {
 // ------------------------------------------------------------------------------------------------------------
 // count
 // ------------------------------------------------------------------------------------------------------------
+// What a count launch does with its workspace of 1 + bins * replicas words: tickets, then global accumulators.
+struct CountLayout {
+  int replicas;  // of the accumulator
+  int groups;    // of tickets (last_block_ticket)
+  int acc;       // first word of the accumulators
+};
+
 template <int REG_BINS>
 struct RegCounters {
   uint32_t c[REG_BINS];
@@ -100,19 +122,19 @@ struct RegCounters {
 // REG_BINS > 0: wave-uniform register counters via ballot (num_bins <= REG_BINS): a handful of bins would make every
 //               lane of an LDS atomic hit the same few addresses.
 // REG_BINS == 0: LDS atomics on per-wave copies of the histogram.
-template <typename id_t, int REG_BINS>
-__global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ ids, int64_t n, int num_bins,
-                                                        int lds_copies, int replicas, uint32_t* __restrict__ counts,
+template <typename id_t, int REG_BINS, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void count_kernel(const id_t* __restrict__ ids, int64_t n, int num_bins,
+                                                        int lds_copies, CountLayout layout, uint32_t* __restrict__ counts,
                                                         uint32_t* __restrict__ ends, uint32_t* __restrict__ starts,
                                                         uint32_t* __restrict__ ws) {
-  extern __shared__ uint32_t lds[];  // [lds_copies][num_bins] then kWavesPerBlock + 1 words of scan scratch
+  extern __shared__ uint32_t lds[];  // [lds_copies][num_bins] then (BLOCK / kWave) + 1 words of scan scratch
   uint32_t* hist = lds;
   uint32_t* tmp = lds + (size_t)lds_copies * num_bins;
   const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
 
-  for (int i = t; i < lds_copies * num_bins; i += kBlock) hist[i] = 0;
+  for (int i = t; i < lds_copies * num_bins; i += BLOCK) hist[i] = 0;
   __syncthreads();
-  uint32_t* my_hist = hist + (size_t)(lds_copies > 1 ? wave : 0) * num_bins;
+  uint32_t* my_hist = hist + (size_t)(lds_copies > 1 ? wave % lds_copies : 0) * num_bins;
 
   constexpr int VEC = 16 / sizeof(id_t);
   // scalar head up to the first 16-byte boundary, vector body, scalar tail
@@ -132,8 +154,8 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
   };
 
   const id_t* body = ids + head;
-  const int64_t gthreads = (int64_t)gridDim.x * kBlock;
-  const int64_t gtid = (int64_t)blockIdx.x * kBlock + t;
+  const int64_t gthreads = (int64_t)gridDim.x * BLOCK;
+  const int64_t gtid = (int64_t)blockIdx.x * BLOCK + t;
   constexpr int UNROLL = 4;
   // every wave runs the same number of iterations so that ballots see whole waves
   const int64_t iters = (nvec + gthreads * UNROLL - 1) / (gthreads * UNROLL);
@@ -162,7 +184,7 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
   }
   if (blockIdx.x == 0) {  // ragged ends, at most VEC-1 ids each; whole waves participate (ballot)
     const int64_t ragged = head + (n - tail_begin);
-    for (int64_t base = 0; base < ragged; base += kBlock) {
+    for (int64_t base = 0; base < ragged; base += BLOCK) {
       const int64_t r = base + t;
       int id = -1;
       if (r < ragged) id = load_id(ids + (r < head ? r : tail_begin + (r - head)));
@@ -179,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
   }
   __syncthreads();
   if (lds_copies > 1) {
-    for (int e = t; e < num_bins; e += kBlock) {
+    for (int e = t; e < num_bins; e += BLOCK) {
       uint32_t s = 0;
       for (int c = 0; c < lds_copies; ++c) s += hist[(size_t)c * num_bins + e];
       hist[e] = s;  // copy 0 row becomes the block total; other rows are not read again
@@ -187,33 +209,32 @@ __global__ __launch_bounds__(kBlock) void count_kernel(const id_t* __restrict__ 
     __syncthreads();
   }
 
-  // Blocks merge into one of `replicas` global accumulators (thousands of atomics on one cache line would serialise in a
+  // Blocks merge into one of several global accumulators (thousands of atomics on one cache line would serialise in a
   // single L2 channel); the last block adds the replicas up and puts them back to zero.
-  uint32_t* acc = ws + 1;
+  uint32_t* acc = ws + layout.acc;
   if (gridDim.x > 1) {
-    uint32_t* my_acc = acc + (size_t)(blockIdx.x % replicas) * num_bins;
-    for (int e = t; e < num_bins; e += kBlock)
+    uint32_t* my_acc = acc + (size_t)(blockIdx.x % layout.replicas) * num_bins;
+    for (int e = t; e < num_bins; e += BLOCK)
       if (hist[e]) atomicAdd(&my_acc[e], hist[e]);
-    if (!last_block_ticket(ws, tmp + kWavesPerBlock)) return;
+    const int used = min(layout.replicas, (int)gridDim.x);
+    if (!last_block_ticket(ws, layout.groups, tmp + (BLOCK / kWave))) return;
     // Sum the replicas that were used and put them back to zero. Device-scope atomic loads read the values where the
     // other blocks' atomics left them; the loads of one thread are independent, so their latencies overlap.
-    const int used = min(replicas, (int)gridDim.x);
-    for (int e = t; e < num_bins; e += kBlock) hist[e] = 0;
+    for (int e = t; e < num_bins; e += BLOCK) hist[e] = 0;
     __syncthreads();
-    for (int idx = t; idx < used * num_bins; idx += kBlock) {  // (replica, bin) pairs spread over the whole block
+    for (int idx = t; idx < used * num_bins; idx += BLOCK) {  // (replica, bin) pairs spread over the whole block
       const uint32_t v = __hip_atomic_load(&acc[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       acc[idx] = 0u;  // visible to the next launch at the kernel boundary; nobody reads it before
       if (v) atomicAdd(&hist[idx % num_bins], v);
     }
-    if (t == 0) ws[0] = 0u;
     __syncthreads();
   }
   // hist[0..num_bins) now holds the global counts
-  for (int e = t; e < num_bins; e += kBlock) counts[e] = hist[e];
+  for (int e = t; e < num_bins; e += BLOCK) counts[e] = hist[e];
   if (ends != nullptr || starts != nullptr) {
     __syncthreads();
-    block_exclusive_scan(hist, num_bins, tmp);
-    for (int e = t; e < num_bins; e += kBlock) {
+    block_exclusive_scan<BLOCK>(hist, num_bins, tmp);
+    for (int e = t; e < num_bins; e += BLOCK) {
       const uint32_t s = hist[e];
       if (starts) starts[e] = s;
       if (ends) ends[e] = s + counts[e];  // counts[e] was written by this same thread above
@@ -486,11 +507,25 @@ __global__ __launch_bounds__(kSmallBlock) void sort_small_kernel(const id_t* __r
 
 using namespace ck;
 
-// global accumulator replicas: as many as fit in 16384 words, at most 32
+// global accumulators that the workspace holds beside one word: as many as fit in 16384 words, at most 32
 static int count_replicas(int num_bins) {
   int r = kMaxCountBins / (num_bins > 0 ? num_bins : 1);
   return r < 1 ? 1 : (r > 32 ? 32 : r);
 }
+
+namespace {
+constexpr int kNarrowCount = 512, kWideCount = 1024;  // threads of a block
+constexpr int64_t kMaxCountBlocks = 512;
+
+// Half of the accumulators' words are enough for as many blocks as there are; the tickets of up to 16 groups take what they
+// need of the rest, where there is room for two groups or more.
+CountLayout count_layout(int num_bins) {
+  const int replicas = count_replicas(num_bins), half = replicas / 2;
+  const int groups = half >= 1 ? min(16, (1 + num_bins * (replicas - half)) / kTicketWords - 1) : 0;
+  if (groups < 2) return {replicas, 0, 1};
+  return {half, groups, (1 + groups) * kTicketWords};
+}
+}  // namespace
 
 extern "C" int64_t ck_count_workspace_words(int32_t num_bins) {
   return 1 + (int64_t)(num_bins > 0 ? num_bins : 0) * count_replicas(num_bins);
@@ -510,21 +545,34 @@ int launch_count(const char* name, const void* ids, int32_t ids_are_i64, int64_t
   CK_REQUIRE((reinterpret_cast<uintptr_t>(ids) & (esz - 1)) == 0, "%s: ids is not element-aligned", name);
 
   const int64_t vec = 16 / (int64_t)esz;
-  // 4 vectors per thread per trip; one block for small inputs. Large inputs: 2 blocks per CU stream fastest with the LDS
-  // path (6.5 TB/s at 512 blocks, 6.1 at 1024, 3.7 at 256); the ballot path is VALU-heavier and wants 4 per CU.
-  int64_t blocks = ceil_div(n, (int64_t)kBlock * vec * 4 * 4);
-  if (blocks < 1) blocks = 1;
-  const int64_t max_blocks = num_bins <= 8 ? 1024 : 512;
-  if (blocks > max_blocks) blocks = max_blocks;
-  // up to 8 bins: ballot counters in registers (5.8 TB/s; LDS atomics on so few addresses serialise: 2.1-5.1 TB/s);
-  // more bins: LDS atomics (6.3-6.5 TB/s; 16 register counters measured 3.3 TB/s)
-  const int reg_bins = num_bins <= 8 ? 8 : 0;  // 16 register counters measured slower (3.3 TB/s) than LDS atomics (5.6)
-  const int copies = reg_bins > 0 ? 1 : (num_bins <= 1024 ? kWavesPerBlock : 1);
-  const size_t lds_bytes = ((size_t)copies * num_bins + kWavesPerBlock + 2) * sizeof(uint32_t);
-#define CK_LAUNCH_COUNT(ID_T, RB)                                                                              \
-  hipLaunchKernelGGL((count_kernel<ID_T, RB>), dim3((unsigned)blocks), dim3(kBlock), lds_bytes, s,            \
-                     static_cast<const ID_T*>(ids), n, (int)num_bins, copies, count_replicas(num_bins), counts, ends,   \
-                     starts, workspace)
+  // up to 8 bins: ballot counters in registers (LDS atomics on so few addresses serialise); more bins: LDS atomics (16 register
+  // counters measured half as fast)
+  const int reg_bins = num_bins <= 8 ? 8 : 0;
+  // A thread starts with 4 vectors (64 bytes) and goes round only once the launch is as large as the chip takes at once:
+  // 512 blocks of 16 waves. (With 4 trips from the start and at most 512 blocks of 4 waves, int32 / int64 ids over 64 experts,
+  // now / then: 65,536 ids 4.8 / 7.8 and 6.4 / 12.7 us, 2^20 6.3 / 10.0 and 7.5 / 14.0, 2^22 7.6 / 12.6 and 10.3 / 19.4, 2^26
+  // 44.5 / 50.2 and 82.4 / 162.8; a ticket for each block on one address alone cost 4 us of a launch of 512 blocks.) Small
+  // inputs want blocks of 8 waves, whose barriers and merge are shorter (1,024 ids 2.6 us against 3.0), as long as
+  // that makes few blocks -- up to 16, or 512 where a block's merge is short (32 bins or fewer: 2^20 ids over 16 experts 5.4 us
+  // against 6.7; over 128 experts 7.6 against 7.0).
+  const int64_t narrow = ceil_div(n, (int64_t)kNarrowCount * vec * 4);
+  const bool wide = narrow > (num_bins <= 32 ? 512 : 16);
+  const int threads = wide ? kWideCount : kNarrowCount;
+  int64_t blocks = wide ? ceil_div(n, (int64_t)kWideCount * vec * 4) : narrow;
+  blocks = blocks < 1 ? 1 : blocks > kMaxCountBlocks ? kMaxCountBlocks : blocks;
+  // copies of the histogram in LDS: one a wave, at most 32 KiB of them
+  int copies = reg_bins > 0 ? 1 : kMaxCountBins / 2 / num_bins;
+  copies = copies < 1 ? 1 : copies > threads / kWave ? threads / kWave : copies;
+  const size_t lds_bytes = ((size_t)copies * num_bins + threads / kWave + 2) * sizeof(uint32_t);
+  const CountLayout layout = count_layout(num_bins);
+#define CK_LAUNCH_COUNT_W(ID_T, RB, THREADS)                                                                              \
+  hipLaunchKernelGGL((count_kernel<ID_T, RB, THREADS>), dim3((unsigned)blocks), dim3(THREADS), lds_bytes, s,             \
+                     static_cast<const ID_T*>(ids), n, (int)num_bins, copies, layout, counts, ends, starts, workspace)
+#define CK_LAUNCH_COUNT(ID_T, RB)                          \
+  do {                                                     \
+    if (wide) CK_LAUNCH_COUNT_W(ID_T, RB, kWideCount);     \
+    else CK_LAUNCH_COUNT_W(ID_T, RB, kNarrowCount);        \
+  } while (0)
   if (ids_are_i64) {
     if (reg_bins == 8) CK_LAUNCH_COUNT(int64_t, 8);
     else CK_LAUNCH_COUNT(int64_t, 0);
@@ -533,6 +581,7 @@ int launch_count(const char* name, const void* ids, int32_t ids_are_i64, int64_t
     else CK_LAUNCH_COUNT(int32_t, 0);
   }
 #undef CK_LAUNCH_COUNT
+#undef CK_LAUNCH_COUNT_W
   CK_CHECK_LAUNCH(name);
   return CK_OK;
 }

@@ -78,6 +78,21 @@ def test_count_misaligned_views_out_of_range_and_shortcut(device):
     )
 
 
+# narrow and wide blocks, one trip and several: 16 and 512 blocks of 512 threads (8,192 int32 or 4,096 int64 ids each) and 512
+# of 1,024 threads, and one id more
+@pytest.mark.parametrize("dtype", [torch.int32, torch.long])
+@pytest.mark.parametrize("bins", [1, 8, 9, 32, 33, 128])
+def test_count_launch_forms(device, bins, dtype):
+    per_block = 8192 if dtype == torch.int32 else 4096
+    for n in (1, 512, per_block, per_block + 1, 16 * per_block, 16 * per_block + 1, 512 * per_block, 512 * per_block + 1, 1024 * per_block + 1):
+        x = torch.randint(0, bins, (n,), dtype=dtype, device=device)
+        expect = torch.bincount(x, minlength=bins).cpu().numpy()
+        for repeat in range(2):  # tickets and accumulators come back to zero
+            counts, ends, _ = cute_kernels.continuous_count_and_offsets_cute(x, bins)
+            np.testing.assert_array_equal(counts.cpu().numpy(), expect, err_msg=f"n={n} call {repeat}")
+            np.testing.assert_array_equal(ends.cpu().numpy(), expect.cumsum())
+
+
 def test_count_large_sum_property(device):
     # full-size property at 2^28 ids (1 GiB): counts sum to N and match a strided sample's histogram scaled check
     n = 1 << 28
