@@ -67,6 +67,10 @@ constexpr int kLineBM = 256, kLineK = 64;
 int launch_line(const GemmParams& prm, int mode, int bn, bool bt, int dtype, unsigned blocks, hipStream_t stream,
                 const char* name);
 
+// Weight gradients from row-major operands on 128 x 256 tiles, two workgroups per compute unit (grouped_gemm_dw.hip); sets
+// prm's tile counts itself.
+int launch_dw_short(const GemmParams& prm, int dtype, hipStream_t stream, const char* name);
+
 // Tiles of 16, 32 or 64 rows (grouped_gemm_skinny.hip): forward GEMMs of inference batches with few rows per expert, modes
 // kGrouped, kScatter, kSwiglu, 16-bit or e4m3 operands; prm.align is the tile height.
 inline bool skinny_align(int align) { return align == 16 || align == 32 || align == 64; }
@@ -287,6 +291,42 @@ __device__ inline void dw_tile(const GemmParams& prm, int pid, int& position, in
   }
   mt = m_major ? a : b;
   nt = m_major ? b : a;
+}
+// The same for tiles of half the height (grouped_gemm_dw.hip; 64 at a time on an XCD): blocks of 8 m tiles x 4 n tiles.
+__device__ inline void dw_rows_first_tile(const GemmParams& prm, int pid, int& position, int& mt, int& nt) {
+  if (prm.m_tiles % kXcds == 0 && prm.m_tiles / kXcds >= 8) {
+    const int slice = prm.m_tiles / kXcds, per_slice = slice * prm.n_tiles, j = pid / kXcds;
+    position = j / per_slice;
+    grouped_order(j - position * per_slice, slice, prm.n_tiles, mt, nt);
+    mt += pid % kXcds * slice;
+  } else {
+    dw_chunk_tile<32, 8>(pid, prm.m_tiles, prm.n_tiles, prm.num_experts, position, mt, nt);
+  }
+}
+
+// The expert with the position-th largest count, ties by index: the longest contractions go first (the hardware hands tiles
+// out in block order), so that the tiles still running when the grid drains are the short ones. One thread ranks one
+// expert against the counts parked in LDS (sh: THREADS + 1 words, free again on return); more experts than threads keep
+// their order.
+template <int THREADS>
+__device__ inline int longest_first(const GemmParams& prm, int position, int* sh) {
+  const int E = prm.num_experts, t = threadIdx.x;
+  if (E > THREADS) return position;
+  if (t < E) sh[t] = (int)prm.counts[t];
+  __syncthreads();
+  if (t < E) {
+    const int c = sh[t];
+    int rank = 0;
+    for (int i = 0; i < E; ++i) {
+      const int ci = sh[i];
+      rank += (ci > c || (ci == c && i < t)) ? 1 : 0;
+    }
+    if (rank == position) sh[THREADS] = t;
+  }
+  __syncthreads();
+  const int expert = sh[THREADS];
+  __syncthreads();  // everyone holds its expert before the first loads land there
+  return expert;
 }
 
 

@@ -90,28 +90,7 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
   [[maybe_unused]] int split_slot = -1, split_part = -1, split_parts = kSplitParts;
   if constexpr (MODE == kDw) {
     dw_tile(prm, blockIdx.x, expert, mt, nt);
-    // `expert` so far is a position in the launch order. Experts differ in contraction length (their row counts), and
-    // the hardware hands tiles out in block order: the longest contractions go first, so that the tiles still running
-    // when the grid drains are the short ones (position r takes the expert with the r-th largest count, ties by index).
-    // Up to NT experts: one thread ranks one expert against the counts parked in LDS (the stages are not in use yet).
-    if (prm.num_experts <= NT) {
-      int* sh = reinterpret_cast<int*>(lds_c);
-      const int E = prm.num_experts;
-      if (tid < E) sh[tid] = (int)prm.counts[tid];
-      __syncthreads();
-      if (tid < E) {
-        const int c = sh[tid];
-        int rank = 0;
-        for (int i = 0; i < E; ++i) {
-          const int ci = sh[i];
-          rank += (ci > c || (ci == c && i < tid)) ? 1 : 0;
-        }
-        if (rank == expert) sh[NT] = tid;
-      }
-      __syncthreads();
-      expert = sh[NT];
-      __syncthreads();  // everyone holds its expert before the first loads land in the stages
-    }
+    expert = longest_first<NT>(prm, expert, reinterpret_cast<int*>(lds_c));  // `expert` so far is a position (the stages are not in use yet)
     k_begin = prm.seg_starts[expert];
     k_len = (int)((prm.counts[expert] + BK - 1) / BK * BK);  // the transposed operands are zero up to the tile boundary
   } else {

@@ -40,10 +40,15 @@ def test_forward_tiles(counts, columns):
         assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())  # |sum| <= 256: exact in bf16
 
 
-# tiles along the longer side: 32 (4 per XCD: slices, or chunks of 32 from 4,096 rows per expert on), 16 and 11 (chunks of 16; 8 experts: 128 and 176 tiles, whole rounds of
-# chunks and a rest), 1; the longer side is the rows' or the columns'
-@pytest.mark.parametrize("M,N", [(8192, 256), (256, 4096), (2816, 512), (512, 2568), (256, 256)])
-@pytest.mark.parametrize("counts", [[70, 0, 64, 65, 1, 128, 3, 200], [33], [4000, 4200, 0, 8300]])
+# 256 x 256 tiles along the longer side: 32 (4 per XCD: slices, or chunks of 32 from 4,096 rows per expert on), 16 and 11 (chunks
+# of 16; 8 experts: 128 and 176 tiles, whole rounds of chunks and a rest), 1; the longer side is the rows' or the columns'.
+# The first three lists average fewer than 512 rows: 128 x 256 tiles, in slices of 8 of them or chunks of 32, contractions of one
+# step of 32 rows, of two and more, ragged and whole; ragged tiles of both kernels.
+@pytest.mark.parametrize("M,N", [(8192, 256), (256, 4096), (2816, 512), (512, 2568), (256, 256), (328, 264)])
+@pytest.mark.parametrize(
+    "counts",
+    [[70, 0, 64, 65, 1, 128, 3, 200], [33], [31, 32, 97, 511], [600, 0, 1100, 513, 512, 700, 3, 1500], [4000, 4200, 0, 8300]],
+)
 def test_weight_gradient_tiles(counts, M, N):
     g = torch.Generator().manual_seed(1)
     seg = _segments(counts)
