@@ -54,7 +54,10 @@ struct GemmParams {
   uint64_t split_tag;
 };
 uint64_t next_split_tag();  // grouped_gemm.hip
-constexpr int kSplitParts = 4, kSplitMaxTail = 64, kSplitMaxRounds = 64, kSplitMinSteps = 16;
+constexpr int kSplitParts = 4, kSplitMaxTail = 64, kSplitMaxRounds = 64;
+// K steps that splitting has to take off the last round. A step of a 256 x 256 tile takes 1.5 to 1.7 us, and the parts'
+// device-wide fences and the exchange of their accumulators 60 to 80 us however short they are.
+constexpr int kSplitMinSaved = 40;
 constexpr int64_t kSplitPartFloats = 4 * 64 * 64 * 4;  // one workgroup's 256 x 256 fp32 tile
 constexpr int64_t kSplitWorkspaceBytes = kSplitMaxTail * kSplitParts * kSplitPartFloats * 4 + 2 * kSplitMaxTail * 8;
 

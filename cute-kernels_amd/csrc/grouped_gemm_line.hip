@@ -101,14 +101,15 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
     if constexpr (kSplit) {
       // The tiles of the last, partial round (the highest block indices: the hardware hands blocks out in order) would
       // each keep one CU busy for a whole tile time while the rest of the chip idles. When that round is at most half
-      // full, every such tile is computed by 2 to 4 workgroups (as many as fill the chip), an equal share of the contraction each: part
+      // full, and splitting takes steps enough off it (kSplitMinSaved), every such tile is computed by 2 to 4 workgroups (as many as fill the chip), an equal share of the contraction each: part
       // 0 is the tile's own block, parts 1.. are extra blocks behind the regular grid. All write their fp32 accumulators
       // to the workspace; the last to arrive (ticket) adds the parts up in part order and runs the epilogue.
       const int cus = kXcds * 32;
       const int tail = total % cus;
+      const int k_steps = prm.K / BK, parts = tail > 0 ? min(kSplitParts, cus / tail) : kSplitParts;
       const bool active = prm.split_ws != nullptr && tail > 0 && tail <= 2 * kSplitMaxTail && total / cus <= kSplitMaxRounds &&
-                          prm.K / BK >= kSplitMinSteps;
-      split_parts = active ? min(kSplitParts, cus / tail) : kSplitParts;  // as many parts as fill the chip: 4, 3 or 2
+                          k_steps - (k_steps + parts - 1) / parts >= kSplitMinSaved;
+      split_parts = active ? parts : kSplitParts;  // as many parts as fill the chip: 4, 3 or 2
       if (pid >= prm.split_base) {  // an extra block
         const int x = pid - prm.split_base;
         split_slot = x / (split_parts - 1);

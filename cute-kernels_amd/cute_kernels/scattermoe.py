@@ -133,16 +133,16 @@ SMALL_TILES = ((6, 16), (14, 32), (30, 64))  # (rows per expert up to which, til
 def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
     """256 or 128 rows for 16-bit layers below 512 rows per expert, whichever makes the sum of the layer's launches shorter.
     launches: (columns, contraction, whether the epilogue may split its last round, input gradient) of every grouped GEMM
-    that depends on the height. In us, with the constants fitted to layers of 8 to 128 experts, 768 to 4,096 wide, 512 to
-    14,336 inside, gated and not, at 16 to 450 rows per expert (1,850 training steps, 2,590 inference calls):
+    that depends on the height. In us, with the constants fitted to measured layers:
       * a 64-deep step of a 256 x 256 tile takes 1.7 on a CU; contractions that are no multiple of 64 run on the general
         kernel, 1.6 with fewer loads in flight and no split; of a 128 x 128 tile 0.7, or 1.4 for the two that share a CU;
-      * splitting the last round of 256-row tiles costs 60 for its device-wide fences (32 experts of 1,024 x 1,024 at 64 rows:
-        137 us in 256-row tiles, 53 in 128-row ones);
+      * splitting the last round of 256-row tiles costs 60 for its device-wide fences, and happens where it takes 40 steps or
+        more off that round;
       * no launch is shorter than its weights' stream, 4.2 TB/s, and the input gradient of 128-row tiles (or of such a
         contraction) transposes the weights first.
-    The chosen height is 0.3 % slower than the better one on average in training and 0.8 % in inference; always 256 was 11 and
-    26 %, always 128 17 and 11 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
+    Over 432 calls of 8 to 64 experts, 1,024 to 4,096 wide, 1,024 to 14,336 inside, at 16 to 450 rows per expert the chosen
+    height is 0.8 % slower than the better one on average in training and 0.7 % in inference; always 256 3.5 and 25 %, always
+    128 24 and 12 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
     4,096 x 14,336 at 8 / 96 / 400 rows 3,217 / 3,548 / 6,801 against 2,132 / 2,416 / 3,980 us; 32 of 1,024 x 1,024 304 / 335 /
     622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. Inference: 8 of 4,096 x
     14,336 at 34 / 64 / 100 / 128 rows 606 / 630 / 686 / 1,014 against 631 / 643 / 658 / 686; 8 of 1,664 x 5,632 at 64 / 200 /
@@ -161,8 +161,8 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tupl
                 time = steps * (1.4 * pairs + (0.0 if left == 0 else 0.7 if left <= 256 else 1.4))
             elif nt_only:
                 time = 1.6 * steps * -(-tiles // 256)
-            elif splits and 0 < tiles % 256 <= 128 and steps >= 16:
-                time = 1.7 * (steps * (tiles // 256) + -(-steps // min(4, 256 // (tiles % 256)))) + 60.0
+            elif splits and 0 < tiles % 256 <= 128 and steps - (part := -(-steps // min(4, 256 // (tiles % 256)))) >= 40:
+                time = 1.7 * (steps * (tiles // 256) + part) + 60.0
             else:
                 time = 1.7 * steps * -(-tiles // 256)
             total += max(time, stream) + (2 * stream if input_gradient and nt_only else 0.0)

@@ -59,3 +59,37 @@ def test_weight_gradient_tiles(counts, M, N):
     for e in range(len(counts)):
         expect = (a_rows[e].t().contiguous() @ b_rows[e]).to(torch.bfloat16)  # sums below 2^24: exact in fp32, one rounding
         assert torch.equal(dw[e].cpu(), expect), e
+
+
+# 6 experts, 13 row tiles x 20 / 25 / 28 column tiles: a last round of 4 / 69 / 108 tiles, in 4 / 3 / 2 parts where that takes 40 of
+# its K steps off: 54, 60, 80 steps are the fewest, 53 too few for any
+@pytest.mark.parametrize("columns,K", [(5120, 54 * 64), (6400, 60 * 64), (7168, 80 * 64), (5120, 53 * 64)])
+@pytest.mark.parametrize("weights", ["as columns x contraction", "as stored by their owner"])
+def test_split_last_round(monkeypatch, weights, columns, K):
+    """The same launch split and unsplit: equal up to the fp32 re-association of a few partial sums, bit for bit from one split
+    launch to the next, and bit for bit to the unsplit one where the rule says no."""
+    counts = [700, 513, 600, 0, 512, 400]
+    seg = _segments(counts)
+    tiles = sum(-(-c // 256) for c in counts) * (columns // 256)
+    assert 0 < tiles % 256 <= 128
+    g = torch.Generator(device=DEV).manual_seed(2)
+    a = torch.randn(seg.max_rows, K, generator=g, device=DEV).to(torch.bfloat16)
+    shape = (len(counts), columns, K) if weights == "as columns x contraction" else (len(counts), K, columns)
+    w = (torch.randn(shape, generator=g, device=DEV) * K**-0.5).to(torch.bfloat16)
+    outs = []
+    for split in (True, True, False):
+        monkeypatch.setattr(scattermoe.options, "gemm_split", split)
+        out = torch.zeros(seg.max_rows, columns, dtype=torch.bfloat16, device=DEV)
+        if weights == "as columns x contraction":
+            scattermoe._gemm(a, 0, w, seg, _C.CK_EPI_GROUPED, out)
+        else:
+            scattermoe._gemm_dx(a, w, seg, _C.CK_EPI_GROUPED, out)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    same = (outs[0] == outs[2]).float().mean()
+    if K == 53 * 64:
+        assert same == 1
+    else:  # a last round of 4 of 260 tiles and more: some element of its tiles rounds the other way
+        assert 0.99 < float(same) < 1
+        # 256 k of K terms ~ N(0, 1 / K): sums differ by a few 2 ** -24, one rounding step of bf16 (2 ** -8) where they straddle
+        torch.testing.assert_close(outs[0].float(), outs[2].float(), rtol=2.0**-7, atol=2.0**-16)
