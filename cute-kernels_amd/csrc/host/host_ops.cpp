@@ -1070,10 +1070,14 @@ struct NormRoute {
 bool router_rows_fit(int64_t B, int64_t H, int64_t E) {
   return H >= 32 && H % 32 == 0 && H <= 4096 && ((B + 15) / 16) * ((E + 15) / 16) <= 256;
 }
-bool router_rows_take(const Tensor& x, const Tensor& gate_weight) {
-  if (x.dim() < 1 || gate_weight.dim() != 2 || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return false;
+bool router_rows_take(const Tensor& x, const Tensor& gate_weight, const OptTensor& norm_weight) {
+  if (!x.is_cuda() || x.dim() < 1 || gate_weight.dim() != 2 || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return false;
+  const Tensor nw = value_or_undefined(norm_weight);
+  // the kernel reads 16 bytes at a time; what is not contiguous is copied first, to where a new tensor begins
+  for (const Tensor* t : {&x, &gate_weight, &nw})
+    if (t->defined() && t->is_contiguous() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0) return false;
   const int64_t H = x.size(-1);
-  return !any_requires_grad({&x, &gate_weight}) && H > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
+  return !any_requires_grad({&x, &gate_weight, &nw}) && x.numel() > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
 }
 // x @ gate_weight^T of few 16-bit rows (router_rows_take)
 Tensor router_rows(const Tensor& x_in, const Tensor& gate_weight_in) {

@@ -19,11 +19,11 @@ from .utils import is_tracing
 MAX_EXPERTS, MAX_HIDDEN, HIDDEN_STEP = 128, 4096, 512
 
 
-def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
+def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor, norm_weight: torch.Tensor | None = None) -> bool:
     """Whether few enough 16-bit rows meet few enough experts for the kernel that gives 16 rows x 16 experts a workgroup of
     their own (ck_router_rows, with or without the norm), and nothing but plain inference is asked for: a linear layer casts
     under autocast, and gradients take the routes that they always took."""
-    return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight)
+    return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight, norm_weight)
 
 
 def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -31,7 +31,8 @@ def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     tensor types) runs as ck_router_rows where few rows come without gradients: the library's product takes 15 us there."""
     weight = getattr(gate, "weight", None)
     if (
-        type(gate) is torch.nn.Linear
+        not is_tracing()
+        and type(gate) is torch.nn.Linear
         and gate.bias is None
         and type(weight) is torch.nn.Parameter
         and type(x) is torch.Tensor
@@ -89,7 +90,7 @@ def rmsnorm_route_cute(
     )
     if eps is None:
         eps = torch.finfo(x.dtype).eps
-    few_rows = fused is None and router_rows_fit(x, gate_weight)
+    few_rows = fused is None and router_rows_fit(x, gate_weight, norm_weight)
     if fused is None:
         fused = rmsnorm_route_pays(x, gate_weight)
     if few_rows or (fused and rmsnorm_route_fused(x, gate_weight)):

@@ -33,7 +33,7 @@ def _close_logits(logits, y, w):
 @pytest.mark.parametrize("B,H,E", [(1, 32, 1), (3, 1024, 8), (16, 1056, 16), (17, 2048, 60), (130, 2080, 128), (33, 4096, 17), (256, 4096, 8)])
 def test_logits_and_norm(B, H, E, dtype):
     x, w, nw = _inputs(B, H, E, dtype)
-    assert _C.host().router_rows_take(x, w)
+    assert _C.host().router_rows_take(x, w, nw)
     _close_logits(_C.host().router_rows(x, w), x, w)
     for weight in (nw, None):
         y, logits, x8, scale = rmsnorm_route.rmsnorm_route_cute(x, weight, w, 1e-6, quantize=True)
@@ -48,9 +48,24 @@ def test_logits_and_norm(B, H, E, dtype):
 
 def test_sizes_beyond_one_workgroup_per_compute_unit_keep_their_routes():
     x, w, _ = _inputs(257, 512, 256, torch.bfloat16)
-    assert not _C.host().router_rows_take(x, w)  # 17 x 16 workgroups
-    assert _C.host().router_rows_take(x[:256], w)
-    assert not _C.host().router_rows_take(x[:16].float(), w.float())
+    take = _C.host().router_rows_take
+    assert not take(x, w, None)  # 17 x 16 workgroups
+    assert take(x[:256], w, None)
+    assert not take(x[:16].float(), w.float(), None)
+    assert not take(x[:0], w, None)
+
+
+def test_rows_off_a_16_byte_boundary_keep_their_routes():
+    x, w, nw = _inputs(9, 640, 8, torch.bfloat16)
+    off = lambda t: torch.cat([t.new_zeros(3), t.flatten()])[3:].view(t.shape)  # contiguous, 6 bytes past a boundary
+    gate = torch.nn.Linear(640, 8, bias=False, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        gate.weight.copy_(w)
+        _close_logits(rmsnorm_route.router_logits(gate, off(x)), x, w)
+        _close_logits(rmsnorm_route.router_logits(gate, x.t().contiguous().t()), x, w)  # not contiguous: copied
+    assert not _C.host().router_rows_take(off(x), w, None)
+    assert not _C.host().router_rows_take(x, off(w), None)
+    assert not _C.host().router_rows_take(x, w, off(nw))
 
 
 def test_a_watched_or_replaced_gate_is_called():
