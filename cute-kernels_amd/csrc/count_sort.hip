@@ -61,13 +61,17 @@ __device__ uint32_t block_exclusive_scan(uint32_t* data, int n, uint32_t* tmp) {
 
 // Returns true in every thread of exactly one block: the last one to arrive. Blocks must have made their global writes before
 // calling; the caller may read other blocks' writes after a true return. Blocks publish their data only through device-scope
-// atomics: those are coherent across the XCDs by themselves and are complete once the barrier below has drained the wave's
-// memory counters, so the L2 write-back + invalidate of a full fence (about 0.2 us per block, serialised) is not needed.
+// atomics, which are coherent across the XCDs by themselves: the L2 write-back + invalidate of a full fence (about 0.2 us per
+// block, serialised) is not needed. Their completion is: an atomic that returns nothing is on its way to an L2 channel of its
+// own when the wave goes on, and __syncthreads() waits for LDS only. So every wave waits for its own (vmcnt) ahead of
+// the barrier behind which the block takes its ticket, or the last block could read an accumulator that an addition
+// has yet to reach.
 // Atomics on one address follow each other at about 9 ns, so the blocks take tickets of `groups` groups, each kTicketWords
 // apart, and only the last of a group one of the launch (groups = 0: all of the launch). tickets: 1 word, or (1 + groups) *
 // kTicketWords words, zero on entry and again when the last block has returned.
 constexpr int kTicketWords = 16;
 __device__ bool last_block_ticket(uint32_t* tickets, int groups, uint32_t* lds_flag) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t arrivals = gridDim.x;  // at the launch's ticket

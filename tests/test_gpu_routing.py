@@ -93,6 +93,15 @@ def test_count_launch_forms(device, bins, dtype):
             np.testing.assert_array_equal(ends.cpu().numpy(), expect.cumsum())
 
 
+# one accumulator for all 512 blocks (4,097 to 8,192 bins), two and three, and one without groups of tickets: additions queue up
+@pytest.mark.parametrize("bins", [3000, 4097, 5000, 8192, 8193, 16384])
+def test_count_many_blocks_on_few_accumulators(device, bins):
+    x = torch.randint(0, bins, (512 * 16384 + 1,), dtype=torch.int32, device=device)
+    expect = torch.bincount(x, minlength=bins)
+    for _ in range(5):
+        assert torch.equal(cute_kernels.continuous_count_cute(x, bins).long(), expect)
+
+
 def test_count_large_sum_property(device):
     # full-size property at 2^28 ids (1 GiB): counts sum to N and match a strided sample's histogram scaled check
     n = 1 << 28
