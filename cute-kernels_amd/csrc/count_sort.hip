@@ -1,7 +1,7 @@
 // Expert histogram, offset scans and the stable token->expert counting sort.
 //
-// count:  one launch. Waves privatise the histogram (ballot/popcount counters in registers for <= 8 bins, else LDS copies, one a
-//         wave while they fit), blocks merge into a zero-initialised global accumulator, and the last block to finish (ticket
+// count:  one launch. Waves privatise the histogram (ballot/popcount counters in registers for <= 8 bins, LDS copies up to 1,024 bins,
+//         one copy for the block beyond), blocks merge into a zero-initialised global accumulator, and the last block to finish (ticket
 //         counters) scans the bins, writes counts / inclusive ends / exclusive starts and puts the accumulator back to
 //         zero.
 // sort:   up to 4,096 ids one launch of one block (sort_small_kernel), beyond that two. (1) every block histograms its
@@ -558,15 +558,18 @@ int launch_count(const char* name, const void* ids, int32_t ids_are_i64, int64_t
   // 44.5 / 50.2 and 82.4 / 162.8; a ticket for each block on one address alone cost 4 us of a launch of 512 blocks.) Small
   // inputs want blocks of 8 waves, whose barriers and merge are shorter (1,024 ids 2.6 us against 3.0), as long as
   // that makes few blocks -- up to 16, or 512 where a block's merge is short (32 bins or fewer: 2^20 ids over 16 experts 5.4 us
-  // against 6.7; over 128 experts 7.6 against 7.0).
+  // against 6.7; over 128 experts 7.6 against 7.0). What two of them would share fits one wide block, which merges nothing:
+  // 16,384 int32 ids over 64 / 2,048 / 16,384 bins 5.3 / 5.0 / 6.1 us against 6.0 / 9.1 / 21.3.
   const int64_t narrow = ceil_div(n, (int64_t)kNarrowCount * vec * 4);
-  const bool wide = narrow > (num_bins <= 32 ? 512 : 16);
+  const bool wide = narrow == kWideCount / kNarrowCount || narrow > (num_bins <= 32 ? 512 : 16);
   const int threads = wide ? kWideCount : kNarrowCount;
   int64_t blocks = wide ? ceil_div(n, (int64_t)kWideCount * vec * 4) : narrow;
   blocks = blocks < 1 ? 1 : blocks > kMaxCountBlocks ? kMaxCountBlocks : blocks;
-  // copies of the histogram in LDS: one a wave, at most 32 KiB of them
-  int copies = reg_bins > 0 ? 1 : kMaxCountBins / 2 / num_bins;
-  copies = copies < 1 ? 1 : copies > threads / kWave ? threads / kWave : copies;
+  // copies of the histogram in LDS: one a wave up to 1,024 bins, at most 32 KiB of them; beyond, waves seldom meet in a bin, and
+  // clearing and adding up copies costs more than it saves (1,024 ids over 4,096 bins 4.6 us with one, 6.1 with two; 2^20 10.8
+  // and 11.8)
+  int copies = reg_bins > 0 || num_bins > 1024 ? 1 : kMaxCountBins / 2 / num_bins;
+  copies = copies > threads / kWave ? threads / kWave : copies;
   const size_t lds_bytes = ((size_t)copies * num_bins + threads / kWave + 2) * sizeof(uint32_t);
   const CountLayout layout = count_layout(num_bins);
 #define CK_LAUNCH_COUNT_W(ID_T, RB, THREADS)                                                                              \

@@ -78,13 +78,13 @@ def test_count_misaligned_views_out_of_range_and_shortcut(device):
     )
 
 
-# narrow and wide blocks, one trip and several: 16 and 512 blocks of 512 threads (8,192 int32 or 4,096 int64 ids each) and 512
-# of 1,024 threads, and one id more
+# narrow and wide blocks, one trip and several: 1, 16 and 512 blocks of 512 threads (8,192 int32 or 4,096 int64 ids each), 1 and
+# 512 of 1,024 threads, and one id more; the most bins with a histogram per wave and the fewest with one for all waves
 @pytest.mark.parametrize("dtype", [torch.int32, torch.long])
-@pytest.mark.parametrize("bins", [1, 8, 9, 32, 33, 128])
+@pytest.mark.parametrize("bins", [1, 8, 9, 32, 33, 128, 1024, 1025])
 def test_count_launch_forms(device, bins, dtype):
     per_block = 8192 if dtype == torch.int32 else 4096
-    for n in (1, 512, per_block, per_block + 1, 16 * per_block, 16 * per_block + 1, 512 * per_block, 512 * per_block + 1, 1024 * per_block + 1):
+    for n in (1, 512, per_block, per_block + 1, 2 * per_block, 2 * per_block + 1, 16 * per_block, 16 * per_block + 1, 512 * per_block, 512 * per_block + 1, 1024 * per_block + 1):
         x = torch.randint(0, bins, (n,), dtype=dtype, device=device)
         expect = torch.bincount(x, minlength=bins).cpu().numpy()
         for repeat in range(2):  # tickets and accumulators come back to zero
