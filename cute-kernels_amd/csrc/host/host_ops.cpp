@@ -1073,13 +1073,16 @@ bool router_rows_fit(int64_t B, int64_t H, int64_t E) {
 bool router_rows_take(const Tensor& x, const Tensor& gate_weight, const OptTensor& norm_weight) {
   if (!x.is_cuda() || x.dim() < 1 || gate_weight.dim() != 2 || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return false;
   const Tensor nw = value_or_undefined(norm_weight);
-  // the kernel reads 16 bytes at a time; what is not contiguous is copied first, to where a new tensor begins
-  for (const Tensor* t : {&x, &gate_weight, &nw})
-    if (t->defined() && t->is_contiguous() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0) return false;
+  for (const Tensor* t : {&x, &gate_weight, &nw}) {
+    if (!t->defined()) continue;
+    // the kernel reads 16 bytes at a time; what is not contiguous is copied first, to where a new tensor begins
+    if (t->is_contiguous() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0) return false;
+    if (t->_fw_grad(/*level=*/0).defined()) return false;  // forward-mode tangents
+  }
   const int64_t H = x.size(-1);
-  return !any_requires_grad({&x, &gate_weight, &nw}) && x.numel() > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
+  return x.numel() > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
 }
-// x @ gate_weight^T of few 16-bit rows (router_rows_take)
+// x @ gate_weight^T of few 16-bit rows (router_rows_take), without autograd
 Tensor router_rows(const Tensor& x_in, const Tensor& gate_weight_in) {
   require_dims({{&x_in, 2}, {&gate_weight_in, 2}});
   require_gpu(x_in, gate_weight_in);
@@ -1092,7 +1095,9 @@ Tensor router_rows(const Tensor& x_in, const Tensor& gate_weight_in) {
                            dtype_code(x), l.stream));
   return logits;
 }
-NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& gate_weight, double eps, bool quantize, bool want_rstd) {
+// few_rows: ck_router_rows, which the caller has found to take the call, instead of ck_rmsnorm_route
+NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& gate_weight, double eps, bool quantize, bool want_rstd,
+                             bool few_rows) {
   const Launch l(x);
   const int64_t B = x.size(0), H = x.size(1), E = gate_weight.size(0);
   NormRoute r;
@@ -1103,7 +1108,7 @@ NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const T
     r.x8 = new_empty({B, H}, x, at::kFloat8_e4m3fn);
     r.scale8 = new_empty({B}, x, at::kFloat);
   }
-  if (router_rows_fit(B, H, E)) {
+  if (few_rows) {
     check(api.ck_router_rows(ptr(x), ptr(norm_weight), ptr(gate_weight), (float)eps, 1, B, (int32_t)H, (int32_t)E, ptr(r.y), (float*)ptr(r.rstd),
                              ptr(r.logits), ptr(r.x8), (float*)ptr(r.scale8), dtype_code(x), l.stream));
     return r;
@@ -1125,9 +1130,10 @@ Tensor gate_weight_grad(const Tensor& d_logits, const Tensor& y) {
 }
 
 struct NormRouteFn : torch::autograd::Function<NormRouteFn> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x_in, const OptTensor& norm_weight_in, const Tensor& gate_weight_in, double eps) {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x_in, const OptTensor& norm_weight_in, const Tensor& gate_weight_in, double eps,
+                               bool few_rows) {
     const Tensor x = x_in.contiguous(), nw = contiguous(value_or_undefined(norm_weight_in)), gw = gate_weight_in.contiguous();
-    NormRoute r = norm_route_forward(x, nw, gw, eps, false, true);
+    NormRoute r = norm_route_forward(x, nw, gw, eps, false, true, few_rows);
     ctx->save_for_backward({x, nw, gw, r.rstd, r.y});
     ctx->saved_data["eps"] = eps;
     ctx->saved_data["need_gate"] = gate_weight_in.requires_grad();
@@ -1135,7 +1141,7 @@ struct NormRouteFn : torch::autograd::Function<NormRouteFn> {
     return {r.y, r.logits};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    variable_list out(4);
+    variable_list out(5);
     const auto s = ctx->get_saved_variables();
     Tensor d_total = grads[0];
     if (grads[1].defined()) {
@@ -1152,16 +1158,16 @@ struct NormRouteFn : torch::autograd::Function<NormRouteFn> {
 };
 // x [B, H]: (y, logits, x8, scale8)
 std::tuple<Tensor, Tensor, OptTensor, OptTensor> norm_route(const Tensor& x, const OptTensor& norm_weight, const Tensor& gate_weight, double eps,
-                                                            bool quantize) {
+                                                            bool quantize, bool few_rows) {
   const Tensor nw = value_or_undefined(norm_weight);
   require_gpu(x, nw, gate_weight);
   if (any_requires_grad({&x, &nw, &gate_weight})) {
-    auto out = NormRouteFn::apply(x, norm_weight, gate_weight, eps);
+    auto out = NormRouteFn::apply(x, norm_weight, gate_weight, eps, few_rows);
     OptTensor x8, scale8;
     if (quantize) std::tie(x8, scale8) = quantize_rows(out[0].detach());
     return {out[0], out[1], x8, scale8};
   }
-  NormRoute r = norm_route_forward(x.contiguous(), contiguous(nw), gate_weight.contiguous(), eps, quantize, false);
+  NormRoute r = norm_route_forward(x.contiguous(), contiguous(nw), gate_weight.contiguous(), eps, quantize, false, few_rows);
   return {r.y, r.logits, to_opt(r.x8), to_opt(r.scale8)};
 }
 

@@ -21,8 +21,8 @@ MAX_EXPERTS, MAX_HIDDEN, HIDDEN_STEP = 128, 4096, 512
 
 def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor, norm_weight: torch.Tensor | None = None) -> bool:
     """Whether few enough 16-bit rows meet few enough experts for the kernel that gives 16 rows x 16 experts a workgroup of
-    their own (ck_router_rows, with or without the norm), and nothing but plain inference is asked for: a linear layer casts
-    under autocast, and gradients take the routes that they always took."""
+    their own (ck_router_rows, with or without the norm). A linear layer casts under autocast. With the norm ahead the answer
+    is the same with gradients and without, so that both compute the same rows and logits."""
     return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight, norm_weight)
 
 
@@ -41,6 +41,7 @@ def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
         and weight.dtype == x.dtype
         and x.dim() == 2
         and x.size(1) == weight.size(1)
+        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
         and "forward" not in vars(gate)
         and not (gate._forward_hooks or gate._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks)
         and router_rows_fit(x, weight)
@@ -51,8 +52,7 @@ def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
 
 def rmsnorm_route_fused(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
     """Whether ck_rmsnorm_route takes this shape: 16-bit rows, hidden size a multiple of 512 up to 4096, at most 128 experts.
-    Other shapes run rmsnorm_cute followed by the linear layer (and quantize_rows_e4m3), with the same results contract, or,
-    few rows, ck_router_rows (router_rows_fit)."""
+    Other shapes run rmsnorm_cute followed by the linear layer (and quantize_rows_e4m3), with the same results contract."""
     H, E = x.size(-1), gate_weight.size(0)
     return (
         x.dtype in (torch.bfloat16, torch.float16)
@@ -81,7 +81,8 @@ def rmsnorm_route_cute(
     router_logits [tokens, E] is what `nn.Linear(H, E, bias=False)` with `gate_weight` returns for the 16-bit y (fp32
     accumulation, another summation order: equal within the rounding of the logits' dtype).
     fused: True takes the one-pass kernel wherever it supports the shape, False the separate kernels; None (default)
-    the one-pass kernel where it is the faster route (router_rows_fit, rmsnorm_route_pays)."""
+    ck_router_rows for few rows (router_rows_fit), else the one-pass kernel where it is the faster route
+    (rmsnorm_route_pays)."""
     if norm_weight is not None:
         assert norm_weight.dim() == 1 and norm_weight.size(0) == x.size(-1), "hidden size for x and weight tensor is different"
         assert norm_weight.dtype == x.dtype, "tensors weight and y should have same dtype"
@@ -94,7 +95,7 @@ def rmsnorm_route_cute(
     if fused is None:
         fused = rmsnorm_route_pays(x, gate_weight)
     if few_rows or (fused and rmsnorm_route_fused(x, gate_weight)):
-        y, logits, x8, scale8 = _C.host().norm_route(x.reshape(-1, x.size(-1)), norm_weight, gate_weight, eps, quantize)
+        y, logits, x8, scale8 = _C.host().norm_route(x.reshape(-1, x.size(-1)), norm_weight, gate_weight, eps, quantize, few_rows)
         y = y.view(x.shape)
     else:
         y = rmsnorm_cute(x, norm_weight, eps)

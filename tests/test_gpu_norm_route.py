@@ -57,6 +57,43 @@ def test_rmsnorm_route_matches_oracle_composition(device, dtype, B, H, E, with_w
     assert torch.equal(x8.cpu().view(torch.uint8), oq.view(torch.uint8)) and torch.equal(scale8.cpu(), os_)
 
 
+def _one_pass(x, w, gate, eps):
+    """ck_rmsnorm_route through the C ABI: (y, rstd, logits, x8, scale8)."""
+    from cute_kernels import _C
+
+    (B, H), E = x.shape, gate.size(0)
+    new = lambda *shape, dtype: torch.empty(*shape, dtype=dtype, device=x.device)
+    y, logits, rstd = torch.empty_like(x), new(B, E, dtype=x.dtype), new(B, dtype=torch.float32)
+    x8, scale8 = new(B, H, dtype=torch.float8_e4m3fn), new(B, dtype=torch.float32)
+    packed = new((E + 15) // 16 * 16 * H, dtype=x.dtype)
+    _C.check(_C.lib().ck_rmsnorm_route(_C.ptr(x), None if w is None else _C.ptr(w), _C.ptr(gate), eps, B, H, E, _C.ptr(y), _C.ptr(rstd),
+                                       _C.ptr(logits), _C.ptr(x8), _C.ptr(scale8), _C.ptr(packed), _C.dtype_code(x.dtype), _C.stream()))
+    return y, rstd, logits, x8, scale8
+
+
+@pytest.mark.parametrize("needs_grad", [False, True])
+@pytest.mark.parametrize("with_weight", [True, False])
+@pytest.mark.parametrize("H", [512 * s for s in range(1, 9)])
+def test_fused_is_the_one_pass_kernel(device, H, with_weight, needs_grad):
+    """fused=True takes ck_rmsnorm_route for few rows too, with gradients and without: its bits, and its results against float64
+    at every width it has an instantiation for and ragged numbers of rows and experts."""
+    B, E, eps = 300 + H // 512, 60 + H // 512, 1e-6
+    x, w, gate = (None if t is None else t.to(device) for t in _inputs(torch.float16, B, H, E, H, with_weight))
+    y, rstd, logits, x8, scale8 = _one_pass(x, w, gate, eps)
+    exact = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + eps)
+    exact = exact if w is None else exact * w.double()
+    # one rounding of y (2 ** -11) behind a sum of H squares and four fp32 operations; logits as sums of H products in fp32
+    assert bool(((y.double() - exact).abs() <= exact.abs() * (2.0**-11 + (1 + 2.0**-11) * (H + 4) * 2.0**-24) + 2.0**-25).all())
+    own = y.double() @ gate.double().t().contiguous()
+    slack = H * 2.0**-24 * (y.double().abs() @ gate.double().abs().t().contiguous())
+    assert bool(((logits.double() - own).abs() <= 2.0**-11 * own.abs() + (1 + 2.0**-11) * slack + 2.0**-25).all())
+    torch.testing.assert_close(rstd.double(), torch.rsqrt(x.double().square().mean(-1) + eps), rtol=1e-6, atol=0)
+    q, s = cute_kernels.quantize_rows_e4m3(y)
+    assert torch.equal(x8.view(torch.uint8), q.view(torch.uint8)) and torch.equal(scale8, s)
+    fy, flogits = cute_kernels.rmsnorm_route_cute(x.clone().requires_grad_(needs_grad), w, gate, eps, fused=True)
+    assert torch.equal(fy, y) and torch.equal(flogits, logits)
+
+
 def test_rmsnorm_route_rstd_and_all_zero_rows(device):
     x, w, gate = _inputs(torch.bfloat16, 40, 1024, 32, 5)
     x[3] = 0
