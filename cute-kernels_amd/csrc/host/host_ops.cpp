@@ -1082,18 +1082,33 @@ bool router_rows_take(const Tensor& x, const Tensor& gate_weight, const OptTenso
   const int64_t H = x.size(-1);
   return x.numel() > 0 && router_rows_fit(x.numel() / H, H, gate_weight.size(0));
 }
-// x @ gate_weight^T of few 16-bit rows (router_rows_take), without autograd
-Tensor router_rows(const Tensor& x_in, const Tensor& gate_weight_in) {
-  require_dims({{&x_in, 2}, {&gate_weight_in, 2}});
-  require_gpu(x_in, gate_weight_in);
+Tensor router_rows_forward(const Tensor& x_in, const Tensor& gate_weight_in) {
   const int64_t B = x_in.size(0), H = x_in.size(1), E = gate_weight_in.size(0);
-  TORCH_CHECK(gate_weight_in.size(1) == H && gate_weight_in.scalar_type() == x_in.scalar_type(), "router_rows: rows and weight disagree");
   const Tensor x = x_in.contiguous(), gate_weight = gate_weight_in.contiguous();
   const Launch l(x);
   const Tensor logits = new_empty({B, E}, x);
   check(api.ck_router_rows(ptr(x), nullptr, ptr(gate_weight), 0.f, 0, B, (int32_t)H, (int32_t)E, nullptr, nullptr, ptr(logits), nullptr, nullptr,
                            dtype_code(x), l.stream));
   return logits;
+}
+struct RouterRows : torch::autograd::Function<RouterRows> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& gate_weight) {
+    ctx->save_for_backward({x, gate_weight});
+    return router_rows_forward(x, gate_weight);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {  // as a linear layer's
+    const auto s = ctx->get_saved_variables();
+    const Tensor& d_logits = grads[0];
+    return {ctx->needs_input_grad(0) ? at::mm(d_logits, s[1]) : Tensor(), ctx->needs_input_grad(1) ? at::mm(d_logits.t(), s[0]) : Tensor()};
+  }
+};
+// x @ gate_weight^T of few 16-bit rows (router_rows_take)
+Tensor router_rows(const Tensor& x, const Tensor& gate_weight) {
+  require_dims({{&x, 2}, {&gate_weight, 2}});
+  require_gpu(x, gate_weight);
+  TORCH_CHECK(gate_weight.size(1) == x.size(1) && gate_weight.scalar_type() == x.scalar_type(), "router_rows: rows and weight disagree");
+  if (any_requires_grad({&x, &gate_weight})) return RouterRows::apply(x, gate_weight);
+  return router_rows_forward(x, gate_weight);
 }
 // few_rows: ck_router_rows, which the caller has found to take the call, instead of ck_rmsnorm_route
 NormRoute norm_route_forward(const Tensor& x, const Tensor& norm_weight, const Tensor& gate_weight, double eps, bool quantize, bool want_rstd,

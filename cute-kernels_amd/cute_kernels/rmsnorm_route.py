@@ -21,14 +21,14 @@ MAX_EXPERTS, MAX_HIDDEN, HIDDEN_STEP = 128, 4096, 512
 
 def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor, norm_weight: torch.Tensor | None = None) -> bool:
     """Whether few enough 16-bit rows meet few enough experts for the kernel that gives 16 rows x 16 experts a workgroup of
-    their own (ck_router_rows, with or without the norm). A linear layer casts under autocast. With the norm ahead the answer
-    is the same with gradients and without, so that both compute the same rows and logits."""
+    their own (ck_router_rows, with or without the norm). A linear layer casts under autocast. The answer is the same with
+    gradients and without: a segment that is checkpointed by running it twice selects the same experts both times."""
     return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight, norm_weight)
 
 
 def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     """gate(x) for rows x [tokens, H]. A plain bias-free nn.Linear that nobody watches (hooks, a forward of its own, other
-    tensor types) runs as ck_router_rows where few rows come without gradients: the library's product takes 15 us there."""
+    tensor types) runs as ck_router_rows on few rows: the library's product takes 15 us there."""
     weight = getattr(gate, "weight", None)
     if (
         not is_tracing()
@@ -41,9 +41,9 @@ def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
         and weight.dtype == x.dtype
         and x.dim() == 2
         and x.size(1) == weight.size(1)
-        and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
         and "forward" not in vars(gate)
         and not (gate._forward_hooks or gate._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks)
+        and not (gate._backward_hooks or gate._backward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks)
         and router_rows_fit(x, weight)
     ):
         return _C.host().router_rows(x, weight)

@@ -87,3 +87,64 @@ def test_a_watched_or_replaced_gate_is_called():
     x.requires_grad_()
     moe(x)[1].float().sum().backward()
     assert x.grad is not None and moe.gate.weight.grad is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,E,H", [(1024, 64, 2048), (256, 8, 4096), (1500, 16, 1536), (256, 128, 4096)])
+def test_the_same_logits_with_gradients_and_without(T, E, H, dtype):
+    """A reentrant checkpoint runs its segment without gradients first and again with them: the same experts have to be selected."""
+    x, w, nw = _inputs(T, H, E, dtype)
+    gate = torch.nn.Linear(H, E, bias=False, device=DEV, dtype=dtype)
+    with torch.no_grad():
+        gate.weight.copy_(w)
+        plain = rmsnorm_route.router_logits(gate, x)
+        y, logits = rmsnorm_route.rmsnorm_route_cute(x, nw, w, 1e-6)
+    for leaf in (False, True):
+        assert torch.equal(plain, rmsnorm_route.router_logits(gate, x.clone().requires_grad_(leaf)))
+        gy, glogits = rmsnorm_route.rmsnorm_route_cute(x.clone().requires_grad_(leaf), nw, gate.weight, 1e-6)
+        assert torch.equal(y, gy) and torch.equal(logits, glogits)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("needs", [(True, True), (True, False), (False, True)])
+def test_gradients_of_the_few_row_router_are_a_linear_layers(needs, dtype):
+    x, w, _ = _inputs(130, 1056, 60, dtype)
+    g = torch.randn(130, 60, device=DEV).to(dtype)
+    ours, linear = ([t.clone().requires_grad_(n) for t, n in zip((x, w), needs)] for _ in range(2))
+    _C.host().router_rows(*ours).backward(g)
+    torch.nn.functional.linear(*linear).backward(g)
+    for a, b in zip(ours, linear):
+        assert (a.grad is None) == (b.grad is None) and (a.grad is None or torch.equal(a.grad, b.grad))
+
+
+def test_second_gradients_and_tangents_of_the_few_row_router():
+    x, w, _ = _inputs(33, 640, 8, torch.float16)
+    gate = torch.nn.Linear(640, 8, bias=False, device=DEV, dtype=torch.float16)
+    gate.weight.data.copy_(w)
+    v, u = torch.randn_like(x), torch.randn(33, 8, device=DEV).half()
+    seconds = []
+    for f in (lambda rows: rmsnorm_route.router_logits(gate, rows), gate):
+        leaf, upstream = x.clone().requires_grad_(), u.clone().requires_grad_()
+        (first,) = torch.autograd.grad(f(leaf), leaf, upstream, create_graph=True)
+        seconds.append(torch.autograd.grad(first, (upstream, gate.weight), v))
+    for a, b in zip(*seconds):
+        assert torch.equal(a, b)
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():  # a linear layer has a forward-mode rule
+        dual = torch.autograd.forward_ad.make_dual(x, v)
+        assert torch.autograd.forward_ad.unpack_dual(rmsnorm_route.router_logits(gate, dual)).tangent is not None
+
+
+def test_backward_hooks_of_the_gate_run():
+    gate = torch.nn.Linear(640, 8, bias=False, device=DEV, dtype=torch.bfloat16)
+    x = _inputs(9, 640, 8, torch.bfloat16)[0].requires_grad_()
+    seen = []
+    handles = [gate.register_full_backward_hook(lambda m, gi, go: seen.append("hook")), gate.register_full_backward_pre_hook(lambda m, go: seen.append("pre"))]
+    for handle in handles:
+        rmsnorm_route.router_logits(gate, x).float().sum().backward()
+        handle.remove()
+    assert seen == ["pre", "hook", "pre"]
+    for register in (torch.nn.modules.module.register_module_full_backward_hook, torch.nn.modules.module.register_module_full_backward_pre_hook):
+        handle = register(lambda *a: seen.append("global"))
+        rmsnorm_route.router_logits(gate, x).float().sum().backward()
+        handle.remove()
+    assert seen[3:] == ["global"] * 2
