@@ -1068,13 +1068,14 @@ struct NormRoute {
 // Where ck_router_rows is the faster way from rows to router logits: while its workgroups (16 rows x 16 experts) do not outnumber
 // the compute units.
 bool router_rows_fit(int64_t B, int64_t H, int64_t E) {
-  return H >= 32 && H % 32 == 0 && H <= 4096 && ((B + 15) / 16) * ((E + 15) / 16) <= 256;
+  return H >= 32 && H % 32 == 0 && H <= 4096 && E >= 1 && ((B + 15) / 16) * ((E + 15) / 16) <= 256;
 }
 bool router_rows_take(const Tensor& x, const Tensor& gate_weight, const OptTensor& norm_weight) {
   if (!x.is_cuda() || x.dim() < 1 || gate_weight.dim() != 2 || (x.scalar_type() != at::kBFloat16 && x.scalar_type() != at::kHalf)) return false;
   const Tensor nw = value_or_undefined(norm_weight);
   for (const Tensor* t : {&x, &gate_weight, &nw}) {
     if (!t->defined()) continue;
+    if (t->device() != x.device()) return false;
     // the kernel reads 16 bytes at a time; what is not contiguous is copied first, to where a new tensor begins
     if (t->is_contiguous() && (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0) return false;
     if (t->_fw_grad(/*level=*/0).defined()) return false;  // forward-mode tangents

@@ -148,3 +148,10 @@ def test_backward_hooks_of_the_gate_run():
         rmsnorm_route.router_logits(gate, x).float().sum().backward()
         handle.remove()
     assert seen[3:] == ["global"] * 2
+
+
+def test_a_router_without_experts_keeps_its_route():
+    x, _, nw = _inputs(9, 640, 8, torch.bfloat16)
+    w = x.new_empty(0, 640)
+    y, logits = rmsnorm_route.rmsnorm_route_cute(x, nw, w, 1e-6)
+    assert logits.shape == (9, 0) and torch.equal(y, cute_kernels.rmsnorm_cute(x, nw, 1e-6))
