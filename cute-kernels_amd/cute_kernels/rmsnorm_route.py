@@ -11,6 +11,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 import torch.nn.modules.module as _module
+from torch.utils._device import DeviceContext
 
 from . import _C
 from .rmsnorm import rmsnorm_cute
@@ -26,9 +27,17 @@ def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor, norm_weight: tor
     return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight, norm_weight)
 
 
+def _modes_watch() -> bool:
+    """Whether a dispatch or function mode (a FLOP counter, a quantiser) is to see the operators that run. The mode behind
+    `with torch.device(...)` changes where new tensors live and nothing else."""
+    return torch._C._len_torch_dispatch_stack() > 0 or any(
+        not isinstance(torch._C._get_function_stack_at(i), DeviceContext) for i in range(torch._C._len_torch_function_stack())
+    )
+
+
 def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """gate(x) for rows x [tokens, H]. A plain bias-free nn.Linear that nobody watches (hooks, a forward of its own, other
-    tensor types) runs as ck_router_rows on few rows: the library's product takes 15 us there."""
+    """gate(x) for rows x [tokens, H]. A plain bias-free nn.Linear that nobody watches (hooks, modes, a forward of its
+    own, other tensor types) runs as ck_router_rows on few rows: the library's product takes 15 us there."""
     weight = getattr(gate, "weight", None)
     if (
         not is_tracing()
@@ -42,6 +51,7 @@ def router_logits(gate: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
         and x.dim() == 2
         and x.size(1) == weight.size(1)
         and "forward" not in vars(gate)
+        and not _modes_watch()
         and not (gate._forward_hooks or gate._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks)
         and not (gate._backward_hooks or gate._backward_pre_hooks or _module._global_backward_hooks or _module._global_backward_pre_hooks)
         and router_rows_fit(x, weight)

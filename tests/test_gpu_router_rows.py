@@ -3,6 +3,7 @@ gate module."""
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import cute_kernels
 from cute_kernels import _C, rmsnorm_route
@@ -155,3 +156,31 @@ def test_a_router_without_experts_keeps_its_route():
     w = x.new_empty(0, 640)
     y, logits = rmsnorm_route.rmsnorm_route_cute(x, nw, w, 1e-6)
     assert logits.shape == (9, 0) and torch.equal(y, cute_kernels.rmsnorm_cute(x, nw, 1e-6))
+
+
+def test_modes_see_the_linear_layer():
+    x, w, _ = _inputs(9, 640, 8, torch.bfloat16)
+    gate = torch.nn.Linear(640, 8, bias=False, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        gate.weight.copy_(w)
+        seen = []
+
+        class Recorder(TorchDispatchMode):
+            def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+                seen.append(func)
+                return func(*args, **(kwargs or {}))
+
+        with Recorder():
+            rmsnorm_route.router_logits(gate, x)
+        assert torch.ops.aten.mm.default in seen
+
+        class Doubled(torch.overrides.TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                out = func(*args, **(kwargs or {}))
+                return 2 * out if func is torch.nn.functional.linear else out
+
+        plain = rmsnorm_route.router_logits(gate, x)
+        with Doubled():
+            torch.testing.assert_close(rmsnorm_route.router_logits(gate, x), 2 * plain, rtol=2.0**-7, atol=1e-6)
+        with torch.device(DEV):  # not a mode that asks for operators
+            assert torch.equal(rmsnorm_route.router_logits(gate, x), plain)
