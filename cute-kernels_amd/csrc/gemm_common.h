@@ -58,6 +58,7 @@ constexpr int kSplitParts = 4, kSplitMaxTail = 64, kSplitMaxRounds = 64;
 // K steps that splitting has to take off the last round. A step of a 256 x 256 tile takes 1.5 to 1.7 us, and the parts'
 // device-wide fences and the exchange of their accumulators 60 to 80 us however short they are.
 constexpr int kSplitMinSaved = 40;
+constexpr bool split_pays(int k_steps, int parts) { return k_steps - (k_steps + parts - 1) / parts >= kSplitMinSaved; }
 constexpr int64_t kSplitPartFloats = 4 * 64 * 64 * 4;  // one workgroup's 256 x 256 fp32 tile
 constexpr int64_t kSplitWorkspaceBytes = kSplitMaxTail * kSplitParts * kSplitPartFloats * 4 + 2 * kSplitMaxTail * 8;
 

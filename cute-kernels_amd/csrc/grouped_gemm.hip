@@ -902,6 +902,8 @@ extern "C" int ck_grouped_gemm_ws(const void* a, int32_t a_gather_div, const voi
 
 extern "C" int64_t ck_grouped_gemm_workspace_bytes(void) { return kSplitWorkspaceBytes; }
 
+extern "C" int ck_grouped_gemm_uses_workspace(int32_t K) { return K > 0 && K % kLineK == 0 && split_pays(K / kLineK, kSplitParts); }
+
 static int grouped_gemm_nn_impl(const void* a, const void* w, int32_t N, int32_t K, const ck_segments* seg,
                                 int32_t epilogue, void* y, int32_t dtype, void* stream, void* workspace,
                                 int64_t workspace_bytes) {

@@ -101,14 +101,15 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
     if constexpr (kSplit) {
       // The tiles of the last, partial round (the highest block indices: the hardware hands blocks out in order) would
       // each keep one CU busy for a whole tile time while the rest of the chip idles. When that round is at most half
-      // full, and splitting takes steps enough off it (kSplitMinSaved), every such tile is computed by 2 to 4 workgroups (as many as fill the chip), an equal share of the contraction each: part
-      // 0 is the tile's own block, parts 1.. are extra blocks behind the regular grid. All write their fp32 accumulators
-      // to the workspace; the last to arrive (ticket) adds the parts up in part order and runs the epilogue.
+      // full, and splitting takes steps enough off it (split_pays), every such tile is computed by 2 to 4 workgroups (as many
+      // as fill the chip), an equal share of the contraction each: part 0 is the tile's own block, parts 1.. are extra
+      // blocks behind the regular grid. All write their fp32 accumulators to the workspace; the last to arrive
+      // (ticket) adds the parts up in part order and runs the epilogue.
       const int cus = kXcds * 32;
       const int tail = total % cus;
       const int k_steps = prm.K / BK, parts = tail > 0 ? min(kSplitParts, cus / tail) : kSplitParts;
       const bool active = prm.split_ws != nullptr && tail > 0 && tail <= 2 * kSplitMaxTail && total / cus <= kSplitMaxRounds &&
-                          k_steps - (k_steps + parts - 1) / parts >= kSplitMinSaved;
+                          split_pays(k_steps, parts);
       split_parts = active ? parts : kSplitParts;  // as many parts as fill the chip: 4, 3 or 2
       if (pid >= prm.split_base) {  // an extra block
         const int x = pid - prm.split_base;
@@ -875,7 +876,8 @@ int launch_bn(const GemmParams& prm, int mode, bool bt, unsigned blocks, hipStre
 int launch_line(const GemmParams& prm_in, int mode, int bn, bool bt, int dtype, unsigned blocks, hipStream_t stream,
                 const char* name) {
   GemmParams prm = prm_in;
-  if (prm.split_ws != nullptr && (mode == kGrouped || mode == kScatter)) {
+  // no more is taken off a round than by the most parts: where that does not pay there are no extra workgroups either
+  if (prm.split_ws != nullptr && (mode == kGrouped || mode == kScatter) && split_pays(prm.K / kLineK, kSplitParts)) {
     prm.split_base = (int)blocks;  // the extra workgroups of a split last round sit behind the regular grid
     prm.split_tag = next_split_tag();
     blocks += kSplitMaxTail * (kSplitParts - 1);

@@ -36,7 +36,7 @@ using torch::autograd::variable_list;
   X(ck_last_error_string) X(ck_count_workspace_words) X(ck_count_offsets) X(ck_route_topk_softmax_all)                  \
   X(ck_route_topk_softmax_bwd) X(ck_route_topk_softmax_bwd_exact) X(ck_sort_max_rows) X(ck_sort_workspace_words)        \
   X(ck_sort_by_expert) X(ck_combine_rows) X(ck_gate_grad_both) X(ck_group_rows_padded) X(ck_swiglu_bwd_grouped)         \
-  X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
+  X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_uses_workspace) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
   X(ck_grouped_gemm_f32) X(ck_grouped_gemm_dw_f32) X(ck_grouped_gemm_dw) X(ck_grouped_gemm_dw_rows)                     \
   X(ck_quant_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) X(ck_router_rows) \
   X(ck_gelu_tanh_bwd_grouped) X(ck_fused_residual_add_rmsnorm_fwd) X(ck_rmsnorm_fwd) X(ck_rmsnorm_bwd_partial_rows) X(ck_rmsnorm_bwd_typed)         \
@@ -327,9 +327,11 @@ const char* epilogue_name(int64_t epilogue, bool nn) {
 
 bool is_f32(const Tensor& t) { return t.scalar_type() == at::kFloat; }
 
-Tensor split_workspace(const Tensor& like, void* stream, int64_t flags) {
-  return (flags & kGemmSplit) ? workspace(kSplitWs, like, stream, (api.ck_grouped_gemm_workspace_bytes() + 3) / 4) : Tensor();
+Tensor split_workspace(const Tensor& like, void* stream) {
+  return workspace(kSplitWs, like, stream, (api.ck_grouped_gemm_workspace_bytes() + 3) / 4);
 }
+// whether a launch of contraction K may split its last round
+bool may_split(int64_t K, int64_t flags) { return (flags & kGemmSplit) && api.ck_grouped_gemm_uses_workspace((int32_t)K); }
 
 void gemm_f32(const Tensor& a, int64_t gather_div, const Tensor& w, bool w_is_kn, int64_t N, int64_t K, const Segments& seg,
               bool scatter, const Tensor& y, const Tensor& bias, const Tensor& rows_in, const Tensor& rows_out) {
@@ -353,8 +355,8 @@ void gemm(const Tensor& a, int64_t gather_div, const Tensor& w, const Segments& 
   timed(epilogue_name(epilogue, false), N, K, [&] {
     const Launch l(w);
     const ck_segments cs = seg.c(rows_in, rows_out);
-    const bool splits = epilogue == CK_EPI_GROUPED || epilogue == CK_EPI_SCATTER;
-    const Tensor ws = splits ? split_workspace(w, l.stream, flags) : Tensor();
+    const bool splits = (epilogue == CK_EPI_GROUPED || epilogue == CK_EPI_SCATTER) && may_split(K, flags);
+    const Tensor ws = splits ? split_workspace(w, l.stream) : Tensor();
     check(api.ck_grouped_gemm_ws(ptr(a), (int32_t)gather_div, ptr(w), (int32_t)N, (int32_t)K, &cs, (int32_t)epilogue, ptr(y), ptr(y_t),
                                  seg.max_rows, ptr(aux), ptr(aux_in), dtype_code(w), l.stream, ptr(ws), ws.defined() ? ws.nbytes() : 0));
   });
@@ -377,7 +379,7 @@ void gemm_dx(const Tensor& d_y, const Tensor& w, const Segments& seg, int64_t ep
     return timed(epilogue_name(epilogue, true), n_in, n_out, [&] {
       const Launch l(w);
       const ck_segments cs = seg.c(Tensor(), rows_out);
-      const Tensor ws = split_workspace(w, l.stream, flags);
+      const Tensor ws = may_split(n_out, flags) ? split_workspace(w, l.stream) : Tensor();
       check(api.ck_grouped_gemm_nn_ws(ptr(d_y), ptr(w), (int32_t)n_in, (int32_t)n_out, &cs, (int32_t)epilogue, ptr(out), dtype_code(w),
                                       l.stream, ptr(ws), ws.defined() ? ws.nbytes() : 0));
     });
@@ -1357,5 +1359,5 @@ PYBIND11_MODULE(_ck_host, m) {
       }));
   DEF("expert_bias_grad", ([](const Tensor& d_y, py::object seg) { return expert_bias_grad(d_y, Segments::of(seg)); }));
   DEF("slot_experts", slot_experts);
-  DEF("split_workspace", ([](const Tensor& like) { return split_workspace(like, Launch(like).stream, kGemmSplit); }));
+  DEF("split_workspace", ([](const Tensor& like) { return split_workspace(like, Launch(like).stream); }));
 }

@@ -75,6 +75,7 @@ _SIGNATURES = {
         [c_void_p, c_int32, c_void_p, c_int32, c_int32, POINTER(ck_segments), c_int32, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int32, c_void_p],
     ),
     "ck_grouped_gemm_workspace_bytes": (c_int64, []),
+    "ck_grouped_gemm_uses_workspace": (c_int32, [c_int32]),
     "ck_grouped_gemm_ws": (
         c_int32,
         [c_void_p, c_int32, c_void_p, c_int32, c_int32, POINTER(ck_segments), c_int32, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int64],

@@ -244,17 +244,19 @@ int ck_grouped_gemm(const void* a, int32_t a_gather_div, const void* w, int32_t 
                     const ck_segments* seg, int32_t epilogue, void* y, void* y_t, int64_t ld_t, void* aux,
                     const void* aux_in, int32_t dtype, void* stream);
 /* The same call with a workspace that lets the kernel split the contraction of its last, partial round of tiles. A
- * launch of t tiles runs in ceil(t / 256) rounds on the 256 CUs; when the last round is at most half full (and the
- * launch has at most 64 rounds and at least 16 K steps of 64), each of its tiles is computed by two to four workgroups (as
- * many as fill the chip), an equal share of the contraction each, which exchange fp32 partial tiles through the workspace;
- * the last to arrive adds them in a fixed order (results do not depend on arrival order) and runs the epilogue. Grouped and scatter epilogues of the
- * 256-row-tile kernel; every other case behaves like ck_grouped_gemm. No counterpart in the reference (its launches
- * are not tile-quantised the same way).
+ * launch of t tiles runs in ceil(t / 256) rounds on the 256 CUs; when the last round is at most half full, the launch has at
+ * most 64 rounds and splitting takes at least 40 K steps of 64 off the last one, each of its tiles is computed by two to four
+ * workgroups (as many as fill the chip), an equal share of the contraction each, which exchange fp32 partial tiles through
+ * the workspace; the last to arrive adds them in a fixed order (results do not depend on arrival order) and runs the
+ * epilogue. Grouped and scatter epilogues of the 256-row-tile kernel; every other case behaves like ck_grouped_gemm. No
+ * counterpart in the reference (its launches are not tile-quantised the same way).
  * workspace: ck_grouped_gemm_workspace_bytes() bytes, 16-byte aligned, no initial contents required (the arrival words at
  * its end carry a tag of the launch, so whatever an earlier or an interrupted launch left there reads as "nobody has
  * arrived", and the last to arrive clears its word, so a captured launch may be replayed). One buffer per stream: launches that may run concurrently must not share one.
- * workspace NULL or too small: never split. */
+ * workspace NULL or too small: never split. ck_grouped_gemm_uses_workspace: 0 where no launch of contraction K splits (fewer than
+ * 54 K steps), so that none is needed. */
 int64_t ck_grouped_gemm_workspace_bytes(void);
+int ck_grouped_gemm_uses_workspace(int32_t K);
 int ck_grouped_gemm_ws(const void* a, int32_t a_gather_div, const void* w, int32_t N, int32_t K,
                        const ck_segments* seg, int32_t epilogue, void* y, void* y_t, int64_t ld_t, void* aux,
                        const void* aux_in, int32_t dtype, void* stream, void* workspace, int64_t workspace_bytes);

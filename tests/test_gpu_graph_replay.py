@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import cute_kernels
-from cute_kernels import scattermoe
+from cute_kernels import _C, scattermoe
 
 pytestmark = pytest.mark.gpu
 
@@ -38,6 +38,28 @@ def test_replays_of_a_layer_with_a_split_last_round(device, tokens, hidden, inte
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, layer())
+
+
+@pytest.mark.parametrize("steps", [53, 54])
+@pytest.mark.parametrize("form", ["forward", "input gradient"])
+def test_a_graph_holds_a_workspace_only_where_a_launch_can_split(device, form, steps):
+    """53 K steps: no share of a tile's contraction is 40 steps shorter than the whole, whatever the number of tiles."""
+    E, N, K = 4, 512, 64 * steps
+    ids = torch.randint(0, E, (600,), device=device, dtype=torch.int32)
+    seg = cute_kernels.sort_by_expert(ids, E, 256)
+    a, out = (torch.zeros(seg.max_rows, n, device=device, dtype=torch.bfloat16) for n in (K, N))
+    w = torch.zeros(E, *((N, K) if form == "forward" else (K, N)), device=device, dtype=torch.bfloat16)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if form == "forward":
+            scattermoe._gemm(a, 0, w, seg, _C.CK_EPI_GROUPED, out)
+        else:
+            scattermoe._gemm_dx(a, w, seg, _C.CK_EPI_GROUPED, out)
+    taken = torch.cuda.max_memory_allocated() - before
+    assert (taken >= _C.lib().ck_grouped_gemm_workspace_bytes()) == (steps == 54)  # a capture takes a little for itself
 
 
 def test_graphs_that_count_do_not_depend_on_each_other(device):
