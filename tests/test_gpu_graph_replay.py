@@ -9,7 +9,13 @@ from cute_kernels import _C, scattermoe
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,hidden,inter", [(300, 1024, 1024), (520, 2048, 2048)])
+def _splits(seg, experts, columns, K):
+    """Whether a launch on 256-row tiles splits its last round: at most half full, and 40 K steps or more saved by its parts."""
+    tail, steps = int(seg.seg_starts[experts]) // 256 * -(-columns // 256) % 256, K // 64
+    return 0 < tail <= 128 and steps - -(-steps // min(4, 256 // tail)) >= 40
+
+
+@pytest.mark.parametrize("tokens,hidden,inter", [(300, 1024, 3456), (520, 2048, 3840)])
 def test_replays_of_a_layer_with_a_split_last_round(device, tokens, hidden, inter):
     """A layer whose c_proj GEMM is the graph's only launch that splits its last round of tiles, on a stream that runs nothing
     else: every replay finds the workspace as the replay before left it. Each one equals the eager layer bit for bit (the
@@ -26,8 +32,7 @@ def test_replays_of_a_layer_with_a_split_last_round(device, tokens, hidden, inte
 
     with torch.no_grad():
         seg = cute_kernels.sort_by_expert(ids, E, 256)
-        tail = int(seg.seg_starts[-1]) // 256 * (hidden // 256) % 256
-        assert 0 < tail <= 128 and inter // 64 >= 16  # the c_proj launch splits
+        assert _splits(seg, E, hidden, inter)  # the c_proj launch
         layer()
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
@@ -93,11 +98,11 @@ def test_graphs_that_count_do_not_depend_on_each_other(device):
 
 
 @pytest.mark.parametrize("act", ["swiglu", "gelu"])
-@pytest.mark.parametrize("tokens", [40, 700])  # tiles of 128 rows; of 256 rows with split last rounds
-def test_replays_of_a_training_step_of_the_experts(device, act, tokens):
+@pytest.mark.parametrize("tokens,inter", [(40, 1024), (700, 3456)])  # tiles of 128 rows; of 256 rows with split last rounds
+def test_replays_of_a_training_step_of_the_experts(device, act, tokens, inter):
     """Forward and backward of the expert block in one graph (the backward launches from the autograd engine's thread), replayed
     on other inputs with eager steps in between: outputs and gradients bit for bit those of an eager step."""
-    E, k, hidden, inter = 4, 2, 1024, 1024
+    E, k, hidden = 4, 2, 1024
     g = torch.Generator(device=device).manual_seed(3)
     rand = lambda *shape: torch.randn(*shape, device=device, generator=g)
     w_fc = (0.03 * rand(E, 2 * inter if act == "swiglu" else inter, hidden)).bfloat16().requires_grad_()
@@ -107,6 +112,8 @@ def test_replays_of_a_training_step_of_the_experts(device, act, tokens):
     gates = torch.rand(tokens, k, device=device, generator=g).bfloat16().requires_grad_()
     leaves = (x, gates, w_fc, w_proj)
     align = 128 if tokens < 100 else 256
+    if align == 256:  # c_proj, and d_x through c_fc's weights
+        assert _splits(cute_kernels.sort_by_expert(ids, E, align), E, hidden, inter)
 
     def step():
         seg = cute_kernels.sort_by_expert(ids, E, align)
