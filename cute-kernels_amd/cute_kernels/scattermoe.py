@@ -136,13 +136,14 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tupl
     that depends on the height. In us, with the constants fitted to measured layers:
       * a 64-deep step of a 256 x 256 tile takes 1.7 on a CU; contractions that are no multiple of 64 run on the general
         kernel, 1.6 with fewer loads in flight and no split; of a 128 x 128 tile 0.7, or 1.4 for the two that share a CU;
-      * splitting the last round of 256-row tiles costs 60 for its device-wide fences, and happens where it takes 40 steps or
+      * splitting the last round of 256-row tiles costs 75 for its device-wide fences, and happens where it takes 40 steps or
         more off that round;
       * no launch is shorter than its weights' stream, 4.2 TB/s, and the input gradient of 128-row tiles (or of such a
         contraction) transposes the weights first.
-    Over 432 calls of 8 to 64 experts, 1,024 to 4,096 wide, 1,024 to 14,336 inside, at 16 to 450 rows per expert the chosen
-    height is 0.8 % slower than the better one on average in training and 0.7 % in inference; always 256 3.5 and 25 %, always
-    128 24 and 12 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
+    Over 1,568 calls of 8 to 64 experts, 1,024 to 4,096 wide, 768 to 14,336 inside, gated and not, at 16 to 500 rows per expert
+    the chosen height is 0.5 % slower than the better one on average in training and 0.8 % in inference (0.7 and 0.8 %
+    with 60 for the fences: training steps of 8 x 2,048 x 4,096 without a gate at 192 rows 618 us for 546); always 256 1.6 and
+    13 %, always 128 22 and 13 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
     4,096 x 14,336 at 8 / 96 / 400 rows 3,217 / 3,548 / 6,801 against 2,132 / 2,416 / 3,980 us; 32 of 1,024 x 1,024 304 / 335 /
     622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. Inference: 8 of 4,096 x
     14,336 at 34 / 64 / 100 / 128 rows 606 / 630 / 686 / 1,014 against 631 / 643 / 658 / 686; 8 of 1,664 x 5,632 at 64 / 200 /
@@ -162,7 +163,7 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tupl
             elif nt_only:
                 time = 1.6 * steps * -(-tiles // 256)
             elif splits and 0 < tiles % 256 <= 128 and steps - (part := -(-steps // min(4, 256 // (tiles % 256)))) >= 40:
-                time = 1.7 * (steps * (tiles // 256) + part) + 60.0
+                time = 1.7 * (steps * (tiles // 256) + part) + 75.0
             else:
                 time = 1.7 * steps * -(-tiles // 256)
             total += max(time, stream) + (2 * stream if input_gradient and nt_only else 0.0)

@@ -84,6 +84,13 @@ def test_sixteen_bit_layers_take_the_faster_height(H, I, gated, rows, training, 
     assert scattermoe.choose_align(rows * E, E, BF16, not training, (H, I, gated)) == height
 
 
+@pytest.mark.parametrize("experts,H,I,gated,rows", [(8, 2048, 4096, False, 160), (8, 2048, 4096, False, 230), (16, 1024, 2016, True, 16),
+                                                    (16, 1024, 2016, True, 64), (8, 1024, 3840, True, 40)])
+def test_a_split_last_round_does_not_make_up_for_its_fences(experts, H, I, gated, rows):
+    """Training steps of few tiles whose long launches split their last round on 256 rows: 128 rows are 1.07 to 1.14 times faster."""
+    assert scattermoe.choose_align(rows * experts, experts, BF16, False, (H, I, gated)) == 128
+
+
 @pytest.mark.parametrize("act", ["swiglu", "gelu", "silu", "prelu"])
 @pytest.mark.parametrize("rows", [4, 40, 200, 600])
 def test_nothing_to_differentiate_is_inference(monkeypatch, act, rows):
