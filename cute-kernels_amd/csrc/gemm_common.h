@@ -256,19 +256,28 @@ __device__ inline void forward_tile(const GemmParams& prm, int pid, int total, i
 // Tile `pid` of a weight-gradient launch: `position` of its expert in the launch's order of experts, and its place in that
 // expert's m_tiles x n_tiles grid. Experts differ in contraction length, and which XCD computes a workgroup is fixed by its
 // index, so every XCD has to get its share of every length.
-// Chunks: runs of consecutive tiles (blocks of one expert's) go out over the XCDs and back; the experts are sorted by
-// length, so that turning back evens the shares out. Slices: every expert's grid is cut in 8 along its longer side, which
-// makes the shares equal, where each XCD gets 4 tiles or more of that side (4 + 8 operand panels for the 32 tiles an XCD
-// computes at a time). Smaller grids would leave an XCD one row of an expert's tiles, or every eighth tile: 36 panels for 32
-// tiles of 11 x 8 per expert.
-//   small grids: chunks of 16, 4 x 4 blocks (8 + 8 panels). 64 experts of 2,816 x 2,048 at 400 / 1,024 / 2,048 rows each: 496 /
-//     806 / 1,398 us -> 481 / 777 / 1,329, with Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393; 32 of 2,048 x 2,048 178 /
-//     282 / 498 -> 165 / 270 / 476. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at even loads and 5 to
-//     10 % slower at Zipf(0.8): too few of them to even out.
-//   large grids, 4,096 rows per expert and more: chunks of 32. All XCDs together then read 16 + 16 panels where slices read
-//     64 + 4, and the contraction is long enough for that to count. 8 experts of 28,672 x 4,096, slices / chunks at 1,024,
-//     2,048, 4,096, 8,192 rows each: 1,775 / 1,855, 3,029 / 3,079, 5,687 / 5,635, 11,342 / 10,958 us; Zipf(1.0) 1,768 / 1,821,
-//     3,080 / 3,079, 5,820 / 5,755, 11,393 / 11,066.
+// Slices: every expert's grid is cut in 8 along its longer side, which makes the shares equal.
+// Chunks: runs of consecutive tiles (blocks of one expert's) go out over the XCDs and back; the experts are sorted by length,
+// so that turning back evens the shares out, unless experts end in the middle of a round of the XCDs and have few rounds:
+// half of the XCDs then get a chunk more of the longest expert than the others.
+// Which of the two, by the slice's tiles along the longer side:
+//   none (no multiple of 8) or 1: chunks of 16, 4 x 4 blocks (8 + 8 operand panels for the 32 tiles an XCD computes at a time);
+//     slices would leave an XCD one row of an expert's tiles, or every eighth tile: 36 panels for 32 tiles of 11 x 8 per
+//     expert. 64 experts of 2,816 x 2,048 at 400 / 1,024 / 2,048 rows each: 496 / 806 / 1,398 us -> 481 / 777 / 1,329, with
+//     Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at
+//     even loads and 5 to 10 % slower at Zipf(0.8): too few of them to even out. At 8 x 6 tiles per expert (3 rounds of half
+//     the XCDs) and 6,144 rows, chunks are 4 % faster than slices at even loads and 5 to 9 % slower at Zipf(1.0).
+//   2 or 3: the same chunks where they deal the experts evenly or below 2,048 rows per expert. 64 of 4,096 x 2,048 (one whole
+//     round) 1 to 2 % faster than slices at every load from Zipf(0) to Zipf(1.2); 128 of 3,072 x 4,096 (1.5 rounds) at 1,024 rows
+//     3.5 % faster up to Zipf(1.0), at 4,096 rows with Zipf(0) / (0.8) / (1.0) / (1.2) 10,211 / 10,484 / 10,592 / 10,759 us in
+//     slices and 10,262 / 10,830 / 11,100 / 11,469 in chunks.
+//   4 or more (4 + 8 panels in slices): chunks of 32 from 4,096 rows per expert on, where they deal the experts evenly. All XCDs
+//     together then read 16 + 16 panels where slices read 64 + 4, and the contraction is long enough for that to count.
+//     8 experts of 28,672 x 4,096, slices / chunks at 1,024, 2,048, 3,072, 4,096, 6,144 rows each: 1,801 / 1,881, 3,234 / 3,300,
+//     4,655 / 4,702, 6,126 / 6,093, 9,073 / 8,990 us; Zipf(1.0) 1,847 / 1,922, 3,303 / 3,291, 4,800 / 4,724, 6,299 / 6,176, 9,160 /
+//     9,105. 64 of 8,192 x 3,072 (1.5 rounds) at 4,096 rows with the four loads 10,005 / 10,319 / 10,369 / 10,474 in slices and
+//     9,878 / 10,412 / 10,667 / 11,003 in chunks; 32 of 10,240 x 4,096 (2.5 rounds) equal within 1 %; 16 of 14,336 x 4,096 (3.5
+//     rounds) 1.5 to 3 % faster in chunks.
 template <int CHUNK, int HEIGHT>
 __device__ inline void dw_chunk_tile(int pid, int major, int minor, int num_experts, int& position, int& a, int& b) {
   const int per_expert = major * minor, total = per_expert * num_experts;
@@ -283,12 +292,15 @@ __device__ inline void dw_tile(const GemmParams& prm, int pid, int& position, in
   const bool m_major = prm.m_tiles >= prm.n_tiles;
   const int major = m_major ? prm.m_tiles : prm.n_tiles, minor = m_major ? prm.n_tiles : prm.m_tiles;
   int a, b;
-  if (major % kXcds != 0 || major / kXcds < 4) {
+  const int per_expert = major * minor, slice = major % kXcds == 0 ? major / kXcds : 0;
+  const int rows = prm.seg_starts[prm.num_experts] / prm.num_experts;  // of an expert, on average
+  const auto even = [&](int chunk) { return per_expert % (kXcds * chunk) == 0 || per_expert >= 3 * kXcds * chunk; };
+  if (slice < 2 || (slice < 4 && (rows < 2048 || even(16)))) {
     dw_chunk_tile<16, 4>(pid, major, minor, prm.num_experts, position, a, b);
-  } else if (prm.seg_starts[prm.num_experts] / prm.num_experts >= 4096) {
+  } else if (slice >= 4 && rows >= 4096 && even(32)) {
     dw_chunk_tile<32, 8>(pid, major, minor, prm.num_experts, position, a, b);
   } else {
-    const int slice = major / kXcds, per_slice = slice * minor, j = pid / kXcds;
+    const int per_slice = slice * minor, j = pid / kXcds;
     position = j / per_slice;
     grouped_order(j - position * per_slice, slice, minor, a, b);
     a += pid % kXcds * slice;

@@ -40,11 +40,12 @@ def test_forward_tiles(counts, columns):
         assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())  # |sum| <= 256: exact in bf16
 
 
-# 256 x 256 tiles along the longer side: 32 (4 per XCD: slices, or chunks of 32 from 4,096 rows per expert on), 16 and 11 (chunks
-# of 16; 8 experts: 128 and 176 tiles, whole rounds of chunks and a rest), 1; the longer side is the rows' or the columns'.
+# 256 x 256 tiles: 32 x 1 (4 per XCD, an eighth of a round of chunks: slices), 32 x 8 (one round: slices, or chunks of 32 from 4,096
+# rows per expert on), 16 x 1 (chunks of 16, or slices from 2,048 rows on), 16 x 8 (one round: chunks of 16), 11 x 2 (chunks of 16;
+# 8 experts: 176 tiles, whole rounds of chunks and a rest), 1 x 1; the longer side is the rows' or the columns'.
 # The first three lists average fewer than 512 rows: 128 x 256 tiles, in slices of 8 of them or chunks of 32, contractions of one
 # step of 32 rows, of two and more, ragged and whole; ragged tiles of both kernels.
-@pytest.mark.parametrize("M,N", [(8192, 256), (256, 4096), (2816, 512), (512, 2568), (256, 256), (328, 264)])
+@pytest.mark.parametrize("M,N", [(8192, 256), (8192, 2048), (256, 4096), (4096, 2048), (2816, 512), (512, 2568), (256, 256), (328, 264)])
 @pytest.mark.parametrize(
     "counts",
     [[70, 0, 64, 65, 1, 128, 3, 200], [33], [31, 32, 97, 511], [600, 0, 1100, 513, 512, 700, 3, 1500], [4000, 4200, 0, 8300]],
@@ -57,8 +58,9 @@ def test_weight_gradient_tiles(counts, M, N):
     dw = torch.full((len(counts), M, N), 1000.0, dtype=torch.bfloat16, device=DEV)
     scattermoe._gemm_dw_rows(a, b, seg, dw)
     for e in range(len(counts)):
-        expect = (a_rows[e].t().contiguous() @ b_rows[e]).to(torch.bfloat16)  # sums below 2^24: exact in fp32, one rounding
-        assert torch.equal(dw[e].cpu(), expect), e
+        # sums below 2^24: exact in fp32, one rounding
+        expect = (a_rows[e].to(DEV).t().contiguous() @ b_rows[e].to(DEV)).to(torch.bfloat16)
+        assert torch.equal(dw[e], expect), e
 
 
 # 6 experts, 13 row tiles x 20 / 25 / 28 column tiles: a last round of 4 / 69 / 108 tiles, in 4 / 3 / 2 parts where that takes 40 of
