@@ -1096,7 +1096,8 @@ Tensor router_rows_forward(const Tensor& x_in, const Tensor& gate_weight_in) {
 }
 struct RouterRows : torch::autograd::Function<RouterRows> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& gate_weight) {
-    ctx->save_for_backward({x, gate_weight});
+    // what a linear layer saves: a tensor that no gradient is computed from may be written to before the backward pass
+    ctx->save_for_backward({gate_weight.requires_grad() ? x : Tensor(), x.requires_grad() ? gate_weight : Tensor()});
     return router_rows_forward(x, gate_weight);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {  // as a linear layer's

@@ -118,6 +118,23 @@ def test_gradients_of_the_few_row_router_are_a_linear_layers(needs, dtype):
         assert (a.grad is None) == (b.grad is None) and (a.grad is None or torch.equal(a.grad, b.grad))
 
 
+@pytest.mark.parametrize("leaf", [0, 1])
+def test_a_leaf_that_no_gradient_is_computed_from_may_be_written_before_the_backward_pass(leaf):
+    """As a linear layer has it: the rows' gradient takes the weight only, and the weight's the rows only."""
+    x, w, _ = _inputs(33, 640, 8, torch.bfloat16)
+    u = torch.randn(33, 8, device=DEV).bfloat16()
+    grads = []
+    for f in (_C.host().router_rows, torch.nn.functional.linear):
+        tensors = [x.clone(), w.clone()]
+        tensors[leaf].requires_grad_()
+        out = f(*tensors)
+        with torch.no_grad():
+            tensors[leaf].zero_()
+        out.backward(u)
+        grads.append(tensors[leaf].grad)
+    assert torch.equal(*grads)
+
+
 def test_second_gradients_and_tangents_of_the_few_row_router():
     x, w, _ = _inputs(33, 640, 8, torch.float16)
     gate = torch.nn.Linear(640, 8, bias=False, device=DEV, dtype=torch.float16)
