@@ -126,6 +126,21 @@ def test_route_topk_softmax_matches_oracle(device, T, E, k, dtype):
     np.testing.assert_array_equal(vals.float().cpu().numpy(), logits.float().topk(k, dim=-1).values.numpy())
 
 
+# groups of 1, 2, 8, 16 and 64 lanes: as many selections as lanes (a lane writes one each), and one more (lane 0 writes them all)
+@pytest.mark.parametrize("E,k", [(8, 1), (8, 2), (16, 2), (16, 3), (64, 8), (64, 9), (128, 16), (128, 17), (512, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_route_selections_and_lanes_of_a_group(device, E, k, dtype):
+    logits = torch.randn(333, E, generator=torch.Generator().manual_seed(E + k)).to(dtype)
+    sel, gates, vals = cute_kernels.route_topk_softmax_raw(logits.to(device), k)
+    o_sel, o_gates, o_vals = io.topk_softmax(logits.float().numpy(), k)
+    np.testing.assert_array_equal(sel.cpu().numpy(), o_sel)
+    np.testing.assert_array_equal(vals.float().cpu().numpy(), o_vals)
+    np.testing.assert_allclose(gates.cpu().numpy(), o_gates, rtol=2e-6, atol=1e-7)
+    both, long = (cute_kernels.route_topk_softmax(logits.to(device), k, long_indices=wide) for wide in (False, True))
+    assert both[1].dtype == torch.int32 and long[1].dtype == torch.long and torch.equal(both[1].long(), long[1]) and torch.equal(both[1].cpu(), sel.cpu())
+    assert torch.equal(both[0].cpu(), gates.cpu().to(both[0].dtype))
+
+
 def test_route_special_values(device):
     row = torch.tensor([[1.0, 3.0, 3.0, -0.0, 0.0, 3.0, float("nan"), 2.0]])
     sel, _, _ = cute_kernels.route_topk_softmax_raw(row.to(device), 5)
