@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64 * WGM * 2) void grouped_gemm_kernel(const GemmPa
     const int live_m = prm.seg_starts[prm.num_experts] / prm.align;
     const int total = live_m * prm.n_tiles;
     if ((int)blockIdx.x >= total) return;
-    forward_tile(prm, blockIdx.x, total, mt, nt, expert);
+    forward_tile<true>(prm, blockIdx.x, total, mt, nt, expert);
     k_len = prm.K;
   }
   const int64_t m0 = (int64_t)mt * BM;

@@ -40,6 +40,23 @@ def test_forward_tiles(counts, columns):
         assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())  # |sum| <= 256: exact in bf16
 
 
+# the general kernel: fewer than two row tiles per expert (groups over all of them, one of 20 included), exactly two, and more
+@pytest.mark.parametrize("align,K", [(128, 64), (128, 40), (256, 40)])
+@pytest.mark.parametrize("tiles", [[1, 0, 1, 1], [3, 0, 1, 3], [4, 0, 2, 2], [1] * 20, [2] * 9, [0, 0, 0, 9]])
+def test_forward_tiles_of_the_general_kernel(tiles, align, K):
+    g = torch.Generator().manual_seed(1)
+    counts = [max(0, t * align - 3 * e) for e, t in enumerate(tiles)]
+    seg = _segments(counts, align)
+    a, rows = _operand(seg, K, counts, g)
+    w = torch.randint(-2, 3, (len(counts), 648, K), generator=g).to(torch.bfloat16)
+    y = torch.full((seg.max_rows, 648), 1000.0, dtype=torch.bfloat16, device=DEV)
+    scattermoe._gemm(a, 0, w.to(DEV), seg, _C.CK_EPI_GROUPED, y)
+    y = y.cpu().float()
+    for e, c in enumerate(counts):
+        first = int(seg.seg_starts[e])
+        assert torch.equal(y[first : first + c], rows[e] @ w[e].float().t())
+
+
 # 256 x 256 tiles: 32 x 1 (4 per XCD, an eighth of a round of chunks: slices), 32 x 8 (one round: slices, or chunks of 32 from 4,096
 # rows per expert on), 16 x 1 (chunks of 16, or slices from 2,048 rows on), 16 x 8 (one round: chunks of 16), 11 x 2 (chunks of 16;
 # 8 experts: 176 tiles, whole rounds of chunks and a rest), 1 x 1; the longer side is the rows' or the columns'.
