@@ -553,21 +553,22 @@ int launch_count(const char* name, const void* ids, int32_t ids_are_i64, int64_t
   // counters measured half as fast)
   const int reg_bins = num_bins <= 8 ? 8 : 0;
   // A thread starts with 4 vectors (64 bytes) and goes round only once the launch is as large as the chip takes at once:
-  // 512 blocks of 16 waves. (With 4 trips from the start and at most 512 blocks of 4 waves, int32 / int64 ids over 64 experts,
-  // now / then: 65,536 ids 4.8 / 7.8 and 6.4 / 12.7 us, 2^20 6.3 / 10.0 and 7.5 / 14.0, 2^22 7.6 / 12.6 and 10.3 / 19.4, 2^26
-  // 44.5 / 50.2 and 82.4 / 162.8; a ticket for each block on one address alone cost 4 us of a launch of 512 blocks.) Small
-  // inputs want blocks of 8 waves, whose barriers and merge are shorter (1,024 ids 2.6 us against 3.0), as long as
-  // that makes few blocks -- up to 16, or 512 where a block's merge is short (32 bins or fewer: 2^20 ids over 16 experts 5.4 us
-  // against 6.7; over 128 experts 7.6 against 7.0). What two of them would share fits one wide block, which merges nothing:
-  // 16,384 int32 ids over 64 / 2,048 / 16,384 bins 5.3 / 5.0 / 6.1 us against 6.0 / 9.1 / 21.3.
+  // 512 blocks of 16 waves. Figures are us a launch, with all three outputs, in a captured graph of 50 of them. With 4 trips from
+  // the start and at most 512 blocks of 4 waves, int32 / int64 ids over 64 experts, now / then: 65,536 ids 5.7 / 6.5 and 6.4 / 8.1,
+  // 2^20 6.8 / 9.6 and 6.7 / 11.5, 2^22 7.1 / 12.1 and 8.5 / 16.3, 2^26 45.5 / 50.0 and 80.7 / 161.8 (a wave's wait for its additions
+  // ahead of the ticket is 0.3 to 0.4 of each). Small inputs want blocks of 8 waves, whose barriers and merge are shorter (1,024
+  // ids over 64 experts 3.1 against 3.7), as long as that makes few blocks -- up to 16, or 512 where a block's merge is short
+  // (32 bins or fewer: 2^20 int32 ids over 16 experts 6.5 against 7.6; over 64 and 128 the two are within 10 % of each other up
+  // to there, over 512 11.5 against 9.8). What two of them would share fits one wide block, which merges nothing: 16,384
+  // int32 ids over 64 / 2,048 / 16,384 bins 4.5 / 4.8 / 18.5 against 5.3 / 10.2 / 49.4.
   const int64_t narrow = ceil_div(n, (int64_t)kNarrowCount * vec * 4);
   const bool wide = narrow == kWideCount / kNarrowCount || narrow > (num_bins <= 32 ? 512 : 16);
   const int threads = wide ? kWideCount : kNarrowCount;
   int64_t blocks = wide ? ceil_div(n, (int64_t)kWideCount * vec * 4) : narrow;
   blocks = blocks < 1 ? 1 : blocks > kMaxCountBlocks ? kMaxCountBlocks : blocks;
   // copies of the histogram in LDS: one a wave up to 1,024 bins, at most 32 KiB of them; beyond, waves seldom meet in a bin, and
-  // clearing and adding up copies costs more than it saves (1,024 ids over 4,096 bins 4.6 us with one, 6.1 with two; 2^20 10.8
-  // and 11.8)
+  // clearing and adding up copies costs more than it saves (1,024 ids over 4,096 bins 6.1 with one, 7.6 with two; 2^20 11.8
+  // and 12.3)
   int copies = reg_bins > 0 || num_bins > 1024 ? 1 : kMaxCountBins / 2 / num_bins;
   copies = copies > threads / kWave ? threads / kWave : copies;
   const size_t lds_bytes = ((size_t)copies * num_bins + threads / kWave + 2) * sizeof(uint32_t);

@@ -281,11 +281,12 @@ __device__ inline void forward_tile(const GemmParams& prm, int pid, int total, i
 //     expert. 64 experts of 2,816 x 2,048 at 400 / 1,024 / 2,048 rows each: 496 / 806 / 1,398 us -> 481 / 777 / 1,329, with
 //     Zipf(0.8) loads 484 / 860 / 1,462 -> 457 / 820 / 1,393. Chunks of 8 and 12 were slower, chunks of 32 (8 x 4) 1 % faster at
 //     even loads and 5 to 10 % slower at Zipf(0.8): too few of them to even out. At 8 x 6 tiles per expert (3 rounds of half
-//     the XCDs) and 6,144 rows, chunks are 4 % faster than slices at even loads and 5 to 9 % slower at Zipf(1.0).
+//     the XCDs) chunks are 4 to 5 % faster than slices at even loads, and at 600 / 1,500 rows with Zipf(0.8) 4 / 2 % faster,
+//     with Zipf(1.0) equal / 3 % slower, with Zipf(1.2) 6 % slower / 3 % faster; at 6,144 rows 5 to 9 % slower at Zipf(1.0).
 //   2 or 3: the same chunks where they deal the experts evenly or below 2,048 rows per expert. 64 of 4,096 x 2,048 (one whole
 //     round) 1 to 2 % faster than slices at every load from Zipf(0) to Zipf(1.2); 128 of 3,072 x 4,096 (1.5 rounds) at 1,024 rows
-//     3.5 % faster up to Zipf(1.0), at 4,096 rows with Zipf(0) / (0.8) / (1.0) / (1.2) 10,211 / 10,484 / 10,592 / 10,759 us in
-//     slices and 10,262 / 10,830 / 11,100 / 11,469 in chunks.
+//     3.5 % faster up to Zipf(1.0), at 1,500 rows with Zipf(0) / (0.8) / (1.0) / (1.2) 3 % faster, equal, 3 and 4 % slower, at
+//     4,096 rows 10,211 / 10,484 / 10,592 / 10,759 us in slices and 10,262 / 10,830 / 11,100 / 11,469 in chunks.
 //   4 or more (4 + 8 panels in slices): chunks of 32 from 4,096 rows per expert on, where they deal the experts evenly. All XCDs
 //     together then read 16 + 16 panels where slices read 64 + 4, and the contraction is long enough for that to count.
 //     8 experts of 28,672 x 4,096, slices / chunks at 1,024, 2,048, 3,072, 4,096, 6,144 rows each: 1,801 / 1,881, 3,234 / 3,300,

@@ -3,8 +3,8 @@
 //
 // What bounds it: a weight-gradient tile contracts over one expert's rows, a few hundred to a few thousand. On the kernel with
 // 128-byte LDS rows (grouped_gemm_line.hip: one workgroup per compute unit, all registers and 128 KiB of LDS) a 256 x 256 tile
-// of 384 rows takes 36 k cycles, of which its MFMAs are 12 k: the dependent loads of the segment tables, the first
-// operands' latency and the output stores have nothing to run under them. Here a tile is 128 x 256 and two workgroups share
+// of 400 rows takes 22 us (128 experts of 4,096 x 1,536: 48 rounds in 1,056 us), of which its MFMAs are 8: the dependent loads
+// of the segment tables, the first operands' latency and the output stores have nothing to run under them. Here a tile is 128 x 256 and two workgroups share
 // a compute unit, so that one multiplies while the other starts up or stores. Per FLOP that reads half as much again from L2
 // and LDS, which is what a long contraction is bound by.
 //
