@@ -41,7 +41,7 @@ struct GemmParams {
   int act_kind;          // kSwiglu epilogue: CK_ACT_SWIGLU (up * gate * sigmoid(gate)) or CK_ACT_GLU (up * sigmoid(gate));
                          // kGrouped epilogue with aux: CK_ACT_GELU_TANH (aux = gelu(y), second output)
   void* trace;           // measurement builds only (CK_STAMP): per-wave cycle counts, 8 x uint64 each, else NULL
-  // Split contraction for the last, partial round of tiles (128-byte-row kernel, grouped / scatter epilogues):
+  // Split contraction for the last, partial round of tiles (128-byte-row kernel, all forward epilogues):
   // split_ws = [tiles][parts][4 waves][64 blocks][64 lanes] f32x4 partial accumulators (at most kSplitMaxTail tiles in
   // kSplitParts parts or twice as many in half as many parts), followed by 2 * kSplitMaxTail 64-bit arrival words; NULL =
   // never split. split_base = the launch's grid without the extra workgroups (they are blockIdx split_base ..).
@@ -55,8 +55,10 @@ struct GemmParams {
 };
 uint64_t next_split_tag();  // grouped_gemm.hip
 constexpr int kSplitParts = 4, kSplitMaxTail = 64, kSplitMaxRounds = 64;
-// K steps that splitting has to take off the last round. A step of a 256 x 256 tile takes 1.5 to 1.7 us, and the parts'
-// device-wide fences and the exchange of their accumulators 60 to 80 us however short they are.
+// K steps that splitting has to take off the last round. A step of a 256 x 256 tile takes 1.5 to 1.7 us with all CUs at work and 1.1
+// to 1.3 with few (the chip's power is shared by fewer), and the exchange of the parts' accumulators 25 to 40 us: launches of 24 and
+// 32 steps that save 16 to 24 of them gain nothing (-5 to 0 us), of 64 that save 48 gain 14 to 16, of 128 that save 64 gain 37, of
+// 224 that save 168 gain 160.
 constexpr int kSplitMinSaved = 40;
 constexpr bool split_pays(int k_steps, int parts) { return k_steps - (k_steps + parts - 1) / parts >= kSplitMinSaved; }
 constexpr int64_t kSplitPartFloats = 4 * 64 * 64 * 4;  // one workgroup's 256 x 256 fp32 tile

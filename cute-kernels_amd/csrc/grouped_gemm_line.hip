@@ -83,7 +83,7 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
   if constexpr (CK_STAMP != 0) st_begin = clock64();
 
   // ---- which tile (XCD-aware orders: gemm_common.h)
-  constexpr bool kSplit = WGM == 2 && (MODE == kGrouped || MODE == kScatter);  // see the split below
+  constexpr bool kSplit = WGM == 2 && MODE != kDw;  // see the split below
   int mt, nt, expert;
   int64_t k_begin = 0;
   int k_len;
@@ -545,16 +545,21 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
 
   if constexpr (kSplit) {
     if (split_part >= 0) {
-      // every part leaves its accumulators in the workspace, in its own register layout (16 bytes per lane)
+      // Every part leaves its accumulators in the workspace, in its own register layout (16 bytes per lane), by stores that are
+      // performed at device scope (sc1: through the XCD's L2), and waits for them ahead of the ticket; the last part to
+      // arrive reads all of them by loads at device scope. So no fence has to write back and throw away whole L2s, with the other
+      // workgroups' operands in them: 2,000 tokens through 8 experts of 4,096 x 14,336 took 1,380 us with fences (c_proj's last 64
+      // tiles of 320 in 4 parts; c_fc not split then) and take 1,329.
       float* slot_ws = prm.split_ws + (int64_t)split_slot * split_parts * kSplitPartFloats;
-      float* mine = slot_ws + (int64_t)split_part * kSplitPartFloats + ((int64_t)wave * MI * NI * kWave + lane) * 4;
+      const char* mine = uniform_ptr(reinterpret_cast<const char*>(slot_ws + (int64_t)split_part * kSplitPartFloats) + wave * MI * NI * kWave * 16);
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) *reinterpret_cast<f32x4*>(mine + (i * NI + j) * kWave * 4) = acc[i][j];
+        for (int j = 0; j < NI; ++j)
+          asm volatile("global_store_dwordx4 %0, %1, %2 sc1" ::"v"(lane * 16), "a"(acc[i][j]), "s"(mine + (i * NI + j) * kWave * 16) : "memory");
       uint64_t* arrivals = reinterpret_cast<uint64_t*>(prm.split_ws + (int64_t)kSplitMaxTail * kSplitParts * kSplitPartFloats);
       uint32_t* flag = reinterpret_cast<uint32_t*>(lds_c);  // the stages are dead
-      __threadfence();  // the partial tile is visible device-wide before the ticket is taken
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave's own stores are performed
       __syncthreads();
       if (tid == 0) {
         // ticket = arrivals of THIS launch so far: a word left by another launch (any tag but ours) counts as zero
@@ -573,18 +578,43 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
       const bool last = *flag == (uint32_t)split_parts;
       __syncthreads();  // everyone has read the flag before the epilogue reuses LDS
       if (!last) return;
-      __threadfence();  // the other parts' tiles are read from memory, not from a stale cache line
-      const float* theirs = slot_ws + ((int64_t)wave * MI * NI * kWave + lane) * 4;
+      constexpr int kPartBytes = (int)kSplitPartFloats * 4, kDeviceScope = 16;  // sc1 of a buffer load
+      const auto parts = __builtin_amdgcn_make_buffer_rsrc(slot_ws, 0, split_parts * kPartBytes, 0x00027000);
+      auto part_of = [&](int part, int block) {
+        union {
+          u32x4_t u;
+          f32x4 f;
+        } c;
+        c.u = __builtin_amdgcn_raw_buffer_load_b128(parts, lane * 16, part * kPartBytes + (wave * MI * NI + block) * kWave * 16, kDeviceScope);
+        return c.f;
+      };
+      // a fixed order of additions whichever part arrived last; a row block's 16 to 32 loads go out together
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+      for (int i = 0; i < MI; ++i) {
+        f32x4 p[kSplitParts][NI];
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {  // a fixed order of additions whichever part arrived last
-          const float* q = theirs + (i * NI + j) * kWave * 4;
-          f32x4 sum = *reinterpret_cast<const f32x4*>(q) + *reinterpret_cast<const f32x4*>(q + kSplitPartFloats);
-          if (split_parts > 2) sum += *reinterpret_cast<const f32x4*>(q + 2 * kSplitPartFloats);
-          if (split_parts > 3) sum += *reinterpret_cast<const f32x4*>(q + 3 * kSplitPartFloats);
-          acc[i][j] = sum;
+        for (int j = 0; j < NI; ++j) p[0][j] = part_of(0, i * NI + j);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) p[1][j] = part_of(1, i * NI + j);
+        if (split_parts > 2) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j) p[2][j] = part_of(2, i * NI + j);
         }
+        if (split_parts > 3) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j) p[3][j] = part_of(3, i * NI + j);
+        }
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = p[0][j] + p[1][j];
+        if (split_parts > 2) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] += p[2][j];
+        }
+        if (split_parts > 3) {
+#pragma unroll
+          for (int j = 0; j < NI; ++j) acc[i][j] += p[3][j];
+        }
+      }
     }
   }
   if constexpr (CK_STAMP != 0) st_end = clock64();
@@ -885,7 +915,7 @@ int launch_line(const GemmParams& prm_in, int mode, int bn, bool bt, int dtype, 
                 const char* name) {
   GemmParams prm = prm_in;
   // no more is taken off a round than by the most parts: where that does not pay there are no extra workgroups either
-  if (prm.split_ws != nullptr && (mode == kGrouped || mode == kScatter) && split_pays(prm.K / kLineK, kSplitParts)) {
+  if (prm.split_ws != nullptr && mode != kDw && split_pays(prm.K / kLineK, kSplitParts)) {
     prm.split_base = (int)blocks;  // the extra workgroups of a split last round sit behind the regular grid
     prm.split_tag = next_split_tag();
     blocks += kSplitMaxTail * (kSplitParts - 1);

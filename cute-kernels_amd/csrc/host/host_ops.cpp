@@ -355,8 +355,7 @@ void gemm(const Tensor& a, int64_t gather_div, const Tensor& w, const Segments& 
   timed(epilogue_name(epilogue, false), N, K, [&] {
     const Launch l(w);
     const ck_segments cs = seg.c(rows_in, rows_out);
-    const bool splits = (epilogue == CK_EPI_GROUPED || epilogue == CK_EPI_SCATTER) && may_split(K, flags);
-    const Tensor ws = splits ? split_workspace(w, l.stream) : Tensor();
+    const Tensor ws = seg.align == 256 && may_split(K, flags) ? split_workspace(w, l.stream) : Tensor();
     check(api.ck_grouped_gemm_ws(ptr(a), (int32_t)gather_div, ptr(w), (int32_t)N, (int32_t)K, &cs, (int32_t)epilogue, ptr(y), ptr(y_t),
                                  seg.max_rows, ptr(aux), ptr(aux_in), dtype_code(w), l.stream, ptr(ws), ws.defined() ? ws.nbytes() : 0));
   });

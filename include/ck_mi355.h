@@ -248,7 +248,7 @@ int ck_grouped_gemm(const void* a, int32_t a_gather_div, const void* w, int32_t 
  * most 64 rounds and splitting takes at least 40 K steps of 64 off the last one, each of its tiles is computed by two to four
  * workgroups (as many as fill the chip), an equal share of the contraction each, which exchange fp32 partial tiles through
  * the workspace; the last to arrive adds them in a fixed order (results do not depend on arrival order) and runs the
- * epilogue. Grouped and scatter epilogues of the 256-row-tile kernel; every other case behaves like ck_grouped_gemm. No
+ * epilogue. All epilogues of the 256-row-tile kernel; every other case behaves like ck_grouped_gemm. No
  * counterpart in the reference (its launches are not tile-quantised the same way).
  * workspace: ck_grouped_gemm_workspace_bytes() bytes, 16-byte aligned, no initial contents required (the arrival words at
  * its end carry a tag of the launch, so whatever an earlier or an interrupted launch left there reads as "nobody has

@@ -112,3 +112,34 @@ def test_split_last_round(monkeypatch, weights, columns, K):
         assert 0.99 < float(same) < 1
         # 256 k of K terms ~ N(0, 1 / K): sums differ by a few 2 ** -24, one rounding step of bf16 (2 ** -8) where they straddle
         torch.testing.assert_close(outs[0].float(), outs[2].float(), rtol=2.0**-7, atol=2.0**-16)
+
+
+# 13 row tiles x 20 / 28 column tiles: a last round of 4 / 108 tiles, in 4 / 2 parts, or whole (53 steps)
+@pytest.mark.parametrize("columns,K", [(5120, 54 * 64), (7168, 80 * 64), (5120, 53 * 64)])
+@pytest.mark.parametrize("epilogue,bias", [("swiglu", False), ("gelu", True), ("gelu", False), ("scatter", True)])
+def test_split_last_round_of_the_activation_and_bias_epilogues(monkeypatch, epilogue, bias, columns, K):
+    counts = [700, 513, 600, 0, 512, 400]
+    seg = _segments(counts)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a = torch.randn(seg.max_rows, K, generator=g, device=DEV).to(torch.bfloat16)
+    gate = 2 if epilogue == "swiglu" else 1
+    w = (torch.randn((len(counts), columns, K), generator=g, device=DEV) * K**-0.5).to(torch.bfloat16)
+    bias = torch.randn(len(counts), columns, generator=g, device=DEV).to(torch.bfloat16) if bias else None
+    code = {"swiglu": _C.CK_EPI_SWIGLU, "gelu": _C.CK_EPI_GELU_TANH, "scatter": _C.CK_EPI_SCATTER}[epilogue]
+    outs = []
+    for split in (True, True, False):
+        monkeypatch.setattr(scattermoe.options, "gemm_split", split)
+        y = torch.zeros(sum(counts) if epilogue == "scatter" else seg.max_rows, columns, dtype=torch.bfloat16, device=DEV)
+        aux = None if epilogue == "scatter" else torch.zeros(seg.max_rows, columns // gate, dtype=torch.bfloat16, device=DEV)
+        scattermoe._gemm(a, 0, w, seg, code, y, aux=aux, aux_in=bias)
+        outs.append(torch.cat([t.flatten() for t in (y, aux) if t is not None]))
+    assert torch.equal(outs[0], outs[1])
+    differ = int((outs[0] != outs[2]).sum())
+    if K == 53 * 64:
+        assert differ == 0
+    else:
+        assert 0 < differ < 0.01 * outs[0].numel()
+        # sums of K terms ~ N(0, 1 / K) differ by a few 2 ** -24; a pre-activation may then round to the next bf16 value (2 ** -8
+        # of it), and so may the output. Gate: x silu'(x) / silu(x) is at most 1 + |x|, |x| < 6: 7 + 2 steps of 2 ** -8 at most.
+        # GELU: |x gelu'(x)| < 0.2 for negative x, 0.2 * 2 ** -8 in all, and at most 1.2 steps of the output for positive ones.
+        torch.testing.assert_close(outs[0].float(), outs[2].float(), rtol=2.0**-4.8, atol=2.0**-10)
