@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 from dataclasses import dataclass
 
 import torch
@@ -171,6 +172,55 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tupl
     return 256 if cost[256] < cost[128] else 128
 
 
+@functools.lru_cache(64)
+def _zipf_total(num_experts: int) -> float:
+    return sum((e + 1) ** -0.8 for e in range(num_experts))
+
+
+def _zipf_tiles(num_rows: int, num_experts: int, height: int) -> int:
+    """row tiles of experts that share the rows by Zipf(0.8), every expert with some"""
+    tiles, share = 0, num_rows / (height * _zipf_total(num_experts))
+    for e in range(num_experts):
+        rows = share * (e + 1) ** -0.8
+        if rows <= 1:
+            return tiles + num_experts - e
+        tiles += math.ceil(rows)
+    return tiles
+
+
+def _height_in_inference(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
+    """The same choice for a layer's forward alone, by a finer model: the sum of its launches at an even load and at a Zipf(0.8) one
+    together, since the more uneven the load, the fewer experts fit one tile of 128 rows. In us, fitted to measured layers:
+      * a round of 256 x 256 tiles takes 1.6 a 64-deep step with all CUs at work, down to 1.15 with few (the chip's power is
+        shared by fewer), and 8.5 for its start and stores; a split last round takes an equal part of the steps and 43 for
+        the exchange of the parts, and happens where it takes 40 steps or more off that round;
+      * a step of a 128 x 128 tile takes 0.9 alone on a CU and 1.75 for the two that share one;
+      * no launch is shorter than its weights' stream, 6.7 TB/s through 256-row tiles and 3.8 through 128-row ones.
+    Over 262 layers (8 to 64 experts, 768 to 4,096 wide, 512 to 8,900 inside, gated and not, 31 to 500 rows per expert, Zipf(0),
+    (0.8) and (1.0) loads) the chosen height is 0.4 % slower than the better one on average and 12 % at most, where the model
+    of training steps is 3.6 and 45 %, and 256 rows throughout 4.0 %. Both sides, 128 against 256 rows: 32 experts of 3,456 x
+    896 at 94 rows 227 against 170 us, 8 of 1,152 x 8,896 at 136 rows 254 against 198, 16 of 1,920 x 5,632 without a gate at
+    102 rows 203 against 230, 8 of 3,584 x 832 at 81 rows 64 against 88."""
+    cost = {128: 0.0, 256: 0.0}
+    for height in cost:
+        even = num_experts * -(-(num_rows + 24 * num_experts) // (height * num_experts))
+        for tile_rows in (even, _zipf_tiles(num_rows, num_experts, height)):
+            for columns, contraction, *_ in launches:
+                tiles, steps = tile_rows * -(-columns // height), -(-contraction // 64)
+                megabytes = num_experts * columns * contraction * 2 / 1e6
+                if height == 128:
+                    pairs, left = tiles // 512, tiles % 512
+                    time = max(steps * (1.75 * pairs + (0.0 if left == 0 else 0.9 if left <= 256 else 1.75)), megabytes / 3.8)
+                else:
+                    rounds, left = tiles // 256, tiles % 256
+                    time = steps * (1.6 * rounds + ((1.15 + 0.45 * left / 256) if left else 0.0)) + 8.5 * -(-tiles // 256)
+                    if contraction % 64 == 0 and 0 < left <= 128 and steps - (part := -(-steps // min(4, 256 // left))) >= 40:
+                        time = min(time, 1.6 * (steps * rounds + part) + 43.0)
+                    time = max(time, megabytes / 6.7)
+                cost[height] += time
+    return 256 if cost[256] < cost[128] else 128
+
+
 def _plain_tiles(num_rows: int, num_experts: int) -> int:
     return 256 if num_rows >= 512 * num_experts else 128
 
@@ -199,6 +249,8 @@ def _layer_tiles(
     launches = ((c_fc, hidden, not gated, False), (hidden, inter, True, False))
     if not inference:
         launches += ((inter, hidden, True, True), (hidden, c_fc, True, True))
+    if inference and not many and num_rows < 512 * num_experts:
+        return _height_in_inference(num_rows, num_experts, launches)
     return _large_tiles(num_rows, num_experts, dtype, launches, many)
 
 
@@ -221,7 +273,7 @@ def choose_align(
     A caller that says no more than the sizes, and every fp32 layer: 256 rows from 512 rows per expert on, else 128, which
     keeps the padding small.
     widths: (hidden, intermediate, whether the activation is the gated epilogue's) of a 16-bit layer. Below 512 rows per
-    expert its GEMMs decide (_height_of_large_tiles), those of a training step or of the forward alone.
+    expert its GEMMs decide, those of a training step (_height_of_large_tiles) or of the forward alone (_height_in_inference).
     inference (no gradient is asked for): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the
     stream of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights
     fetched once per tile, from L2 at best, so the height follows the load. Whole inference layers at 1 / 8 / 16 / 32 / 64
