@@ -61,3 +61,20 @@ def test_expert_bias_gradient(device, dtype, align, N):
         want, bound = rows.sum(0), rows.abs().sum(0) * 40 * 2.0**-24
         off = (d_bias[e].cpu().double() - want).abs()
         assert torch.all(off <= step * want.abs() + bound + 1e-7), (e, c, float(off.max()))
+
+
+# whole 16-byte pieces of rows (widths of less and more than the 128 columns of a block), and rows that have none: an odd width, and a
+# first row off its 16-byte boundary
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,offset", [(120, 0), (136, 0), (1000, 0), (12, 0), (21, 0), (136, 1)])
+def test_expert_bias_gradient_by_pieces_and_by_elements(device, dtype, N, offset):
+    seg, starts, valid = _segments(device, 128)
+    g = torch.Generator().manual_seed(N)
+    d_y = torch.randint(-8, 9, (seg.max_rows, N), generator=g).to(dtype)  # sums below 2 ** 13: exact in 32 bits
+    d_y[~valid] = float("nan")
+    on_gpu, cs = torch.empty(d_y.numel() + offset, dtype=dtype, device=device)[offset:], seg.c_struct()
+    on_gpu.copy_(d_y.flatten())
+    d_bias = torch.empty(len(COUNTS), N, dtype=dtype, device=device)
+    _C.check(_C.lib().ck_expert_bias_grad(_C.ptr(on_gpu), N, ctypes.byref(cs), _C.ptr(d_bias), _C.dtype_code(dtype), _C.stream()))
+    for e, c in enumerate(COUNTS):
+        assert torch.equal(d_bias[e].cpu(), d_y[starts[e] : starts[e] + c].double().sum(0).to(dtype)), e
