@@ -4,23 +4,31 @@
 // What bounds it: the stream of expert weights out of HBM. A decoding step reads nearly every expert's matrices for a
 // handful of rows each, 2 to 64 multiply-adds per weight, far below what the matrix cores need to matter. So the kernel is
 // built around the weight stream and nothing else:
-//  * weights go straight from memory into MFMA operand registers: no LDS stage and no barrier in the main loop. A lane's
-//    16 bytes are 8 (fp8: 16) contraction values of one output column, which is the operand layout of
-//    v_mfma_f32_16x16x32 (v_mfma_f32_16x16x128_f8f6f4: two such pieces, the same two for both operands);
+//  * weights go straight from memory into MFMA operand registers: no LDS stage and no barrier in the main loop. A load
+//    takes whole 128-byte lines, of 8 columns, and two loads become the two operands of a step by 8 moves between lanes
+//    (to_operands); v_mfma_f32_16x16x32 takes 8 contraction values a lane and operand, v_mfma_f32_16x16x128_f8f6f4 both pieces
+//    at once, 32 values. Because a line is used up by one load, the loads can be non-temporal, and memory then delivers more: bare
+//    reads of 369 to 1,611 MB in this kernel's pattern 6.6 to 7.0 TB/s, of plain loads 5.9 to 6.2 whatever the pattern. With
+//    half lines (16 columns a load) non-temporal loads fetch lines twice, 5 to 20 % slower, and so they do where a row's pitch or
+//    the first row is off a 128-byte boundary: plain loads there (non-temporal 10 to 28 % slower at 200 MB and more);
 //  * the four waves of a workgroup share the output tile and split the contraction, a quarter of every row each, in steps
 //    of one 128-byte line per row; no weight is read twice. The four partial tiles meet once, in LDS, in front of the
-//    epilogue (a fixed order of additions). Waves that take every fourth line instead, and lanes that take 16-byte pieces q
-//    and q + 4 of a line instead of 2 q and 2 q + 1, measured equal in bf16 and 2 to 8 % slower in fp8;
+//    epilogue (a fixed order of additions). Waves that take every fourth line instead measured equal in bf16 and 2 to 8 %
+//    slower in fp8;
 //  * a wave keeps the next step's loads in flight under the current step's MFMAs (two register sets); with 2 to 4
 //    workgroups per CU that is 64 to 128 KiB of weights in flight per CU (eight waves per workgroup: 0 to 10 % slower,
-//    128-column tiles: equal, non-temporal weight loads: 5 to 20 % slower);
+//    128-column tiles: equal);
+//  * the workgroups in flight read one stretch of memory, expert by expert (column tiles of all experts in turn: 2 to 6 %
+//    slower);
 //  * the activations, a few hundred KiB for the whole launch, are re-read by every column tile from L2.
 // An expert with more rows than a tile has several tiles; they are neighbours in launch order on one XCD, so that the
 // second reads the weights from that XCD's L2.
-// Measured (kernel trace; the rate is the weights' bytes by the time): 8 experts of 28,672 x 4,096 with 2 rows each 308 us =
-// 6.1 TB/s, 8 x 4,096 x 14,336 163 us = 5.8, 64 x 2,816 x 2,048 with 8 rows 130 us = 5.7 (128-row tiles of the general kernel:
-// 179), 64 x 2,048 x 1,408 69 us = 5.3, e4m3 128 x 3,072 x 4,096 with 8 rows 281 us = 5.7 and 128 x 4,096 x 1,536 157 us = 5.1
-// (256-row tiles: 348, 205). The memory reads 1.01 to 1.13 times the weights' bytes, most where the activations weigh most.
+// Measured (kernel trace, in decoding layers; the rate is the bytes of the weights with rows by the time; before: plain loads of half
+// lines, column tile by column tile): 8 experts of 28,672 x 4,096, five of them with two to six rows, 199 -> 170 us = 6.9 TB/s,
+// 4,096 x 14,336 112 -> 102 = 5.8; 64 of 2,816 x 2,048 with 8 rows each 132 -> 114 us = 6.5, 2,048 x 1,408 70 -> 57 = 6.4; e4m3, 128 of
+// 3,072 x 4,096 with 8 rows 282 -> 247 us = 6.5, 4,096 x 1,536 156 -> 146 = 5.5 (three steps a wave: start and reduction weigh
+// most there). 224 launches of 4 to 128 experts, 4 MB to 2.1 GB of weights, 0.3 to 60 rows each, even and uneven loads:
+// 26 % less time on average, none slower than by the spread of a 10 us launch; 181 with odd row pitches 17 % less.
 #include "gemm_common.h"
 
 namespace ck {
@@ -72,9 +80,23 @@ __device__ inline void multiply(const vec16 (&w)[2], const vec16 (&a)[2], f32x4&
   }
 }
 
+// The two loads of a column block (columns 0 to 7 and 8 to 15, lane l: piece l / 8 of column l % 8) as the two operands of a step:
+// lane l: pieces 2 (l / 16) and 2 (l / 16) + 1 of column l % 16. The lanes whose bit 3 is the piece's lowest bit in one order and the
+// column's highest in the other change places, 8 lanes apart within a row of 16.
+__device__ inline void to_operands(const vec16 (&lines)[2], vec16 (&w)[2]) {
+  constexpr int kRowRor8 = 0x128, kLow = 0x3, kHigh = 0xc;  // banks of 4 lanes: lanes 0 to 7 / 8 to 15 of a row
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int low = (int)lines[0].w[d], high = (int)lines[1].w[d];
+    w[0].w[d] = (uint32_t)__builtin_amdgcn_update_dpp(low, high, kRowRor8, 0xf, kHigh, false);
+    w[1].w[d] = (uint32_t)__builtin_amdgcn_update_dpp(high, low, kRowRor8, 0xf, kLow, false);
+  }
+}
+
 // TI: operand type, TO: output type; MB: row blocks of 16 per tile, NB: column blocks of 16 per tile. kSwiglu: half of the
-// column blocks are up columns, the other half the gate columns of the same outputs.
-template <typename TI, typename TO, int MODE, int MB, int NB>
+// column blocks are up columns, the other half the gate columns of the same outputs. LINES: every row of the weights starts on
+// a 128-byte boundary.
+template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
 __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
   constexpr int BM = 16 * MB, kEl = Operand<TI>::kBytes;
   constexpr int NH = MODE == kSwiglu ? NB / 2 : NB;  // column blocks of outputs per tile
@@ -84,15 +106,20 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lrow = lane & 15, lq = lane >> 4;
 
-  // ---- which tile: every XCD owns a contiguous run of column tiles, all row tiles of one column tile in a row
+  // ---- which tile: expert by expert, column tile by column tile, the row tiles of one column tile in a row; chunks of kChunk
+  // consecutive tiles go out over the XCDs, so that the chip reads one stretch of memory at a time
   const int live_m = prm.seg_starts[prm.num_experts] / BM;
   const int total = live_m * prm.n_tiles;
   int pid = blockIdx.x;
   if (pid >= total) return;
-  const int per_xcd = total / kXcds;
-  if (pid < per_xcd * kXcds) pid = (pid % kXcds) * per_xcd + pid / kXcds;
-  const int nt = pid / live_m, mt = pid - nt * live_m;
-  const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[mt]);
+  constexpr int kChunk = 32;
+  if (pid < total / (kXcds * kChunk) * (kXcds * kChunk)) {  // the last, partial round keeps its order
+    const int j = pid / kXcds;
+    pid = (j / kChunk * kXcds + pid % kXcds) * kChunk + j % kChunk;
+  }
+  const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[pid / prm.n_tiles]);
+  const int first_m = prm.seg_starts[expert] / BM, expert_m = prm.seg_starts[expert + 1] / BM - first_m;
+  const int local = pid - first_m * prm.n_tiles, nt = local / expert_m, mt = first_m + local - nt * expert_m;
   const int m0 = mt * BM;
   const int valid_end = prm.seg_starts[expert] + (int)prm.counts[expert];
 
@@ -100,20 +127,24 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   const char* w_base = static_cast<const char*>(prm.w) + (int64_t)expert * prm.w_expert_stride * kEl;
   const char* a_base = static_cast<const char*>(prm.a);
   if (prm.a_gather_div <= 0) a_base += (int64_t)m0 * prm.lda * kEl;
-  uint32_t w_off[NB], a_off[MB];
+  uint32_t w_off[NB][2], a_off[MB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     const int p = min(m0 + i * 16 + lrow, valid_end - 1);  // pad rows re-read a valid row; their results are never stored
     const int row = prm.a_gather_div > 0 ? prm.row_slot[p] / prm.a_gather_div : p - m0;
     a_off[i] = (uint32_t)row * (uint32_t)(prm.lda * kEl) + lq * 32;
   }
+  // weights: a load takes the whole lines of 8 columns, lane l 16-byte piece l / 8 of column l % 8; two loads are a column block
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    int n;
-    if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(nt * (NH * 16) + (j % NH) * 16 + lrow, prm.I - 1);
-    else n = min(nt * (NB * 16) + j * 16 + lrow, prm.N - 1);
-    w_off[j] = (uint32_t)n * (uint32_t)(prm.ldw * kEl) + lq * 32;
-  }
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 8 * h + (lane & 7);
+      int n;
+      if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(nt * (NH * 16) + (j % NH) * 16 + c, prm.I - 1);
+      else n = min(nt * (NB * 16) + j * 16 + c, prm.N - 1);
+      w_off[j][h] = (uint32_t)n * (uint32_t)(prm.ldw * kEl) + (lane >> 3) * 16;
+    }
 
   f32x4 acc[MB][NB];
 #pragma unroll
@@ -130,7 +161,7 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) s.w[j][h] = load16(wp + w_off[j] + h * 16);
+      for (int h = 0; h < 2; ++h) s.w[j][h] = LINES ? load16_nt(wp + w_off[j][h]) : load16(wp + w_off[j][h]);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -139,9 +170,12 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   };
   auto step_products = [&](const Set& s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int j = 0; j < NB; ++j) {
+      vec16 w[2];
+      to_operands(s.w[j], w);
 #pragma unroll
-      for (int j = 0; j < NB; ++j) multiply<TI>(s.w[j], s.a[i], acc[i][j]);
+      for (int i = 0; i < MB; ++i) multiply<TI>(w, s.a[i], acc[i][j]);
+    }
     __builtin_amdgcn_sched_barrier(0);
   };
 
@@ -171,9 +205,9 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
     const int left = row_bytes - full * kStepBytes;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const bool in = (2 * lq + h) * 16 < left;
+      const bool in = (2 * lq + h) * 16 < left, in_w = (lane >> 3) * 16 < left;
 #pragma unroll
-      for (int j = 0; j < NB; ++j) s0.w[j][h] = in ? load16(w_base + (int64_t)full * kStepBytes + w_off[j] + h * 16) : zero16();
+      for (int j = 0; j < NB; ++j) s0.w[j][h] = in_w ? load16(w_base + (int64_t)full * kStepBytes + w_off[j][h]) : zero16();
 #pragma unroll
       for (int i = 0; i < MB; ++i) s0.a[i][h] = in ? load16(a_base + (int64_t)full * kStepBytes + a_off[i] + h * 16) : zero16();
     }
@@ -258,7 +292,10 @@ int launch_tile(const GemmParams& prm_in, int64_t m_tiles, int out_cols, hipStre
   prm.n_tiles = (int)ceil_div(out_cols, 16 * (MODE == kSwiglu ? NB / 2 : NB));
   const int64_t blocks = m_tiles * prm.n_tiles;
   CK_REQUIRE(blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
-  hipLaunchKernelGGL((grouped_gemm_skinny_kernel<TI, TO, MODE, MB, NB>), dim3((unsigned)blocks), dim3(kNT), 0, s, prm);
+  constexpr int64_t kLine = 128;
+  const bool lines = prm.ldw * Operand<TI>::kBytes % kLine == 0 && reinterpret_cast<uintptr_t>(prm.w) % kLine == 0;
+  auto kernel = lines ? grouped_gemm_skinny_kernel<TI, TO, MODE, MB, NB, true> : grouped_gemm_skinny_kernel<TI, TO, MODE, MB, NB, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kNT), 0, s, prm);
   CK_CHECK_LAUNCH(name);
   return CK_OK;
 }

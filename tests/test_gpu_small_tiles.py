@@ -114,3 +114,28 @@ def test_inference_on_128_row_tiles_matches_a_forward_on_256(device, monkeypatch
     monkeypatch.setattr(moe_module, "choose_align", lambda *args: 256)
     want, _ = moe(x)
     torch.testing.assert_close(got.float(), want.detach().float(), rtol=RTOL, atol=ATOL)
+
+
+# weights on 128-byte boundaries throughout, with another row pitch, and with another first row; one line a row, several, and a part of
+# one. Column tiles of 64 (32 outputs with a gate) and a rest; enough tiles for whole rounds of chunks over the XCDs and a rest
+@pytest.mark.parametrize("align", [16, 32, 64])
+@pytest.mark.parametrize("K,offset", [(64, 0), (320, 0), (328, 0), (320, 8), (32, 0)])
+@pytest.mark.parametrize("columns", [8, 200, 1032])
+def test_weight_lines(device, align, K, offset, columns):
+    g = torch.Generator().manual_seed(K + columns)
+    counts = [0, 2 * align + 3, 1, 0, align, 5, 70, 0]
+    ids = torch.arange(len(counts), dtype=torch.int32).repeat_interleave(torch.tensor(counts)).to(device)
+    seg = scattermoe.sort_by_expert(ids, len(counts), align)
+    a = torch.full((seg.max_rows, K), float("nan"), dtype=torch.bfloat16)
+    rows = [torch.randint(-2, 3, (c, K), generator=g).to(torch.bfloat16) for c in counts]
+    starts = seg.seg_starts.cpu().tolist()
+    for e, c in enumerate(counts):
+        a[starts[e] : starts[e] + c] = rows[e]
+    w = torch.randint(-1, 2, (len(counts), columns, K), generator=g).to(torch.bfloat16)
+    wd = torch.empty(w.numel() + offset, dtype=torch.bfloat16, device=device)[offset:].view(w.shape).copy_(w)
+    y = torch.full((seg.max_rows, columns), 1000.0, dtype=torch.bfloat16, device=device)
+    scattermoe._gemm(a.to(device), 0, wd, seg, _C.CK_EPI_GROUPED, y)
+    y = y.cpu().float()
+    for e, c in enumerate(counts):
+        want = (rows[e].float() @ w[e].float().t()).to(torch.bfloat16).float()  # whole numbers, exact in fp32 and rounded once
+        assert torch.equal(y[starts[e] : starts[e] + c], want), e
