@@ -24,7 +24,7 @@
 // An expert with more rows than a tile has several tiles; they are neighbours in launch order on one XCD, so that the
 // second reads the weights from that XCD's L2.
 // Measured (kernel trace, in decoding layers; the rate is the bytes of the weights with rows by the time; before: plain loads of half
-// lines, column tile by column tile): 8 experts of 28,672 x 4,096, five of them with two to six rows, 199 -> 170 us = 6.9 TB/s,
+// lines, column tile by column tile): 8 experts of 28,672 x 4,096, five of them with one to seven rows, 199 -> 170 us = 6.9 TB/s,
 // 4,096 x 14,336 112 -> 102 = 5.8; 64 of 2,816 x 2,048 with 8 rows each 132 -> 114 us = 6.5, 2,048 x 1,408 70 -> 57 = 6.4; e4m3, 128 of
 // 3,072 x 4,096 with 8 rows 282 -> 247 us = 6.5, 4,096 x 1,536 156 -> 146 = 5.5 (three steps a wave: start and reduction weigh
 // most there). 224 launches of 4 to 128 experts, 4 MB to 2.1 GB of weights, 0.3 to 60 rows each, even and uneven loads:

@@ -128,7 +128,8 @@ class ExpertSegments:
         return self.max_rows
 
 
-SMALL_TILES = ((6, 16), (14, 32), (30, 64))  # (rows per expert up to which, tile height) of inference batches
+# (rows per expert up to which, tile height) of inference batches: 16-bit layers, and the quantised-expert layer, whose next height is 256
+SMALL_TILES, SMALL_TILES_E4M3 = ((6, 16), (22, 32), (30, 64)), ((6, 16), (22, 32), (40, 64))
 
 
 def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
@@ -239,7 +240,7 @@ def _layer_tiles(
     if dtype is torch.float32 or (widths is None and not inference):
         return _plain_tiles(num_rows, num_experts)
     if inference and not many:
-        for rows, align in SMALL_TILES:
+        for rows, align in SMALL_TILES if widths is not None else SMALL_TILES_E4M3:
             if num_rows <= rows * num_experts:
                 return align
     if widths is None:
@@ -276,11 +277,13 @@ def choose_align(
     expert its GEMMs decide, those of a training step (_height_of_large_tiles) or of the forward alone (_height_in_inference).
     inference (no gradient is asked for): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the
     stream of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights
-    fetched once per tile, from L2 at best, so the height follows the load. Whole inference layers at 1 / 8 / 16 / 32 / 64
-    rows per expert, tiles of 16, 32, 64, 256 rows: 128 experts of 4,096 x 1,536 in e4m3 286, 291, 299, 382 / 522, 509, 522,
-    607 / - / 872, 683, 662, 702 / 1,512, 1,032, 888, 738 us; 8 of 4,096 x 14,336 in bf16, from 8 rows on, 545, 547, 541, 673 /
-    661, 609, 596, 677 / 975, 750, 719, 681 / 1,685, 1,216, 943, 695 us. Without widths, 256 rows beyond: the e4m3 GEMMs have
-    tiles of 16, 32, 64 and 256 rows."""
+    fetched once per tile, from L2 at best, so the height follows the load. 160 bf16 layers of 8 to 128 experts at 3 to 80 rows
+    each and Zipf(0), (0.8), (1.0) loads: the height chosen is 1.6 % slower than the best of 16, 32, 64, 128 and 256 rows on
+    average (14 rows as the end of 32-row tiles: 2.2); at 14 to 20 rows tiles of 16 / 32 / 64 are 20 / 1 / 5 % off it on
+    average, at 20 to 30 44 / 6 / 1, at 30 to 40 59 / 20 / 5 (128: 9, 256: 8). The quantised-expert layer's next height is
+    256: 128 experts of 4,096 x 1,536 at 8 / 18 / 22 / 30 / 40 / 60 rows, even load, tiles of 32 398 / 444 / 470 / 610 / 873 /
+    1,008 us, of 64 438 / 486 / 502 / 543 / 588 / 787, of 256 584 / 584 / 590 / 592 / 603 / 622; with Zipf(0.8) loads at 22 / 30 / 40 rows
+    555 / 633 / 760, 540 / 608 / 670 and 588 / 653 / 675."""
     return _height(_layer_tiles, _layer_tiles_kept, num_rows, num_experts, dtype, inference, widths)
 
 

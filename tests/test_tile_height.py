@@ -170,3 +170,10 @@ def test_graphs_saved_without_a_height_still_call():
 def test_inference_layers_at_uneven_loads(experts, H, I, gated, rows, height):
     """Heights measured at Zipf(0) to Zipf(1.0) loads: the other one is 5 to 35 % slower."""
     assert scattermoe.choose_align(rows * experts, experts, BF16, True, (H, I, gated)) == height
+
+
+@pytest.mark.parametrize("rows,layer,quantised", [(6, 16, 16), (7, 32, 32), (22, 32, 32), (23, 64, 64), (30, 64, 64), (31, 128, 64), (40, 128, 64), (41, 128, 256)])
+def test_few_rows_per_expert(rows, layer, quantised):
+    """The lines between the small tiles; 8 experts of 1,024 x 1,024 take 128 rows behind them."""
+    assert scattermoe.choose_align(rows * E, E, BF16, True, (1024, 1024, True)) == layer
+    assert scattermoe.choose_align(rows * E, E, BF16, True) == quantised
