@@ -303,3 +303,27 @@ def test_softmax_router_logits_shape_and_sharp_rows(device):
     (cute_kernels.softmax_cute(a, 0.5) * w.to(device)).sum().backward()
     (mo.softmax_torch(c, 0.5) * w).sum().backward()
     torch.testing.assert_close(a.grad.cpu(), c.grad, rtol=1e-4, atol=1e-6)
+
+
+# rows of one piece less than a wave's lanes (the kernel by pieces), of as many, one more, and more than a wave's four loads at a time
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pieces", [63, 64, 65, 256, 264])
+@pytest.mark.parametrize("align", [64, 256])
+def test_group_rows_by_waves(device, dtype, pieces, align):
+    g = torch.Generator().manual_seed(pieces)
+    H = pieces * 8 if dtype == torch.bfloat16 else (pieces + pieces % 2) * 4  # whole 16-bit pieces in either type
+    counts, k = [align, 0, 1, align + 1, 0], 3
+    R = sum(counts)
+    ids = torch.arange(len(counts), dtype=torch.int32).repeat_interleave(torch.tensor(counts))[torch.randperm(R, generator=g)]
+    seg = cute_kernels.sort_by_expert(ids.to(device), len(counts), align)
+    src, coeff = torch.randn(-(-R // k), H, generator=g).to(dtype), torch.rand(R, generator=g).to(dtype)
+    slots, starts = seg.row_slot.cpu(), seg.seg_starts.cpu().tolist()
+    for c in (coeff, None):
+        got, _ = scattermoe._group_rows(src.to(device), None if c is None else c.to(device), k, seg, True, False)
+        want = torch.zeros(starts[-1], H, dtype=dtype)
+        for e, n in enumerate(counts):
+            s = slots[starts[e] : starts[e] + n].long()
+            want[starts[e] : starts[e] + n] = src[s // k] if c is None else (src[s // k].float() * c[s, None].float()).to(dtype)
+        assert torch.equal(got.cpu()[: starts[-1]], want)
+    same, _ = scattermoe._group_rows(got, None, 0, seg, True, False)
+    assert torch.equal(same.cpu()[: starts[-1]], want)
