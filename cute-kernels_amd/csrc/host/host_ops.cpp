@@ -186,7 +186,17 @@ std::tuple<Tensor, OptTensor, OptTensor> count(const Tensor& ids_in, int64_t siz
   return {counts, to_opt(ends), to_opt(starts)};
 }
 
+// `words` 32-bit words of `base` from word `offset` on, as a tensor of its own: no view of base, the way an allocation would be,
+// at a quarter of its cost
+Tensor words_of(const Tensor& base, int64_t offset, int64_t words, at::ScalarType t) {
+  Tensor part = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(base.storage()), base.key_set(), c10::scalarTypeToTypeMeta(t));
+  part.unsafeGetTensorImpl()->set_storage_offset(base.storage_offset() + offset);
+  part.unsafeGetTensorImpl()->set_sizes_contiguous({words});
+  return part;
+}
+
 // (sorted_expert_idxs, sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert, max_rows)
+// The tables live and die together: one allocation for the eight, each on a 256-byte boundary.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> sort_by_expert(const Tensor& ids_in,
                                                                                                 int64_t E, int64_t align) {
   require_gpu(ids_in);
@@ -194,10 +204,18 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64
   const Launch l(ids);
   const int64_t R = ids.numel();
   const int64_t max_rows = api.ck_sort_max_rows(R, (int32_t)E, (int32_t)align);
-  const auto i32 = [&](int64_t n) { return new_empty({n}, ids, at::kInt); };
-  const auto u32 = [&](int64_t n) { return new_empty({n}, ids, at::kUInt32); };
-  const Tensor se = i32(R), ss = i32(R), counts = u32(E), ends = u32(E), starts = u32(E), seg_starts = i32(E + 1);
-  const Tensor row_slot = i32(std::max<int64_t>(max_rows, 1)), tile_expert = i32(std::max<int64_t>(max_rows / align, 1));
+  const int64_t slots = std::max<int64_t>(max_rows, 1), tiles = std::max<int64_t>(max_rows / align, 1);
+  const auto room = [](int64_t n) { return (n + 63) / 64 * 64; };
+  const Tensor tables = new_empty({2 * room(R) + 3 * room(E) + room(E + 1) + room(slots) + room(tiles)}, ids, at::kInt);
+  int64_t used = 0;
+  const auto next = [&](int64_t n, at::ScalarType t) {
+    const Tensor part = words_of(tables, used, n, t);
+    used += room(n);
+    return part;
+  };
+  const Tensor se = next(R, at::kInt), ss = next(R, at::kInt), counts = next(E, at::kUInt32), ends = next(E, at::kUInt32);
+  const Tensor starts = next(E, at::kUInt32), seg_starts = next(E + 1, at::kInt), row_slot = next(slots, at::kInt);
+  const Tensor tile_expert = next(tiles, at::kInt);
   const Tensor ws = workspace(kSortWs, ids, l.stream, api.ck_sort_workspace_words(R, (int32_t)E));
   check(api.ck_sort_by_expert(ptr(ids), ids.scalar_type() == at::kLong, R, (int32_t)E, (int32_t)align, (int32_t*)ptr(se),
                               (int32_t*)ptr(ss), (uint32_t*)ptr(counts), (uint32_t*)ptr(ends), (uint32_t*)ptr(starts),
