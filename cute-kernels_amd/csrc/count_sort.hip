@@ -438,7 +438,144 @@ __global__ __launch_bounds__(WAVES * kWave) void sort_scatter_kernel(
   }
 }
 
-// The whole sort in one block and one launch, for the few ids of a decoding step or a small batch. What bounds it: latency.
+// Exclusive scan over the bins as a wave holds them: lane l bins l, 64 + l, ..
+template <int NB>
+__device__ inline void bins_exclusive_scan(const uint32_t (&v)[NB], uint32_t (&before)[NB], int lane) {
+  uint32_t total = 0;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    uint32_t incl = v[b];
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t u = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += u;
+    }
+    before[b] = total + incl - v[b];
+    total += __shfl(incl, kWave - 1, kWave);
+  }
+}
+
+// The sort over up to 64 NB experts: the whole of it in one block (SMALL: the ids fit its registers) or the second of two launches.
+// What bounds it is latency, and most of that was the block's barriers: three block-wide scans of two or three barriers each
+// beside four more. With a bin (or two) per lane every wave scans all bins in its own registers, and sums over the waves as it
+// reads them: one barrier, behind which no wave waits for another. 50 sorts in a replayed graph, the kernels for any number of
+// experts -> these: 16 ids over 64 experts 4.6 -> 3.3 us, 512 over 64 4.75 -> 3.45, 1,024 over 128 5.4 -> 4.7, 4,096 over 64 8.9 -> 7.0, in
+// two launches 8,192 over 64 9.3 -> 7.05, 32,768 over 64 9.9 -> 7.6, over 128 10.9 -> 9.15, 65,536 over 64 10.6 -> 7.7, 524,288 over
+// 128 18.3 -> 16.9, 2,000,003 over 60 34.5 -> 30.4.
+constexpr int kLaneWaves = 16, kLaneBins = 2 * kWave;
+template <typename id_t, int NB, bool SMALL>
+__global__ __launch_bounds__(kLaneWaves * kWave) void sort_lanes_kernel(
+    const id_t* __restrict__ ids, int64_t R, int E, int64_t seg_len, int id_bits, int align, int64_t max_tiles,
+    const uint32_t* __restrict__ table, int32_t* __restrict__ sorted_expert_idxs, int32_t* __restrict__ sorted_scattered_idxs,
+    uint32_t* __restrict__ counts, uint32_t* __restrict__ ends, uint32_t* __restrict__ starts, int32_t* __restrict__ seg_starts,
+    int32_t* __restrict__ row_slot, int32_t* __restrict__ tile_expert) {
+  constexpr int W = kLaneWaves, BINS = NB * kWave;
+  __shared__ uint32_t hist[W][BINS];                                 // a wave's own ids by bin
+  __shared__ uint32_t all[SMALL ? 1 : W][BINS], before[SMALL ? 1 : W][BINS];  // a wave's share of the table: of all blocks, of those ahead
+  __shared__ uint32_t next[W][BINS], padded[W][BINS + 1];            // a wave's own: the bins' next places; their padded starts
+  const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave, me = blockIdx.x;
+  const int64_t per_wave = seg_len / W, begin = (int64_t)me * seg_len + wave * per_wave, end = min(R, begin + per_wave);
+  constexpr int kRound = kSortPer * kWave;
+  int id[kSortPer];
+  auto fetch = [&](int64_t base) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kSortPer; ++u) {
+      const int64_t i = base + u * kWave + lane;
+      id[u] = u * kWave < per_wave && i < end ? load_id(ids + i) : -1;
+    }
+  };
+  fetch(begin);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) hist[wave][b * kWave + lane] = 0;
+  if constexpr (!SMALL) {
+    uint32_t a[NB] = {}, n_before[NB] = {};
+#pragma unroll 4
+    for (int s = wave; s < (int)gridDim.x; s += W)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const uint32_t n = b * kWave + lane < E ? table[(int64_t)s * E + b * kWave + lane] : 0;
+        a[b] += n;
+        if (s < me) n_before[b] += n;
+      }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      all[wave][b * kWave + lane] = a[b];
+      before[wave][b * kWave + lane] = n_before[b];
+    }
+  }
+  for (int64_t base = begin; base < end; base += kRound) {
+    if (base > begin) fetch(base);
+#pragma unroll
+    for (int u = 0; u < kSortPer; ++u)
+      if ((unsigned)id[u] < (unsigned)E) atomicAdd(&hist[wave][id[u]], 1u);
+  }
+  __syncthreads();
+
+  // ---- every wave for itself: the bins' counts, starts and padded starts, and how many ids of a bin lie ahead of its own
+  uint32_t count[NB] = {}, ahead[NB] = {}, start[NB], size[NB], pad[NB];
+#pragma unroll
+  for (int w = 0; w < W; ++w)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const uint32_t mine = hist[w][b * kWave + lane];
+      if constexpr (SMALL) {
+        count[b] += mine;
+      } else {
+        count[b] += all[w][b * kWave + lane];
+        ahead[b] += before[w][b * kWave + lane];
+      }
+      if (w < wave) ahead[b] += mine;
+    }
+  bins_exclusive_scan<NB>(count, start, lane);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) size[b] = (count[b] + (uint32_t)align - 1) / (uint32_t)align * (uint32_t)align;
+  bins_exclusive_scan<NB>(size, pad, lane);
+  uint32_t padded_total = __shfl(pad[NB - 1] + size[NB - 1], kWave - 1, kWave);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int e = b * kWave + lane;
+    next[wave][e] = start[b] + ahead[b];
+    padded[wave][e] = pad[b];
+    if (me == 0 && wave == 0 && e < E) {
+      counts[e] = count[b];
+      starts[e] = start[b];
+      ends[e] = start[b] + count[b];
+      seg_starts[e] = (int32_t)pad[b];
+      if (e == E - 1) seg_starts[E] = (int32_t)padded_total;
+    }
+  }
+  __builtin_amdgcn_wave_barrier();  // the wave's own LDS words, in order
+  write_tile_experts(padded[wave], E, padded_total, align, max_tiles, tile_expert, (int64_t)me * W * kWave + t, (int64_t)gridDim.x * W * kWave);
+  const uint64_t lanes_below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
+  const bool again = per_wave > kRound;  // more than the registers hold: read once more, out of L2
+  for (int64_t base = begin; base < end; base += kRound) {
+    if (again) fetch(base);
+#pragma unroll
+    for (int u = 0; u < kSortPer; ++u) {
+      if (u * kWave >= per_wave || base + u * kWave >= end) break;
+      const bool valid = (unsigned)id[u] < (unsigned)E;
+      const uint64_t peers = lanes_with_same_id(id[u], valid, id_bits);
+      const int bin = valid ? id[u] : 0;
+      uint32_t shift = 0;  // padded start less start of the id's bin
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const uint32_t v = __shfl(pad[b] - start[b], bin & (kWave - 1), kWave);
+        if (bin / kWave == b) shift = v;
+      }
+      if (valid) {
+        uint32_t* mine = &next[wave][bin];  // this wave's word alone; its LDS operations keep their order
+        const uint32_t pos = *mine + (uint32_t)__popcll(peers & lanes_below);
+        if ((peers >> lane) == 1ull) *mine = pos + 1;  // the highest lane of the group advances the bin
+        const int32_t i = (int32_t)(base + u * kWave + lane);
+        sorted_expert_idxs[pos] = bin;
+        sorted_scattered_idxs[pos] = i;
+        row_slot[pos + shift] = i;
+      }
+    }
+  }
+}
+
+// The whole sort in one block and one launch, for few ids over more than kLaneBins experts. What bounds it: latency.
 // An id is read once and stays in registers, and the table in LDS; the second launch and the way of the table through memory
 // go. Measured, 50 sorts in a replayed graph, one launch against two: 16 / 512 / 4,096 ids over 64 experts 4.5 / 4.7 / 8.9
 // against 7.6 / 7.7 / 9.0 us, over 512 experts 7.6 / 8.0 / 13.0 against 9.5 / 9.9 / 11.3. The line lies where the two meet for
@@ -773,6 +910,23 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
   const int64_t max_tiles = ck_sort_max_rows(R, E, align) / align;
   int id_bits = 0;
   while ((1 << id_bits) < E) ++id_bits;
+#define CK_LAUNCH_LANES(ID_T, NB, SMALL, BLOCKS, SEG_LEN, TABLE)                                                              \
+  hipLaunchKernelGGL((sort_lanes_kernel<ID_T, NB, SMALL>), dim3(BLOCKS), dim3(kLaneWaves * kWave), 0, static_cast<hipStream_t>(stream), \
+                     static_cast<const ID_T*>(expert_ids), R, (int)E, (int64_t)(SEG_LEN), id_bits, (int)align, max_tiles, TABLE,         \
+                     sorted_expert_idxs, sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert)
+#define CK_LAUNCH_LANES_OF(ID_T, SMALL, BLOCKS, SEG_LEN, TABLE)                        \
+  do {                                                                                 \
+    if (E <= kWave) CK_LAUNCH_LANES(ID_T, 1, SMALL, BLOCKS, SEG_LEN, TABLE);           \
+    else CK_LAUNCH_LANES(ID_T, 2, SMALL, BLOCKS, SEG_LEN, TABLE);                      \
+  } while (0)
+  if (R <= kSmallIds && E <= kLaneBins) {
+    const int64_t seg_len = round_up(R > 0 ? R : 1, (int64_t)kLaneWaves * kWave);
+    const uint32_t* none = nullptr;
+    if (ids_are_i64) CK_LAUNCH_LANES_OF(int64_t, true, 1, seg_len, none);
+    else CK_LAUNCH_LANES_OF(int32_t, true, 1, seg_len, none);
+    CK_CHECK_LAUNCH("ck_sort_by_expert");
+    return CK_OK;
+  }
   if (R <= kSmallIds && E <= kSmallBins) {
     const size_t lds = ((size_t)E * (kSmallWaves + 2) + 1 + kSmallWaves) * sizeof(uint32_t);
 #define CK_LAUNCH_SMALL(ID_T)                                                                                                \
@@ -794,6 +948,10 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
     const size_t hist_words = (size_t)WAVES * E, words = (size_t)(WAVES + 4) * E + 1 + WAVES;                                  \
     hipLaunchKernelGGL((sort_hist_kernel<ID_T, WAVES>), dim3(p.blocks), dim3(WAVES * kWave), hist_words * sizeof(uint32_t), s, \
                        ids, R, (int)E, p.seg_len, table);                                                                      \
+    if (E <= kLaneBins) {                                                                                                      \
+      CK_LAUNCH_LANES_OF(ID_T, false, p.blocks, p.seg_len, table);                                                             \
+      break;                                                                                                                   \
+    }                                                                                                                          \
     hipLaunchKernelGGL((sort_scatter_kernel<ID_T, WAVES>), dim3(p.blocks), dim3(WAVES * kWave), words * sizeof(uint32_t), s,   \
                        ids, R, (int)E, p.seg_len, id_bits, (int)align, max_tiles, table, sorted_expert_idxs,                   \
                        sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert);                        \
@@ -806,6 +964,8 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
     else CK_LAUNCH_SORT(int32_t, kNarrowWaves);
   }
 #undef CK_LAUNCH_SORT
+#undef CK_LAUNCH_LANES_OF
+#undef CK_LAUNCH_LANES
   CK_CHECK_LAUNCH("ck_sort_by_expert");
   return CK_OK;
 }

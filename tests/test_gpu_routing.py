@@ -332,3 +332,28 @@ def test_sort_over_many_blocks(device, R, E, dtype):
     """Two launches: a ragged last block and one with no ids left, both widths of block (to 512 bins and beyond), bins that do
     not divide the block, the most blocks that the table of counts allows, and segments longer than the registers hold."""
     test_sort_of_few_ids_in_one_block(device, R, E, 128, dtype)
+
+
+# a bin per lane, two, and the kernels for any number; one block and several; counts of no, one and several rounds of 256 ids a wave
+@pytest.mark.parametrize("E", [63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("R", [1, 4095, 4096, 4097, 70000, 600001])
+def test_sort_by_bins_per_lane(device, R, E):
+    g = torch.Generator().manual_seed(R + E)
+    ids = torch.randint(-1, E + 1, (R,), generator=g, dtype=torch.int32)  # ids outside [0, E) are dropped
+    ids[ids == 5] = 6
+    seg = cute_kernels.sort_by_expert(ids.to(device), E, 64)
+    kept = torch.nonzero((ids >= 0) & (ids < E)).flatten()
+    order = kept[torch.sort(ids[kept], stable=True)[1]]
+    counts = torch.bincount(ids[kept].long(), minlength=E)
+    n = kept.numel()
+    assert torch.equal(seg.counts.cpu().long(), counts) and torch.equal(seg.ends.cpu().long(), counts.cumsum(0))
+    assert torch.equal(seg.sorted_scattered_idxs.cpu()[:n].long(), order)
+    assert torch.equal(seg.sorted_expert_idxs.cpu()[:n], ids[order])
+    padded = (counts + 63) // 64 * 64
+    starts = torch.cat((torch.zeros(1, dtype=torch.long), padded.cumsum(0)))
+    assert torch.equal(seg.seg_starts.cpu().long(), starts)
+    rows = torch.arange(n) - (counts.cumsum(0) - counts)[ids[order].long()] + starts[ids[order].long()]
+    assert torch.equal(seg.row_slot.cpu().long()[rows], order)
+    tiles = torch.repeat_interleave(torch.arange(E), padded // 64)
+    owners = seg.tile_expert.cpu().long()
+    assert torch.equal(owners[: tiles.numel()], tiles) and bool((owners[tiles.numel() :] == -1).all())
