@@ -196,9 +196,10 @@ Tensor words_of(const Tensor& base, int64_t offset, int64_t words, at::ScalarTyp
 }
 
 // (sorted_expert_idxs, sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert, max_rows)
-// The tables live and die together: one allocation for the eight, each on a 256-byte boundary.
+// The tables live and die together: one allocation for the eight, each on a 256-byte boundary. apart: eight, for a registered
+// operator, whose outputs may not share storage.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> sort_by_expert(const Tensor& ids_in,
-                                                                                                int64_t E, int64_t align) {
+                                                                                                int64_t E, int64_t align, bool apart) {
   require_gpu(ids_in);
   const Tensor ids = ids_in.contiguous();
   const Launch l(ids);
@@ -206,9 +207,11 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64
   const int64_t max_rows = api.ck_sort_max_rows(R, (int32_t)E, (int32_t)align);
   const int64_t slots = std::max<int64_t>(max_rows, 1), tiles = std::max<int64_t>(max_rows / align, 1);
   const auto room = [](int64_t n) { return (n + 63) / 64 * 64; };
-  const Tensor tables = new_empty({2 * room(R) + 3 * room(E) + room(E + 1) + room(slots) + room(tiles)}, ids, at::kInt);
+  Tensor tables;
+  if (!apart) tables = new_empty({2 * room(R) + 3 * room(E) + room(E + 1) + room(slots) + room(tiles)}, ids, at::kInt);
   int64_t used = 0;
   const auto next = [&](int64_t n, at::ScalarType t) {
+    if (apart) return new_empty({n}, ids, t);
     const Tensor part = words_of(tables, used, n, t);
     used += room(n);
     return part;

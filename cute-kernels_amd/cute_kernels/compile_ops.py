@@ -318,7 +318,7 @@ _SEG_FIELDS = ("sorted_expert_idxs", "sorted_scattered_idxs", "counts", "ends", 
 
 @custom_op(f"{NS}::sort_by_expert", mutates_args=())
 def sort_by_expert(expert_ids: Tensor, num_experts: int, align: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
-    seg = _moe._sort_by_expert_eager(expert_ids, num_experts, align)
+    seg = _moe._sort_by_expert_eager(expert_ids, num_experts, align, apart=True)  # outputs of an operator share no storage
     return tuple(getattr(seg, f) for f in _SEG_FIELDS)
 
 

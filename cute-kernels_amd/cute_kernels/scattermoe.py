@@ -312,8 +312,8 @@ def sort_by_expert(
     return seg
 
 
-def _sort_by_expert_eager(expert_ids: torch.Tensor, num_experts: int, align: int) -> ExpertSegments:
-    *tables, max_rows = _C.host().sort_by_expert(expert_ids, num_experts, align)
+def _sort_by_expert_eager(expert_ids: torch.Tensor, num_experts: int, align: int, apart: bool = False) -> ExpertSegments:
+    *tables, max_rows = _C.host().sort_by_expert(expert_ids, num_experts, align, apart)
     return ExpertSegments(*tables, max_rows, num_experts, align)
 
 
