@@ -23,12 +23,14 @@
 //  * the activations, a few hundred KiB for the whole launch, are re-read by every column tile from L2.
 // An expert with more rows than a tile has several tiles; they are neighbours in launch order on one XCD, so that the
 // second reads the weights from that XCD's L2.
-// Measured (kernel trace, in decoding layers; the rate is the bytes of the weights with rows by the time; before: plain loads of half
-// lines, column tile by column tile): 8 experts of 28,672 x 4,096, five of them with one to seven rows, 199 -> 170 us = 6.9 TB/s,
-// 4,096 x 14,336 112 -> 102 = 5.8; 64 of 2,816 x 2,048 with 8 rows each 132 -> 114 us = 6.5, 2,048 x 1,408 70 -> 57 = 6.4; e4m3, 128 of
-// 3,072 x 4,096 with 8 rows 282 -> 247 us = 6.5, 4,096 x 1,536 156 -> 146 = 5.5 (three steps a wave: start and reduction weigh
-// most there). 224 launches of 4 to 128 experts, 4 MB to 2.1 GB of weights, 0.3 to 60 rows each, even and uneven loads:
-// 26 % less time on average, none slower than by the spread of a 10 us launch; 181 with odd row pitches 17 % less.
+// Measured (kernel trace, all experts with as many rows; the rate is the weights' bytes by the time; before: plain loads of half lines,
+// column tile by column tile): 8 experts of 28,672 x 4,096 with 2 rows each 308 -> 271 us = 6.9 TB/s, 4,096 x 14,336 163 -> 152 = 6.2,
+// 64 of 2,816 x 2,048 with 8 rows 130 -> 116 = 6.4, 2,048 x 1,408 69 -> 58.5 = 6.3, e4m3, 128 of 3,072 x 4,096 with 8 rows 281 -> 237 =
+// 6.8, 4,096 x 1,536 157 -> 141 = 5.7 (three steps a wave: start and reduction weigh most there; several column tiles a workgroup, the
+// next one's first loads ahead of the reduction, take registers that a third workgroup has now: 2 % faster there with two, slower
+// with more and elsewhere). The memory reads 1.000 to 1.007 times the weights' bytes (1.01 to 1.13 before). 224 launches of 4 to 128
+// experts, 4 MB to 2.1 GB of weights, 0.3 to 60 rows each, even and uneven loads: 26 % less time on average, none slower than by the
+// spread of a 10 us launch; 181 with odd row pitches 17 % less.
 #include "gemm_common.h"
 
 namespace ck {

@@ -133,24 +133,22 @@ SMALL_TILES, SMALL_TILES_E4M3 = ((6, 16), (22, 32), (30, 64)), ((6, 16), (22, 32
 
 
 def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
-    """256 or 128 rows for 16-bit layers below 512 rows per expert, whichever makes the sum of the layer's launches shorter.
+    """256 or 128 rows for 16-bit training steps and single linears below 512 rows per expert, by the shorter sum of launches.
     launches: (columns, contraction, whether the epilogue may split its last round, input gradient) of every grouped GEMM
     that depends on the height. In us, with the constants fitted to measured layers:
       * a 64-deep step of a 256 x 256 tile takes 1.7 on a CU; contractions that are no multiple of 64 run on the general
         kernel, 1.6 with fewer loads in flight and no split; of a 128 x 128 tile 0.7, or 1.4 for the two that share a CU;
-      * splitting the last round of 256-row tiles costs 75 for its device-wide fences, and happens where it takes 40 steps or
-        more off that round;
+      * splitting the last round of 256-row tiles costs 75, and happens where it takes 40 steps or more off that round (fitted
+        while the parts met through device-wide fences, and kept for training steps: the exchange takes 25 to 40 now, but with
+        60 already training steps of 8 x 2,048 x 4,096 without a gate at 192 rows got the slower height, 618 us for 546);
       * no launch is shorter than its weights' stream, 4.2 TB/s, and the input gradient of 128-row tiles (or of such a
         contraction) transposes the weights first.
     Over 1,568 calls of 8 to 64 experts, 1,024 to 4,096 wide, 768 to 14,336 inside, gated and not, at 16 to 500 rows per expert
-    the chosen height is 0.5 % slower than the better one on average in training and 0.8 % in inference (0.7 and 0.8 %
-    with 60 for the fences: training steps of 8 x 2,048 x 4,096 without a gate at 192 rows 618 us for 546); always 256 1.6 and
-    13 %, always 128 22 and 13 %. (+ 24 rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
+    the chosen height is 0.5 % slower than the better one on average in training; always 256 1.6 %, always 128 22 %. (+ 24
+    rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
     4,096 x 14,336 at 8 / 96 / 400 rows 3,217 / 3,548 / 6,801 against 2,132 / 2,416 / 3,980 us; 32 of 1,024 x 1,024 304 / 335 /
-    622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. Inference: 8 of 4,096 x
-    14,336 at 34 / 64 / 100 / 128 rows 606 / 630 / 686 / 1,014 against 631 / 643 / 658 / 686; 8 of 1,664 x 5,632 at 64 / 200 /
-    300 rows 154 / 214 / 301 against 243 / 265 / 279; 16 of 1,536 x 4,096 without a gate at 64 / 300 rows 121 / 264 against
-    193 / 188."""
+    622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. The gated
+    epilogue splits its last round as well; the fit counts it whole, as it was when the layers were measured."""
     cost = {}
     for height in (128, 256):
         tile_rows = num_experts * -(-(num_rows + 24 * num_experts) // (height * num_experts))
