@@ -196,8 +196,9 @@ Tensor words_of(const Tensor& base, int64_t offset, int64_t words, at::ScalarTyp
 }
 
 // (sorted_expert_idxs, sorted_scattered_idxs, counts, ends, starts, seg_starts, row_slot, tile_expert, max_rows)
-// The tables live and die together: one allocation for the eight, each on a 256-byte boundary. apart: eight, for a registered
-// operator, whose outputs may not share storage.
+// The tables live and die together: one allocation for those of a word per routed row and one for those of a word per expert, which
+// a caller may keep of every step; each table on a 256-byte boundary. apart: eight, for a registered operator, whose outputs may
+// not share storage.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64_t> sort_by_expert(const Tensor& ids_in,
                                                                                                 int64_t E, int64_t align, bool apart) {
   require_gpu(ids_in);
@@ -207,18 +208,24 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, int64
   const int64_t max_rows = api.ck_sort_max_rows(R, (int32_t)E, (int32_t)align);
   const int64_t slots = std::max<int64_t>(max_rows, 1), tiles = std::max<int64_t>(max_rows / align, 1);
   const auto room = [](int64_t n) { return (n + 63) / 64 * 64; };
-  Tensor tables;
-  if (!apart) tables = new_empty({2 * room(R) + 3 * room(E) + room(E + 1) + room(slots) + room(tiles)}, ids, at::kInt);
-  int64_t used = 0;
-  const auto next = [&](int64_t n, at::ScalarType t) {
+  struct Tables {
+    Tensor all;
+    int64_t used = 0;
+  } of_rows, of_experts;
+  if (!apart) {
+    of_rows.all = new_empty({2 * room(R) + room(slots) + room(tiles)}, ids, at::kInt);
+    of_experts.all = new_empty({3 * room(E) + room(E + 1)}, ids, at::kInt);
+  }
+  const auto next = [&](Tables& from, int64_t n, at::ScalarType t) {
     if (apart) return new_empty({n}, ids, t);
-    const Tensor part = words_of(tables, used, n, t);
-    used += room(n);
+    const Tensor part = words_of(from.all, from.used, n, t);
+    from.used += room(n);
     return part;
   };
-  const Tensor se = next(R, at::kInt), ss = next(R, at::kInt), counts = next(E, at::kUInt32), ends = next(E, at::kUInt32);
-  const Tensor starts = next(E, at::kUInt32), seg_starts = next(E + 1, at::kInt), row_slot = next(slots, at::kInt);
-  const Tensor tile_expert = next(tiles, at::kInt);
+  const Tensor se = next(of_rows, R, at::kInt), ss = next(of_rows, R, at::kInt), row_slot = next(of_rows, slots, at::kInt);
+  const Tensor tile_expert = next(of_rows, tiles, at::kInt), counts = next(of_experts, E, at::kUInt32);
+  const Tensor ends = next(of_experts, E, at::kUInt32), starts = next(of_experts, E, at::kUInt32);
+  const Tensor seg_starts = next(of_experts, E + 1, at::kInt);
   const Tensor ws = workspace(kSortWs, ids, l.stream, api.ck_sort_workspace_words(R, (int32_t)E));
   check(api.ck_sort_by_expert(ptr(ids), ids.scalar_type() == at::kLong, R, (int32_t)E, (int32_t)align, (int32_t*)ptr(se),
                               (int32_t*)ptr(ss), (uint32_t*)ptr(counts), (uint32_t*)ptr(ends), (uint32_t*)ptr(starts),
