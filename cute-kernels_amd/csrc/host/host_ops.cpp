@@ -1094,7 +1094,7 @@ std::tuple<Tensor, Tensor> residual_rmsnorm(const Tensor& x, const Tensor& resid
 struct NormRoute {
   Tensor y, logits, rstd, x8, scale8;
 };
-// Where ck_router_rows is the faster way from rows to router logits: while its workgroups (16 rows x 16 experts) do not outnumber
+// Where ck_router_rows is the faster way from rows to router logits: while its workgroups of 16 rows x 16 experts do not outnumber
 // the compute units.
 bool router_rows_fit(int64_t B, int64_t H, int64_t E) {
   return H >= 32 && H % 32 == 0 && H <= 4096 && E >= 1 && ((B + 15) / 16) * ((E + 15) / 16) <= 256;

@@ -252,99 +252,130 @@ __global__ __launch_bounds__(kNT, 3) void rmsnorm_route_kernel(const T* __restri
 }
 
 // ---- the same for few rows -----------------------------------------------------------------------------------------
-// What bounds it: latency. The kernel above gives 16 rows to one workgroup of 4 waves, each of which walks through a quarter
-// of the contraction for all experts, behind a launch that re-orders the gate weight; a handful of workgroups takes 13 us
-// for what is 1 MiB of reads. Here a workgroup owns 16 rows x 16 experts and has 16 waves: wave w takes the 64-column pieces
-// w, w + 16, ..., all of its loads (at most 8 of x, 8 of the gate weight) go out at once, and the 16 partial 16 x 16 blocks
-// are added through LDS in a fixed order. The workgroups of a row block all normalise it; the first writes y and rstd, the
-// last the e4m3 rows. The gate weight is read as stored: the channel conflicts of its row pitch do not show at this
-// size. In a decoding step: 64 rows x 2,048, 64 experts 8.0 us (re-ordering 4.2 + 12.9 above); 128 x 4,096, 128 experts with
-// e4m3 rows 17.5 (norm 4.5, library product 14.8, quantiser 4.4); without the norm, 8 rows x 4,096 and 8 experts 7.0 (library
-// 15.4), 2,000 rows 9.3 (16.1). A workgroup takes its 256 KiB at what one compute unit can fetch, which is most of the time:
-// more of them than compute units, and the kernels that read the gate weight once per more rows win (1,024 x 4,096, 128
-// experts: 28.5 us against 24.0 in separate kernels).
+// What bounds it: latency, and the vector work of the norm that every workgroup of a row block repeats. The kernel above gives 16
+// rows to one workgroup of 4 waves, each of which walks through a quarter of the contraction for all experts, behind a launch that
+// re-orders the gate weight; a handful of workgroups takes 13 us for what is 1 MiB of reads. Here a workgroup owns 4, 8 or 16 rows
+// x 16 experts and has 16 waves: wave w takes the 64-column pieces w, w + 16, ..., all of its loads (at most 8 of x, 8 of the gate
+// weight) go out at once, and the 16 partial blocks are added through LDS in a fixed order. The workgroups of a row block all
+// normalise it; the first writes y and rstd, the last the e4m3 rows. The gate weight is read as stored: the channel conflicts of its
+// row pitch do not show at this size.
+// Rows of a workgroup: the fewest whose workgroups are no more than the compute units, since a unit does their norms in turn. With
+// 16 / 8 / 4 in a replayed graph: 64 rows x 2,048, 64 experts 7.8 / 5.9 / 5.0 us; 128 x 4,096, 128 experts with e4m3 rows 15.3 /
+// 10.6 / 8.6, 256 of them 15.1 / 10.7 / 13.3 and 512 15.6 / 18.1 / 22.8; without the norm 1,024 x 4,096 and 8 experts 7.4 / 6.1 /
+// 5.4, 2,000 rows 7.8 / 6.3 / 8.4. (With loads that waited for one another behind conditions, 16 rows took 7.7, 16.8, 16.5 and
+// 17.1 us; in separate kernels the 128 rows take norm 4.5, library product 14.8, quantiser 4.4.) More workgroups of 16 rows than
+// compute units, and the kernels that read the gate weight once per more rows win (1,024 x 4,096, 128 experts).
 constexpr int kRowWaves = 16;
+constexpr int kRowBlocks = 256;  // workgroups up to which fewer rows in each pay: one per compute unit
 
 // S: 32-column pieces per wave, H <= 512 S and H % 32 == 0. NORM: rmsnorm(x) goes to the router (norm_w may be NULL), else x
-// itself.
-template <typename T, int S, bool NORM>
+// itself. ROWS: 16, or 8 or 4 with FOLD = 2 or 4 pieces of a row side by side in the 16 columns of an operand: each then meets FOLD
+// pieces of the gate weight in products of their own, and of the FOLD blocks a column counts in the one of its piece.
+template <typename T, int S, bool NORM, int ROWS>
 __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T* __restrict__ x, const T* __restrict__ norm_w,
                                                                          const T* __restrict__ gate_w, float eps, int64_t B,
                                                                          int H, int E, T* __restrict__ y,
                                                                          float* __restrict__ rstd_out, T* __restrict__ logits,
                                                                          uint8_t* __restrict__ x8, float* __restrict__ scale8) {
-  __shared__ float part[kRowWaves][kRows][17];  // 16 experts, one column of padding
-  __shared__ float red[2][kRowWaves][kRows];
-  __shared__ __attribute__((aligned(16))) T w_lds[NORM ? 512 * S : 8];  // the norm weight: read by all 16 rows of every wave
+  constexpr int FOLD = 16 / ROWS, XS = S / FOLD;
+  static_assert(XS * FOLD == S, "whole operands");
+  __shared__ float part[kRowWaves][16][17];  // 16 experts, one column of padding
+  __shared__ float red[2][kRowWaves][ROWS];
+  __shared__ __attribute__((aligned(16))) T w_lds[NORM ? 512 * S : 8];  // the norm weight: read by all rows of every wave
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int r = lane & 15, q = lane >> 4;
-  const int64_t row0 = (int64_t)blockIdx.x * kRows, row = row0 + r;
+  const int col = lane & 15, q = lane >> 4, r = col % ROWS, fold = col / ROWS;
+  const int64_t row0 = (int64_t)blockIdx.x * ROWS, row = row0 + r;
   const int e0 = blockIdx.y * 16;
   const bool row_ok = row < B;
-  const bool writer = row_ok && blockIdx.y == 0;
   const int pieces = H / 32;
-  const T* xr = x + (row_ok ? row : B - 1) * H + 8 * q;     // rows past the end re-read the last row
-  const T* gr = gate_w + (int64_t)min(e0 + r, E - 1) * H + 8 * q;  // experts past the end the last expert
-  auto piece = [&](int s) { return (s / 2 * kRowWaves + wave) * 2 + s % 2; };  // pairs: the halves of 128-byte lines
+  const bool whole = pieces == 16 * S;  // no piece past the end of the rows
+  auto piece = [&](int t) { return (t / 2 * kRowWaves + wave) * 2 + t % 2; };  // pairs: the halves of 128-byte lines
+  auto at = [&](int t) { return 32 * min(piece(t), pieces - 1); };             // pieces past the end re-read the last one
+  // rows past the end re-read the last row, experts past the end the last expert
+  const T* xb = x + row0 * H;
+  const uint32_t x_lane = (uint32_t)min((int64_t)r, B - 1 - row0) * H + 8 * q;
+  const T* gb = gate_w + (int64_t)e0 * H;
+  const uint32_t g_lane = (uint32_t)min(col, E - 1 - e0) * H + 8 * q;
 
-  vec16 xa[S], g[S];
+  // the order of the loads is the order they are waited for in, and none hangs on a condition: the wait for x leaves the others
+  // in flight
+  vec16 xa[XS], g[S];
 #pragma unroll
-  for (int s = 0; s < S; ++s) xa[s] = piece(s) < pieces ? load16(xr + piece(s) * 32) : zero16();
-  if constexpr (NORM) {
-    if (norm_w != nullptr && tid < H / 8) *reinterpret_cast<vec16*>(&w_lds[8 * tid]) = load16(norm_w + 8 * tid);
+  for (int s = 0; s < XS; ++s) xa[s] = load16(xb + (x_lane + (uint32_t)at(s * FOLD + fold)));
+  Pack16<T> nw;
+  if constexpr (NORM) nw.v = load16((norm_w != nullptr ? norm_w : gate_w) + min(8 * tid, H - 8));
+#pragma unroll
+  for (int t = 0; t < S; ++t) g[t] = load16(gb + at(t) + g_lane);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!whole) {
+#pragma unroll
+    for (int s = 0; s < XS; ++s)
+      if (piece(s * FOLD + fold) >= pieces) xa[s] = zero16();
   }
-#pragma unroll
-  for (int s = 0; s < S; ++s) g[s] = piece(s) < pieces ? load16(gr + piece(s) * 32) : zero16();
 
-  auto row_total = [&](float (&of)[kRowWaves][kRows], auto&& join) {  // over the waves, in order
+  auto row_total = [&](float (&of)[kRowWaves][ROWS], auto&& join) {  // over the waves, in order
     float total = of[0][r];
 #pragma unroll
     for (int w = 1; w < kRowWaves; ++w) total = join(total, of[w][r]);
     return total;
   };
+  auto lanes_total = [](float v, auto&& join) {  // over the lanes of a row
+#pragma unroll
+    for (int step = ROWS; step < kWave; step *= 2) v = join(v, __shfl_xor(v, step, kWave));
+    return v;
+  };
+  const auto add = [](float a, float b) { return a + b; };
+  const auto larger = [](float a, float b) { return fmaxf(a, b); };
   if constexpr (NORM) {
     float ss = 0.f;
 #pragma unroll
-    for (int s = 0; s < S; ++s)
+    for (int s = 0; s < XS; ++s)
 #pragma unroll
       for (int i = 0; i < 4; ++i) ss = dot2_acc<T>(xa[s].w[i], ss);
-    ss += __shfl_xor(ss, 16, kWave);
-    ss += __shfl_xor(ss, 32, kWave);
-    if (q == 0) red[0][wave][r] = ss;
-    __syncthreads();
-    ss = row_total(red[0], [](float a, float b) { return a + b; });
-    const float rs = rsqrtf(ss * (1.0f / (float)H) + eps);
-    if (rstd_out != nullptr && writer && wave == 0 && q == 0) rstd_out[row] = rs;
-    uint32_t amax_bits = 0;
+    ss = lanes_total(ss, add);
+    if (lane < ROWS) red[0][wave][r] = ss;
+    if (tid < 64 * S) {  // a weight of one changes no bit; zero past the end of the rows
+      if (norm_w == nullptr || 8 * tid >= H) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
+        for (int i = 0; i < 8; ++i) nw.e[i] = Elem<T>::down(8 * tid >= H ? 0.f : 1.f);
+      }
+      *reinterpret_cast<vec16*>(&w_lds[8 * tid]) = nw.v;
+    }
+    __syncthreads();
+    ss = row_total(red[0], add);
+    const float rs = rsqrtf(ss * (1.0f / (float)H) + eps);
+    if (rstd_out != nullptr && blockIdx.y == 0 && row_ok && wave == 0 && lane < ROWS) rstd_out[row] = rs;
+#pragma unroll
+    for (int s = 0; s < XS; ++s) {
       Pack16<T> p, w;
       p.v = xa[s];
-      if (norm_w != nullptr && piece(s) < pieces) w.v = *reinterpret_cast<const vec16*>(&w_lds[piece(s) * 32 + 8 * q]);
+      w.v = *reinterpret_cast<const vec16*>(&w_lds[piece(s * FOLD + fold) * 32 + 8 * q]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v0 = Elem<T>::up(p.e[2 * i]) * rs, v1 = Elem<T>::up(p.e[2 * i + 1]) * rs;
-        if (norm_w != nullptr) {
-          v0 *= Elem<T>::up(w.e[2 * i]);
-          v1 *= Elem<T>::up(w.e[2 * i + 1]);
-        }
-        xa[s].w[i] = piece(s) < pieces ? pack_pair<T>(v0, v1) : 0u;
-        amax_bits = pk_max_u16(amax_bits, xa[s].w[i] & 0x7fff7fffu);
-      }
-      if (writer && piece(s) < pieces) store16(y + row * H + piece(s) * 32 + 8 * q, xa[s]);
+      for (int i = 0; i < 4; ++i)
+        xa[s].w[i] = pack_pair<T>(Elem<T>::up(p.e[2 * i]) * rs * Elem<T>::up(w.e[2 * i]),
+                                  Elem<T>::up(p.e[2 * i + 1]) * rs * Elem<T>::up(w.e[2 * i + 1]));
+    }
+    if (blockIdx.y == 0) {
+#pragma unroll
+      for (int s = 0; s < XS; ++s)
+        if (row_ok && piece(s * FOLD + fold) < pieces) store16(y + row * H + piece(s * FOLD + fold) * 32 + 8 * q, xa[s]);
     }
     if (x8 != nullptr && blockIdx.y == gridDim.y - 1) {  // as ck_quant_rows_e4m3 computes them from the stored y
-      float amax = fmaxf(half_bits_to_float<T>(amax_bits & 0xffffu), half_bits_to_float<T>(amax_bits >> 16));
-      amax = fmaxf(amax, __shfl_xor(amax, 16, kWave));
-      amax = fmaxf(amax, __shfl_xor(amax, 32, kWave));
-      if (q == 0) red[1][wave][r] = amax;
-      __syncthreads();
-      amax = row_total(red[1], [](float a, float b) { return fmaxf(a, b); });
-      const float inv = amax > 0.f ? kE4M3Max / amax : 1.0f;
-      if (wave == 0 && q == 0 && row_ok) scale8[row] = amax > 0.f ? amax / kE4M3Max : 1.0f;
+      uint32_t amax_bits = 0;
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
+      for (int s = 0; s < XS; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) amax_bits = pk_max_u16(amax_bits, xa[s].w[i] & 0x7fff7fffu);
+      float amax = fmaxf(half_bits_to_float<T>(amax_bits & 0xffffu), half_bits_to_float<T>(amax_bits >> 16));
+      amax = lanes_total(amax, larger);
+      if (lane < ROWS) red[1][wave][r] = amax;
+      __syncthreads();
+      amax = row_total(red[1], larger);
+      const float inv = amax > 0.f ? kE4M3Max / amax : 1.0f;
+      if (wave == 0 && lane < ROWS && row_ok) scale8[row] = amax > 0.f ? amax / kE4M3Max : 1.0f;
+#pragma unroll
+      for (int s = 0; s < XS; ++s) {
         Pack16<T> a;
         a.v = xa[s];
         int lo = 0, hi = 0;
@@ -352,25 +383,40 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
         lo = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[2]) * inv, Elem<T>::up(a.e[3]) * inv, lo, true);
         hi = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[4]) * inv, Elem<T>::up(a.e[5]) * inv, hi, false);
         hi = __builtin_amdgcn_cvt_pk_fp8_f32(Elem<T>::up(a.e[6]) * inv, Elem<T>::up(a.e[7]) * inv, hi, true);
-        if (row_ok && piece(s) < pieces)
-          *reinterpret_cast<uint2*>(x8 + row * H + piece(s) * 32 + 8 * q) = uint2{(uint32_t)lo, (uint32_t)hi};
+        if (row_ok && piece(s * FOLD + fold) < pieces)
+          *reinterpret_cast<uint2*>(x8 + row * H + piece(s * FOLD + fold) * 32 + 8 * q) = uint2{(uint32_t)lo, (uint32_t)hi};
       }
     }
   }
 
+  if (!whole) {  // x is zero there, but what was read again may be infinite
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+      if (piece(t) >= pieces) g[t] = zero16();
+  }
   auto frag = [](const vec16& v) { return __builtin_bit_cast(typename Mfma16<T>::frag, v); };
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[FOLD] = {};
 #pragma unroll
-  for (int s = 0; s < S; ++s) acc = Mfma16<T>::run(frag(g[s]), frag(xa[s]), acc);  // 4 consecutive experts of one row
+  for (int s = 0; s < XS; ++s)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) part[wave][r][4 * q + i] = acc[i];
+    for (int f = 0; f < FOLD; ++f) acc[f] = Mfma16<T>::run(frag(g[s * FOLD + f]), frag(xa[s]), acc[f]);  // 4 experts of one column
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float v = acc[0][i];
+#pragma unroll
+    for (int f = 1; f < FOLD; ++f) v = fold == f ? acc[f][i] : v;
+    part[wave][col][4 * q + i] = v;
+  }
   __syncthreads();
-  if (tid < kRows * 16) {
-    const int orow = tid >> 4, e = tid & 15;
-    float v = part[0][orow][e];
+  if (tid < 16 * 16) {
+    // the columns of one row lie in one wave, side by side
+    const int u = tid >> 4, e = tid & 15, of = u / FOLD, c = u % FOLD * ROWS + of;
+    float v = part[0][c][e];
 #pragma unroll
-    for (int w = 1; w < kRowWaves; ++w) v += part[w][orow][e];
-    if (row0 + orow < B && e0 + e < E) logits[(row0 + orow) * E + e0 + e] = Elem<T>::down(v);
+    for (int w = 1; w < kRowWaves; ++w) v += part[w][c][e];
+#pragma unroll
+    for (int step = 16; step < 16 * FOLD; step *= 2) v += __shfl_xor(v, step, kWave);
+    if (u % FOLD == 0 && row0 + of < B && e0 + e < E) logits[(row0 + of) * E + e0 + e] = Elem<T>::down(v);
   }
 }
 
@@ -394,24 +440,35 @@ extern "C" int ck_router_rows(const void* x, const void* norm_weight, const void
   CK_REQUIRE((x8 == nullptr) == (scale8 == nullptr), "%s: x8 and scale8 go together", name);
   CK_REQUIRE(aligned16(x) && aligned16(gate_weight) && aligned16(y) && aligned16(norm_weight) && aligned16(x8),
              "%s: pointers must be 16-byte aligned", name);
-  const int64_t row_blocks = ceil_div(B, kRows);
+  const int64_t expert_blocks = ceil_div(E, 16);
+  const int rows = H > 1024 && ceil_div(B, 4) * expert_blocks <= kRowBlocks ? 4 : ceil_div(B, 8) * expert_blocks <= kRowBlocks ? 8 : 16;
+  const int64_t row_blocks = ceil_div(B, rows);
   CK_REQUIRE(row_blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
-  const dim3 grid((unsigned)row_blocks, (unsigned)ceil_div(E, 16));
+  const dim3 grid((unsigned)row_blocks, (unsigned)expert_blocks);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CK_RR_N(S, NORM)                                                                                                   \
-  hipLaunchKernelGGL((router_rows_kernel<scalar_t, S, NORM>), grid, dim3(kRowWaves * kWave), 0, s,                         \
+#define CK_RR_N(S, NORM, ROWS)                                                                                             \
+  hipLaunchKernelGGL((router_rows_kernel<scalar_t, S, NORM, ROWS>), grid, dim3(kRowWaves * kWave), 0, s,                   \
                      static_cast<const scalar_t*>(x), static_cast<const scalar_t*>(norm_weight),                           \
                      static_cast<const scalar_t*>(gate_weight), eps, B, (int)H, (int)E, static_cast<scalar_t*>(y), rstd,   \
                      static_cast<scalar_t*>(logits), static_cast<uint8_t*>(x8), scale8)
-#define CK_RR(S)                     \
-  do {                               \
-    if (normalize) CK_RR_N(S, true); \
-    else CK_RR_N(S, false);          \
+#define CK_RR(S, ROWS)                     \
+  do {                                     \
+    if (normalize) CK_RR_N(S, true, ROWS); \
+    else CK_RR_N(S, false, ROWS);          \
   } while (0)
   CK_DISPATCH_HALF(dtype, name, {
-    if (H <= 1024) CK_RR(2);
-    else if (H <= 2048) CK_RR(4);
-    else CK_RR(8);
+    if (H <= 1024) {
+      if (rows == 8) CK_RR(2, 8);
+      else CK_RR(2, 16);
+    } else if (H <= 2048) {
+      if (rows == 4) CK_RR(4, 4);
+      else if (rows == 8) CK_RR(4, 8);
+      else CK_RR(4, 16);
+    } else {
+      if (rows == 4) CK_RR(8, 4);
+      else if (rows == 8) CK_RR(8, 8);
+      else CK_RR(8, 16);
+    }
   });
 #undef CK_RR
 #undef CK_RR_N

@@ -47,6 +47,20 @@ def test_logits_and_norm(B, H, E, dtype):
         assert torch.equal(x8.view(torch.uint8), q.view(torch.uint8)) and torch.equal(scale, s)
 
 
+# 4, 8 or 16 rows a workgroup, by how many there are: edges of each, at whole and ragged widths of each instantiation
+@pytest.mark.parametrize(
+    "B,H,E",
+    [(4, 2048, 16), (5, 3072, 33), (500, 1088, 17), (8, 32, 16), (9, 1024, 8), (515, 2016, 32), (1023, 4096, 17), (2049, 992, 1),
+     (1030, 2048, 20), (1033, 4064, 32)],
+)
+def test_rows_of_a_workgroup(B, H, E):
+    test_logits_and_norm(B, H, E, torch.bfloat16)
+    x, w, nw = _inputs(B, H, E, torch.bfloat16)
+    w[E // 2, H - 1] = float("inf")  # read again by the pieces past the end of a row: in no other product
+    _, logits = rmsnorm_route.rmsnorm_route_cute(x, nw, w, 1e-6)
+    assert bool((torch.isfinite(logits).all(0) == (torch.arange(E, device=DEV) != E // 2)).all()) and bool(torch.isinf(logits[:, E // 2]).all())
+
+
 def test_sizes_beyond_one_workgroup_per_compute_unit_keep_their_routes():
     x, w, _ = _inputs(257, 512, 256, torch.bfloat16)
     take = _C.host().router_rows_take
