@@ -97,32 +97,15 @@ __device__ inline void to_operands(const vec16 (&lines)[2], vec16 (&w)[2]) {
 
 // TI: operand type, TO: output type; MB: row blocks of 16 per tile, NB: column blocks of 16 per tile. kSwiglu: half of the
 // column blocks are up columns, the other half the gate columns of the same outputs. LINES: every row of the weights starts on
-// a 128-byte boundary.
+// a 128-byte boundary. The tile of rows m0.. and outputs n0..
 template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
-__global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
-  constexpr int BM = 16 * MB, kEl = Operand<TI>::kBytes;
+__device__ __attribute__((always_inline)) inline void skinny_tile(const GemmParams& prm, f32x4 (*red)[kWave], int expert, int m0, int n0) {
+  constexpr int kEl = Operand<TI>::kBytes;
   constexpr int NH = MODE == kSwiglu ? NB / 2 : NB;  // column blocks of outputs per tile
   static_assert(MODE != kSwiglu || NB % 2 == 0, "whole up / gate block pairs");
-  __shared__ f32x4 red[kWaves][MB * NB][kWave];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lrow = lane & 15, lq = lane >> 4;
-
-  // ---- which tile: expert by expert, column tile by column tile, the row tiles of one column tile in a row; chunks of kChunk
-  // consecutive tiles go out over the XCDs, so that the chip reads one stretch of memory at a time
-  const int live_m = prm.seg_starts[prm.num_experts] / BM;
-  const int total = live_m * prm.n_tiles;
-  int pid = blockIdx.x;
-  if (pid >= total) return;
-  constexpr int kChunk = 32;
-  if (pid < total / (kXcds * kChunk) * (kXcds * kChunk)) {  // the last, partial round keeps its order
-    const int j = pid / kXcds;
-    pid = (j / kChunk * kXcds + pid % kXcds) * kChunk + j % kChunk;
-  }
-  const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[pid / prm.n_tiles]);
-  const int first_m = prm.seg_starts[expert] / BM, expert_m = prm.seg_starts[expert + 1] / BM - first_m;
-  const int local = pid - first_m * prm.n_tiles, nt = local / expert_m, mt = first_m + local - nt * expert_m;
-  const int m0 = mt * BM;
   const int valid_end = prm.seg_starts[expert] + (int)prm.counts[expert];
 
   // ---- operand rows of this lane, as 32-bit byte offsets from a uniform base (the host checks that they fit)
@@ -143,8 +126,8 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
     for (int h = 0; h < 2; ++h) {
       const int c = 8 * h + (lane & 7);
       int n;
-      if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(nt * (NH * 16) + (j % NH) * 16 + c, prm.I - 1);
-      else n = min(nt * (NB * 16) + j * 16 + c, prm.N - 1);
+      if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(n0 + (j % NH) * 16 + c, prm.I - 1);
+      else n = min(n0 + j * 16 + c, prm.N - 1);
       w_off[j][h] = (uint32_t)n * (uint32_t)(prm.ldw * kEl) + (lane >> 3) * 16;
     }
 
@@ -221,12 +204,12 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) red[wave][i * NB + j][lane] = acc[i][j];
+    for (int j = 0; j < NB; ++j) red[wave * MB * NB + i * NB + j][lane] = acc[i][j];
   __syncthreads();
   auto total_of = [&](int b, int l) {
-    f32x4 v = red[0][b][l];
+    f32x4 v = red[b][l];
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w) v += red[w][b][l];
+    for (int w = 1; w < kWaves; ++w) v += red[w * MB * NB + b][l];
     return v;
   };
   constexpr int kItems = MB * NH * kWave;
@@ -235,7 +218,7 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   for (int it = tid; it < kItems; it += kNT) {
     const int b = it / kWave, i = b / NH, j = b % NH;  // lane of the item: this thread's (kNT is a multiple of kWave)
     const int p = m0 + i * 16 + lrow;
-    const int n = nt * (NH * 16) + j * 16 + 4 * lq;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
+    const int n = n0 + j * 16 + 4 * lq;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
     const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N);
     f32x4 v = total_of(i * NB + j, lane);
     [[maybe_unused]] f32x4 g = v;
@@ -288,11 +271,50 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   }
 }
 
+// Narrow weights of few experts are few tiles, and a compute unit streams 28 bytes a ns however many it holds (256 of them: what
+// memory gives), so that a launch takes as long as the unit with the most tiles: 128, 256, 384, ... tiles of 32 x 14,336 took 37, 40, 69,
+// 73, 102, 107 and 136 us. Where the last round of one tile per unit is at most half full, its tiles go out in two halves of the columns
+// therefore: 28, 41, 59, 74, 93, 107 and 125 us (a half's single wave per SIMD does not get the full rate out of its unit, so halves
+// are no better for a fuller round). No sum changes. A SwiGLU tile of one block of up and one of gate columns has no halves.
+constexpr int kCus = 256;
+template <int MODE, int NB>
+constexpr bool kHalves = MODE == kSwiglu ? NB > 2 : NB > 1;
+
+template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
+__global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
+  constexpr int BM = 16 * MB, kColumns = 16 * (MODE == kSwiglu ? NB / 2 : NB);
+  __shared__ f32x4 red[kWaves * MB * NB][kWave];
+
+  // ---- which tile: expert by expert, column tile by column tile, the row tiles of one column tile in a row; chunks of kChunk
+  // consecutive tiles go out over the XCDs, so that the chip reads one stretch of memory at a time
+  const int live_m = prm.seg_starts[prm.num_experts] / BM;
+  const int total = live_m * prm.n_tiles;
+  constexpr int kChunk = 32;
+  static_assert(kXcds * kChunk == kCus, "the partial round of the chunks is that of the compute units");
+  const int whole = total / kCus * kCus;
+  int pid = blockIdx.x, half = -1;
+  if (pid < whole) {
+    const int j = pid / kXcds;
+    pid = (j / kChunk * kXcds + pid % kXcds) * kChunk + j % kChunk;
+  } else if (kHalves<MODE, NB> && total - whole <= kCus / 2) {
+    half = (pid - whole) % 2;
+    pid = whole + (pid - whole) / 2;
+  }
+  if (pid >= total) return;
+  const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[pid / prm.n_tiles]);
+  const int first_m = prm.seg_starts[expert] / BM, expert_m = prm.seg_starts[expert + 1] / BM - first_m;
+  const int local = pid - first_m * prm.n_tiles, nt = local / expert_m, mt = first_m + local - nt * expert_m;
+  if constexpr (kHalves<MODE, NB>) {
+    if (half >= 0) return skinny_tile<TI, TO, MODE, MB, NB / 2, LINES>(prm, red, expert, mt * BM, nt * kColumns + half * (kColumns / 2));
+  }
+  skinny_tile<TI, TO, MODE, MB, NB, LINES>(prm, red, expert, mt * BM, nt * kColumns);
+}
+
 template <typename TI, typename TO, int MODE, int MB, int NB>
 int launch_tile(const GemmParams& prm_in, int64_t m_tiles, int out_cols, hipStream_t s, const char* name) {
   GemmParams prm = prm_in;
   prm.n_tiles = (int)ceil_div(out_cols, 16 * (MODE == kSwiglu ? NB / 2 : NB));
-  const int64_t blocks = m_tiles * prm.n_tiles;
+  const int64_t blocks = m_tiles * prm.n_tiles + (kHalves<MODE, NB> ? kCus / 2 : 0);  // where a last round has halves, each of them
   CK_REQUIRE(blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
   constexpr int64_t kLine = 128;
   const bool lines = prm.ldw * Operand<TI>::kBytes % kLine == 0 && reinterpret_cast<uintptr_t>(prm.w) % kLine == 0;

@@ -139,3 +139,15 @@ def test_weight_lines(device, align, K, offset, columns):
     for e, c in enumerate(counts):
         want = (rows[e].float() @ w[e].float().t()).to(torch.bfloat16).float()  # whole numbers, exact in fp32 and rounded once
         assert torch.equal(y[starts[e] : starts[e] + c], want), e
+
+
+# Four experts have rows, of 16 to 64 a tile: 128 column tiles of 64 (the last one ragged) and so on, that is a launch that goes out in
+# halves of tiles, one of more than half a round, whole rounds, and these behind a whole round
+@pytest.mark.parametrize("align", [16, 32, 64])
+@pytest.mark.parametrize("N", [2032, 2064, 4096, 4112, 6160])
+@pytest.mark.parametrize("epilogue", ["grouped_bias", "scatter", "swiglu", "fp8"])
+def test_last_round_in_halves(device, align, N, epilogue):
+    if epilogue == "fp8":
+        test_small_tiles_fp8(device, align, 9, 1152, N)
+    else:
+        test_small_tiles_match_fp32(device, torch.bfloat16, align, 9, 200, N, epilogue)
