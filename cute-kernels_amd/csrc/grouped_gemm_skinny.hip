@@ -96,13 +96,14 @@ __device__ inline void to_operands(const vec16 (&lines)[2], vec16 (&w)[2]) {
 }
 
 // TI: operand type, TO: output type; MB: row blocks of 16 per tile, NB: column blocks of 16 per tile. kSwiglu: half of the
-// column blocks are up columns, the other half the gate columns of the same outputs. LINES: every row of the weights starts on
-// a 128-byte boundary. The tile of rows m0.. and outputs n0..
+// column blocks are up columns, the other half the gate columns of the same outputs; of one block, the first and the last 8 columns.
+// LINES: every row of the weights starts on a 128-byte boundary. The tile of rows m0.. and outputs n0..
 template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
 __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmParams& prm, f32x4 (*red)[kWave], int expert, int m0, int n0) {
   constexpr int kEl = Operand<TI>::kBytes;
-  constexpr int NH = MODE == kSwiglu ? NB / 2 : NB;  // column blocks of outputs per tile
-  static_assert(MODE != kSwiglu || NB % 2 == 0, "whole up / gate block pairs");
+  constexpr bool kPair = MODE == kSwiglu && NB == 1;              // up and gate columns share a block
+  constexpr int NH = MODE == kSwiglu && !kPair ? NB / 2 : NB;  // column blocks of outputs per tile
+  static_assert(MODE != kSwiglu || kPair || NB % 2 == 0, "whole up / gate block pairs");
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lrow = lane & 15, lq = lane >> 4;
@@ -126,7 +127,8 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
     for (int h = 0; h < 2; ++h) {
       const int c = 8 * h + (lane & 7);
       int n;
-      if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(n0 + (j % NH) * 16 + c, prm.I - 1);
+      if constexpr (kPair) n = h * prm.I + min(n0 + (lane & 7), prm.I - 1);
+      else if constexpr (MODE == kSwiglu) n = (j / NH) * prm.I + min(n0 + (j % NH) * 16 + c, prm.I - 1);
       else n = min(n0 + j * 16 + c, prm.N - 1);
       w_off[j][h] = (uint32_t)n * (uint32_t)(prm.ldw * kEl) + (lane >> 3) * 16;
     }
@@ -219,10 +221,10 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
     const int b = it / kWave, i = b / NH, j = b % NH;  // lane of the item: this thread's (kNT is a multiple of kWave)
     const int p = m0 + i * 16 + lrow;
     const int n = n0 + j * 16 + 4 * lq;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
-    const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N);
+    const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N) && (!kPair || lq < 2);
     f32x4 v = total_of(i * NB + j, lane);
     [[maybe_unused]] f32x4 g = v;
-    if constexpr (MODE == kSwiglu) g = total_of(i * NB + j + NH, lane);
+    if constexpr (MODE == kSwiglu) g = kPair ? total_of(i, lane ^ 32) : total_of(i * NB + j + NH, lane);
     if (!inside) continue;
     if constexpr (kFp8) {
       const float rs = prm.a_scale[prm.a_gather_div > 0 ? prm.row_slot[p] / prm.a_gather_div : p];
@@ -275,10 +277,10 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
 // memory gives), so that a launch takes as long as the unit with the most tiles: 128, 256, 384, ... tiles of 32 x 14,336 took 37, 40, 69,
 // 73, 102, 107 and 136 us. Where the last round of one tile per unit is at most half full, its tiles go out in two halves of the columns
 // therefore: 28, 41, 59, 74, 93, 107 and 125 us (a half's single wave per SIMD does not get the full rate out of its unit, so halves
-// are no better for a fuller round). No sum changes. A SwiGLU tile of one block of up and one of gate columns has no halves.
+// are no better for a fuller round). No sum changes. SwiGLU tiles likewise, 4 experts of 2,000 x 3,072 with a row or two in all 11.8 ->
+// 10.1 us; where more than a dozen rounds go by, the units are out of step anyway and a last one is worth 1 % or nothing. Of 265 launches
+// in all (4 to 128 experts, 4 MB to 2.1 GB) 2 to 3 % less time on average; 3 % of a 10 us launch more for the longer program.
 constexpr int kCus = 256;
-template <int MODE, int NB>
-constexpr bool kHalves = MODE == kSwiglu ? NB > 2 : NB > 1;
 
 template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
 __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
@@ -296,7 +298,7 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   if (pid < whole) {
     const int j = pid / kXcds;
     pid = (j / kChunk * kXcds + pid % kXcds) * kChunk + j % kChunk;
-  } else if (kHalves<MODE, NB> && total - whole <= kCus / 2) {
+  } else if (total - whole <= kCus / 2) {
     half = (pid - whole) % 2;
     pid = whole + (pid - whole) / 2;
   }
@@ -304,9 +306,7 @@ __global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kern
   const int expert = __builtin_amdgcn_readfirstlane(prm.tile_expert[pid / prm.n_tiles]);
   const int first_m = prm.seg_starts[expert] / BM, expert_m = prm.seg_starts[expert + 1] / BM - first_m;
   const int local = pid - first_m * prm.n_tiles, nt = local / expert_m, mt = first_m + local - nt * expert_m;
-  if constexpr (kHalves<MODE, NB>) {
-    if (half >= 0) return skinny_tile<TI, TO, MODE, MB, NB / 2, LINES>(prm, red, expert, mt * BM, nt * kColumns + half * (kColumns / 2));
-  }
+  if (half >= 0) return skinny_tile<TI, TO, MODE, MB, NB / 2, LINES>(prm, red, expert, mt * BM, nt * kColumns + half * (kColumns / 2));
   skinny_tile<TI, TO, MODE, MB, NB, LINES>(prm, red, expert, mt * BM, nt * kColumns);
 }
 
@@ -314,7 +314,7 @@ template <typename TI, typename TO, int MODE, int MB, int NB>
 int launch_tile(const GemmParams& prm_in, int64_t m_tiles, int out_cols, hipStream_t s, const char* name) {
   GemmParams prm = prm_in;
   prm.n_tiles = (int)ceil_div(out_cols, 16 * (MODE == kSwiglu ? NB / 2 : NB));
-  const int64_t blocks = m_tiles * prm.n_tiles + (kHalves<MODE, NB> ? kCus / 2 : 0);  // where a last round has halves, each of them
+  const int64_t blocks = m_tiles * prm.n_tiles + kCus / 2;  // where a last round has halves, each of them
   CK_REQUIRE(blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
   constexpr int64_t kLine = 128;
   const bool lines = prm.ldw * Operand<TI>::kBytes % kLine == 0 && reinterpret_cast<uintptr_t>(prm.w) % kLine == 0;
