@@ -282,8 +282,11 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
 // in all (4 to 128 experts, 4 MB to 2.1 GB) 2 to 3 % less time on average; 3 % of a 10 us launch more for the longer program.
 constexpr int kCus = 256;
 
+// Workgroups per compute unit: three of 32-row tiles. Left to itself the compiler takes 174 to 178 registers for e4m3 operands, for
+// which there is room twice: 128 experts of 4,096 x 1,536 with 8 rows on average, Zipf(0.8), 150 us and now 133, 64 gated ones of 11,264
+// x 1,024 176 and 156.
 template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
-__global__ __launch_bounds__(kNT, MB == 1 ? 4 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
+__global__ __launch_bounds__(kNT, MB == 1 ? 4 : MB == 2 ? 3 : 2) void grouped_gemm_skinny_kernel(const GemmParams prm) {
   constexpr int BM = 16 * MB, kColumns = 16 * (MODE == kSwiglu ? NB / 2 : NB);
   __shared__ f32x4 red[kWaves * MB * NB][kWave];
 
