@@ -406,9 +406,12 @@ constexpr float kE4M3Max = 448.0f;
 // scale[r] = amax(x[r, :]) / 448 (1 for an all-zero row); q[r, c] = e4m3(x[r, c] * (448 / amax)), round to nearest even.
 // A row is owned by TPR = 64 lanes (one wave, no block synchronisation) or 256 (the block); a lane keeps its NC chunks of
 // 16 elements in registers between the reduction and the conversion, so x is read once (NC == 0: long rows, re-read).
-template <typename T, int TPR, int NC>
+// SEGMENTS: the rows of the padded grouped layout; those that stand for nothing are left out. With few rows per
+// expert most do: 1,024 rows of 1,536 in 4,992, 7.2 us with all of them and 5.9 to 6.0 without. A row's own look-up is two dependent reads.
+template <typename T, int TPR, int NC, bool SEGMENTS>
 __global__ __launch_bounds__(kQuantBlock) void quant_rows_e4m3_kernel(const T* __restrict__ x, int64_t rows, int cols,
-                                                                       uint8_t* __restrict__ q, float* __restrict__ scales) {
+                                                                       uint8_t* __restrict__ q, float* __restrict__ scales,
+                                                                       [[maybe_unused]] const ck_segments seg) {
   __shared__ float red[kQuantBlock / kWave];
   constexpr int ROWS = kQuantBlock / TPR;
   const int chunks = cols / 16;  // 16 elements: 32 bytes in, 16 bytes out
@@ -433,6 +436,11 @@ __global__ __launch_bounds__(kQuantBlock) void quant_rows_e4m3_kernel(const T* _
   };
   // TPR == 256: every thread of the block runs the same trip count (the reduction synchronises the block)
   for (int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / TPR; row < rows; row += (int64_t)gridDim.x * ROWS) {
+    if constexpr (SEGMENTS) {  // the same answer in all lanes of the row
+      if (row >= seg.seg_starts[seg.num_experts]) break;
+      const int expert = __builtin_amdgcn_readfirstlane(seg.tile_expert[__builtin_amdgcn_readfirstlane((int)(row / seg.align))]);
+      if (row >= seg.seg_starts[expert] + (int64_t)seg.counts[expert]) continue;
+    }
     const T* xr = x + row * cols;
     uint8_t* qr = q + row * cols;
     float amax = 0.f;
@@ -486,21 +494,22 @@ __global__ __launch_bounds__(kQuantBlock) void quant_rows_e4m3_kernel(const T* _
 
 using namespace ck;
 
-extern "C" int ck_quant_rows_e4m3(const void* x, int64_t rows, int32_t cols, void* q, float* scales, int32_t dtype,
-                                  void* stream) {
-  CK_REQUIRE(rows >= 0 && cols >= 16 && cols % 16 == 0, "ck_quant_rows_e4m3: cols=%d must be a positive multiple of 16", cols);
+static int quant_impl(const char* name, const void* x, int64_t rows, int32_t cols, void* q, float* scales, const ck_segments* seg,
+                      int32_t dtype, void* stream) {
+  CK_REQUIRE(rows >= 0 && cols >= 16 && cols % 16 == 0, "%s: cols=%d must be a positive multiple of 16", name, cols);
   if (rows == 0) return CK_OK;
-  CK_REQUIRE(x && q && scales && aligned16(x) && aligned16(q), "ck_quant_rows_e4m3: NULL or misaligned pointer");
+  CK_REQUIRE(x && q && scales && aligned16(x) && aligned16(q), "%s: NULL or misaligned pointer", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int chunks = cols / 16;
 #define CK_QUANT(TPR, NC)                                                                                          \
   do {                                                                                                             \
     const int64_t want = ceil_div(rows, (int64_t)(kQuantBlock / (TPR)));                                           \
     const unsigned blocks = (unsigned)(want < 65535 * 4 ? want : 65535 * 4);                                       \
-    hipLaunchKernelGGL((quant_rows_e4m3_kernel<scalar_t, TPR, NC>), dim3(blocks), dim3(kQuantBlock), 0, s,         \
-                       static_cast<const scalar_t*>(x), rows, (int)cols, static_cast<uint8_t*>(q), scales);        \
+    auto kernel = seg != nullptr ? quant_rows_e4m3_kernel<scalar_t, TPR, NC, true> : quant_rows_e4m3_kernel<scalar_t, TPR, NC, false>; \
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kQuantBlock), 0, s, static_cast<const scalar_t*>(x), rows,       \
+                       (int)cols, static_cast<uint8_t*>(q), scales, seg != nullptr ? *seg : ck_segments{});        \
   } while (0)
-  CK_DISPATCH_HALF(dtype, "ck_quant_rows_e4m3", {
+  CK_DISPATCH_HALF(dtype, name, {
     if (chunks <= kWave) CK_QUANT(kWave, 1);
     else if (chunks <= 2 * kWave) CK_QUANT(kWave, 2);
     else if (chunks <= kQuantBlock) CK_QUANT(kQuantBlock, 1);
@@ -509,8 +518,20 @@ extern "C" int ck_quant_rows_e4m3(const void* x, int64_t rows, int32_t cols, voi
     else CK_QUANT(kQuantBlock, 0);
   });
 #undef CK_QUANT
-  CK_CHECK_LAUNCH("ck_quant_rows_e4m3");
+  CK_CHECK_LAUNCH(name);
   return CK_OK;
+}
+
+extern "C" int ck_quant_rows_e4m3(const void* x, int64_t rows, int32_t cols, void* q, float* scales, int32_t dtype,
+                                  void* stream) {
+  return quant_impl("ck_quant_rows_e4m3", x, rows, cols, q, scales, nullptr, dtype, stream);
+}
+extern "C" int ck_quant_grouped_rows_e4m3(const void* x, const ck_segments* seg, int32_t cols, void* q, float* scales, int32_t dtype,
+                                          void* stream) {
+  const char* name = "ck_quant_grouped_rows_e4m3";
+  CK_REQUIRE(seg && seg->seg_starts && seg->counts && seg->tile_expert && seg->align > 0 && seg->num_experts > 0 &&
+                 seg->max_rows / seg->align < (int64_t)0x7fffffff, "%s: incomplete segment tables", name);
+  return quant_impl(name, x, seg->max_rows, cols, q, scales, seg, dtype, stream);
 }
 
 extern "C" int ck_grouped_gemm_fp8(const void* a8, const float* a_scale, int32_t a_gather_div, const void* w8,

@@ -38,7 +38,7 @@ using torch::autograd::variable_list;
   X(ck_sort_by_expert) X(ck_combine_rows) X(ck_gate_grad_both) X(ck_group_rows_padded) X(ck_swiglu_bwd_grouped)         \
   X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_uses_workspace) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
   X(ck_grouped_gemm_f32) X(ck_grouped_gemm_dw_f32) X(ck_grouped_gemm_dw) X(ck_grouped_gemm_dw_rows)                     \
-  X(ck_quant_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) X(ck_router_rows) \
+  X(ck_quant_rows_e4m3) X(ck_quant_grouped_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) X(ck_router_rows) \
   X(ck_gelu_tanh_bwd_grouped) X(ck_fused_residual_add_rmsnorm_fwd) X(ck_rmsnorm_fwd) X(ck_rmsnorm_bwd_partial_rows) X(ck_rmsnorm_bwd_typed)         \
   X(ck_softmax_fwd) X(ck_softmax_bwd) X(ck_add_expert_bias) X(ck_expert_bias_grad)
 
@@ -863,12 +863,17 @@ Tensor gelu_experts(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, c
 }
 
 // ---- quantised-expert forward (inference) ------------------------------------------------------------------------
-std::pair<Tensor, Tensor> quantize_rows(const Tensor& x_in) {
+// seg: x holds the rows of that padded grouped layout; those that stand for nothing stay undefined
+std::pair<Tensor, Tensor> quantize_rows(const Tensor& x_in, const Segments* seg = nullptr) {
   require_gpu(x_in);
   const Tensor x = x_in.contiguous();
   const Launch l(x);
   const Tensor q = new_empty({x.size(0), x.size(1)}, x, at::kFloat8_e4m3fn), scale = new_empty({x.size(0)}, x, at::kFloat);
-  check(api.ck_quant_rows_e4m3(ptr(x), x.size(0), (int32_t)x.size(1), ptr(q), (float*)ptr(scale), dtype_code(x), l.stream));
+  if (seg != nullptr) {
+    const ck_segments cs = seg->c();
+    check(api.ck_quant_grouped_rows_e4m3(ptr(x), &cs, (int32_t)x.size(1), ptr(q), (float*)ptr(scale), dtype_code(x), l.stream));
+  } else
+    check(api.ck_quant_rows_e4m3(ptr(x), x.size(0), (int32_t)x.size(1), ptr(q), (float*)ptr(scale), dtype_code(x), l.stream));
   return {q, scale};
 }
 
@@ -900,9 +905,10 @@ Tensor swiglu_experts_e4m3(const Tensor& x, const Tensor& w_fc8, const Tensor& w
     std::tie(x8, x_scale) = quantize_rows(x);  // per token
   }
   const Tensor none;
-  const Tensor act = new_empty({g.max_rows, I}, x);  // pad rows: never written, quantised, never used
+  const Tensor act = new_empty({g.max_rows, I}, x);  // pad rows: never written, quantised perhaps, never used
   gemm_fp8(x8, x_scale, k, w_fc8, w_fc_scale, g, CK_EPI_SWIGLU, none, act, x.scalar_type());
-  auto [act8, act_scale] = quantize_rows(act);  // per routed row
+  // per routed row; the look-up that leaves padding out where that may be more than a quarter of the rows (at 6 % it gains nothing)
+  auto [act8, act_scale] = quantize_rows(act, 4 * T * k < 3 * g.max_rows ? &g : nullptr);
   const Tensor expanded = new_empty({T * k, H}, x);
   gemm_fp8(act8, act_scale, 0, w_proj8, w_proj_scale, g, CK_EPI_SCATTER, expanded, none, x.scalar_type());
   return combine(expanded, gates_in.to(x.scalar_type()).contiguous(), T, k, H);
@@ -1280,7 +1286,7 @@ PYBIND11_MODULE(_ck_host, m) {
   DEF("experts_up", experts_up);
   DEF("experts_down", experts_down);
   DEF("gelu_experts", gelu_experts);
-  DEF("quantize_rows", quantize_rows);
+  DEF("quantize_rows", ([](const Tensor& x) { return quantize_rows(x); }));
   DEF("swiglu_experts_e4m3", swiglu_experts_e4m3);
   DEF("swiglu", swiglu);
   DEF("swiglu_packed", swiglu_packed);

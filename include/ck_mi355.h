@@ -312,6 +312,8 @@ int ck_grouped_gemm_dw_rows(const void* a, const void* b, int32_t M, int32_t N, 
  * round to nearest even. x [rows, cols] bf16 / f16, q [rows, cols] bytes, cols % 16 == 0. Used per token for
  * activations and per output channel ([E * out, in] rows) for expert weights. */
 int ck_quant_rows_e4m3(const void* x, int64_t rows, int32_t cols, void* q, float* scales, int32_t dtype, void* stream);
+/* The same for the rows of the padded grouped layout, x and q [max_rows, cols]: padding rows are neither read nor written. */
+int ck_quant_grouped_rows_e4m3(const void* x, const ck_segments* seg, int32_t cols, void* q, float* scales, int32_t dtype, void* stream);
 /* Y = (A_e * diag(a_scale)) * (W[e] * diag(w_scale[e]))^T over tile-aligned expert segments (align 16, 32, 64 or 256).
  * a8: e4m3 rows [*, K], gathered like ck_grouped_gemm (a_gather_div); a_scale is indexed by the row of a8 that is read.
  * w8 [E, N, K] e4m3, w_scale [E, N]. K % 128 == 0. Epilogues: CK_EPI_GROUPED (y [max_rows, N]), CK_EPI_SCATTER

@@ -162,3 +162,24 @@ def test_fp8_rejects_unsupported(device):
         fp8._gemm_fp8(x8, s, 1, w8, ws, seg128, _C.CK_EPI_GROUPED, y, None, torch.bfloat16)
     with pytest.raises(RuntimeError, match="multiple of 16"):
         _C.check(_C.lib().ck_quant_rows_e4m3(1, 4, 24, 1, 1, _C.CK_BF16, None))
+
+
+# a wave a row (one chunk of 16, two trips), a block a row (an odd chunk over, kept in registers and read again)
+@pytest.mark.parametrize("align", [16, 256])
+@pytest.mark.parametrize("cols", [16, 1536, 4112, 16400])
+def test_grouped_rows_are_quantised_and_padding_is_left_alone(device, align, cols):
+    counts = torch.tensor([0, align, 1, align + 1, 0, 15, 0])
+    ids = torch.arange(7, dtype=torch.int32).repeat_interleave(counts).to(device)
+    seg = cute_kernels.sort_by_expert(ids, 7, align)
+    x = torch.randn(seg.max_rows, cols, generator=torch.Generator().manual_seed(cols)).to(torch.bfloat16).to(device)
+    q = torch.full((seg.max_rows, cols), 0x55, dtype=torch.uint8, device=device)
+    scale = torch.full((seg.max_rows,), -3.0, device=device)
+    _C.check(_C.lib().ck_quant_grouped_rows_e4m3(_C.ptr(x), seg.c_struct(), cols, _C.ptr(q), _C.ptr(scale), _C.CK_BF16, _C.stream()))
+    starts = seg.seg_starts.cpu()
+    valid = torch.zeros(seg.max_rows, dtype=torch.bool)
+    for e, c in enumerate(counts.tolist()):
+        valid[int(starts[e]) : int(starts[e]) + c] = True
+    valid = valid.to(device)
+    want, want_scale = cute_kernels.quantize_rows_e4m3(x)
+    assert torch.equal(q[valid], want.view(torch.uint8)[valid]) and torch.equal(scale[valid], want_scale[valid])
+    assert bool((q[~valid] == 0x55).all()) and bool((scale[~valid] == -3.0).all())
