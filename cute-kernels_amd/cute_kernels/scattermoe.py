@@ -256,12 +256,30 @@ def _layer_tiles(
 _large_tiles_kept, _layer_tiles_kept = functools.lru_cache(4096)(_large_tiles), functools.lru_cache(4096)(_layer_tiles)
 
 
+def _least(known) -> int:
+    """The largest of 0 .. 2^48 for which known(value) holds, if it holds below one value and not from there on."""
+    low, high = 0, 1 << 48
+    while low < high:
+        middle = (low + high + 1) // 2
+        if known(middle):
+            low = middle
+        else:
+            high = middle - 1
+    return low
+
+
 def _height(rule, kept, num_rows: int, *rest) -> int:
     """A rule of sizes alone, looked up where it has been asked before. A traced row count that stands for many takes part in
-    one comparison only (many), so that a graph is compiled for two ranges of it and no more."""
+    one comparison only (many), so that a graph is compiled for two ranges of it and no more. If the caller has said between what
+    bounds it lies, in none, as any comparison that holds for a part of them has the graph refused: one height for all of them,
+    that of their geometric mean."""
     if not is_tracing():
         return kept(num_rows, *rest, False)
-    return rule(num_rows, *rest, not statically_known_true(num_rows < 1 << 48))
+    if not statically_known_true(num_rows < 1 << 48):
+        return rule(num_rows, *rest, True)
+    low = _least(lambda v: statically_known_true(num_rows >= v))
+    high = (1 << 48) - _least(lambda v: statically_known_true(num_rows <= (1 << 48) - v))
+    return rule(low if low == high else math.isqrt(low * high), *rest, False)
 
 
 def choose_align(

@@ -1,6 +1,8 @@
 """Which tile height a call gets (scattermoe.choose_align): one rule for the eager layer, the traced one and the reference's
 expert-linear interface. Nothing is launched; traced calls end at the first real operator, which refuses the CPU tensor."""
 
+import math
+
 import pytest
 import torch
 
@@ -125,6 +127,23 @@ def test_a_dynamic_row_count_compiles_two_graphs(grad):
         with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="runs on the GPU only"):
             compiled(torch.randn(T, 256, dtype=BF16))
     assert backend.aligns == [128, 256] and backend.graphs == 2
+
+
+@pytest.mark.parametrize("act,H,I", [("swiglu", 256, 320), ("gelu", 768, 3072), ("swiglu", 1024, 2048)])
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("least,most", [(4, 20), (30, 60), (200, 400), (900, 2000), (1500, 3000), (20000, 40000)])
+def test_a_bounded_row_count_compiles_one_graph(act, H, I, grad, least, most):
+    """A token count that the caller says may be anything between two bounds: no rule narrows it, which would have the graph refused
+    (ConstraintViolationError). The height is that of the bounds' geometric mean."""
+    moe, backend = _layer(act, H, I), _Backend()
+    x = torch.randn((least + most) // 2, H, dtype=BF16)
+    torch._dynamo.reset()
+    torch._dynamo.mark_dynamic(x, 0, min=least, max=most)
+    compiled = torch.compile(lambda x: moe(x)[0], fullgraph=True, backend=backend)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="runs on the GPU only"):
+        compiled(x)
+    rows = math.isqrt(2 * least * 2 * most)
+    assert backend.graphs == 1 and backend.aligns == [scattermoe.choose_align(rows, E, BF16, not grad, (H, I, act == "swiglu"))]
 
 
 @pytest.mark.parametrize("dtype,rows,grad,height", [
