@@ -189,33 +189,40 @@ def _zipf_tiles(num_rows: int, num_experts: int, height: int) -> int:
 
 def _height_in_inference(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
     """The same choice for a layer's forward alone, by a finer model: the sum of its launches at an even load and at a Zipf(0.8) one
-    together, since the more uneven the load, the fewer experts fit one tile of 128 rows. In us, fitted to measured layers:
+    together, since the more uneven the load, the fewer experts fit one tile of 128 rows. In us:
       * a round of 256 x 256 tiles takes 1.6 a 64-deep step with all CUs at work, down to 1.15 with few (the chip's power is
         shared by fewer), and 8.5 for its start and stores; a split last round takes an equal part of the steps and 43 for
         the exchange of the parts, and happens where it takes 40 steps or more off that round;
-      * a step of a 128 x 128 tile takes 0.9 alone on a CU and 1.75 for the two that share one;
-      * no launch is shorter than its weights' stream, 6.7 TB/s through 256-row tiles and 3.8 through 128-row ones.
-    Over 262 layers (8 to 64 experts, 768 to 4,096 wide, 512 to 8,900 inside, gated and not, 31 to 500 rows per expert, Zipf(0),
-    (0.8) and (1.0) loads) the chosen height is 0.4 % slower than the better one on average and 12 % at most, where the model
-    of training steps is 3.6 and 45 %, and 256 rows throughout 4.0 %. Both sides, 128 against 256 rows: 32 experts of 3,456 x
-    896 at 94 rows 227 against 170 us, 8 of 1,152 x 8,896 at 136 rows 254 against 198, 16 of 1,920 x 5,632 without a gate at
-    102 rows 203 against 230, 8 of 3,584 x 832 at 81 rows 64 against 88."""
+      * contractions that are no multiple of 64 run on the general kernel, 2.1 and 1.6 a step and no split (single launches with
+        256 / 32 tiles: 2,848 deep 121 / 97, 2,816 deep 92 / 59);
+      * a step of a 128 x 128 tile takes 0.9 alone on a CU, and 1.6 where the first CUs have two to 1.95 where all do (single
+        launches of 272 tiles 1.5 times those of 512 and 256: 117 against 138 and 70, 62 against 77 and 39);
+      * no launch is shorter than its weights' stream, 6.7 TB/s through 256-row tiles, 4.2 through the general kernel's and 3.8 through
+        128-row ones.
+    Over 370 layers (8 to 128 experts, 768 to 4,096 wide, 512 to 8,900 inside in steps of 32, gated and not, 31 to 500 rows per
+    expert, Zipf(0), (0.8) and (1.0) loads) the chosen height is 0.5 % slower than the better one on average, 256 rows throughout 6.2 %.
+    (With the general kernel's step as the other's, and 1.75 for a CU with two tiles, 0.8 %, and layers of 8 experts at 170 to 390
+    rows up to 36 %.) Both sides at Zipf(0.8), 128 against 256 rows: 32 experts of 3,456 x 896 at 94 rows 211 against 161 us, 8 of 1,152 x
+    8,896 at 136 rows 234 against 185, 128 of 2,048 x 1,408 at 60 rows 623 against 556; 8 of 3,584 x 832 at 81 rows 60 against 83,
+    8 of 1,408 x 3,552 at 168 rows 106 against 123, 8 of 1,664 x 1,088 without a gate at 392 rows 69 against 83."""
     cost = {128: 0.0, 256: 0.0}
     for height in cost:
         even = num_experts * -(-(num_rows + 24 * num_experts) // (height * num_experts))
         for tile_rows in (even, _zipf_tiles(num_rows, num_experts, height)):
             for columns, contraction, *_ in launches:
-                tiles, steps = tile_rows * -(-columns // height), -(-contraction // 64)
+                tiles, steps, general = tile_rows * -(-columns // height), -(-contraction // 64), contraction % 64 != 0
                 megabytes = num_experts * columns * contraction * 2 / 1e6
                 if height == 128:
                     pairs, left = tiles // 512, tiles % 512
-                    time = max(steps * (1.75 * pairs + (0.0 if left == 0 else 0.9 if left <= 256 else 1.75)), megabytes / 3.8)
+                    one_or_two = 0.0 if left == 0 else 0.9 if left <= 256 else 1.6 + 0.35 * (left - 256) / 256
+                    time = max(steps * (1.95 * pairs + one_or_two), megabytes / 3.8)
                 else:
                     rounds, left = tiles // 256, tiles % 256
-                    time = steps * (1.6 * rounds + ((1.15 + 0.45 * left / 256) if left else 0.0)) + 8.5 * -(-tiles // 256)
-                    if contraction % 64 == 0 and 0 < left <= 128 and steps - (part := -(-steps // min(4, 256 // left))) >= 40:
+                    few, all_cus = (1.6, 2.1) if general else (1.15, 1.6)
+                    time = steps * (all_cus * rounds + ((few + (all_cus - few) * left / 256) if left else 0.0)) + 8.5 * -(-tiles // 256)
+                    if not general and 0 < left <= 128 and steps - (part := -(-steps // min(4, 256 // left))) >= 40:
                         time = min(time, 1.6 * (steps * rounds + part) + 43.0)
-                    time = max(time, megabytes / 6.7)
+                    time = max(time, megabytes / (4.2 if general else 6.7))
                 cost[height] += time
     return 256 if cost[256] < cost[128] else 128
 
