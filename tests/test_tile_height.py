@@ -2,6 +2,7 @@
 expert-linear interface. Nothing is launched; traced calls end at the first real operator, which refuses the CPU tensor."""
 
 import math
+import sys
 
 import pytest
 import torch
@@ -199,6 +200,42 @@ def test_inference_layers_of_odd_widths_and_many_experts(experts, H, I, gated, r
     """Measured at Zipf(0), (0.8) and (1.0) loads: the other height is 4 to 41 % slower at each of them (10 to 35 % in the first four,
     whose 128-row launches give few CUs a second tile, or run c_proj on the general kernel)."""
     assert scattermoe.choose_align(rows * experts, experts, BF16, True, (H, I, gated)) == height
+
+
+@pytest.mark.parametrize("experts", [1, 2, 8, 60, 128, 512])
+def test_tiles_of_an_uneven_load(experts):
+    """The closed form against the experts' loads one by one: within 10 %, and the tile that one expert's rounding is worth."""
+    weights = [(e + 1) ** -0.8 for e in range(experts)]
+    assert abs(scattermoe._zipf_sum(experts) / sum(weights) - 1) < 0.006
+    for tiles in (0.1, 0.5, 1.3, 3.0, 10.0):  # per expert, on average
+        share = tiles * experts / sum(weights)
+        want = sum(max(1, math.ceil(share * w)) for w in weights)
+        assert abs(scattermoe._zipf_tiles(share, experts) - want) <= 0.1 * want + 1, tiles
+
+
+@pytest.mark.parametrize("inference", [True, False])
+def test_an_unseen_row_count_costs_no_loop_over_the_experts(inference):
+    """Lines of the rule that run for it: a server's row count differs from call to call, so that nothing is looked up."""
+    def lines(experts):
+        ran = 0
+
+        def trace(frame, event, arg):
+            nonlocal ran
+            if frame.f_code.co_filename != scattermoe.__file__:
+                return None
+            ran += event == "line"
+            return trace
+
+        scattermoe._layer_tiles_kept.cache_clear()
+        before = sys.gettrace()
+        sys.settrace(trace)
+        try:
+            scattermoe.choose_align(200 * experts, experts, BF16, inference, (2048, 1408, True))
+        finally:
+            sys.settrace(before)
+        return ran
+
+    assert lines(128) <= lines(8) + 10 <= 200
 
 
 @pytest.mark.parametrize("rows,layer,quantised", [(6, 16, 16), (7, 32, 32), (22, 32, 32), (23, 64, 64), (30, 64, 64), (31, 128, 64), (40, 128, 64), (41, 128, 256)])
