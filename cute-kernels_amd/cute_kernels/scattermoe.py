@@ -132,45 +132,6 @@ class ExpertSegments:
 SMALL_TILES, SMALL_TILES_E4M3 = ((6, 16), (22, 32), (30, 64)), ((6, 16), (22, 32), (40, 64))
 
 
-def _height_of_large_tiles(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
-    """256 or 128 rows for 16-bit training steps and single linears below 512 rows per expert, by the shorter sum of launches.
-    launches: (columns, contraction, whether the epilogue may split its last round, input gradient) of every grouped GEMM
-    that depends on the height. In us, with the constants fitted to measured layers:
-      * a 64-deep step of a 256 x 256 tile takes 1.7 on a CU; contractions that are no multiple of 64 run on the general
-        kernel, 1.6 with fewer loads in flight and no split; of a 128 x 128 tile 0.7, or 1.4 for the two that share a CU;
-      * splitting the last round of 256-row tiles costs 75, and happens where it takes 40 steps or more off that round (fitted
-        while the parts met through device-wide fences, and kept for training steps: the exchange takes 25 to 40 now, but with
-        60 already training steps of 8 x 2,048 x 4,096 without a gate at 192 rows got the slower height, 618 us for 546);
-      * no launch is shorter than its weights' stream, 4.2 TB/s, and the input gradient of 128-row tiles (or of such a
-        contraction) transposes the weights first.
-    Over 1,568 calls of 8 to 64 experts, 1,024 to 4,096 wide, 768 to 14,336 inside, gated and not, at 16 to 500 rows per expert
-    the chosen height is 0.5 % slower than the better one on average in training; always 256 1.6 %, always 128 22 %. (+ 24
-    rows: the load is not even.) Both sides, 128 against 256 rows, training: 8 experts of
-    4,096 x 14,336 at 8 / 96 / 400 rows 3,217 / 3,548 / 6,801 against 2,132 / 2,416 / 3,980 us; 32 of 1,024 x 1,024 304 / 335 /
-    622 against 488 / 494 / 419; 8 of 3,200 x 1,120 at 32 / 400 rows 312 / 568 against 413 / 483. The gated
-    epilogue splits its last round as well; the fit counts it whole, as it was when the layers were measured."""
-    cost = {}
-    for height in (128, 256):
-        tile_rows = num_experts * -(-(num_rows + 24 * num_experts) // (height * num_experts))
-        total = 0.0
-        for columns, contraction, splits, input_gradient in launches:
-            tiles, steps = tile_rows * -(-columns // height), -(-contraction // 64)
-            stream = num_experts * columns * contraction * 2 / 4.2e6
-            nt_only = height == 128 or contraction % 64 != 0
-            if height == 128:
-                pairs, left = tiles // 512, tiles % 512
-                time = steps * (1.4 * pairs + (0.0 if left == 0 else 0.7 if left <= 256 else 1.4))
-            elif nt_only:
-                time = 1.6 * steps * -(-tiles // 256)
-            elif splits and 0 < tiles % 256 <= 128 and steps - (part := -(-steps // min(4, 256 // (tiles % 256)))) >= 40:
-                time = 1.7 * (steps * (tiles // 256) + part) + 75.0
-            else:
-                time = 1.7 * steps * -(-tiles // 256)
-            total += max(time, stream) + (2 * stream if input_gradient and nt_only else 0.0)
-        cost[height] = total
-    return 256 if cost[256] < cost[128] else 128
-
-
 def _zipf_sum(num_experts: int) -> float:
     """sum of e ** -0.8 over e = 1 .. num_experts by Euler and Maclaurin, 0.5 % off for one expert and less beyond; -4.4375 is zeta(0.8)"""
     return 5.0 * num_experts**0.2 - 4.4375 + 0.5 * num_experts**-0.8 - num_experts**-1.8 / 15
@@ -183,41 +144,52 @@ def _zipf_tiles(share: float, num_experts: int) -> int:
     return num_experts - several + (int(share * _zipf_sum(several) + 0.5 * several + 0.5) if several else 0)
 
 
-def _height_in_inference(num_rows: int, num_experts: int, launches: tuple[tuple[int, int, bool, bool], ...]) -> int:
-    """The same choice for a layer's forward alone, by a finer model: the sum of its launches at an even load and at a Zipf(0.8) one
-    together, since the more uneven the load, the fewer experts fit one tile of 128 rows. In us:
+def _height_of_large_tiles(num_rows: int, num_experts: int, inference: bool, launches: tuple[tuple[int, int, bool], ...]) -> int:
+    """256 or 128 rows for 16-bit layers and single linears below 512 rows per expert, by the shorter sum of launches.
+    launches: (columns, contraction, input gradient) of every grouped GEMM that depends on the height. An inference layer is
+    judged at an even load and at a Zipf(0.8) one together, since the more uneven the load, the fewer experts fit one tile of 128
+    rows; a training step, whose heights lie further apart, at the Zipf(0.8) one alone. In us:
       * a round of 256 x 256 tiles takes 1.6 a 64-deep step with all CUs at work, down to 1.15 with few (the chip's power is
         shared by fewer), and 8.5 for its start and stores; a split last round takes an equal part of the steps and 43 for
         the exchange of the parts, and happens where it takes 40 steps or more off that round;
       * contractions that are no multiple of 64 run on the general kernel, 2.1 and 1.6 a step and no split (single launches with
         256 / 32 tiles: 2,848 deep 121 / 97, 2,816 deep 92 / 59);
       * a step of a 128 x 128 tile takes 0.9 alone on a CU, and 1.6 where the first CUs have two to 1.95 where all do (single
-        launches of 272 tiles 1.5 times those of 512 and 256: 117 against 138 and 70, 62 against 77 and 39);
+        launches with 256, 272 and 512 tiles: 4,096 deep 70, 117 and 138, 2,048 deep 39, 62 and 77);
       * no launch is shorter than its weights' stream, 6.7 TB/s through 256-row tiles, 4.2 through the general kernel's and 3.8 through
-        128-row ones.
-    Over 370 layers (8 to 128 experts, 768 to 4,096 wide, 512 to 8,900 inside in steps of 32, gated and not, 31 to 500 rows per
-    expert, Zipf(0), (0.8) and (1.0) loads) the chosen height is 0.5 % slower than the better one on average, 256 rows throughout 6.2 %.
-    (With the general kernel's step as the other's, and 1.75 for a CU with two tiles, 0.8 %, and layers of 8 experts at 170 to 390
-    rows up to 36 %.) Both sides at Zipf(0.8), 128 against 256 rows: 32 experts of 3,456 x 896 at 94 rows 211 against 161 us, 8 of 1,152 x
-    8,896 at 136 rows 234 against 185, 128 of 2,048 x 1,408 at 60 rows 623 against 556; 8 of 3,584 x 832 at 81 rows 60 against 83,
-    8 of 1,408 x 3,552 at 168 rows 106 against 123, 8 of 1,664 x 1,088 without a gate at 392 rows 69 against 83."""
+        128-row ones; the input gradient of 128-row tiles, or of the general kernel, transposes the weights first, at 4.2.
+    Over 370 inference layers (8 to 128 experts, 768 to 4,096 wide, 512 to 8,900 inside in steps of 32, gated and not, 31 to 500 rows
+    per expert, Zipf(0), (0.8) and (1.0) loads) the chosen height is 0.5 % slower than the better one on average, 256 rows throughout
+    6.2 %. (With the general kernel's step as the other's, and 1.75 for a CU with two tiles, 0.8 %, and layers of 8 experts at 170 to
+    390 rows up to 36 %.) Both sides at Zipf(0.8), 128 against 256 rows: 32 experts of 3,456 x 896 at 94 rows 211 against 161 us, 8 of
+    1,152 x 8,896 at 136 rows 234 against 185, 128 of 2,048 x 1,408 at 60 rows 623 against 556; 8 of 3,584 x 832 at 81 rows 60 against
+    83, 8 of 1,408 x 3,552 at 168 rows 106 against 123, 8 of 1,664 x 1,088 without a gate at 392 rows 69 against 83.
+    Over 350 training steps of such layers from 12 rows on it is 0.03 % slower on average and 4.5 % at most, 256 rows throughout 1.0
+    and 47 %. (By the kernels whose parts met through device-wide fences, 75 us, and with a gated epilogue that did not split: 1.5 and
+    51 %.) Both sides: 8 of 2,048 x 4,096 without a gate at 160 / 192 / 230 rows 498 / 510 / 617 against 401 / 412 / 461, 16 of 1,024 x
+    2,016 at 16 / 64 rows 307 / 359 against 276 / 312, 8 of 1,024 x 3,840 at 40 rows 363 against 275, 8 of 3,200 x 1,120 at 400 rows 543
+    against 419; at 32 rows 299 against 306, 8 of 1,024 x 1,024 at 96 / 300 rows 162 / 186 against 180 / 200."""
     even_rows, zipf_rows = num_rows / num_experts + 24, num_rows / _zipf_sum(num_experts)
     cost = {}
     for height in (128, 256):
-        tile_rows = (num_experts * math.ceil(even_rows / height), _zipf_tiles(zipf_rows / height, num_experts))
+        loads = [_zipf_tiles(zipf_rows / height, num_experts)]
+        if inference:
+            loads.append(num_experts * math.ceil(even_rows / height))
         total = 0.0
-        for columns, contraction, *_ in launches:
+        for columns, contraction, input_gradient in launches:
             column_tiles, steps, general = -(-columns // height), -(-contraction // 64), contraction % 64 != 0
             megabytes = num_experts * columns * contraction * 2e-6
+            if input_gradient and (height == 128 or general):
+                total += 2 * megabytes / 4.2
             if height == 128:
                 stream = megabytes / 3.8
-                for rows in tile_rows:
+                for rows in loads:
                     pairs, left = divmod(rows * column_tiles, 512)
                     time = steps * (1.95 * pairs + (0.0 if left == 0 else 0.9 if left <= 256 else 1.25 + left * (0.35 / 256)))
                     total += time if time > stream else stream
                 continue
             few, all_cus, stream = (1.6, 2.1, megabytes / 4.2) if general else (1.15, 1.6, megabytes / 6.7)
-            for rows in tile_rows:
+            for rows in loads:
                 rounds, left = divmod(rows * column_tiles, 256)
                 time = (steps * all_cus + 8.5) * rounds
                 if left:
@@ -235,11 +207,11 @@ def _plain_tiles(num_rows: int, num_experts: int) -> int:
 
 
 def _large_tiles(
-    num_rows: int, num_experts: int, dtype: torch.dtype | None, launches: tuple[tuple[int, int, bool, bool], ...], many: bool
+    num_rows: int, num_experts: int, dtype: torch.dtype | None, inference: bool, launches: tuple[tuple[int, int, bool], ...], many: bool
 ) -> int:
     if many or dtype is torch.float32 or num_rows >= 512 * num_experts:  # fp32 GEMMs run on 64-row tiles either way
         return _plain_tiles(num_rows, num_experts)
-    return _height_of_large_tiles(num_rows, num_experts, launches)
+    return _height_of_large_tiles(num_rows, num_experts, inference, launches)
 
 
 def _layer_tiles(
@@ -255,12 +227,10 @@ def _layer_tiles(
         return 256
     hidden, inter, gated = widths
     c_fc = 2 * inter if gated else inter
-    launches = ((c_fc, hidden, not gated, False), (hidden, inter, True, False))
+    launches = ((c_fc, hidden, False), (hidden, inter, False))
     if not inference:
-        launches += ((inter, hidden, True, True), (hidden, c_fc, True, True))
-    if inference and not many and num_rows < 512 * num_experts:
-        return _height_in_inference(num_rows, num_experts, launches)
-    return _large_tiles(num_rows, num_experts, dtype, launches, many)
+        launches += ((inter, hidden, True), (hidden, c_fc, True))
+    return _large_tiles(num_rows, num_experts, dtype, inference, launches, many)
 
 
 _large_tiles_kept, _layer_tiles_kept = functools.lru_cache(4096)(_large_tiles), functools.lru_cache(4096)(_layer_tiles)
@@ -300,7 +270,7 @@ def choose_align(
     A caller that says no more than the sizes, and every fp32 layer: 256 rows from 512 rows per expert on, else 128, which
     keeps the padding small.
     widths: (hidden, intermediate, whether the activation is the gated epilogue's) of a 16-bit layer. Below 512 rows per
-    expert its GEMMs decide, those of a training step (_height_of_large_tiles) or of the forward alone (_height_in_inference).
+    expert its GEMMs decide, those of a training step or of the forward alone (_height_of_large_tiles).
     inference (no gradient is asked for): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the
     stream of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights
     fetched once per tile, from L2 at best, so the height follows the load. 160 bf16 layers of 8 to 128 experts at 3 to 80 rows
@@ -719,10 +689,10 @@ def scattered_experts(
         gates_in = gates
         gates = gates.to(inputs.dtype)
     E, N, K = (plain_size(n) for n in w.shape)
-    launches = ((N, K, True, False),)
-    if torch.is_grad_enabled() and inputs.requires_grad:
-        launches += ((K, N, True, True),)
-    align = _height(_large_tiles, _large_tiles_kept, plain_size(sorted_expert_idxs.numel()), E, inputs.dtype, launches)
+    launches, forward_alone = ((N, K, False),), not (torch.is_grad_enabled() and inputs.requires_grad)
+    if not forward_alone:
+        launches += ((K, N, True),)
+    align = _height(_large_tiles, _large_tiles_kept, plain_size(sorted_expert_idxs.numel()), E, inputs.dtype, forward_alone, launches)
     if is_tracing():
         out = _ops.scattered_experts(
             inputs, w, gates, bias, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, grouped_in, grouped_out, align
