@@ -156,6 +156,9 @@ struct Mfma16<f16_t> {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
   }
 };
+// The lane's number, counted anew: what an epilogue derives from it needs no register while the products are under way.
+__device__ inline int lane_again() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
 // After the last run_acc, before anything else reads the accumulators: longer than any MFMA's result latency. The wait
 // alone is not enough: nothing ties the compiler's own reads of the accumulators (v_accvgpr_read, spills) to it, and the
 // scheduler is free to hoist them above the wait, right behind the MFMA that writes them (it did: a few stale values

@@ -619,7 +619,9 @@ __global__ __launch_bounds__(64 * 2 * WGM) void grouped_gemm_line_kernel(const G
   }
   if constexpr (CK_STAMP != 0) st_end = clock64();
   auto store_out = [](void* p, const vec16& v) { store16(p, v); };
-  const int lrow = lane & 15, lg = lane >> 4;
+  // counted anew: beside the parts of a split there is no register for it
+  const int epilogue_lane = lane_again();
+  const int lrow = epilogue_lane & 15, lg = epilogue_lane >> 4;
   const bool odd_group = (lg & 1) != 0;
   const T kZero = Elem<T>::down(0.f);
   // 8 consecutive columns for this lane out of the column blocks j (packed pairs p0, p1) and j + 1 (q0, q1) of one row block

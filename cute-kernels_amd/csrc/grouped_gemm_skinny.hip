@@ -146,6 +146,14 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
   auto fetch = [&](Set& s, int step) __attribute__((always_inline)) {
     const char* wp = w_base + (int64_t)step * kStepBytes;
     const char* ap = a_base + (int64_t)step * kStepBytes;
+    // As 32-bit values that it knows nothing of, the offsets stay one register each, behind a scalar base. Otherwise the compiler
+    // widens them ahead of the loop, to pairs of which one is zero, and has 2 others in scratch for it.
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) asm("" : "+v"(w_off[j][h]));
+#pragma unroll
+    for (int i = 0; i < MB; ++i) asm("" : "+v"(a_off[i]));
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -204,10 +212,11 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
 
   // ---- the four partial tiles meet in LDS; the weight operand is the MFMA's first, so a lane holds 4 consecutive output
   // columns (16 j + 4 (lane / 16) ..) of tile row 16 i + lane % 16
+  const int out_lane = lane_again(), out_row = out_lane & 15, out_q = out_lane >> 4;
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) red[wave * MB * NB + i * NB + j][lane] = acc[i][j];
+    for (int j = 0; j < NB; ++j) red[wave * MB * NB + i * NB + j][out_lane] = acc[i][j];
   __syncthreads();
   auto total_of = [&](int b, int l) {
     f32x4 v = red[b][l];
@@ -218,14 +227,14 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
   constexpr int kItems = MB * NH * kWave;
   constexpr bool kFp8 = std::is_same_v<TI, fp8_t>;
 #pragma unroll
-  for (int it = tid; it < kItems; it += kNT) {
+  for (int it = wave * kWave + out_lane; it < kItems; it += kNT) {
     const int b = it / kWave, i = b / NH, j = b % NH;  // lane of the item: this thread's (kNT is a multiple of kWave)
-    const int p = m0 + i * 16 + lrow;
-    const int n = n0 + j * 16 + 4 * lq;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
-    const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N) && (!kPair || lq < 2);
-    f32x4 v = total_of(i * NB + j, lane);
+    const int p = m0 + i * 16 + out_row;
+    const int n = n0 + j * 16 + 4 * out_q;  // first of 4 columns; widths are multiples of 8, so all 4 exist or none
+    const bool inside = p < valid_end && n < (MODE == kSwiglu ? prm.I : prm.N) && (!kPair || out_q < 2);
+    f32x4 v = total_of(i * NB + j, out_lane);
     [[maybe_unused]] f32x4 g = v;
-    if constexpr (MODE == kSwiglu) g = kPair ? total_of(i, lane ^ 32) : total_of(i * NB + j + NH, lane);
+    if constexpr (MODE == kSwiglu) g = kPair ? total_of(i, out_lane ^ 32) : total_of(i * NB + j + NH, out_lane);
     if (!inside) continue;
     if constexpr (kFp8) {
       const float rs = prm.a_scale[prm.a_gather_div > 0 ? prm.row_slot[p] / prm.a_gather_div : p];
@@ -283,7 +292,7 @@ __device__ __attribute__((always_inline)) inline void skinny_tile(const GemmPara
 // in all (4 to 128 experts, 4 MB to 2.1 GB) 2 to 3 % less time on average; 3 % of a 10 us launch more for the longer program.
 constexpr int kCus = 256;
 
-// Workgroups per compute unit: three of 32-row tiles. Left to itself the compiler takes 174 to 178 registers for e4m3 operands, for
+// Workgroups per compute unit: three of 32-row tiles. Left to itself the compiler takes 174 registers for e4m3 operands, for
 // which there is room twice: 128 experts of 4,096 x 1,536 with 8 rows on average, Zipf(0.8), 150 us and now 133, 64 gated ones of 11,264
 // x 1,024 176 and 156.
 template <typename TI, typename TO, int MODE, int MB, int NB, bool LINES>
