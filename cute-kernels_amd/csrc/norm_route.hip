@@ -335,10 +335,10 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
       for (int i = 0; i < 4; ++i) ss = dot2_acc<T>(xa[s].w[i], ss);
     ss = lanes_total(ss, add);
     if (lane < ROWS) red[0][wave][r] = ss;
-    if (tid < 64 * S) {  // a weight of one changes no bit; zero past the end of the rows
-      if (norm_w == nullptr || 8 * tid >= H) {
+    if (tid < 64 * S) {  // a weight of one changes no bit
+      if (norm_w == nullptr) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) nw.e[i] = Elem<T>::down(8 * tid >= H ? 0.f : 1.f);
+        for (int i = 0; i < 8; ++i) nw.e[i] = Elem<T>::down(1.f);
       }
       *reinterpret_cast<vec16*>(&w_lds[8 * tid]) = nw.v;
     }
@@ -355,6 +355,11 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
       for (int i = 0; i < 4; ++i)
         xa[s].w[i] = pack_pair<T>(Elem<T>::up(p.e[2 * i]) * rs * Elem<T>::up(w.e[2 * i]),
                                   Elem<T>::up(p.e[2 * i + 1]) * rs * Elem<T>::up(w.e[2 * i + 1]));
+    }
+    if (!whole) {  // zero again: of a row whose squares vanish the reciprocal root may be infinite (eps = 0)
+#pragma unroll
+      for (int s = 0; s < XS; ++s)
+        if (piece(s * FOLD + fold) >= pieces) xa[s] = zero16();
     }
     if (blockIdx.y == 0) {
 #pragma unroll

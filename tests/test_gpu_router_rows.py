@@ -61,6 +61,19 @@ def test_rows_of_a_workgroup(B, H, E):
     assert bool((torch.isfinite(logits).all(0) == (torch.arange(E, device=DEV) != E // 2)).all()) and bool(torch.isinf(logits[:, E // 2]).all())
 
 
+# 4, 8 and 16 rows a workgroup, at whole and ragged widths
+@pytest.mark.parametrize("B,H,E", [(4, 1088, 8), (5, 2048, 8), (600, 1056, 16), (8, 96, 8), (9, 1024, 8), (2050, 992, 8), (2050, 2080, 16)])
+def test_rows_whose_squares_vanish(B, H, E):
+    """2 ** -80 squared is no fp32 number: without eps the row's reciprocal root is infinite, and so are its values, its logits and its
+    e4m3 scale. No NaN out of the columns that a ragged width leaves over."""
+    x, w = torch.full((B, H), 2.0**-80, device=DEV, dtype=torch.bfloat16), torch.full((E, H), 0.5, device=DEV, dtype=torch.bfloat16)
+    x[1] = 1.0
+    y, logits, _, scale = rmsnorm_route.rmsnorm_route_cute(x, None, w, 0.0, quantize=True)
+    ordinary = torch.arange(B, device=DEV) == 1
+    for t in (y, logits, scale[:, None]):
+        assert bool((torch.isinf(t) == ~ordinary[:, None]).all()) and not bool(torch.isnan(t).any())
+
+
 def test_sizes_beyond_one_workgroup_per_compute_unit_keep_their_routes():
     x, w, _ = _inputs(257, 512, 256, torch.bfloat16)
     take = _C.host().router_rows_take
