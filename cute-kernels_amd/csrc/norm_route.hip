@@ -259,19 +259,21 @@ __global__ __launch_bounds__(kNT, 3) void rmsnorm_route_kernel(const T* __restri
 // weight) go out at once, and the 16 partial blocks are added through LDS in a fixed order. The workgroups of a row block all
 // normalise it; the first writes y and rstd, the last the e4m3 rows. The gate weight is read as stored: the channel conflicts of its
 // row pitch do not show at this size.
-// Rows of a workgroup: the fewest whose workgroups are no more than the compute units, since a unit does their norms in turn. With
-// 16 / 8 / 4 in a replayed graph: 64 rows x 2,048, 64 experts 7.8 / 5.9 / 5.0 us; 128 x 4,096, 128 experts with e4m3 rows 15.3 /
-// 10.6 / 8.6, 256 of them 15.1 / 10.7 / 13.3 and 512 15.6 / 18.1 / 22.8; without the norm 1,024 x 4,096 and 8 experts 7.4 / 6.1 /
-// 5.4, 2,000 rows 7.8 / 6.3 / 8.4. (With loads that waited for one another behind conditions, 16 rows took 7.7, 16.8, 16.5 and
-// 17.1 us; in separate kernels the 128 rows take norm 4.5, library product 14.8, quantiser 4.4.) More workgroups of 16 rows than
-// compute units, and the kernels that read the gate weight once per more rows win (1,024 x 4,096, 128 experts).
+// Rows of a workgroup: the fewest of 16, 8 and (beyond 1,024 columns, where a wave has four pieces to fold) 4 whose workgroups are no
+// more than the compute units, since a unit does their norms in turn. With 16 / 8 / 4 in a replayed graph: 64 rows x 2,048, 64
+// experts 7.8 / 5.9 / 5.0 us; 128 x 4,096, 128 experts with e4m3 rows 15.3 / 10.6 / 8.6, 256 of them 15.1 / 10.7 / 13.3 and 512 15.6
+// / 18.1 / 22.8; without the norm 1,024 x 4,096 and 8 experts 7.4 / 6.1 / 5.4, 2,000 rows 7.8 / 6.3 / 8.4. A logit's sum is folded
+// accordingly: its last bits depend on how many rows there are. (With loads that waited for one another behind conditions, 16 rows
+// took 7.7, 16.8, 16.5 and 17.1 us; 16 rows x 256 columns without the norm 2.1, and 2.2 now. In separate kernels the 128 rows take
+// norm 4.5, library product 14.8, quantiser 4.4.) More workgroups of 16 rows than compute units, and the kernels that read the
+// gate weight once per more rows win (1,024 x 4,096, 128 experts).
 constexpr int kRowWaves = 16;
 constexpr int kRowBlocks = 256;  // workgroups up to which fewer rows in each pay: one per compute unit
 
-// S: 32-column pieces per wave, H <= 512 S and H % 32 == 0. NORM: rmsnorm(x) goes to the router (norm_w may be NULL), else x
-// itself. ROWS: 16, or 8 or 4 with FOLD = 2 or 4 pieces of a row side by side in the 16 columns of an operand: each then meets FOLD
-// pieces of the gate weight in products of their own, and of the FOLD blocks a column counts in the one of its piece.
-template <typename T, int S, bool NORM, int ROWS>
+// S: 32-column pieces per wave, H <= 512 S and H % 32 == 0; WHOLE: H == 512 S. NORM: rmsnorm(x) goes to the router (norm_w may be
+// NULL), else x itself. ROWS: 16, or 8 or 4 with FOLD = 2 or 4 pieces of a row side by side in the 16 columns of an operand: each then
+// meets FOLD pieces of the gate weight in products of their own, and of the FOLD blocks a column counts in the one of its piece.
+template <typename T, int S, bool NORM, int ROWS, bool WHOLE>
 __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T* __restrict__ x, const T* __restrict__ norm_w,
                                                                          const T* __restrict__ gate_w, float eps, int64_t B,
                                                                          int H, int E, T* __restrict__ y,
@@ -289,30 +291,48 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
   const int e0 = blockIdx.y * 16;
   const bool row_ok = row < B;
   const int pieces = H / 32;
-  const bool whole = pieces == 16 * S;  // no piece past the end of the rows
   auto piece = [&](int t) { return (t / 2 * kRowWaves + wave) * 2 + t % 2; };  // pairs: the halves of 128-byte lines
-  auto at = [&](int t) { return 32 * min(piece(t), pieces - 1); };             // pieces past the end re-read the last one
-  // rows past the end re-read the last row, experts past the end the last expert
-  const T* xb = x + row0 * H;
-  const uint32_t x_lane = (uint32_t)min((int64_t)r, B - 1 - row0) * H + 8 * q;
-  const T* gb = gate_w + (int64_t)e0 * H;
-  const uint32_t g_lane = (uint32_t)min(col, E - 1 - e0) * H + 8 * q;
+  // Rows past the end re-read the last row, experts past the end the last expert. A piece past the end of the rows lies outside of
+  // the buffer: such a load is as unconditional as the others, but asks memory for nothing and returns zeros. (Re-reading the last
+  // piece instead took 16 rows x 256 without the norm from 2.1 to 2.8 us, 1,000 x 1,536 over 64 experts from 4.7 to 5.7, now 2.2 and
+  // 5.0. WHOLE rows have no such piece, and plain loads: 64 x 4,096 with the norm 5.8 us, of buffers 6.2.)
+  constexpr int kOutside = 1 << 30;
+  auto rows_of = [](const T* p, int64_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, (int)bytes, 0x00027000); };
+  const int x_left = (int)min((int64_t)ROWS, B - row0), g_left = min(16, E - e0), pitch = H * (int)sizeof(T);
+  const T *x0 = x + row0 * H, *g0 = gate_w + (int64_t)e0 * H;
+  const auto xb = rows_of(x0, (int64_t)x_left * pitch), gb = rows_of(g0, (int64_t)g_left * pitch);
+  auto load = [&](const T* base, const auto& buffer, uint32_t lane_bytes, int at) {
+    if constexpr (WHOLE) return load16(reinterpret_cast<const char*>(base) + (lane_bytes + (uint32_t)(64 * at)));
+    const auto u = __builtin_amdgcn_raw_buffer_load_b128(buffer, at < pieces ? (int)lane_bytes + 64 * at : kOutside, 0, 0);
+    vec16 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v.w[i] = u[i];
+    return v;
+  };
+  const uint32_t x_lane = (uint32_t)(min(r, x_left - 1) * pitch + 16 * q), g_lane = (uint32_t)(min(col, g_left - 1) * pitch + 16 * q);
 
-  // the order of the loads is the order they are waited for in, and none hangs on a condition: the wait for x leaves the others
-  // in flight
+  // the order of the loads is the order they are waited for in, and none hangs on a condition of its own: the wait for x leaves the
+  // others in flight. Of rows of fewer than 1,024 columns some waves have no piece (256 columns with the norm 3.1 us, with loads
+  // outside of the buffer 3.4).
   vec16 xa[XS], g[S];
-#pragma unroll
-  for (int s = 0; s < XS; ++s) xa[s] = load16(xb + (x_lane + (uint32_t)at(s * FOLD + fold)));
   Pack16<T> nw;
-  if constexpr (NORM) nw.v = load16((norm_w != nullptr ? norm_w : gate_w) + min(8 * tid, H - 8));
+  auto load_norm_weight = [&]() {
+    if constexpr (NORM) nw.v = load16((norm_w != nullptr ? norm_w : gate_w) + min(8 * tid, H - 8));
+  };
+  if (!WHOLE && S == 2 && 2 * wave >= pieces) {
+    load_norm_weight();
 #pragma unroll
-  for (int t = 0; t < S; ++t) g[t] = load16(gb + at(t) + g_lane);
-  __builtin_amdgcn_sched_barrier(0);
-  if (!whole) {
+    for (int s = 0; s < XS; ++s) xa[s] = zero16();
 #pragma unroll
-    for (int s = 0; s < XS; ++s)
-      if (piece(s * FOLD + fold) >= pieces) xa[s] = zero16();
+    for (int t = 0; t < S; ++t) g[t] = zero16();
+  } else {
+#pragma unroll
+    for (int s = 0; s < XS; ++s) xa[s] = load(x0, xb, x_lane, piece(s * FOLD + fold));
+    load_norm_weight();
+#pragma unroll
+    for (int t = 0; t < S; ++t) g[t] = load(g0, gb, g_lane, piece(t));
   }
+  __builtin_amdgcn_sched_barrier(0);
 
   auto row_total = [&](float (&of)[kRowWaves][ROWS], auto&& join) {  // over the waves, in order
     float total = of[0][r];
@@ -356,7 +376,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
         xa[s].w[i] = pack_pair<T>(Elem<T>::up(p.e[2 * i]) * rs * Elem<T>::up(w.e[2 * i]),
                                   Elem<T>::up(p.e[2 * i + 1]) * rs * Elem<T>::up(w.e[2 * i + 1]));
     }
-    if (!whole) {  // zero again: of a row whose squares vanish the reciprocal root may be infinite (eps = 0)
+    if constexpr (!WHOLE) {  // zero again: of a row whose squares vanish the reciprocal root may be infinite (eps = 0)
 #pragma unroll
       for (int s = 0; s < XS; ++s)
         if (piece(s * FOLD + fold) >= pieces) xa[s] = zero16();
@@ -394,11 +414,6 @@ __global__ __launch_bounds__(kRowWaves * kWave) void router_rows_kernel(const T*
     }
   }
 
-  if (!whole) {  // x is zero there, but what was read again may be infinite
-#pragma unroll
-    for (int t = 0; t < S; ++t)
-      if (piece(t) >= pieces) g[t] = zero16();
-  }
   auto frag = [](const vec16& v) { return __builtin_bit_cast(typename Mfma16<T>::frag, v); };
   f32x4 acc[FOLD] = {};
 #pragma unroll
@@ -451,15 +466,20 @@ extern "C" int ck_router_rows(const void* x, const void* norm_weight, const void
   CK_REQUIRE(row_blocks < (int64_t)0x7fffffff, "%s: grid too large", name);
   const dim3 grid((unsigned)row_blocks, (unsigned)expert_blocks);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CK_RR_N(S, NORM, ROWS)                                                                                             \
-  hipLaunchKernelGGL((router_rows_kernel<scalar_t, S, NORM, ROWS>), grid, dim3(kRowWaves * kWave), 0, s,                   \
+#define CK_RR_N(S, NORM, ROWS, WHOLE)                                                                                      \
+  hipLaunchKernelGGL((router_rows_kernel<scalar_t, S, NORM, ROWS, WHOLE>), grid, dim3(kRowWaves * kWave), 0, s,            \
                      static_cast<const scalar_t*>(x), static_cast<const scalar_t*>(norm_weight),                           \
                      static_cast<const scalar_t*>(gate_weight), eps, B, (int)H, (int)E, static_cast<scalar_t*>(y), rstd,   \
                      static_cast<scalar_t*>(logits), static_cast<uint8_t*>(x8), scale8)
+#define CK_RR_W(S, NORM, ROWS)                              \
+  do {                                                      \
+    if (H == 512 * S) CK_RR_N(S, NORM, ROWS, true);         \
+    else CK_RR_N(S, NORM, ROWS, false);                     \
+  } while (0)
 #define CK_RR(S, ROWS)                     \
   do {                                     \
-    if (normalize) CK_RR_N(S, true, ROWS); \
-    else CK_RR_N(S, false, ROWS);          \
+    if (normalize) CK_RR_W(S, true, ROWS); \
+    else CK_RR_W(S, false, ROWS);          \
   } while (0)
   CK_DISPATCH_HALF(dtype, name, {
     if (H <= 1024) {
@@ -476,6 +496,7 @@ extern "C" int ck_router_rows(const void* x, const void* norm_weight, const void
     }
   });
 #undef CK_RR
+#undef CK_RR_W
 #undef CK_RR_N
   CK_CHECK_LAUNCH(name);
   return CK_OK;

@@ -22,7 +22,8 @@ MAX_EXPERTS, MAX_HIDDEN, HIDDEN_STEP = 128, 4096, 512
 
 def router_rows_fit(x: torch.Tensor, gate_weight: torch.Tensor, norm_weight: torch.Tensor | None = None) -> bool:
     """Whether few enough 16-bit rows meet few enough experts for the kernel that gives 4 to 16 rows x 16 experts a workgroup of
-    their own (ck_router_rows, with or without the norm). A linear layer casts under autocast. The answer is the same with
+    their own (ck_router_rows, with or without the norm; the last bits of a token's logits follow how many rows share a
+    workgroup, and so the batch). A linear layer casts under autocast. The answer is the same with
     gradients and without: a segment that is checkpointed by running it twice selects the same experts both times."""
     return not is_tracing() and not torch.is_autocast_enabled("cuda") and _C.host().router_rows_take(x, gate_weight, norm_weight)
 

@@ -47,11 +47,12 @@ def test_logits_and_norm(B, H, E, dtype):
         assert torch.equal(x8.view(torch.uint8), q.view(torch.uint8)) and torch.equal(scale, s)
 
 
-# 4, 8 or 16 rows a workgroup, by how many there are: edges of each, at whole and ragged widths of each instantiation
+# 4, 8 or 16 rows a workgroup, by how many there are: edges of each, at whole and ragged widths of each instantiation; widths that
+# leave whole waves, or half of their pieces, without columns
 @pytest.mark.parametrize(
     "B,H,E",
     [(4, 2048, 16), (5, 3072, 33), (500, 1088, 17), (8, 32, 16), (9, 1024, 8), (515, 2016, 32), (1023, 4096, 17), (2049, 992, 1),
-     (1030, 2048, 20), (1033, 4064, 32)],
+     (1030, 2048, 20), (1033, 4064, 32), (3, 256, 8), (17, 512, 33), (2100, 288, 16), (6, 1536, 16), (1000, 1536, 64), (7, 3072, 8)],
 )
 def test_rows_of_a_workgroup(B, H, E):
     test_logits_and_norm(B, H, E, torch.bfloat16)
