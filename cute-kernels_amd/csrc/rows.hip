@@ -436,10 +436,13 @@ __global__ __launch_bounds__(kBlock) void expert_bias_grad_kernel(const T* __res
   }
 }
 
-// The same for rows of whole 16-byte pieces: a lane sums one piece (8 columns of 16 bits), a wave reads 4 rows x 256 bytes with one
-// load, eight loads in flight, and the 8 waves of a block cover 128 columns. Latency and the number of loads bound it, not
-// memory: one value a lane took 16.3 us for 6,000 f16 rows of 4,096 over 16 experts and 12.8 for
-// 1,536, this 13.7 and 7.6 (16 waves a block the same).
+// The same for rows of whole 16-byte pieces, and many of them per expert: a lane sums one piece (8 columns of 16 bits), a wave reads
+// 4 rows x 256 bytes with one load, eight loads in flight, and the 8 waves of a block cover 128 columns. Latency and the number of
+// loads bound it, not memory: one value a lane took 16.3 us for 6,000 f16 rows of 4,096 over 16 experts and 12.8 for 1,536, this 13.7
+// and 7.6 (16 waves a block the same). Eight waves of eight loads are too many for few rows: of bf16 64 experts of 14,336 columns at 8 /
+// 64 / 192 rows each take 20.4 / 27.3 / 61.6 us and one value a lane 7.1 / 18.4 / 67.3, 8 of 1,536 at 64 / 256 / 320 rows 3.4 / 3.6 / 4.1
+// and 2.5 / 3.5 / 3.9, 16 at 375 rows 4.4 and 5.0; of fp32 64 of 1,536 at 64 rows 5.3 and 3.2, 8 at 256 rows 3.3 and 3.4. So the line is
+// 350 rows per expert on average, 192 of 32 bits and of sums as many as the 64 x 14,336, which memory bounds.
 constexpr int kBiasBlock = 512, kBiasLanes = 16;
 template <typename T>
 __global__ __launch_bounds__(kBiasBlock) void expert_bias_grad_wide_kernel(const T* __restrict__ d_y, int N,
@@ -720,9 +723,12 @@ extern "C" int ck_expert_bias_grad(const void* d_y, int32_t N, const ck_segments
   CK_REQUIRE(d_bias != nullptr && (seg->max_rows == 0 || d_y != nullptr), "%s: NULL argument", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)ceil_div(N, kWave), (unsigned)seg->num_experts);
+  // rows in the padded layout, to half a tile (ck_sort_max_rows); where the line lies: at the wide kernel
+  const int64_t rows = seg->max_rows - (int64_t)seg->num_experts * (seg->align - 1) - seg->align / 2;
   CK_DISPATCH_FLOAT(dtype, name, {
     constexpr int P = Elem<scalar_t>::per16;
-    if (N % P == 0 && aligned16(d_y)) {
+    const int64_t many = (P == 8 && (int64_t)seg->num_experts * N < (1 << 19) ? 350 : 192) * (int64_t)seg->num_experts;
+    if (N % P == 0 && aligned16(d_y) && rows >= many) {
       hipLaunchKernelGGL((expert_bias_grad_wide_kernel<scalar_t>), dim3((unsigned)ceil_div(N, kBiasLanes * P), (unsigned)seg->num_experts),
                          dim3(kBiasBlock), 0, s, static_cast<const scalar_t*>(d_y), (int)N, seg->seg_starts, seg->counts,
                          static_cast<scalar_t*>(d_bias));

@@ -78,3 +78,23 @@ def test_expert_bias_gradient_by_pieces_and_by_elements(device, dtype, N, offset
     _C.check(_C.lib().ck_expert_bias_grad(_C.ptr(on_gpu), N, ctypes.byref(cs), _C.ptr(d_bias), _C.dtype_code(dtype), _C.stream()))
     for e, c in enumerate(COUNTS):
         assert torch.equal(d_bias[e].cpu(), d_y[starts[e] : starts[e] + c].double().sum(0).to(dtype)), e
+
+
+# which of the two kernels sums goes by the rows per expert, 350 on average (192 of 32 bits or of many sums): both sides, one expert with none and one with
+# nearly all rows
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("total", [3 * 64, 3 * 150, 3 * 250, 3 * 340, 3 * 351, 3 * 700])
+@pytest.mark.parametrize("N", [8, 136, 1000])
+def test_expert_bias_gradient_of_few_and_many_rows(device, dtype, total, N):
+    counts = [5, 0, total - 5]
+    seg = cute_kernels.sort_by_expert(torch.tensor([0] * 5 + [2] * (total - 5), dtype=torch.int32, device=device), 3, 128)
+    g = torch.Generator().manual_seed(N + total)
+    d_y = torch.full((seg.max_rows, N), float("nan"))
+    starts, want = seg.seg_starts.cpu().tolist(), torch.zeros(3, N, dtype=torch.float64)
+    for e, c in enumerate(counts):
+        rows = torch.randint(-8, 9, (c, N), generator=g).float()  # sums below 2 ** 15: exact in 32 bits
+        d_y[starts[e] : starts[e] + c], want[e] = rows, rows.double().sum(0)
+    on_gpu, cs = d_y.to(dtype).to(device), seg.c_struct()
+    d_bias = torch.empty(3, N, dtype=dtype, device=device)
+    _C.check(_C.lib().ck_expert_bias_grad(_C.ptr(on_gpu), N, ctypes.byref(cs), _C.ptr(d_bias), _C.dtype_code(dtype), _C.stream()))
+    assert torch.equal(d_bias.cpu(), want.to(dtype))
