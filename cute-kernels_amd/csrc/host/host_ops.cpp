@@ -35,7 +35,7 @@ using torch::autograd::variable_list;
 #define CK_API(X)                                                                                                       \
   X(ck_last_error_string) X(ck_count_workspace_words) X(ck_count_offsets) X(ck_route_topk_softmax_all)                  \
   X(ck_route_topk_softmax_bwd) X(ck_route_topk_softmax_bwd_exact) X(ck_sort_max_rows) X(ck_sort_workspace_words)        \
-  X(ck_sort_by_expert) X(ck_combine_rows) X(ck_gate_grad_both) X(ck_group_rows_padded) X(ck_swiglu_bwd_grouped)         \
+  X(ck_sort_by_expert) X(ck_combine_rows) X(ck_gate_grad_both) X(ck_group_segment_rows) X(ck_swiglu_bwd_grouped)         \
   X(ck_transpose_batched) X(ck_grouped_gemm_workspace_bytes) X(ck_grouped_gemm_uses_workspace) X(ck_grouped_gemm_ws) X(ck_grouped_gemm_nn_ws)             \
   X(ck_grouped_gemm_f32) X(ck_grouped_gemm_dw_f32) X(ck_grouped_gemm_dw) X(ck_grouped_gemm_dw_rows)                     \
   X(ck_quant_rows_e4m3) X(ck_quant_grouped_rows_e4m3) X(ck_grouped_gemm_fp8) X(ck_swiglu_fwd) X(ck_swiglu_bwd) X(ck_gelu_tanh_bwd) X(ck_rmsnorm_route) X(ck_router_rows) \
@@ -458,10 +458,9 @@ std::pair<Tensor, Tensor> group_rows(const Tensor& src, const Tensor& coeff, int
   if (want_grouped) grouped = new_empty({seg.max_rows, H}, src);
   if (want_transposed) grouped_t = new_empty({H, seg.max_rows}, src);
   const Launch l(src);
-  check(api.ck_group_rows_padded(ptr(src), ptr(coeff), (int32_t)fan_out, (int32_t)H, (const int32_t*)ptr(rows.defined() ? rows : seg.row_slot),
-                                 (const int32_t*)ptr(seg.seg_starts), (const uint32_t*)ptr(seg.counts),
-                                 (const int32_t*)ptr(seg.tile_expert), (int32_t)seg.align, seg.max_rows, ptr(grouped), ptr(grouped_t),
-                                 seg.max_rows, dtype_code(src), l.stream));
+  const ck_segments cs = seg.c(rows);
+  check(api.ck_group_segment_rows(ptr(src), ptr(coeff), (int32_t)fan_out, (int32_t)H, &cs, ptr(grouped), ptr(grouped_t), seg.max_rows,
+                                  dtype_code(src), l.stream));
   return {grouped, grouped_t};
 }
 

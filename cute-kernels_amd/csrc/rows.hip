@@ -252,6 +252,11 @@ __global__ __launch_bounds__(kBlock) void group_rows_stream_kernel(
 // division deep. Bound by the rows written and the source read k times past the L2s (bare copies: 5.9 TB/s, bare stores 6.3).
 // 65,536 rows of 2,048 bf16 values out of 8,192 (268 + 302 MB with the pad rows) 97 -> 78 us, 32,768 of 4,096 out of 16,384 99 -> 81,
 // 6,000 f16 rows of 1,536 11.2 -> 8.4.
+// Where nearly all rows are padding, and wide, there is little to ask and the kernel above writes faster: of 512 rows over 64 experts
+// (16,896 padded) 8,192 / 14,336 bf16 values 50 / 79 against 55 / 96 us here, 14,336 of fp32 149 against 203, 4,096 bf16 values the
+// same. With a third of the rows to copy the waves win at any width (64 / 113 against 79 / 138, 227 against 257). So rows of more than
+// 512 pieces are left to it where not a quarter of them stands for something. (Behind 0.5 GB of other traffic, as in a training step;
+// in a loop that repeats one copy the waves lose 2 to 15 % from 512 pieces on.)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void group_rows_wave_kernel(
     const T* __restrict__ src, const T* __restrict__ coeff, int fan_out, const int32_t* __restrict__ row_slot,
@@ -570,34 +575,35 @@ extern "C" int ck_gate_grad_both(const void* expanded, const void* grad_out, int
   return gate_grad_impl(name, expanded, grad_out, T, k, H, d_gates, d_gates_rounded, dtype, stream);
 }
 
-extern "C" int ck_group_rows_padded(const void* src, const void* coeff, int32_t fan_out, int32_t H,
-                                    const int32_t* row_slot, const int32_t* seg_starts, const uint32_t* counts,
-                                    const int32_t* tile_expert, int32_t align, int64_t max_rows, void* grouped,
-                                    void* grouped_t, int64_t ld_t, int32_t dtype, void* stream) {
-  CK_REQUIRE(H >= 8 && H % 8 == 0, "ck_group_rows_padded: H=%d must be a positive multiple of 8", H);
-  CK_REQUIRE(fan_out >= 0 && (fan_out > 0 || coeff == nullptr), "ck_group_rows_padded: fan_out=%d (0 takes no coeff)", fan_out);
-  CK_REQUIRE(align >= kTile && align % kTile == 0, "ck_group_rows_padded: align=%d must be a multiple of %d", align, kTile);
-  CK_REQUIRE(max_rows >= 0 && max_rows % align == 0, "ck_group_rows_padded: max_rows=%lld is not a multiple of align",
+// rows: how many of max_rows stand for something (an estimate chooses as well)
+static int group_rows_impl(const char* name, const void* src, const void* coeff, int32_t fan_out, int32_t H, const int32_t* row_slot,
+                           const int32_t* seg_starts, const uint32_t* counts, const int32_t* tile_expert, int32_t align, int64_t max_rows,
+                           int64_t rows, void* grouped, void* grouped_t, int64_t ld_t, int32_t dtype, void* stream) {
+  CK_REQUIRE(H >= 8 && H % 8 == 0, "%s: H=%d must be a positive multiple of 8", name, H);
+  CK_REQUIRE(fan_out >= 0 && (fan_out > 0 || coeff == nullptr), "%s: fan_out=%d (0 takes no coeff)", name, fan_out);
+  CK_REQUIRE(align >= kTile && align % kTile == 0, "%s: align=%d must be a multiple of %d", name, align, kTile);
+  CK_REQUIRE(max_rows >= 0 && max_rows % align == 0, "%s: max_rows=%lld is not a multiple of align", name,
              (long long)max_rows);
   if (max_rows == 0) return CK_OK;
-  CK_REQUIRE(src && row_slot && seg_starts && counts && tile_expert, "ck_group_rows_padded: NULL argument");
-  CK_REQUIRE(grouped || grouped_t, "ck_group_rows_padded: nothing to write");
+  CK_REQUIRE(src && row_slot && seg_starts && counts && tile_expert, "%s: NULL argument", name);
+  CK_REQUIRE(grouped || grouped_t, "%s: nothing to write", name);
   CK_REQUIRE(grouped_t == nullptr || (ld_t >= max_rows && ld_t % 8 == 0),
-             "ck_group_rows_padded: ld_t=%lld must be >= max_rows and a multiple of 8", (long long)ld_t);
+             "%s: ld_t=%lld must be >= max_rows and a multiple of 8", name, (long long)ld_t);
   CK_REQUIRE(aligned16(src) && (!grouped || aligned16(grouped)) && (!grouped_t || aligned16(grouped_t)),
-             "ck_group_rows_padded: pointers must be 16-byte aligned");
-  CK_REQUIRE(max_rows / kTile <= 65535, "ck_group_rows_padded: too many rows for one launch");
+             "%s: pointers must be 16-byte aligned", name);
+  CK_REQUIRE(max_rows / kTile <= 65535, "%s: too many rows for one launch", name);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)ceil_div(H, kTile), (unsigned)(max_rows / kTile));
   if (grouped_t == nullptr) {  // the row-major copy alone: also for fp32 rows
-    CK_DISPATCH_FLOAT(dtype, "ck_group_rows_padded", {
+    CK_DISPATCH_FLOAT(dtype, name, {
       constexpr int P = Elem<scalar_t>::per16;
-      CK_REQUIRE(H % P == 0, "ck_group_rows_padded: H=%d must be a multiple of %d", H, P);
-      if (H / P >= kWave) {  // a piece for every lane
+      CK_REQUIRE(H % P == 0, "%s: H=%d must be a multiple of %d", name, H, P);
+      // a piece for every lane; wide rows not where nearly all are padding
+      if (H / P >= kWave && (H / P <= 512 || 4 * rows >= max_rows)) {
         hipLaunchKernelGGL((group_rows_wave_kernel<scalar_t>), dim3((unsigned)ceil_div(max_rows, (int64_t)(kBlock / kWave))), dim3(kBlock), 0,
                            s, static_cast<const scalar_t*>(src), static_cast<const scalar_t*>(coeff), (int)fan_out, row_slot,
                            seg_starts, counts, tile_expert, (int)align, (int)max_rows, (int)(H / P), static_cast<scalar_t*>(grouped));
-        CK_CHECK_LAUNCH("ck_group_rows_padded");
+        CK_CHECK_LAUNCH(name);
         return CK_OK;
       }
       hipLaunchKernelGGL((group_rows_stream_kernel<scalar_t>), dim3(grid_for(max_rows * (H / P), 2)), dim3(kBlock), 0, s,
@@ -605,17 +611,34 @@ extern "C" int ck_group_rows_padded(const void* src, const void* coeff, int32_t 
                          seg_starts, counts, tile_expert, (int)align, max_rows, (int)(H / P),
                          static_cast<scalar_t*>(grouped));
     });
-    CK_CHECK_LAUNCH("ck_group_rows_padded");
+    CK_CHECK_LAUNCH(name);
     return CK_OK;
   }
-  CK_DISPATCH_HALF(dtype, "ck_group_rows_padded", {
+  CK_DISPATCH_HALF(dtype, name, {
     hipLaunchKernelGGL((group_rows_padded_kernel<scalar_t>), grid, dim3(kBlock), 0, s,
                        static_cast<const scalar_t*>(src), static_cast<const scalar_t*>(coeff), (int)fan_out, (int)H,
                        row_slot, seg_starts, counts, tile_expert, (int)align, static_cast<scalar_t*>(grouped),
                        static_cast<scalar_t*>(grouped_t), ld_t);
   });
-  CK_CHECK_LAUNCH("ck_group_rows_padded");
+  CK_CHECK_LAUNCH(name);
   return CK_OK;
+}
+
+extern "C" int ck_group_rows_padded(const void* src, const void* coeff, int32_t fan_out, int32_t H,
+                                    const int32_t* row_slot, const int32_t* seg_starts, const uint32_t* counts,
+                                    const int32_t* tile_expert, int32_t align, int64_t max_rows, void* grouped,
+                                    void* grouped_t, int64_t ld_t, int32_t dtype, void* stream) {
+  return group_rows_impl("ck_group_rows_padded", src, coeff, fan_out, H, row_slot, seg_starts, counts, tile_expert, align, max_rows,
+                         max_rows, grouped, grouped_t, ld_t, dtype, stream);
+}
+extern "C" int ck_group_segment_rows(const void* src, const void* coeff, int32_t fan_out, int32_t H, const ck_segments* seg,
+                                     void* grouped, void* grouped_t, int64_t ld_t, int32_t dtype, void* stream) {
+  const char* name = "ck_group_segment_rows";
+  CK_REQUIRE(seg != nullptr && seg->num_experts >= 0 && seg->align >= 1, "%s: incomplete segment tables", name);
+  // at most so many rows lie in the padded layout (ck_sort_max_rows)
+  const int64_t rows = seg->max_rows - (int64_t)seg->num_experts * (seg->align - 1);
+  return group_rows_impl(name, src, coeff, fan_out, H, seg->row_slot, seg->seg_starts, seg->counts, seg->tile_expert, seg->align,
+                         seg->max_rows, rows, grouped, grouped_t, ld_t, dtype, stream);
 }
 
 extern "C" int ck_gelu_tanh_bwd_grouped(const void* pre, const void* d_act, int32_t N, const ck_segments* seg, void* d_pre,

@@ -65,6 +65,10 @@ _SIGNATURES = {
         c_int32,
         [c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_int64, c_int32, c_void_p],
     ),
+    "ck_group_segment_rows": (
+        c_int32,
+        [c_void_p, c_void_p, c_int32, c_int32, POINTER(ck_segments), c_void_p, c_void_p, c_int64, c_int32, c_void_p],
+    ),
     "ck_swiglu_bwd_grouped": (
         c_int32,
         [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p],

@@ -206,6 +206,9 @@ typedef struct ck_segments {
                                   epilogues. Differs from row_slot when input and output are indexed differently, e.g. token
                                   rows in, unpadded grouped rows out (row_pos of ck_segments_from_sorted). */
 } ck_segments;
+/* ck_group_rows_padded for a caller with these tables: knows how much of the layout is padding, and chooses by it. */
+int ck_group_segment_rows(const void* src, const void* coeff, int32_t fan_out, int32_t H, const ck_segments* seg, void* grouped,
+                          void* grouped_t, int64_t ld_t, int32_t dtype, void* stream);
 
 /* Y = A_e * W[e]^T for every expert segment e. W [E, N, K].
  * A rows: a_gather_div > 0 : row p reads a[row_slot[p] / a_gather_div, :]   (a is [*, K], token order)

@@ -327,3 +327,24 @@ def test_group_rows_by_waves(device, dtype, pieces, align):
         assert torch.equal(got.cpu()[: starts[-1]], want)
     same, _ = scattermoe._group_rows(got, None, 0, seg, True, False)
     assert torch.equal(same.cpu()[: starts[-1]], want)
+
+
+# wide rows go by pieces where nearly all of them are padding, and by waves where not; up to 512 pieces by waves either way
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("pieces", [512, 514, 1090])
+@pytest.mark.parametrize("counts", [[1, 0, 3, 1, 0, 2], [128, 0, 100, 129, 0, 200]])
+def test_wide_rows_mostly_padding_and_not(device, dtype, pieces, counts):
+    g = torch.Generator().manual_seed(pieces)
+    H, k, R = pieces * 16 // dtype.itemsize, 2, sum(counts)
+    ids = torch.arange(len(counts), dtype=torch.int32).repeat_interleave(torch.tensor(counts))[torch.randperm(R, generator=g)]
+    seg = cute_kernels.sort_by_expert(ids.to(device), len(counts), 128)
+    src, coeff = torch.randn(-(-R // k), H, generator=g).to(dtype), torch.rand(R, generator=g).to(dtype)
+    slots, starts = seg.row_slot.cpu(), seg.seg_starts.cpu().tolist()
+    want = torch.zeros(starts[-1], H, dtype=dtype)
+    for e, n in enumerate(counts):
+        s = slots[starts[e] : starts[e] + n].long()
+        want[starts[e] : starts[e] + n] = (src[s // k].float() * coeff[s, None].float()).to(dtype)
+    got, _ = scattermoe._group_rows(src.to(device), coeff.to(device), k, seg, True, False)
+    assert torch.equal(got.cpu()[: starts[-1]], want)
+    same, _ = scattermoe._group_rows(got, None, 0, seg, True, False)
+    assert torch.equal(same.cpu()[: starts[-1]], want)
