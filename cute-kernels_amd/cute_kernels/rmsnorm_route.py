@@ -77,11 +77,14 @@ def rmsnorm_route_fused(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
 def rmsnorm_route_pays(x: torch.Tensor, gate_weight: torch.Tensor) -> bool:
     """Where the one-pass kernel is the faster route. It re-reads the gate weight from L2 for every 16 rows, so its time
     grows with E * H: 28 us against 40 us for the separate kernels at 8,192 x 2,048 with 64 experts (30 against 53 with the
-    e4m3 rows), 62 against 89 at 16,384 x 4,096 with 8. Beyond 64 x 4,096 it pays up to 16,384 rows: 128 experts and rows of 4,096, 513 /
-    4,096 / 16,384 / 65,536 of them, one pass and separate, 35 / 38 / 89 / 325 and 36 / 49 / 94 / 321 us, with the e4m3 rows 40 / 42 /
-    117 / 436 and 45 / 58 / 124 / 442 (a layer of 65,536 rows 1 % slower all the same); rows of 2,560 24 / 28 / 66 / 242 and 34 / 39 / 75 /
-    222, with the e4m3 rows 30 / 34 / 80 / 310 and 41 / 50 / 94 / 309."""
-    return gate_weight.size(0) * x.size(-1) <= 64 * 4096 or x.numel() <= 16384 * x.size(-1)
+    e4m3 rows), 62 against 89 at 16,384 x 4,096 with 8. Beyond 64 x 4,096 it pays from
+    2,048 rows, where its workgroups begin to fill the chip, up to 16,384. GPU time of 128 experts and rows of 4,096, 513 / 1,024 /
+    2,048 / 2,560 / 4,096 / 16,384 of them, one pass 36 / 35 / 36 / 36 / 38 / 90 us, separate 19 / 21 / 28 / 44 / 51 / 113, with the e4m3
+    rows 39 / 39 / 40 / 40 / 42 / 122 and 23 / 25 / 33 / 49 / 59 / 139 (65,536 rows: 325 and 321, 436 and 442, a layer 1 % slower); of 96
+    experts 1,024 / 2,560 / 4,096 rows 32 / 32 / 34 and 21 / 30 / 49."""
+    if gate_weight.size(0) * x.size(-1) <= 64 * 4096:
+        return True
+    return 2048 * x.size(-1) < x.numel() <= 16384 * x.size(-1)
 
 
 def rmsnorm_route_cute(

@@ -133,7 +133,8 @@ def test_launch_timer_may_be_taken_off_while_another_thread_launches():
     assert len(launched) == 2002
 
 
-@pytest.mark.parametrize("rows,hidden,experts,pays", [(100_000, 4096, 64, True), (16384, 4096, 128, True), (16385, 4096, 128, False), (65536, 2560, 128, False)])
+@pytest.mark.parametrize("rows,hidden,experts,pays", [(100_000, 4096, 64, True), (16384, 4096, 128, True), (16385, 4096, 128, False), (65536, 2560, 128, False),
+                                                       (1, 4096, 64, True), (513, 4096, 128, False), (2048, 4096, 96, False), (2049, 2560, 128, True)])
 def test_where_the_one_pass_norm_and_router_pays(rows, hidden, experts, pays):
     from cute_kernels.rmsnorm_route import rmsnorm_route_pays
 
