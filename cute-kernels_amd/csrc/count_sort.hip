@@ -463,6 +463,7 @@ __device__ inline void bins_exclusive_scan(const uint32_t (&v)[NB], uint32_t (&b
 // two launches 8,192 over 64 9.3 -> 7.05, 32,768 over 64 9.9 -> 7.6, over 128 10.9 -> 9.15, 65,536 over 64 10.6 -> 7.7, 524,288 over
 // 128 18.3 -> 16.9, 2,000,003 over 60 34.5 -> 30.4.
 constexpr int kLaneWaves = 16, kLaneBins = 2 * kWave;
+constexpr int kLaneIds = kLaneWaves * kWave * kSortPer;  // R up to which one block sorts
 template <typename id_t, int NB, bool SMALL>
 __global__ __launch_bounds__(kLaneWaves * kWave) void sort_lanes_kernel(
     const id_t* __restrict__ ids, int64_t R, int E, int64_t seg_len, int id_bits, int align, int64_t max_tiles,
@@ -577,12 +578,14 @@ __global__ __launch_bounds__(kLaneWaves * kWave) void sort_lanes_kernel(
 
 // The whole sort in one block and one launch, for few ids over more than kLaneBins experts. What bounds it: latency.
 // An id is read once and stays in registers, and the table in LDS; the second launch and the way of the table through memory
-// go. Measured, 50 sorts in a replayed graph, one launch against two: 16 / 512 / 4,096 ids over 64 experts 4.5 / 4.7 / 8.9
-// against 7.6 / 7.7 / 9.0 us, over 512 experts 7.6 / 8.0 / 13.0 against 9.5 / 9.9 / 11.3. The line lies where the two meet for
-// few experts; past it one block's rounds of 64 take longer than launches that spread them over the chip.
+// go. Measured, 40 sorts in a replayed graph, one launch against two: 8 / 512 / 2,048 / 3,500 / 4,096 ids over 129 experts 4.9 / 5.1
+// / 6.9 / 9.0 / 9.9 against 8.2 / 8.5 / 9.2 / 9.6 / 9.6 us, over 384 5.7 / 6.1 / 7.8 / 10.5 / 11.1 against 9.0 / 9.7 / 10.5 / 11.0 / 10.8;
+// over 512 3,000 / 3,500 / 4,096 ids 11.2 / 12.2 / 13.2 against 11.1 / 11.3 / 11.4. The line lies where the two meet: past it one
+// block's rounds of 64, and its scan of a word per expert and wave, take longer than launches that spread them over the chip.
 constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
 constexpr int kSmallPer = 4;                                  // ids per lane
 constexpr int kSmallIds = kSmallBlock * kSmallPer;            // R up to which the one-block sort runs, up to kSmallBins bins
+constexpr int small_ids(int E) { return E <= 384 ? kSmallIds : kSmallIds * 3 / 4; }
 
 template <typename id_t>
 __global__ __launch_bounds__(kSmallBlock) void sort_small_kernel(const id_t* __restrict__ ids, int R, int E, int align, int64_t max_tiles,
@@ -919,7 +922,7 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
     if (E <= kWave) CK_LAUNCH_LANES(ID_T, 1, SMALL, BLOCKS, SEG_LEN, TABLE);           \
     else CK_LAUNCH_LANES(ID_T, 2, SMALL, BLOCKS, SEG_LEN, TABLE);                      \
   } while (0)
-  if (R <= kSmallIds && E <= kLaneBins) {
+  if (R <= kLaneIds && E <= kLaneBins) {
     const int64_t seg_len = round_up(R > 0 ? R : 1, (int64_t)kLaneWaves * kWave);
     const uint32_t* none = nullptr;
     if (ids_are_i64) CK_LAUNCH_LANES_OF(int64_t, true, 1, seg_len, none);
@@ -927,7 +930,7 @@ extern "C" int ck_sort_by_expert(const void* expert_ids, int32_t ids_are_i64, in
     CK_CHECK_LAUNCH("ck_sort_by_expert");
     return CK_OK;
   }
-  if (R <= kSmallIds && E <= kSmallBins) {
+  if (E <= kSmallBins && R <= small_ids(E)) {
     const size_t lds = ((size_t)E * (kSmallWaves + 2) + 1 + kSmallWaves) * sizeof(uint32_t);
 #define CK_LAUNCH_SMALL(ID_T)                                                                                                \
   hipLaunchKernelGGL((sort_small_kernel<ID_T>), dim3(1), dim3(kSmallBlock), lds, static_cast<hipStream_t>(stream),           \

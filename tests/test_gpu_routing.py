@@ -326,6 +326,13 @@ def test_sort_of_few_ids_in_one_block(device, R, E, align, dtype):
     assert torch.equal(seg.counts.cpu().long(), torch.bincount(ids[kept].long(), minlength=E))
 
 
+# where one block hands over to two launches: 3,072 ids over more than 384 experts, 4,096 over fewer
+@pytest.mark.parametrize("R,E", [(4096, 129), (4097, 129), (4096, 384), (4097, 384), (3072, 385), (3073, 385), (3072, 512), (3073, 512), (4096, 128)])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.long])
+def test_sort_on_both_sides_of_one_block(device, R, E, dtype):
+    test_sort_of_few_ids_in_one_block(device, R, E, 64, dtype)
+
+
 @pytest.mark.parametrize("R,E", [(5121, 60), (4099, 512), (4099, 513), (66000, 1), (262145, 512), (131073, 384), (20001, 4096), (300001, 128)])
 @pytest.mark.parametrize("dtype", [torch.int32, torch.long])
 def test_sort_over_many_blocks(device, R, E, dtype):
