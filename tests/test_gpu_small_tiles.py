@@ -117,10 +117,11 @@ def test_inference_on_128_row_tiles_matches_a_forward_on_256(device, monkeypatch
 
 
 # weights on 128-byte boundaries throughout, with another row pitch, and with another first row; one line a row, several, and a part of
-# one. Column tiles of 64 (32 outputs with a gate) and a rest; enough tiles for whole rounds of chunks over the XCDs and a rest
+# one. Column tiles of 64 (32 outputs with a gate) and a rest; with 4,104 columns, 520 to 715 tiles: whole rounds of chunks over the
+# XCDs and a rest, at every height, with experts of several row tiles
 @pytest.mark.parametrize("align", [16, 32, 64])
 @pytest.mark.parametrize("K,offset", [(64, 0), (320, 0), (328, 0), (320, 8), (32, 0)])
-@pytest.mark.parametrize("columns", [8, 200, 1032])
+@pytest.mark.parametrize("columns", [8, 200, 1032, 4104])
 def test_weight_lines(device, align, K, offset, columns):
     g = torch.Generator().manual_seed(K + columns)
     counts = [0, 2 * align + 3, 1, 0, align, 5, 70, 0]
