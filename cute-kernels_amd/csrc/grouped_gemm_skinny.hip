@@ -26,10 +26,10 @@
 // Measured (kernel trace, all experts with as many rows; the rate is the weights' bytes by the time; before: plain loads of half lines,
 // column tile by column tile): 8 experts of 28,672 x 4,096 with 2 rows each 308 -> 271 us = 6.9 TB/s, 4,096 x 14,336 163 -> 152 = 6.2,
 // 64 of 2,816 x 2,048 with 8 rows 130 -> 116 = 6.4, 2,048 x 1,408 69 -> 58.5 = 6.3, e4m3, 128 of 3,072 x 4,096 with 8 rows 281 -> 237 =
-// 6.8, 4,096 x 1,536 157 -> 141 = 5.7 with two workgroups per CU (three now, see there; three steps a wave: start and reduction weigh
-// most; several column tiles a workgroup, the next one's first loads ahead of the reduction, take registers that a third workgroup
-// has now: 2 % faster there with two, slower
-// with more and elsewhere). The memory reads 1.000 to 1.007 times the weights' bytes (1.01 to 1.13 before). 224 launches of 4 to 128
+// 6.8, 4,096 x 1,536 157 -> 141 = 5.7 with two workgroups per CU, three now (see the kernel). That launch's waves have three steps each, so
+// start and reduction weigh most; several column tiles a workgroup, the next one's first loads ahead of the reduction, made it 2 % faster
+// with two workgroups, but take the registers that a third one has now, and were slower with more tiles and in other launches.
+// The memory reads 1.000 to 1.007 times the weights' bytes (1.01 to 1.13 before). 224 launches of 4 to 128
 // experts, 4 MB to 2.1 GB of weights, 0.3 to 60 rows each, even and uneven loads: 26 % less time on average, none slower than by the
 // spread of a 10 us launch; 181 with odd row pitches 17 % less.
 #include "gemm_common.h"

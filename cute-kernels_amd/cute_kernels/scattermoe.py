@@ -273,13 +273,15 @@ def choose_align(
     expert its GEMMs decide, those of a training step or of the forward alone (_height_of_large_tiles).
     inference (no gradient is asked for): tiles of 16, 32 or 64 rows while the experts average few rows and the load is the
     stream of their weights (grouped_gemm_skinny.hip stages no weights in LDS). An expert of several tiles has its weights
-    fetched once per tile, from L2 at best, so the height follows the load. 160 bf16 layers of 8 to 128 experts at 3 to 80 rows
-    each and Zipf(0), (0.8), (1.0) loads: the height chosen is 1.6 % slower than the best of 16, 32, 64, 128 and 256 rows on
-    average (14 rows as the end of 32-row tiles: 2.2); at 14 to 20 rows tiles of 16 / 32 / 64 are 20 / 1 / 5 % off it on
-    average, at 20 to 30 44 / 6 / 1, at 30 to 40 59 / 20 / 5 (128: 9, 256: 8). The quantised-expert layer's next height is
-    256: 128 experts of 4,096 x 1,536 at 8 / 18 / 22 / 30 / 40 / 60 rows, even load, tiles of 32 398 / 444 / 470 / 610 / 873 /
-    1,008 us, of 64 438 / 486 / 502 / 543 / 588 / 787, of 256 584 / 584 / 590 / 592 / 603 / 622; with Zipf(0.8) loads at 22 / 30 / 40 rows
-    555 / 633 / 760, 540 / 608 / 670 and 588 / 653 / 675."""
+    fetched once per tile, from L2 at best, so the height follows the load. Six gated shapes of 8 to 128 experts, 1,024 to 4,096 wide, at
+    3 to 50 rows each and Zipf(0) and (0.8) loads, 156 calls of either layer: the height chosen is 1.1 % (16 bits) and 1.3 % (e4m3) slower
+    than the best of 16, 32, 64 and the next one on average (with 14 rows as the end of 32-row tiles and 30 of e4m3's 64-row ones 1.7
+    and 3.9). On average over the shapes tiles of 16 / 32 / 64 / 128 rows are at 8 rows 4 / 1 / 11 / 33 % off the best, at 14 16 / 0 / 7 /
+    27, at 22 45 / 1 / 4 / 19, at 30 58 / 14 / 1 / 7, at 40 80 / 37 / 3 / 2; the quantised-expert layer's, whose next height is 256, at 8
+    rows 4 / 2 / 13 / 53, at 14 15 / 0 / 11 / 44, at 22 39 / 0 / 7 / 29, at 30 44 / 6 / 1 / 16, at 40 58 / 24 / 1 / 7, at 50 76 / 29 / 3 / 3.
+    In e4m3, even load, 128 experts of 4,096 x 1,536 at 5 / 8 / 22 / 30 / 40 / 50 rows: tiles of 16 390 / 401 / 774 / 926 / 1,093 / 1,337 us,
+    of 32 379 / 394 / 466 / 627 / 891 / 952, of 64 422 / 436 / 515 / 553 / 596 / 646, of 256 571 / 573 / 591 / 600 / 605 / 616; 64 of 2,048 x
+    1,408 at 8 / 22 rows: of 16 115 / 197, of 32 111 / 135, of 64 135 / 146."""
     return _height(_layer_tiles, _layer_tiles_kept, num_rows, num_experts, dtype, inference, widths)
 
 
