@@ -157,18 +157,19 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, inference: bool, lau
       * a step of a 128 x 128 tile takes 0.9 alone on a CU, and 1.6 where the first CUs have two to 1.95 where all do (single
         launches with 256, 272 and 512 tiles: 4,096 deep 70, 117 and 138, 2,048 deep 39, 62 and 77);
       * no launch is shorter than its weights' stream, 6.7 TB/s through 256-row tiles, 4.2 through the general kernel's and 3.8 through
-        128-row ones; the input gradient of 128-row tiles, or of the general kernel, transposes the weights first, at 4.2.
-    Over 370 inference layers (8 to 128 experts, 768 to 4,096 wide, 512 to 8,900 inside in steps of 32, gated and not, 31 to 500 rows
-    per expert, Zipf(0), (0.8) and (1.0) loads) the chosen height is 0.5 % slower than the better one on average, 256 rows throughout
-    6.2 %. (With the general kernel's step as the other's, and 1.75 for a CU with two tiles, 0.8 %, and layers of 8 experts at 170 to
-    390 rows up to 36 %.) Both sides at Zipf(0.8), 128 against 256 rows: 32 experts of 3,456 x 896 at 94 rows 211 against 161 us, 8 of
+        128-row ones; the input gradient of 128-row tiles, or of the general kernel, transposes the weights first, at 4.2 and in 5 more.
+    Over 520 inference layers (8 to 128 experts, 256 to 4,096 wide, 256 to 8,900 inside in steps of 32, gated and not, 31 to 500 rows
+    per expert, Zipf(0), (0.8) and (1.0) loads) the chosen height is 0.6 % slower than the better one on average, 256 rows throughout
+    15 %. (With the general kernel's step as the other's, and 1.75 for a CU with two tiles, layers of 8 experts at 170 to 390 rows were
+    up to 36 % slower.) Both sides at Zipf(0.8), 128 against 256 rows: 32 experts of 3,456 x 896 at 94 rows 211 against 161 us, 8 of
     1,152 x 8,896 at 136 rows 234 against 185, 128 of 2,048 x 1,408 at 60 rows 623 against 556; 8 of 3,584 x 832 at 81 rows 60 against
     83, 8 of 1,408 x 3,552 at 168 rows 106 against 123, 8 of 1,664 x 1,088 without a gate at 392 rows 69 against 83.
-    Over 350 training steps of such layers from 12 rows on it is 0.03 % slower on average and 4.5 % at most, 256 rows throughout 1.0
-    and 47 %. (By the kernels whose parts met through device-wide fences, 75 us, and with a gated epilogue that did not split: 1.5 and
-    51 %.) Both sides: 8 of 2,048 x 4,096 without a gate at 160 / 192 / 230 rows 498 / 510 / 617 against 401 / 412 / 461, 16 of 1,024 x
-    2,016 at 16 / 64 rows 307 / 359 against 276 / 312, 8 of 1,024 x 3,840 at 40 rows 363 against 275, 8 of 3,200 x 1,120 at 400 rows 543
-    against 419; at 32 rows 299 against 306, 8 of 1,024 x 1,024 at 96 / 300 rows 162 / 186 against 180 / 200."""
+    Over 500 training steps of such layers from 12 rows on it is 0.1 % slower on average and 7 % at most, 256 rows throughout 3.5 and
+    47 %, over 440 single linears 0.5 % forward and 0.1 % with the backward (always 128: 6 and 10 %). (By the kernels whose parts met
+    through device-wide fences, 75 us, and with a gated epilogue that did not split, training steps up to 51 % slower.) Both sides: 8
+    of 2,048 x 4,096 without a gate at 160 / 192 / 230 rows 498 / 510 / 617 against 401 / 412 / 461, 16 of 1,024 x 2,016 at 16 / 64 rows
+    307 / 359 against 276 / 312, 8 of 1,024 x 3,840 at 40 rows 363 against 275, 8 of 3,200 x 1,120 at 400 rows 543 against 419; at 32
+    rows 299 against 306, 8 of 1,024 x 1,024 at 96 / 300 rows 162 / 186 against 180 / 200."""
     even_rows, zipf_rows = num_rows / num_experts + 24, num_rows / _zipf_sum(num_experts)
     cost = {}
     for height in (128, 256):
@@ -180,7 +181,7 @@ def _height_of_large_tiles(num_rows: int, num_experts: int, inference: bool, lau
             column_tiles, steps, general = -(-columns // height), -(-contraction // 64), contraction % 64 != 0
             megabytes = num_experts * columns * contraction * 2e-6
             if input_gradient and (height == 128 or general):
-                total += 2 * megabytes / 4.2
+                total += 2 * megabytes / 4.2 + 5.0
             if height == 128:
                 stream = megabytes / 3.8
                 for rows in loads:
